@@ -1144,7 +1144,8 @@ hipError_t dispatch(const IgemmParams& p, int epi_vec, hipStream_t s) {
 }  // namespace
 
 bool igemm_wants_wfrag(const IgemmParams& p) {
-  return wreg_shape(p) || lean_steps(p) > 0 || taps_shape(p).nkk > 0 || igemm_stream_q8_geometry(p) || igemm_c3_geometry(p);
+  return wreg_shape(p) || lean_steps(p) > 0 || taps_shape(p).nkk > 0 || igemm_stream_q8_geometry(p) || igemm_c3_geometry(p) ||
+         igemm_slim_variant(p, true) > 0;
 }
 
 hipError_t launch_wfrag_pack(const WfragPackParams& p, hipStream_t stream) {
@@ -1157,7 +1158,7 @@ hipError_t launch_wfrag_pack(const WfragPackParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
-const char* igemm_variant_name(const IgemmParams& p) {
+const char* igemm_variant_name(const IgemmParams& p, const bool small_tiles) {
   switch (igemm_big_variant(p)) {
     case 1: return "256x256";
     case 2: return "256x128";
@@ -1165,6 +1166,14 @@ const char* igemm_variant_name(const IgemmParams& p) {
     default: break;
   }
   if (gemm_rowdot_shape(p)) return "rowdot";
+  if (small_tiles) {
+    switch (igemm_slim_variant(p, p.w_frag != nullptr)) {
+      case 1: return "16x16k16";
+      case 2: return "32x32k8";
+      case 3: return "64x64";
+      default: break;
+    }
+  }
   if (p.w_frag != nullptr && igemm_c3_geometry(p)) return "patch3x3";
   if (p.w_frag != nullptr && igemm_stream_q8_geometry(p)) return "stream";
   if (p.w_frag != nullptr && lean_steps(p) > 0) return "128x128s";
@@ -1257,6 +1266,7 @@ hipError_t launch_igemm(const IgemmParams& p_in, hipStream_t stream) {
   if (gemm_rowdot_shape(p)) return launch_gemm_rowdot(p, stream);
   if (p.row_softmax != 0) return hipErrorInvalidValue;   // (no other kernel finishes with a Softmax)
   if (const int big = igemm_big_variant(p)) return launch_igemm_big(p, epi_vec, big, stream);
+  if (const int slim = igemm_slim_variant(p, p.w_frag != nullptr)) return launch_igemm_slim(p, epi_vec, slim, stream);
   if (p.w_frag != nullptr && igemm_c3_geometry(p)) return launch_igemm_c3(p, epi_vec, stream);
 
   switch (p.in_dt) {

@@ -81,33 +81,33 @@ __device__ __forceinline__ float epi_act(float v, ActKind act, float a, float b)
     default: return v;
   }
 }
-// Eight values at once: the (wavefront-uniform) switch is taken once, not per
+// Several values at once: the (wavefront-uniform) switch is taken once, not per
 // element - per element it compiles to a tree of scalar branches that costs
 // more than the arithmetic of the whole epilogue.
-template <bool kRich = false>
-__device__ __forceinline__ void epi_act8(float (&v)[8], ActKind act, float a, float b) {
+template <bool kRich = false, int N>
+__device__ __forceinline__ void epi_act_n(float (&v)[N], ActKind act, float a, float b) {
   if constexpr (kRich) {
     // Variant with the transcendental activations (GELU behind a feed-forward
     // GEMM, Sigmoid / Tanh gates): a separate instantiation, so that the common
     // epilogue stays small.
-    // (one element after the other: interleaving eight polynomial evaluations
+    // (one element after the other: interleaving several polynomial evaluations
     // would take the registers the accumulators of the other slices live in)
     switch (act) {
       case ACT_GELU_ERF:
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { v[e] = gelu_erf(v[e]); __builtin_amdgcn_sched_barrier(0); }
+        for (int e = 0; e < N; ++e) { v[e] = gelu_erf(v[e]); __builtin_amdgcn_sched_barrier(0); }
         return;
       case ACT_GELU_TANH:
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { v[e] = gelu_tanh(v[e]); __builtin_amdgcn_sched_barrier(0); }
+        for (int e = 0; e < N; ++e) { v[e] = gelu_tanh(v[e]); __builtin_amdgcn_sched_barrier(0); }
         return;
       case ACT_SIGMOID:
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { v[e] = 1.0f / (1.0f + expf(-v[e])); __builtin_amdgcn_sched_barrier(0); }
+        for (int e = 0; e < N; ++e) { v[e] = 1.0f / (1.0f + expf(-v[e])); __builtin_amdgcn_sched_barrier(0); }
         return;
       case ACT_TANH:
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { v[e] = tanhf(v[e]); __builtin_amdgcn_sched_barrier(0); }
+        for (int e = 0; e < N; ++e) { v[e] = tanhf(v[e]); __builtin_amdgcn_sched_barrier(0); }
         return;
       default: break;
     }
@@ -115,15 +115,15 @@ __device__ __forceinline__ void epi_act8(float (&v)[8], ActKind act, float a, fl
   switch (act) {
     case ACT_RELU:
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = v[e] > 0.f ? v[e] : 0.f;
+      for (int e = 0; e < N; ++e) v[e] = v[e] > 0.f ? v[e] : 0.f;
       break;
     case ACT_LEAKY:
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = v[e] > 0.f ? v[e] : a * v[e];
+      for (int e = 0; e < N; ++e) v[e] = v[e] > 0.f ? v[e] : a * v[e];
       break;
     case ACT_CLAMP:
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = fminf(fmaxf(v[e], a), b);
+      for (int e = 0; e < N; ++e) v[e] = fminf(fmaxf(v[e], a), b);
       break;
     default: break;
   }
@@ -144,7 +144,7 @@ struct EpiFloat {
     for (int e = 0; e < 8; ++e) v[e] = __builtin_fmaf(acc[e], p.alpha, b8[e]);
     // the activation comes before the residual in networks whose shortcut joins
     // an already activated branch, behind it in the ResNet order
-    if (p.res_after_act) epi_act8<kRich>(v, p.act, p.act_a, p.act_b);
+    if (p.res_after_act) epi_act_n<kRich>(v, p.act, p.act_a, p.act_b);
     if (vec) {
       if (r != nullptr) {
         if constexpr (sizeof(TOut) == 4) {
@@ -163,7 +163,7 @@ struct EpiFloat {
           for (int e = 0; e < 8; ++e) v[e] += rv.get(e);
         }
       }
-      if (!p.res_after_act) epi_act8<kRich>(v, p.act, p.act_a, p.act_b);
+      if (!p.res_after_act) epi_act_n<kRich>(v, p.act, p.act_a, p.act_b);
       if constexpr (sizeof(TOut) == 4) {
         *reinterpret_cast<floatx4*>(y) = (floatx4){v[0], v[1], v[2], v[3]};
         *reinterpret_cast<floatx4*>(y + 4) = (floatx4){v[4], v[5], v[6], v[7]};
@@ -185,7 +185,7 @@ struct EpiFloat {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         if (e < nvalid && r != nullptr) v[e] += Store<TOut>::ld(r + e);
-      if (!p.res_after_act) epi_act8<kRich>(v, p.act, p.act_a, p.act_b);
+      if (!p.res_after_act) epi_act_n<kRich>(v, p.act, p.act_a, p.act_b);
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         if (e < nvalid) Store<TOut>::st(y + e, v[e]);
@@ -222,7 +222,7 @@ struct EpiQuant {
         f[e] = (float)acc[e] * m8[e];
         if (e < nvalid && r != nullptr) f[e] += r[e];
       }
-      epi_act8(f, p.act, p.act_a, p.act_b);
+      epi_act_n(f, p.act, p.act_a, p.act_b);
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         if (e < nvalid) y[e] = f[e];

@@ -1,0 +1,512 @@
+// Implicit GEMM for launches with few output tiles: batch-1 .. batch-16 images, single
+// sequences, the small feature maps at the end of a network.
+//
+// What bounds such a launch is not bandwidth or the matrix cores but one workgroup's chain of
+// K stages (128-pixel x 128-channel tiles: ResNet-50's last 3x3 layer at one image is four
+// workgroups of 72 stages, 32 us) on a mostly idle chip.  Here
+//   - the output tile is small (16 .. 64 pixels x 16 .. 64 channels, 16x16 MFMA blocks), so that
+//     a layer of 49 pixels x 512 channels is 128 workgroups instead of four;
+//   - the wavefronts of a workgroup (4 .. 16) all own the SAME tile and split K: each walks a
+//     contiguous share of the 64-byte K steps, so the chain is a few steps long and its loads
+//     are all in flight together;
+//   - both operands go straight from global memory into MFMA registers (16 bytes per lane; the
+//     caches serve what workgroups share), no staging, no barrier in the K loop;
+//   - the partial tiles are added through LDS in a fixed order by the threads that then apply
+//     the epilogue to four consecutive channels of one pixel each.
+// Any tap geometry, stride, dilation, padding, grid.z batch and operand type of IgemmParams is
+// served; weights are read from the fragment-ordered copy where one exists, from the packed
+// rows otherwise.
+#include "igemm_common.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+namespace ohip {
+
+// 16x16 blocks: lane l feeds row l % 16 of either operand with the 16 bytes l / 16 of a 64-byte
+// K step, and ends up with four consecutive channels ((l / 16) * 4 ..) of pixel l % 16.
+template <typename T> struct Mma16;
+template <> struct Mma16<float> {
+  using Acc = floatx4;
+  __device__ static __forceinline__ Acc run(uintx4 a, uintx4 b, Acc c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
+    return c;
+  }
+};
+template <> struct Mma16<f16_t> {
+  using Acc = floatx4;
+  __device__ static __forceinline__ Acc run(uintx4 a, uintx4 b, Acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  }
+};
+template <> struct Mma16<bf16_t> {
+  using Acc = floatx4;
+  __device__ static __forceinline__ Acc run(uintx4 a, uintx4 b, Acc c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+};
+template <> struct Mma16<int8_t> {
+  using Acc = intx4;
+  __device__ static __forceinline__ Acc run(uintx4 a, uintx4 b, Acc c) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(intx4, a), __builtin_bit_cast(intx4, b), c, 0, 0, 0);
+  }
+};
+
+// What the launcher works out once per launch.
+struct SlimArgs {
+  int tiles_m = 0, tiles_n = 0;
+  int m_fast = 0;        // neighbouring workgroups share channels (1) or pixels (0)
+  int steps = 0;         // 64-byte K steps, the last one possibly partial
+  int cvec = 1;          // 16-byte vectors per tap
+  unsigned cv_magic = 0, s_magic = 0;
+  int cv_shift = 0, s_shift = 0;
+};
+
+// How K maps to taps: one contiguous run per pixel / a step inside one tap / any.
+enum SlimMode { SLIM_ROW = 0, SLIM_TAP = 1, SLIM_ANY = 2 };
+
+template <typename TIn, typename Epi, int MB, int NB, int NW, int MODE>
+__global__ void __launch_bounds__(NW * 64, 4)
+igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
+  using Acc = typename Mma16<TIn>::Acc;
+  using AccE = typename Epi::AccE;
+  using TOut = typename EpiTraits<Epi>::TOut;
+  typedef AccE accx4 __attribute__((ext_vector_type(4)));
+  constexpr int ES = sizeof(TIn);
+  constexpr int BM = MB * 16, BN = NB * 16;
+  constexpr int PITCH = BN + 4;             // words per pixel of a partial tile
+  constexpr int U = MB + NB <= 2 ? 4 : 2;   // K steps requested together
+  constexpr int REGION = BM * PITCH * 4;    // bytes of a wavefront's partial tile
+  constexpr int UNITS = BM * BN / 4;        // (pixel, four channels) pairs of the tile
+  constexpr int UPT = (UNITS + NW * 64 - 1) / (NW * 64);
+  static_assert(UNITS % 64 == 0, "whole wavefronts in the epilogue");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int M = p.N * p.Ho * p.Wo;
+  // workgroups that share operands stay on one XCD (they are dealt round-robin)
+  int bid = blockIdx.x;
+  {
+    const int per = gridDim.x >> 3;
+    if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
+  }
+  const int tile_m = a.m_fast ? bid % a.tiles_m : bid / a.tiles_n;
+  const int tile_n = a.m_fast ? bid / a.tiles_m : bid % a.tiles_n;
+  const int z = blockIdx.z;
+
+  const unsigned char* x = reinterpret_cast<const unsigned char*>(reinterpret_cast<const TIn*>(p.x) + (int64_t)z * p.x_bs);
+
+  // ---- weights: lane base address and bytes per 64 bytes of K ----
+  const unsigned char* w_ptr[NB];
+  const bool frag = p.w_frag != nullptr;
+  const int w_step = frag ? 2048 : 64;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    int n = tile_n * BN + j * 16 + l16;
+    if (frag) {
+      int t = n >> 5;
+      t = t < p.wf_tiles ? t : p.wf_tiles - 1;   // surplus channels are computed and never stored
+      w_ptr[j] = reinterpret_cast<const unsigned char*>(p.w_frag) +
+                 (((int64_t)z * p.wf_tiles + t) * p.wf_chunks + (g >> 1)) * 1024 + ((g & 1) * 32 + (n & 31)) * 16;
+    } else {
+      n = n < p.w_rows ? n : p.w_rows - 1;
+      w_ptr[j] = reinterpret_cast<const unsigned char*>(reinterpret_cast<const TIn*>(p.w) + (int64_t)z * p.w_bs + (int64_t)n * p.w_rs) + g * 16;
+    }
+  }
+
+  // ---- pixels: lane base address at tap (0, 0), channel 0 ----
+  const unsigned char* a_ptr[MB];
+  int a_hi[MB], a_wi[MB];
+  const int HoWo = p.Ho * p.Wo;
+#pragma unroll
+  for (int i = 0; i < MB; ++i) {
+    int m = tile_m * BM + i * 16 + l16;
+    m = m < M ? m : M - 1;                       // surplus rows are computed and never stored
+    const int n_img = fast_div(m, p.howo_magic, p.howo_shift);
+    const int rem = m - n_img * HoWo;
+    const int ho = fast_div(rem, p.wo_magic, p.wo_shift);
+    const int wo = rem - ho * p.Wo;
+    a_hi[i] = ho * p.sh - p.ph;
+    a_wi[i] = wo * p.sw - p.pw;
+    a_ptr[i] = x + (((int64_t)n_img * p.H + a_hi[i]) * p.W + a_wi[i]) * p.xcs * ES + (MODE == SLIM_ANY ? 0 : g * 16);
+  }
+  const unsigned f = (unsigned)(p.a_fill & 0xff) * 0x01010101u;
+  const uintx4 fillv = {f, f, f, f}, zerov = {0u, 0u, 0u, 0u};
+
+  // ---- this wavefront's share of the K steps ----
+  const int per = a.steps / NW, extra = a.steps - per * NW;
+  const int k0 = wave * per + (wave < extra ? wave : extra);
+  const int k1 = k0 + per + (wave < extra ? 1 : 0);
+  const int kvecs = p.R * p.S * a.cvec;          // valid 16-byte vectors of K
+
+  // walk of SLIM_TAP: wavefront-uniform tap and step inside the tap
+  int kc = 0, kr = 0, ks = 0;
+  const int cps = a.cvec >> 2;
+  if constexpr (MODE == SLIM_TAP) {
+    const int tap = fast_div(k0 * 4, a.cv_magic, a.cv_shift);
+    kc = k0 - tap * cps;
+    kr = fast_div(tap, a.s_magic, a.s_shift);
+    ks = tap - kr * p.S;
+  }
+
+  auto load = [&](const int k, uintx4 (&A)[MB], uintx4 (&W)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      if (!frag && MODE != SLIM_TAP) {
+        // (packed rows end at w_cols: the last step may reach behind them)
+        const bool in = k * 4 + g < kvecs;
+        const uintx4 v = *reinterpret_cast<const uintx4*>(w_ptr[j] + (in ? (int64_t)k * 64 : (int64_t)0));
+        W[j] = in ? v : zerov;
+      } else {
+        W[j] = *reinterpret_cast<const uintx4*>(w_ptr[j] + (int64_t)k * w_step);
+      }
+    }
+    if constexpr (MODE == SLIM_ROW) {
+      const bool in = k * 4 + g < kvecs;
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const uintx4 v = *reinterpret_cast<const uintx4*>(a_ptr[i] + (in ? k * 64 : -g * 16));
+        A[i] = in ? v : zerov;
+      }
+    } else {
+      int hoff, woff, coff;
+      bool in = true;
+      if constexpr (MODE == SLIM_TAP) {
+        hoff = kr * p.dh; woff = ks * p.dw; coff = kc * 64;
+        if (++kc == cps) { kc = 0; if (++ks == p.S) { ks = 0; ++kr; } }
+      } else {
+        const int kv = k * 4 + g;
+        in = kv < kvecs;
+        const int tap = fast_div(kv, a.cv_magic, a.cv_shift);
+        const int r = fast_div(tap, a.s_magic, a.s_shift);
+        hoff = r * p.dh; woff = (tap - r * p.S) * p.dw; coff = (kv - tap * a.cvec) * 16;
+      }
+      const int off = (hoff * p.W + woff) * p.xcs * ES + coff;
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const bool ok = in && (unsigned)(a_hi[i] + hoff) < (unsigned)p.H && (unsigned)(a_wi[i] + woff) < (unsigned)p.W;
+        const unsigned char* src = ok ? a_ptr[i] + off : x;
+        const uintx4 v = *reinterpret_cast<const uintx4*>(src);
+        A[i] = ok ? v : fillv;
+      }
+    }
+  };
+
+  Acc acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = Acc{0, 0, 0, 0};
+  auto mul = [&](const uintx4 (&A)[MB], const uintx4 (&W)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = Mma16<TIn>::run(W[j], A[i], acc[i][j]);
+  };
+
+  {
+    uintx4 A0[U][MB], W0[U][NB], A1[U][MB], W1[U][NB];
+    int k = k0;
+    const bool first = k + U <= k1;
+    if (first) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) load(k + u, A0[u], W0[u]);
+      k += U;
+      // two batches in turn: the next one is requested before the current one is used
+      for (; k + 2 * U <= k1; k += 2 * U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) load(k + u, A1[u], W1[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mul(A0[u], W0[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) load(k + U + u, A0[u], W0[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mul(A1[u], W1[u]);
+      }
+    }
+    // fewer than 2 U steps are left beside the batch in hand
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k + u < k1) load(k + u, A1[u], W1[u]);
+    if (first) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) mul(A0[u], W0[u]);
+    }
+#pragma unroll
+    for (int u = 0; u + 1 < U; ++u)
+      if (k + U + u < k1) load(k + U + u, A0[u], W0[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k + u < k1) mul(A1[u], W1[u]);
+#pragma unroll
+    for (int u = 0; u + 1 < U; ++u)
+      if (k + U + u < k1) mul(A0[u], W0[u]);
+  }
+
+  unsigned char* mine = smem + wave * REGION;
+  // ---- operands of the epilogue, requested ahead of the barrier ----
+  const AccE* bias = p.bias ? reinterpret_cast<const AccE*>(p.bias) + (int64_t)z * p.bias_bs : nullptr;
+  TOut* ybase = reinterpret_cast<TOut*>(p.y) + (EpiTraits<Epi>::quant ? (int64_t)z * p.y_bs : y_batch_off(p, z));
+  const TOut* rbase = p.residual ? reinterpret_cast<const TOut*>(p.residual) + (int64_t)z * p.r_bs : nullptr;
+  constexpr bool kQ8 = std::is_same<Epi, EpiQuant<0>>::value;
+  const bool wide = (epi_vec & 1) != 0;
+  AccE b4[UPT][4];
+  float m4[UPT][4], r4[UPT][4];
+  unsigned rq[UPT];
+#pragma unroll
+  for (int t = 0; t < UPT; ++t) {
+    const int u = tid + t * NW * 64;
+    const int m = tile_m * BM + u / (BN / 4), n = tile_n * BN + (u % (BN / 4)) * 4;
+    rq[t] = 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { b4[t][e] = 0; m4[t][e] = 0.f; r4[t][e] = 0.f; }
+    if (u < UNITS && m < M && n < p.Kout) {
+      if (wide && n + 4 <= p.Kout) {
+        if (bias != nullptr) __builtin_memcpy(b4[t], __builtin_assume_aligned(bias + n, 16), 16);
+        if (rbase != nullptr) {
+          const TOut* r = rbase + (int64_t)m * p.rcs + n;
+          if constexpr (kQ8) rq[t] = *reinterpret_cast<const unsigned*>(r);
+          else if constexpr (sizeof(TOut) == 4) __builtin_memcpy(r4[t], __builtin_assume_aligned(r, 16), 16);
+          else {
+            const uintx2 v = *reinterpret_cast<const uintx2*>(r);
+            const TOut* e4 = reinterpret_cast<const TOut*>(&v);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r4[t][e] = Store<TOut>::ld(e4 + e);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (n + e >= p.Kout) break;
+          if (bias != nullptr) b4[t][e] = bias[n + e];
+          if (rbase != nullptr) {
+            if constexpr (kQ8) rq[t] |= (unsigned)(uint8_t)rbase[(int64_t)m * p.rcs + n + e] << (8 * e);
+            else if constexpr (sizeof(TOut) == 4) r4[t][e] = (float)rbase[(int64_t)m * p.rcs + n + e];
+            else r4[t][e] = Store<TOut>::ld(rbase + (int64_t)m * p.rcs + n + e);
+          }
+        }
+      }
+      if constexpr (EpiTraits<Epi>::quant) {
+        if (p.qmul != nullptr) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < p.Kout) m4[t][e] = p.qmul[n + e];
+        }
+      }
+    }
+  }
+
+  // ---- partial tiles through LDS ----
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      *reinterpret_cast<accx4*>(reinterpret_cast<AccE*>(mine) + (i * 16 + l16) * PITCH + j * 16 + g * 4) = acc[i][j];
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < UPT; ++t) {
+    const int u = tid + t * NW * 64;
+    const int pix = u / (BN / 4), c = (u % (BN / 4)) * 4;
+    const int m = tile_m * BM + pix, n = tile_n * BN + c;
+    if (u >= UNITS || m >= M || n >= p.Kout) continue;
+    accx4 s = *reinterpret_cast<const accx4*>(smem + (pix * PITCH + c) * 4);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += *reinterpret_cast<const accx4*>(smem + w * REGION + (pix * PITCH + c) * 4);
+    const bool vec = wide && n + 4 <= p.Kout;
+    if constexpr (kQ8) {
+      const floatx4 mq = {m4[t][0], m4[t][1], m4[t][2], m4[t][3]};
+      const int a0 = s.x + b4[t][0], a1 = s.y + b4[t][1], a2 = s.z + b4[t][2], a3 = s.w + b4[t][3];
+      const unsigned w = rbase != nullptr ? requant4<true>(a0, a1, a2, a3, mq, rq[t], p) : requant4<false>(a0, a1, a2, a3, mq, 0u, p);
+      int8_t* y = ybase + (int64_t)m * p.ycs + n;
+      if (vec) *reinterpret_cast<unsigned*>(y) = w;
+      else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < p.Kout) y[e] = (int8_t)(w >> (8 * e));
+      }
+    } else if constexpr (EpiTraits<Epi>::quant) {
+      TOut* y = ybase + (int64_t)m * p.ycs + n;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= p.Kout) break;
+        const int v = s[e] + b4[t][e];
+        if constexpr (std::is_same<TOut, int>::value) y[e] = v;
+        else y[e] = epi_act((float)v * m4[t][e] + r4[t][e], p.act, p.act_a, p.act_b);
+      }
+    } else {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(s[e], p.alpha, b4[t][e]);
+      if (p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += r4[t][e];
+      if (!p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+      TOut* y = ybase + y_row_off(p, m) + y_col_off(p, n);
+      if (vec) {
+        if constexpr (sizeof(TOut) == 4) *reinterpret_cast<floatx4*>(y) = (floatx4){v[0], v[1], v[2], v[3]};
+        else {
+          uintx2 o;
+          TOut* e4 = reinterpret_cast<TOut*>(&o);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) Store<TOut>::st(e4 + e, v[e]);
+          *reinterpret_cast<uintx2*>(y) = o;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (n + e >= p.Kout) break;
+          if constexpr (sizeof(TOut) == 4) y[e] = v[e];
+          else Store<TOut>::st(y + e, v[e]);
+        }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+namespace {
+
+
+template <typename TIn, typename Epi, int MB, int NB, int NW>
+hipError_t launch_tile(const IgemmParams& p, const int epi_vec, SlimArgs a, const int mode, hipStream_t stream) {
+  const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
+  const int64_t tm = (M + MB * 16 - 1) / (MB * 16), tn = ((int64_t)p.Kout + NB * 16 - 1) / (NB * 16);
+  if (tm * tn <= 0 || tm * tn > 0x7fffffff || p.batch > 65535) return hipErrorInvalidValue;
+  a.tiles_m = (int)tm;
+  a.tiles_n = (int)tn;
+  constexpr size_t lds = (size_t)NW * MB * 16 * (NB * 16 + 4) * 4;
+  const dim3 grid((unsigned)(tm * tn), 1, (unsigned)p.batch), block(NW * 64);
+#define SLIM_LAUNCH(MODE_)                                                                                            \
+  do {                                                                                                                \
+    if constexpr (lds > 65536) {                                                                                      \
+      static bool ready = false; /* (repeating the call is harmless: no lock) */                                      \
+      if (!ready) {                                                                                                   \
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&igemm_slim_kernel<TIn, Epi, MB, NB, NW, MODE_>), \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
+        if (e != hipSuccess) return e;                                                                                \
+        ready = true;                                                                                                 \
+      }                                                                                                               \
+    }                                                                                                                 \
+    hipLaunchKernelGGL((igemm_slim_kernel<TIn, Epi, MB, NB, NW, MODE_>), grid, block, lds, stream, p, epi_vec, a);    \
+  } while (0)
+  if (mode == SLIM_ROW) SLIM_LAUNCH(SLIM_ROW);
+  else if (mode == SLIM_TAP) SLIM_LAUNCH(SLIM_TAP);
+  else SLIM_LAUNCH(SLIM_ANY);
+#undef SLIM_LAUNCH
+  return hipGetLastError();
+}
+
+template <typename TIn, typename Epi>
+hipError_t launch_slim(const IgemmParams& p, const int epi_vec, const int variant, hipStream_t stream) {
+  constexpr int ES = sizeof(TIn);
+  SlimArgs a;
+  a.cvec = p.C * ES / 16;
+  const int64_t vecs = (int64_t)p.R * p.S * a.cvec;
+  if (vecs <= 0 || vecs > (1 << 28)) return hipErrorInvalidValue;
+  a.steps = (int)((vecs + 3) / 4);
+  div_magic(a.cvec, &a.cv_magic, &a.cv_shift);
+  div_magic(p.S, &a.s_magic, &a.s_shift);
+  const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
+  // one XCD keeps the larger operand's tiles: with fewer pixels than channels the workgroups of one channel tile sit together
+  a.m_fast = M < p.Kout;
+  const bool row = p.R == 1 && p.S == 1 && p.ph == 0 && p.pw == 0 && (int64_t)(p.Ho - 1) * p.sh < p.H && (int64_t)(p.Wo - 1) * p.sw < p.W;
+  const int mode = row ? SLIM_ROW : (a.cvec % 4 == 0 ? SLIM_TAP : SLIM_ANY);
+  switch (variant) {
+    case 1: return launch_tile<TIn, Epi, 1, 1, 16>(p, epi_vec, a, mode, stream);
+    case 2: return launch_tile<TIn, Epi, 2, 2, 8>(p, epi_vec, a, mode, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+
+// Which kernel a launch gets, by an estimate of its time in us (beside the launch itself):
+//   c0 + c1 * chain + c2 * tiles / 256 + c3 * tiles * stages / 256
+// chain: K stages of 128 bytes that one wavefront walks; tiles: of the kernel's own size.  The
+// coefficients are a least-squares fit to some 1300 launches (ResNet-50 at 1 .. 48 images in
+// three types, BERT-base at 1 .. 64 sequences, YOLOv3 at 1 .. 16 images) of which each kernel's
+// fit saw those where it came within a factor of two of the best (three for the 128 x 128 row,
+// which stands for all kernels of igemm.hip and its siblings); rms errors 10 .. 20 %.  Chosen
+// by these estimates the launches take 3 % more than with the best kernel for each, and as much
+// as a fifth of what the 128 x 128 tiles take: ResNet-50 fp16, sums of the launches of a step,
+// 1 / 4 / 16 images 0.63 / 0.66 / 0.75 -> 0.18 / 0.28 / 0.51 ms, fp32 at 4 images 3.6 -> 0.75 ms,
+// BERT-base fp32 at 2 x 128 tokens 5.0 -> 1.2 ms.
+namespace {
+struct SlimCost { float fix, chain, tile, work; };
+struct SlimCosts { SlimCost wide, k16, k8, mid; };
+constexpr SlimCosts kCost1 = {{4.3f, .37f, .98f, .117f}, {.05f, .62f, 2.27f, .056f}, {.73f, .88f, .82f, .108f}, {1.74f, .18f, 1.06f, .16f}};
+constexpr SlimCosts kCost2 = {{4.4f, .42f, 1.0f, .42f}, {.05f, .62f, 2.27f, .056f}, {.73f, .88f, .82f, .108f}, {1.74f, .18f, 1.06f, .16f}};
+constexpr SlimCosts kCost4 = {{1.8f, 2.05f, 6.9f, .144f}, {0.f, .59f, 2.07f, .075f}, {1.14f, .93f, 1.15f, .19f}, {2.5f, .344f, 1.78f, .42f}};
+// How much faster than the 128 x 128 tiles the choice has to be.  (0.85 .. 1 cost the same over
+// all launches.)  More than two 64 x 64 tiles per compute unit: 0.7 - they ask the L2s for twice
+// the bytes per operation, which a launch that runs beside this one (the other half of a batch)
+// feels: YOLOv3 at 16 images in two halves 2.27 -> 2.34 ms with 0.88 there.
+constexpr float kSlimMargin = 0.88f, kSlimMarginFull = 0.7f;
+}  // namespace
+
+int igemm_slim_variant(const IgemmParams& p, const bool frag, float* us) {
+  if (us != nullptr) *us = 0.f;
+  if (p.f_y != nullptr || p.row_softmax != 0 || p.fixed_order) return 0;
+  // what the kernels' addressing assumes: 32-bit offsets inside an image, no column of K behind the packed rows
+  const int es = dtype_size(p.in_dt);
+  if (es == 0 || (int64_t)p.H * p.W * p.xcs * es >= (1ll << 31) || (int64_t)p.R * p.S * p.C > p.w_cols) return 0;
+  if (const char* force = getenv("ODLA_HIP_IGEMM_TILE")) {  // tuning aid: "slim1", "slim2", "mid"
+    if (strncmp(force, "slim", 4) == 0 && force[4] >= '1' && force[4] <= '2') return force[4] - '0';
+    if (strcmp(force, "mid") == 0) return frag ? 3 : 0;
+    if (force[0] != 0) return 0;
+  }
+  // (a tuning aid of another kernel asks for that kernel)
+  for (const char* aid : {"ODLA_HIP_WREG_SLICES", "ODLA_HIP_WREG_KSPLIT", "ODLA_HIP_C3_MIN_FILL", "ODLA_HIP_C3_BC", "ODLA_HIP_C3_SLICES",
+                          "ODLA_HIP_LEAN_TILES", "ODLA_HIP_STREAM_WGS"})
+    if (getenv(aid) != nullptr) return 0;
+  const SlimCosts& c = es == 1 ? kCost1 : es == 2 ? kCost2 : kCost4;
+  const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
+  const float stages = (float)(((int64_t)p.R * p.S * p.C * es + 127) / 128);
+  auto cost = [&](const SlimCost& k, const int tile, const int waves) {
+    const float tiles = (float)((M + tile - 1) / tile) * (float)((p.Kout + tile - 1) / tile) * (float)p.batch / 256.f;
+    return k.fix + k.chain * stages / (float)waves + k.tile * tiles + k.work * tiles * stages;
+  };
+  const float t1 = cost(c.k16, 16, 16), t2 = cost(c.k8, 32, 8), t3 = cost(c.mid, 64, 1);
+  int v = t1 < t2 ? 1 : 2;
+  float t = t1 < t2 ? t1 : t2;
+  if (frag && t3 < t) { v = 3; t = t3; }
+  if (us != nullptr) *us = t;
+  const int64_t tiles64 = ((M + 63) / 64) * (((int64_t)p.Kout + 63) / 64) * p.batch;
+  const float margin = v == 3 && es < 4 && tiles64 > 512 ? kSlimMarginFull : kSlimMargin;
+  return t < margin * cost(c.wide, 128, 1) ? v : 0;
+}
+
+hipError_t launch_igemm_slim(const IgemmParams& p, int epi_vec, int variant, hipStream_t stream) {
+  if (variant == 3) return launch_igemm_mid(p, epi_vec, stream);
+  const bool rich = p.act == ACT_GELU_ERF || p.act == ACT_GELU_TANH || p.act == ACT_SIGMOID || p.act == ACT_TANH;
+  switch (p.in_dt) {
+    case DT_F32:
+      if (p.out_dt != DT_F32) return hipErrorInvalidValue;
+      if (rich) return launch_slim<float, EpiFloat<float, true>>(p, epi_vec, variant, stream);
+      return launch_slim<float, EpiFloat<float>>(p, epi_vec, variant, stream);
+    case DT_F16:
+      if (p.out_dt == DT_F16 && rich) return launch_slim<f16_t, EpiFloat<f16_t, true>>(p, epi_vec, variant, stream);
+      if (p.out_dt == DT_F16) return launch_slim<f16_t, EpiFloat<f16_t>>(p, epi_vec, variant, stream);
+      if (p.out_dt == DT_F32) return launch_slim<f16_t, EpiFloat<float>>(p, epi_vec, variant, stream);
+      return hipErrorInvalidValue;
+    case DT_BF16:
+      if (p.out_dt == DT_BF16 && rich) return launch_slim<bf16_t, EpiFloat<bf16_t, true>>(p, epi_vec, variant, stream);
+      if (p.out_dt == DT_BF16) return launch_slim<bf16_t, EpiFloat<bf16_t>>(p, epi_vec, variant, stream);
+      if (p.out_dt == DT_F32) return launch_slim<bf16_t, EpiFloat<float>>(p, epi_vec, variant, stream);
+      return hipErrorInvalidValue;
+    case DT_I8:
+      if (p.out_dt == DT_I8) return p.qmul == nullptr ? hipErrorInvalidValue : launch_slim<int8_t, EpiQuant<0>>(p, epi_vec, variant, stream);
+      if (p.out_dt == DT_F32) return p.qmul == nullptr ? hipErrorInvalidValue : launch_slim<int8_t, EpiQuant<1>>(p, 0, variant, stream);
+      if (p.out_dt == DT_I32) return launch_slim<int8_t, EpiQuant<2>>(p, 0, variant, stream);
+      return hipErrorInvalidValue;
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace ohip

@@ -124,6 +124,9 @@ struct IgemmParams {
   float act_a = 0.0f, act_b = 0.0f;  // leaky slope / clamp lo,hi
   bool res_after_act = false;        // float types: y = act(..) + residual instead of act(.. + residual)
   bool stream_out = false;           // 2-byte results leave with non-temporal stores (results far larger than the last-level cache)
+  // fp32 sums of an 8-bit plan keep one order whatever the number of rows (an image's results do
+  // not depend on its batch, bit for bit): no small-tile kernel.
+  bool fixed_order = false;
   // Softmax (1) or LogSoftmax (2) over the Kout columns of every result row, behind bias and
   // activation: only the one-wavefront-per-row kernel computes it (gemm_rowdot_shape).
   int row_softmax = 0;
@@ -155,8 +158,9 @@ struct IgemmParams {
   float f_q_add = 0.f, f_q_lo = 0.f;
 };
 hipError_t launch_igemm(const IgemmParams& p, hipStream_t stream);
-// Name of the kernel variant launch_igemm would pick (for reports).
-const char* igemm_variant_name(const IgemmParams& p);
+// Name of the kernel variant launch_igemm would pick (for reports); small_tiles = false: of the
+// variant it would pick without the small-tile kernels.
+const char* igemm_variant_name(const IgemmParams& p, bool small_tiles = true);
 
 // Products with at most 16 output columns, a long reduction and few rows (gemm_rowdot.hip): one
 // wavefront per output row.  Whether the shape qualifies, and the launch (launch_igemm uses both).
@@ -167,6 +171,13 @@ hipError_t launch_gemm_rowdot(const IgemmParams& p, hipStream_t stream);
 // launch_igemm uses for this shape (0: none), and the launch itself.
 int igemm_big_variant(const IgemmParams& p);
 hipError_t launch_igemm_big(const IgemmParams& p, int epi_vec, int variant, hipStream_t stream);
+
+// Small-tile kernels for launches with few output tiles: the variant launch_igemm uses for this
+// shape (0: none; 1, 2: igemm_slim.hip; 3: igemm_mid.hip), and the launches themselves.  frag:
+// the weights exist in fragment order; us: the estimated time in us, beside the launch itself.
+int igemm_slim_variant(const IgemmParams& p, bool frag, float* us = nullptr);
+hipError_t launch_igemm_slim(const IgemmParams& p, int epi_vec, int variant, hipStream_t stream);
+hipError_t launch_igemm_mid(const IgemmParams& p, int epi_vec, hipStream_t stream);
 
 // Streaming kernel for 8-bit 1x1 filters over short pixel rows (igemm_stream.hip):
 // whether the layer's geometry qualifies (no pointer is looked at), and the launch

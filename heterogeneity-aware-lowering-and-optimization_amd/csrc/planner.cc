@@ -589,6 +589,8 @@ class Planner {
     ip.w_frag = has_wfrag ? &dummy : nullptr;
     ip.residual = has_residual ? &dummy : nullptr;
     OHIP_DEBUG("%s: kernel %s", name.c_str(), igemm_variant_name(ip));
+    if (igemm_slim_variant(ip, has_wfrag) > 0)
+      OHIP_DEBUG("%s: the small tile is estimated to beat kernel %s", name.c_str(), igemm_variant_name(ip, false));
   }
   // A value whose only use is Reshape -> [B, S, heads, d] -> Transpose (0, 2, 1, 3): the
   // GEMM that computes it can store [B, heads, S, d] directly (IgemmParams::y_rdiv).
@@ -1527,6 +1529,7 @@ void Planner::lower_conv(int ni) {
   ip.dh = dil_h; ip.dw = dil_w; ip.ph = pad_t; ip.pw = pad_l;
   ip.w_rows = Oge; ip.w_cols = w_rs; ip.w_rs = w_rs;
   ip.in_dt = dt; ip.out_dt = odt;
+  ip.fixed_order = comp_->opts.int8 && dt == DT_F32;
   ip.batch = Ge;
   ip.alpha = ep.scalar;
   if (Ge > 1) { ip.x_bs = Cg; ip.w_bs = (int64_t)Og * w_rs; ip.y_bs = Og; ip.r_bs = Og; ip.bias_bs = Og; }
@@ -1825,6 +1828,7 @@ void Planner::lower_gemm(int ni) {
   ip.C = Kp; ip.xcs = Kp;
   ip.Kout = (int)Nn;
   ip.in_dt = dt; ip.out_dt = odt;
+  ip.fixed_order = comp_->opts.int8 && dt == DT_F32;
   ip.alpha = alpha * ep.scalar;
   ip.ycs = (int)Nn;
   int tw;
@@ -1914,6 +1918,10 @@ void Planner::lower_gemm(int ni) {
         while (splits < 16 && Kp % (splits * 2 * stage) == 0 && Kp / (splits * 2) >= 4 * stage && tiles * splits * 2 <= 1024)
           splits *= 2;
       }
+      // (few rows: the small-tile kernels split K inside the workgroup, one launch instead of the
+      //  products and their sum, which take 7 us together)
+      float us = 0.f;
+      if (splits > 1 && igemm_slim_variant(ip, true, &us) > 0 && us < 7.f) splits = 1;
       if (splits > 1) {
         const int Kc = Kp / splits;
         Shape ps;
