@@ -229,7 +229,7 @@ hipError_t launch_pack_weights(const PackWeightsParams& p, hipStream_t stream);
 // One-launch attention (attention.hip):
 //   out[b, h] = softmax(scale * q[b, h] . k[b, h]^T + mask[b]) . v[b, h]
 // q, k, v: [S][d] matrices of 16-bit elements per (batch, head), rows of d = 64
-// contiguous values; S = 32, 64, 96 or 128.  mask: one row of S values per batch
+// contiguous values; any S.  mask: one row of S values per batch
 // (added to every query's scores), of the operands' type or fp32, or null.
 // All strides in elements.
 struct AttentionParams {

@@ -1706,7 +1706,7 @@ bool Planner::try_fused_attention(int ni) {
   if (ti >= 0) { ap.o_bs = S * heads * d; ap.o_hs = d; ap.o_rs = heads * d; }
   else { ap.o_bs = heads * S * d; ap.o_hs = S * d; ap.o_rs = d; }
   ap.mask_bs = mask_bs;
-  if (B * heads > 0x7fffffff || !attention_supported(ap)) return false;
+  if (!attention_supported(ap)) return false;
 
   // ---- from here on the plan changes
   const int tq = get(Q, L_ROWMAJOR, FORM_OPERAND), tk = get(K, L_ROWMAJOR, FORM_OPERAND), tv = get(V, L_ROWMAJOR, FORM_OPERAND);
