@@ -255,7 +255,8 @@ odla_status stage_inputs(_odla_context* ctx, const Plan& plan, char* arena, std:
       OHIP_ERR("argument '%s' is not bound", io.v->name.c_str());
       return ODLA_INVALID_PARAM;
     }
-    if (ext != nullptr && io.in_place_ok && !ctx->in_place_off && in_place_args_enabled() && is_device_memory(it->second)) {
+    if (ext != nullptr && io.in_place_ok && !ctx->in_place_off && in_place_args_enabled() &&
+        (!io.align16 || (reinterpret_cast<uintptr_t>(it->second) & 15u) == 0) && is_device_memory(it->second)) {
       (*ext)[k] = static_cast<const char*>(it->second);
       OHIP_DEBUG("argument '%s' is read in place", io.v->name.c_str());
       continue;

@@ -177,11 +177,12 @@ struct Plan {
     int tensor = -1;  // staging tensor in the arena: row-major, declared element type
     size_t offset = 0;  // byte offset inside that tensor (results that are slices of a merged launch)
     size_t bytes = 0;
-    // arguments: every step that touches the staging tensor reads exactly its elements and
-    // checks alignment itself, and nothing writes it: a device buffer can be read in place;
-    // results: only the final conversion to the declared type touches the tensor, and it
-    // writes exactly its elements: a device buffer can be written in place
+    // arguments: every step that touches the staging tensor reads exactly its elements, and
+    // nothing writes it: a device buffer can be read in place;
+    // results: no step reads the tensor and those that write it write exactly its elements: a
+    // device buffer can be written in place
     bool in_place_ok = false;
+    bool align16 = false;    // ... at a 16-byte aligned address
   };
   std::vector<IO> inputs, outputs;
   std::unordered_map<const _odla_value*, int> final_tensor;  // for odla_GetValueData

@@ -56,26 +56,18 @@ unary_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t n, ActKind act,
   }
 }
 
-// y = x * scale[c] + shift[c].  inner == 1: channel is the innermost index
-// (channels-last), so a vector spans V consecutive channels; when the grid
-// stride is a multiple of the channel count every thread meets the same V
-// channels in every iteration and keeps their parameters in registers.
-// inner > 1 (row-major N,C,HW): the channel is constant across a vector when
-// inner % V == 0.
+// y = x * scale[c] + shift[c] on row-major N,C,inner tensors (inner > 1): the channel is constant
+// across a vector when inner % V == 0.  (Channels-last tensors: channel_rows_kernel.)
 template <typename T, int U>
 __global__ void __launch_bounds__(kThreads)
 channel_affine_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t n, int64_t inner,
                       int channels, const float* __restrict__ scale,
                       const float* __restrict__ shift) {
   constexpr int V = Vec16<T>::N;
-  const bool vec_ok = (inner == 1) ? (channels % V == 0) : (inner % V == 0);
-  if (vec_ok) {
+  if (inner % V == 0) {
     // tiled like unary_kernel: a workgroup owns kThreads * U consecutive vectors
     const int64_t nvec = n / V;
-    const int64_t tile0 = (int64_t)blockIdx.x * (kThreads * U);
-    const int64_t base = tile0 + threadIdx.x;
-    // channel of the tile's first element (wavefront-uniform), then 32-bit arithmetic per vector
-    const unsigned c_tile = inner == 1 ? (unsigned)((tile0 * V) % channels) : 0u;
+    const int64_t base = (int64_t)blockIdx.x * (kThreads * U) + threadIdx.x;
     Vec16<T> v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -86,34 +78,86 @@ channel_affine_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t n, int
     for (int u = 0; u < U; ++u) {
       const int64_t i = base + u * kThreads;
       if (i >= nvec) continue;
-      if (inner == 1) {
-        const unsigned c0 = (c_tile + (unsigned)(u * kThreads + threadIdx.x) * V) % (unsigned)channels;
-        float sc[V], sh[V];
-        if constexpr (V == 8) {
-          const floatx4 s0 = *reinterpret_cast<const floatx4*>(scale + c0), s1 = *reinterpret_cast<const floatx4*>(scale + c0 + 4);
-          const floatx4 t0 = *reinterpret_cast<const floatx4*>(shift + c0), t1 = *reinterpret_cast<const floatx4*>(shift + c0 + 4);
-          sc[0] = s0.x; sc[1] = s0.y; sc[2] = s0.z; sc[3] = s0.w; sc[4] = s1.x; sc[5] = s1.y; sc[6] = s1.z; sc[7] = s1.w;
-          sh[0] = t0.x; sh[1] = t0.y; sh[2] = t0.z; sh[3] = t0.w; sh[4] = t1.x; sh[5] = t1.y; sh[6] = t1.z; sh[7] = t1.w;
-        } else {
+      const int c = (int)(((i * V) / inner) % channels);
+      const float sc = scale[c], sh = shift[c];
 #pragma unroll
-          for (int e = 0; e < V; ++e) { sc[e] = scale[c0 + e]; sh[e] = shift[c0 + e]; }
-        }
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[u].set(e, v[u].get(e) * sc[e] + sh[e]);
-      } else {
-        const int c = (int)(((i * V) / inner) % channels);
-        const float sc = scale[c], sh = shift[c];
-#pragma unroll
-        for (int e = 0; e < V; ++e) v[u].set(e, v[u].get(e) * sc + sh);
-      }
+      for (int e = 0; e < V; ++e) v[u].set(e, v[u].get(e) * sc + sh);
       out_store(v[u], y + i * V);
     }
   } else {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x * U;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += stride / U) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += stride) {
       const int c = (int)((i / inner) % channels);
       Store<T>::st(y + i, Store<T>::ld(x + i) * scale[c] + shift[c]);
     }
+  }
+}
+
+__device__ __forceinline__ float bin_op(float a, float b, BinKind op) {
+  switch (op) {
+    case BIN_ADD: return a + b;
+    case BIN_SUB: return a - b;
+    case BIN_MUL: return a * b;
+    case BIN_DIV: return a / b;
+    case BIN_MAX: return fmaxf(a, b);
+    case BIN_MIN: return fminf(a, b);
+  }
+  return a;
+}
+
+// Channels-last rows (pixels) of C channels, each tensor with its own pitch:
+//   y[m][c] = act((x[m][c] * scale[c] + shift[c]) op r[m][c])
+// with the affine part, the operand r and the activation optional - BatchNorm with its activation,
+// an element-wise operator, an activation - so that the result can be a channel slice of a wider
+// tensor (the place it has in a Concat) and nothing is copied there afterwards.
+// HBM-bound; one pass over what each operand holds.  W = 8 (2-byte types) or 4: vectors of W
+// channels; W = 1: single elements, where the channel count or a pitch is odd.  Tiled like
+// unary_kernel.  OP / KIND >= 0 fix the operator / the activation at compile time.
+template <typename T, int W, bool AFFINE, int OP, int KIND, int U>
+__global__ void __launch_bounds__(kThreads) channel_rows_kernel(const ChannelRowsParams p) {
+  const T* x = reinterpret_cast<const T*>(p.x);
+  const T* r = reinterpret_cast<const T*>(p.r);
+  T* y = reinterpret_cast<T*>(p.y);
+  constexpr bool kOp = OP != -2;   // -2: no second operand
+  const ActKind kind = KIND >= 0 ? (ActKind)KIND : p.act;
+  const BinKind op = OP >= 0 ? (BinKind)OP : p.op;
+  const int cw = p.C / W;
+  const int64_t n = p.rows * cw;   // (the launcher checks n < 2^31)
+  const int64_t base = (int64_t)blockIdx.x * (kThreads * U) + threadIdx.x;
+  struct alignas(W == 1 ? sizeof(T) : 16) Unit { T v[W]; };
+  Unit vx[U], vr[U];
+  int64_t m[U];
+  int c[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = base + u * kThreads;
+    if (i < n) {
+      m[u] = fast_div((int)i, p.cw_magic, p.cw_shift);
+      c[u] = ((int)i - (int)m[u] * cw) * W;
+      vx[u] = *reinterpret_cast<const Unit*>(x + m[u] * p.xcs + c[u]);
+      if constexpr (kOp) vr[u] = *reinterpret_cast<const Unit*>(r + m[u] * p.rcs + c[u]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = base + u * kThreads;
+    if (i >= n) continue;
+    float f[W];
+#pragma unroll
+    for (int e = 0; e < W; ++e) f[e] = Store<T>::ld(&vx[u].v[e]);
+    if constexpr (AFFINE) {
+      float sc[W], sh[W];
+#pragma unroll
+      for (int e = 0; e < W; ++e) { sc[e] = p.scale[c[u] + e]; sh[e] = p.shift[c[u] + e]; }
+#pragma unroll
+      for (int e = 0; e < W; ++e) f[e] = f[e] * sc[e] + sh[e];
+    }
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      if constexpr (kOp) f[e] = bin_op(f[e], Store<T>::ld(&vr[u].v[e]), op);
+      Store<T>::st(&vx[u].v[e], apply_act(f[e], kind, p.act_a, p.act_b));
+    }
+    *reinterpret_cast<Unit*>(y + m[u] * p.ycs + c[u]) = vx[u];
   }
 }
 
@@ -127,18 +171,6 @@ __global__ void bn_fold_kernel(const float* mean, const float* var, const float*
   const float m = g / sqrtf(var[c] + eps);
   scale[c] = m;
   shift[c] = b - mean[c] * m;
-}
-
-__device__ __forceinline__ float bin_op(float a, float b, BinKind op) {
-  switch (op) {
-    case BIN_ADD: return a + b;
-    case BIN_SUB: return a - b;
-    case BIN_MUL: return a * b;
-    case BIN_DIV: return a / b;
-    case BIN_MAX: return fmaxf(a, b);
-    case BIN_MIN: return fminf(a, b);
-  }
-  return a;
 }
 
 // Same-shape, contiguous operands; tiled like unary_kernel.  OP / KIND >= 0 fix the
@@ -598,6 +630,42 @@ hipError_t launch_channel_affine(const void* x, void* y, DType dt, int64_t n, in
   const unsigned grid = (unsigned)(tiles > 0 ? tiles : 1);
   FLOAT_DISPATCH(dt, hipLaunchKernelGGL((channel_affine_kernel<T, U>), dim3(grid), dim3(kThreads), 0,
                                         stream, (const T*)x, (T*)y, n, inner, channels, scale, shift));
+  return hipGetLastError();
+}
+
+hipError_t launch_channel_rows(const ChannelRowsParams& p_in, hipStream_t stream) {
+  ChannelRowsParams p = p_in;
+  const bool affine = p.scale != nullptr, has_r = p.r != nullptr;
+  if (!p.x || !p.y || p.rows <= 0 || p.C <= 0 || p.xcs < p.C || p.ycs < p.C || (has_r && p.rcs < p.C) || (affine && !p.shift))
+    return hipErrorInvalidValue;
+  const int v = 16 / dtype_size(p.dt);
+  const bool vec = p.C % v == 0 && p.xcs % v == 0 && p.ycs % v == 0 && al16(p.x) && al16(p.y) &&
+                   (!has_r || (p.rcs % v == 0 && al16(p.r)));
+  const int w = vec ? v : 1;
+  if (p.rows * (p.C / w) >= (1ll << 31)) return hipErrorInvalidValue;
+  div_magic(p.C / w, &p.cw_magic, &p.cw_shift);
+  constexpr int U = 4;
+  const dim3 grid((unsigned)((p.rows * (p.C / w) + kThreads * U - 1) / (kThreads * U)));
+#define ROWS_GO(W_, A_, OP_, K_) hipLaunchKernelGGL((channel_rows_kernel<T, W_, A_, OP_, K_, U>), grid, dim3(kThreads), 0, stream, p)
+#define ROWS_ACT(W_, A_, OP_)                                         \
+  do {                                                                \
+    if (p.act == ACT_NONE) ROWS_GO(W_, A_, OP_, (int)ACT_NONE);       \
+    else if (p.act == ACT_RELU) ROWS_GO(W_, A_, OP_, (int)ACT_RELU);  \
+    else if (p.act == ACT_LEAKY) ROWS_GO(W_, A_, OP_, (int)ACT_LEAKY); \
+    else ROWS_GO(W_, A_, OP_, -1);                                    \
+  } while (0)
+#define ROWS_CASE(W_)                                                                            \
+  do {                                                                                           \
+    if (affine && !has_r) ROWS_ACT(W_, true, -2);                                                \
+    else if (!affine && has_r && p.op == BIN_ADD) ROWS_ACT(W_, false, (int)BIN_ADD);             \
+    else if (!affine && has_r) ROWS_GO(W_, false, -1, -1);                                       \
+    else if (!affine) ROWS_ACT(W_, false, -2);                                                   \
+    else ROWS_GO(W_, true, -1, -1);                                                              \
+  } while (0)
+  FLOAT_DISPATCH(p.dt, do { if (vec) ROWS_CASE(16 / (int)sizeof(T)); else ROWS_CASE(1); } while (0));
+#undef ROWS_CASE
+#undef ROWS_ACT
+#undef ROWS_GO
   return hipGetLastError();
 }
 

@@ -295,10 +295,24 @@ hipError_t launch_dequantize(const QuantParams& p, hipStream_t stream);  // src 
 // Streaming element-wise kernels (flat, 16-byte vectorised).
 hipError_t launch_unary(const void* x, void* y, DType dt, int64_t n, ActKind act,
                         float a, float b, hipStream_t stream);
-// y = x * scale[c] + shift[c], c = (i / inner) % channels   (folded BatchNorm)
+// y = x * scale[c] + shift[c], c = (i / inner) % channels   (folded BatchNorm, row-major)
 hipError_t launch_channel_affine(const void* x, void* y, DType dt, int64_t n,
                                  int64_t inner, int channels, const float* scale,
                                  const float* shift, hipStream_t stream);
+// y[m][c] = act((x[m][c] * scale[c] + shift[c]) op r[m][c]) on channels-last rows of C channels with
+// one pitch per tensor; scale / shift and r may be null.  rows * C < 2^31.
+struct ChannelRowsParams {
+  const void* x = nullptr; const void* r = nullptr; void* y = nullptr;
+  DType dt = DT_F32;
+  int64_t rows = 0;
+  int C = 0, xcs = 0, rcs = 0, ycs = 0;
+  const float* scale = nullptr; const float* shift = nullptr;
+  BinKind op = BIN_ADD;
+  ActKind act = ACT_NONE; float act_a = 0.f, act_b = 0.f;
+  // filled in by the launcher: division by the vectors per row
+  unsigned cw_magic = 0; int cw_shift = 0;
+};
+hipError_t launch_channel_rows(const ChannelRowsParams& p, hipStream_t stream);
 // scale/shift from BatchNorm statistics, computed on the device for
 // non-constant operands.  Any of gamma/beta may be null (scalars used instead).
 hipError_t launch_bn_fold(const float* mean, const float* var, const float* gamma,
@@ -407,7 +421,10 @@ enum ReduceKind : int {
 };
 hipError_t launch_reduce(const void* x, void* y, DType in_dt, DType out_dt, int64_t outer,
                          int64_t len, int64_t inner, ReduceKind kind, hipStream_t stream,
-                         float eps = 0.f);
+                         float eps = 0.f, float* ws = nullptr);
+// Slices of the middle axis a column reduction is split into when it is given `ws`, outer *
+// slices * inner floats of scratch memory (1: not split, no scratch needed).
+int reduce_slices(DType dt, int64_t outer, int64_t len, int64_t inner);
 // Index (int32 / int64) of the largest or smallest element along the middle
 // axis; ties resolve to the first index, or to the last when `last` is set.
 hipError_t launch_arg_extreme(const void* x, void* y, DType in_dt, DType out_dt, int64_t outer,
@@ -447,8 +464,9 @@ hipError_t launch_strided_copy(const StridedCopyParams& p, hipStream_t stream);
 hipError_t launch_transpose2d(const void* x, void* y, int elem_size, int batch, int rows, int cols,
                               int dst_pitch, hipStream_t stream);
 // Nearest-neighbour resize, channels-last: src index = floor(dst * in / out).
-hipError_t launch_resize_nearest_nhwc(const void* x, void* y, int elem_size, int N, int H,
-                                      int W, int cs, int Ho, int Wo, hipStream_t stream);
+// cs / ycs: element pitch of x's / y's pixels, of which C are moved.
+hipError_t launch_resize_nearest_nhwc(const void* x, void* y, int elem_size, int N, int H, int W, int C, int cs, int ycs,
+                                      int Ho, int Wo, hipStream_t stream);
 // Bilinear resize, channels-last, float types: half-pixel centres, edges clamped.
 hipError_t launch_resize_linear_nhwc(const void* x, void* y, DType dt, int N, int H, int W, int cs,
                                      int Ho, int Wo, hipStream_t stream);

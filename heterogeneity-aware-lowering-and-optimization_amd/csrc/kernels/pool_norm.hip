@@ -6,6 +6,8 @@
 
 #include "device_utils.h"
 
+#include <algorithm>
+
 namespace ohip {
 namespace {
 
@@ -92,16 +94,16 @@ __global__ void __launch_bounds__(kThreads) pool2d_vec_kernel(PoolParams p) {
 // Scalar-channel fallback (C not a multiple of the vector width).
 template <typename T, bool IS_MAX>
 __global__ void __launch_bounds__(kThreads) pool2d_scalar_kernel(PoolParams p) {
-  const int64_t total = (int64_t)p.N * p.Ho * p.Wo * p.C;
   const T* x = reinterpret_cast<const T*>(p.x);
   T* y = reinterpret_cast<T*>(p.y);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int c = (int)(i % p.C);
-    int64_t t = i / p.C;
-    const int wo = (int)(t % p.Wo); t /= p.Wo;
-    const int ho = (int)(t % p.Ho);
-    const int n = (int)(t / p.Ho);
+  const int i = blockIdx.x * kThreads + threadIdx.x;   // position and channel within an image
+  const int row_units = p.Wo * p.C;
+  if (i >= p.Ho * row_units) return;
+  const int ho = fast_div(i, p.row_magic, p.row_shift);
+  const int rem = i - ho * row_units;
+  const int wo = fast_div(rem, p.cv_magic, p.cv_shift);
+  const int c = rem - wo * p.C;
+  for (int n = blockIdx.y; n < p.N; n += gridDim.y) {
     const int h0 = ho * p.sh - p.ph, w0 = wo * p.sw - p.pw;
     float acc = IS_MAX ? -INFINITY : 0.f;
     int cnt = 0;
@@ -327,9 +329,11 @@ reduce_cols_vec_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t out
 // long sequence): one thread per column leaves most of the chip idle.  Here a
 // workgroup owns `cl` 16-byte column groups of one outer index, its NT / cl
 // thread rows stride the reduced axis, and the partial results meet in LDS.
+// `slices` (grid.z slices of the axis, reduce_slices): the slices' partial results go there as
+// [outer][slice][inner] instead of a result to y.
 template <typename TI, typename TO, int A, int NT>
 __global__ void __launch_bounds__(NT)
-reduce_cols_split_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t len, int64_t inner,
+reduce_cols_split_kernel(const TI* __restrict__ x, TO* __restrict__ y, float* __restrict__ slices, int64_t len, int64_t inner,
                          int cl, ReduceKind kind, float eps) {
   constexpr int V = Vec16<TI>::N;
   __shared__ float part[NT * V];
@@ -337,13 +341,15 @@ reduce_cols_split_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t l
   const int64_t iv = inner / V;
   const int64_t cv = blockIdx.x * (int64_t)cl + c;
   const int64_t o = blockIdx.y;
+  const int64_t per = (len + gridDim.z - 1) / gridDim.z;
+  const int64_t k0 = blockIdx.z * per, k1 = k0 + per < len ? k0 + per : len;
   float acc[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) acc[e] = red_init<A>();
-  if (cv < iv) {
+  if (cv < iv && s < S) {
     const TI* col = x + o * len * inner + cv * V;
-    int64_t k = s;
-    for (; k + 3 * (int64_t)S < len; k += 4 * (int64_t)S) {
+    int64_t k = k0 + s;
+    for (; k + 3 * (int64_t)S < k1; k += 4 * (int64_t)S) {
       Vec16<TI> v[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) v[u].load(col + (k + u * (int64_t)S) * inner);
@@ -352,7 +358,7 @@ reduce_cols_split_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t l
 #pragma unroll
         for (int e = 0; e < V; ++e) acc[e] = red_step<A>(acc[e], v[u].get(e));
     }
-    for (; k < len; k += S) {
+    for (; k < k1; k += S) {
       Vec16<TI> v;
       v.load(col + k * inner);
 #pragma unroll
@@ -361,14 +367,55 @@ reduce_cols_split_kernel(const TI* __restrict__ x, TO* __restrict__ y, int64_t l
   }
   const int width = cl * V;
 #pragma unroll
-  for (int e = 0; e < V; ++e) part[s * width + c * V + e] = acc[e];
+  for (int e = 0; e < V; ++e)
+    if (s < S) part[s * width + c * V + e] = acc[e];
   __syncthreads();
   for (int j = threadIdx.x; j < width; j += NT) {
     const int64_t col = blockIdx.x * (int64_t)width + j;
     if (col >= inner) break;
     float r = part[j];
     for (int t = 1; t < S; ++t) r = red_merge<A>(r, part[t * width + j]);
-    Store<TO>::st(y + o * inner + col, red_final(r, len, kind, eps));
+    if (slices != nullptr) slices[(o * gridDim.z + blockIdx.z) * inner + col] = r;
+    else Store<TO>::st(y + o * inner + col, red_final(r, len, kind, eps));
+  }
+}
+// Columns that form no 16-byte groups (odd channel counts): a thread keeps one column and the
+// workgroup reads runs of whole rows, NT / inner of them per pass (one run of NT columns per
+// pass where a row is longer), so that its lanes read consecutive elements whatever `inner` is.
+// One thread per column walked the axis alone: ReduceMean [1, 162, 66 x 66] fp16 1000 -> 8 us.
+// total: elements of the axis behind the result (the second pass over slices divides by it).
+template <typename TI, typename TO, int A, int NT>
+__global__ void __launch_bounds__(NT)
+reduce_cols_flat_kernel(const TI* __restrict__ x, TO* __restrict__ y, float* __restrict__ slices, int64_t len, int64_t inner,
+                        int64_t total, ReduceKind kind, float eps) {
+  __shared__ float part[NT];
+  const int cols = inner < NT ? (int)inner : NT;
+  const int R = NT / cols;                       // rows per pass
+  const int r0 = threadIdx.x / cols, c = threadIdx.x - r0 * cols;
+  const int64_t col = blockIdx.x * (int64_t)NT + c;
+  const int64_t o = blockIdx.y;
+  const int64_t per = (len + gridDim.z - 1) / gridDim.z;
+  const int64_t k0 = blockIdx.z * per, k1 = k0 + per < len ? k0 + per : len;
+  float acc = red_init<A>();
+  if (r0 < R && col < inner) {
+    const TI* p = x + o * len * inner + col;
+    int64_t k = k0 + r0;
+    for (; k + 7 * (int64_t)R < k1; k += 8 * (int64_t)R) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = Store<TI>::ld(p + (k + u * (int64_t)R) * inner);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc = red_step<A>(acc, v[u]);
+    }
+    for (; k < k1; k += R) acc = red_step<A>(acc, Store<TI>::ld(p + k * inner));
+  }
+  part[threadIdx.x] = acc;
+  __syncthreads();
+  if (r0 == 0 && col < inner) {
+    float r = part[c];
+    for (int t = 1; t < R; ++t) r = red_merge<A>(r, part[t * cols + c]);
+    if (slices != nullptr) slices[(o * gridDim.z + blockIdx.z) * inner + col] = r;
+    else Store<TO>::st(y + o * inner + col, red_final(r, total, kind, eps));
   }
 }
 // Few long rows (inner == 1): a workgroup per row, 16-byte loads.
@@ -453,7 +500,7 @@ reduce_cols_q8_split_kernel(const int8_t* __restrict__ x, float* __restrict__ y,
   int acc[16];
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = 0;
-  if (cv < iv) {
+  if (cv < iv && s < S) {
     const int8_t* col = x + o * len * inner + cv * 16;
     for (int64_t k = s; k < len; k += S) {
       const uintx4 v = *reinterpret_cast<const uintx4*>(col + k * inner);
@@ -464,7 +511,8 @@ reduce_cols_q8_split_kernel(const int8_t* __restrict__ x, float* __restrict__ y,
   }
   const int width = cl * 16;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) part[s * width + c * 16 + e] = acc[e];
+  for (int e = 0; e < 16; ++e)
+    if (s < S) part[s * width + c * 16 + e] = acc[e];
   __syncthreads();
   for (int j = threadIdx.x; j < width; j += kThreads) {
     const int64_t col = blockIdx.x * (int64_t)width + j;
@@ -868,10 +916,13 @@ hipError_t launch_pool2d(const PoolParams& p_in, hipStream_t stream) {
     else { if (p.is_max) { POOL_LAUNCH(true, 0, 0); } else { POOL_LAUNCH(false, 0, 0); } }
 #undef POOL_LAUNCH
   } else {
-    const int64_t total = (int64_t)p.N * p.Ho * p.Wo * p.C;
-    const int grid = grid_for(total, kThreads);
-    if (p.is_max) { FLOAT_DISPATCH(p.dt, hipLaunchKernelGGL((pool2d_scalar_kernel<T, true>), dim3(grid), dim3(kThreads), 0, stream, p)); }
-    else { FLOAT_DISPATCH(p.dt, hipLaunchKernelGGL((pool2d_scalar_kernel<T, false>), dim3(grid), dim3(kThreads), 0, stream, p)); }
+    const int64_t per_image = (int64_t)p.Ho * p.Wo * p.C;
+    if (per_image >= (1ll << 31)) return hipErrorInvalidValue;
+    div_magic(p.Wo * p.C, &p.row_magic, &p.row_shift);
+    div_magic(p.C, &p.cv_magic, &p.cv_shift);
+    const dim3 grid((unsigned)((per_image + kThreads - 1) / kThreads), (unsigned)(p.N < 65535 ? p.N : 65535));
+    if (p.is_max) { FLOAT_DISPATCH(p.dt, hipLaunchKernelGGL((pool2d_scalar_kernel<T, true>), grid, dim3(kThreads), 0, stream, p)); }
+    else { FLOAT_DISPATCH(p.dt, hipLaunchKernelGGL((pool2d_scalar_kernel<T, false>), grid, dim3(kThreads), 0, stream, p)); }
   }
   return hipGetLastError();
 }
@@ -879,11 +930,8 @@ hipError_t launch_pool2d(const PoolParams& p_in, hipStream_t stream) {
 // Below this many column threads (half the chip's resident threads at 512 per
 // CU) the reductions split the reduced axis over the workgroup as well.
 static constexpr int64_t kSplitBelow = 256 * 512;
-static int split_columns(int64_t groups) {
-  int cl = 64;
-  while (cl > 1 && cl > groups) cl >>= 1;
-  return cl;
-}
+// 16-byte column groups of a workgroup (threads beyond a whole number of rows idle)
+static int split_columns(int64_t groups) { return groups < 64 ? (int)groups : 64; }
 
 hipError_t launch_reduce_q8_mean(const void* x, float* y, int64_t outer, int64_t len, int64_t inner,
                                  float scale, int zp, hipStream_t stream) {
@@ -899,9 +947,29 @@ hipError_t launch_reduce_q8_mean(const void* x, float* y, int64_t outer, int64_t
   return hipGetLastError();
 }
 
+// Slices of the reduced axis that column reductions take: enough for two workgroups per compute
+// unit where the columns alone leave them idle, none shorter than 64 rows or 32 KiB.
+int reduce_slices(DType dt, int64_t outer, int64_t len, int64_t inner) {
+  if (inner <= 1 || outer > 65535) return 1;
+  const int64_t V = 16 / dtype_size(dt);
+  int64_t wgs;
+  if (inner % V == 0) {
+    const int cl = split_columns(inner / V);
+    if (outer * (inner / V) >= kSplitBelow) return 1;
+    wgs = outer * ((inner / V + cl - 1) / cl);
+  } else {
+    wgs = outer * ((inner + 255) / 256);
+  }
+  int64_t n = 512 / wgs;
+  const int64_t most = std::min(len / 64, len * inner * dtype_size(dt) / 32768);
+  if (n > most) n = most;
+  return n < 2 ? 1 : (int)n;
+}
+
 template <typename TI>
 static hipError_t reduce_out(const void* x, void* y, DType out_dt, int64_t outer, int64_t len,
-                             int64_t inner, ReduceKind kind, float eps, hipStream_t stream) {
+                             int64_t inner, ReduceKind kind, float eps, float* ws, hipStream_t stream) {
+  const int slices = ws != nullptr ? reduce_slices(Store<TI>::dt, outer, len, inner) : 1;
   auto go = [&](auto tag, auto rule) -> hipError_t {
     using TO = decltype(tag);
     constexpr int A = decltype(rule)::value;
@@ -912,13 +980,14 @@ static hipError_t reduce_out(const void* x, void* y, DType out_dt, int64_t outer
     } else if (inner > 1 && inner % V == 0 && al16(x) && outer * (inner / V) < kSplitBelow && len >= 32 &&
                outer <= 65535) {
       const int cl = split_columns(inner / V);
-      const dim3 grid((unsigned)((inner / V + cl - 1) / cl), (unsigned)outer);
-      if (len >= 1024)
+      const dim3 grid((unsigned)((inner / V + cl - 1) / cl), (unsigned)outer, (unsigned)slices);
+      float* part = slices > 1 ? ws : nullptr;
+      if (len / slices >= 1024)
         hipLaunchKernelGGL((reduce_cols_split_kernel<TI, TO, A, 1024>), grid, dim3(1024), 0, stream,
-                           (const TI*)x, (TO*)y, len, inner, cl, kind, eps);
+                           (const TI*)x, (TO*)y, part, len, inner, cl, kind, eps);
       else
         hipLaunchKernelGGL((reduce_cols_split_kernel<TI, TO, A, kThreads>), grid, dim3(kThreads), 0, stream,
-                           (const TI*)x, (TO*)y, len, inner, cl, kind, eps);
+                           (const TI*)x, (TO*)y, part, len, inner, cl, kind, eps);
     } else if (inner == 1) {
       const int grid = grid_for(outer * 64, kThreads);
       hipLaunchKernelGGL((reduce_rows_kernel<TI, TO, A>), dim3(grid), dim3(kThreads), 0, stream,
@@ -927,10 +996,20 @@ static hipError_t reduce_out(const void* x, void* y, DType out_dt, int64_t outer
       const int grid = grid_for(outer * (inner / (16 / (int)sizeof(TI))), kThreads);
       hipLaunchKernelGGL((reduce_cols_vec_kernel<TI, TO, A>), dim3(grid), dim3(kThreads), 0, stream,
                          (const TI*)x, (TO*)y, outer, len, inner, kind, eps);
+    } else if (outer <= 65535 && len >= 8) {
+      const dim3 grid((unsigned)((inner + kThreads - 1) / kThreads), (unsigned)outer, (unsigned)slices);
+      hipLaunchKernelGGL((reduce_cols_flat_kernel<TI, TO, A, kThreads>), grid, dim3(kThreads), 0, stream,
+                         (const TI*)x, (TO*)y, slices > 1 ? ws : nullptr, len, inner, len, kind, eps);
     } else {
       const int grid = grid_for(outer * inner, kThreads);
       hipLaunchKernelGGL((reduce_cols_kernel<TI, TO, A>), dim3(grid), dim3(kThreads), 0, stream,
                          (const TI*)x, (TO*)y, outer, len, inner, kind, eps);
+    }
+    if (slices > 1) {   // the slices' partial results meet (magnitudes and squares are sums by now)
+      constexpr int A2 = A == ACC_ABS || A == ACC_SQ ? (int)ACC_SUM : A;
+      const dim3 grid((unsigned)((inner + kThreads - 1) / kThreads), (unsigned)outer);
+      hipLaunchKernelGGL((reduce_cols_flat_kernel<float, TO, A2, kThreads>), grid, dim3(kThreads), 0, stream, (const float*)ws,
+                         (TO*)y, (float*)nullptr, (int64_t)slices, inner, len, kind, eps);
     }
     return hipGetLastError();
   };
@@ -951,12 +1030,12 @@ static hipError_t reduce_out(const void* x, void* y, DType out_dt, int64_t outer
 }
 
 hipError_t launch_reduce(const void* x, void* y, DType in_dt, DType out_dt, int64_t outer,
-                         int64_t len, int64_t inner, ReduceKind kind, hipStream_t stream, float eps) {
+                         int64_t len, int64_t inner, ReduceKind kind, hipStream_t stream, float eps, float* ws) {
   if (!x || !y || outer <= 0 || len <= 0 || inner <= 0) return hipErrorInvalidValue;
   switch (in_dt) {
-    case DT_F32: return reduce_out<float>(x, y, out_dt, outer, len, inner, kind, eps, stream);
-    case DT_F16: return reduce_out<f16_t>(x, y, out_dt, outer, len, inner, kind, eps, stream);
-    case DT_BF16: return reduce_out<bf16_t>(x, y, out_dt, outer, len, inner, kind, eps, stream);
+    case DT_F32: return reduce_out<float>(x, y, out_dt, outer, len, inner, kind, eps, ws, stream);
+    case DT_F16: return reduce_out<f16_t>(x, y, out_dt, outer, len, inner, kind, eps, ws, stream);
+    case DT_BF16: return reduce_out<bf16_t>(x, y, out_dt, outer, len, inner, kind, eps, ws, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -154,7 +154,8 @@ class Planner {
     plan_->tensors.push_back(t);
     return (int)plan_->tensors.size() - 1;
   }
-  std::unordered_set<int> arena_only_;   // root tensors that some step writes, or reads relying on the arena
+  // by root tensor: some launch relies on the arena for it; needs a 16-byte aligned base; reads it; writes it
+  std::unordered_set<int> arena_only_, aligned_only_, read_, written_;
   // The 8-bit convolution steps, kept so that a plain 1x1 layer over the result of one can ride in
   // its launch (lower_conv; igemm_stream_q8_fusable decides).
   struct FuseProducer {
@@ -185,16 +186,21 @@ class Planner {
   };
   Ref ref(int t) const { return Ref{plan_, t}; }
 
-  // exact_reader: the launch reads exactly the elements of its sources and tests their alignment
-  // itself (the layout conversions launch_nchw_to_nhwc / launch_nchw_to_s2d do), so a source that
-  // is an argument's staging tensor may be the caller's own device buffer.  Every other reader
-  // may rely on the arena (256-byte bases, slack behind a tensor) and pins its sources to it.
+  // What a launch demands of the buffers it reads and writes, beside their elements.  Every launch
+  // may rely on the arena (256-byte bases, slack behind a tensor) unless it says otherwise:
+  //   kReadsAny     it reads exactly the elements of its sources, at any alignment (the layout
+  //                 conversions launch_nchw_to_nhwc / launch_nchw_to_s2d test it themselves)
+  //   kReads16      the same from 16-byte aligned bases
+  //   kWrites16     it writes exactly the elements of its results, at 16-byte aligned bases
+  // A source that is an argument's staging tensor may then be the caller's own device buffer, and
+  // so may a result that no launch reads.
+  enum : unsigned { kReadsAny = 1, kReads16 = 2, kWrites16 = 4 };
   void emit(const std::string& name, std::initializer_list<int> reads, std::initializer_list<int> writes,
-            std::function<hipError_t(const ExecEnv&, hipStream_t)> fn, bool exact_reader = false) {
-    emit_lists(name, std::vector<int>(reads), std::vector<int>(writes), std::move(fn), exact_reader);
+            std::function<hipError_t(const ExecEnv&, hipStream_t)> fn, unsigned exact = 0) {
+    emit_lists(name, std::vector<int>(reads), std::vector<int>(writes), std::move(fn), exact);
   }
   void emit_lists(const std::string& name, const std::vector<int>& reads, const std::vector<int>& writes,
-                  std::function<hipError_t(const ExecEnv&, hipStream_t)> fn, bool exact_reader = false) {
+                  std::function<hipError_t(const ExecEnv&, hipStream_t)> fn, unsigned exact = 0) {
     if (in_init_) {
       plan_->init_steps.push_back({name, std::move(fn)});
       return;
@@ -209,8 +215,17 @@ class Planner {
     };
     for (int t : reads) touch(t);
     for (int t : writes) touch(t);
-    for (int t : reads) if (t >= 0 && !exact_reader) arena_only_.insert(root(t));
-    for (int t : writes) if (t >= 0) arena_only_.insert(root(t));
+    for (int t : reads) {
+      if (t < 0) continue;
+      read_.insert(root(t));
+      if (!(exact & (kReadsAny | kReads16))) arena_only_.insert(root(t));
+      if (!(exact & kReadsAny)) aligned_only_.insert(root(t));
+    }
+    for (int t : writes) {
+      if (t < 0) continue;
+      written_.insert(root(t));
+      if (!(exact & kWrites16)) arena_only_.insert(root(t));
+    }
     plan_->steps.push_back({name, std::move(fn)});
   }
 
@@ -431,7 +446,7 @@ class Planner {
         emit("to_nhwc:" + v->name, {from}, {dst}, [=](const ExecEnv& e, hipStream_t st) {
           LayoutParams p = lp; p.src = a(e); p.dst = b(e);
           return launch_nchw_to_nhwc(p, st);
-        }, /*exact_reader=*/true);
+        }, kReadsAny);
         return dst;
       } else {
         lp.cs = s2.cs;
@@ -472,7 +487,7 @@ class Planner {
       });
     } else if (src.dt != fdt) {
       const DType sdt = src.dt, ddt = fdt;
-      emit("cast:" + v->name, {have}, {dst}, [=](const ExecEnv& e, hipStream_t st) { return launch_cast(a(e), sdt, b(e), ddt, n, st); });
+      emit("cast:" + v->name, {have}, {dst}, [=](const ExecEnv& e, hipStream_t st) { return launch_cast(a(e), sdt, b(e), ddt, n, st); }, kReads16 | kWrites16);
     } else {
       fail(ODLA_INTERNAL_LOGIC_ERR, "no conversion needed for '%s'", v->name.c_str());
     }
@@ -528,6 +543,68 @@ class Planner {
     return s.main >= 0 && T(s.main).quant;
   }
   int use_count(const _odla_value* v) const { return (int)consumers_[v->index].size() + (v->is_output ? 1 : 0); }
+  // Does the rank-4 value reach, through element-wise operators of its own shape, an operator that
+  // works on channels-last tensors?  Its producer then changes the layout while it reads (the
+  // conversion of an argument's type is part of that), instead of every later reader for itself.
+  bool feeds_channels_last(const _odla_value* v, int depth = 0) const {
+    if (calib_ || comp_->opts.int8 || v == nullptr || v->shape.rank != 4 || depth > 8 || dtype_from_odla(v->etype) != DT_F32) return false;
+    for (int ci : consumers_[v->index]) {
+      const Node& c = comp_->nodes[ci];
+      // (a convolution wants whole 16-byte vectors of channels: it makes its padded copy from the row-major tensor)
+      if (c.op == OP_POOL || (c.op == OP_CONV && v->shape.d[1] % 8 == 0)) { if (c.in[0] == v && c.i[0] != ODLA_CHANNELS_LAST) return true; }
+      else if (c.op == OP_RESIZE) return true;
+      else if ((c.op == OP_UNARY || c.op == OP_BINARY || c.op == OP_BATCHNORM) && c.out->shape == v->shape && c.in[0] == v) {
+        if (c.op == OP_BATCHNORM && c.i[0] == ODLA_CHANNELS_LAST) continue;
+        if (feeds_channels_last(c.out, depth + 1)) return true;
+      }
+    }
+    return false;
+  }
+  // Where the channels-last result `v` belongs if its only reader is a Concat along the channels: a
+  // channel slice of the Concat's result (its pixels have that tensor's pitch), or -1.
+  std::unordered_map<int, int> concat_dst_;   // Concat node -> its result, made by the first part that is stored there
+  int concat_slice(const _odla_value* v, DType dt) {
+    if (calib_ || comp_->opts.int8 || v->is_output || v->shape.rank != 4 || consumers_[v->index].size() != 1) return -1;
+    const int ci = consumers_[v->index][0];
+    const Node& c = comp_->nodes[ci];
+    if (c.op != OP_CONCAT || c.absorbed || c.i[0] != 1 || c.out->shape.rank != 4 || storage_dtype(c.out) != dt || storage_dtype(v) != dt) return -1;
+    int64_t off = 0;
+    for (const _odla_value* part : c.in) {
+      if (part == v) break;
+      off += part->shape.d[1];
+    }
+    auto it = concat_dst_.find(ci);
+    if (it == concat_dst_.end())
+      it = concat_dst_.emplace(ci, new_tensor(dt, L_NHWC, c.out->shape, (int)c.out->shape.d[1], SP_ARENA)).first;
+    PTensor t = T(it->second);
+    t.shape = v->shape;
+    t.alias_of = root(it->second);
+    t.alias_off = T(it->second).alias_off + (size_t)off * dtype_size(dt);
+    plan_->tensors.push_back(t);
+    return (int)plan_->tensors.size() - 1;
+  }
+  // A channels-last result: its Concat slice, or a tensor of its own.
+  int channels_last_result(const _odla_value* v, DType dt) {
+    const int s = concat_slice(v, dt);
+    return s >= 0 ? s : new_tensor(dt, L_NHWC, v->shape, (int)v->shape.d[1], SP_ARENA);
+  }
+  // The activation behind `v` that the launch which makes it can apply (cheap ones; `v` has no other
+  // reader): marks it as done and moves *v to its result.
+  void take_activation(_odla_value** v, ActKind* act, float* fa, float* fb) {
+    if (calib_ || (*v)->is_output || consumers_[(*v)->index].size() != 1) return;
+    Node& nx = comp_->nodes[consumers_[(*v)->index][0]];
+    if (nx.op != OP_UNARY || nx.absorbed) return;
+    const ActKind k = (ActKind)nx.i[0];
+    if (k != ACT_RELU && k != ACT_LEAKY && k != ACT_CLAMP && k != ACT_SIGMOID && k != ACT_TANH) return;
+    *act = k; *fa = nx.f[0]; *fb = nx.f[1];
+    nx.absorbed = true;
+    *v = nx.out;
+  }
+  // Scratch tensor of a column reduction that is split over its axis, or -1.
+  int reduce_scratch(DType dt, int64_t outer, int64_t len, int64_t inner) {
+    const int n = reduce_slices(dt, outer, len, inner);
+    return n > 1 ? raw_buffer((size_t)(outer * n * inner) * sizeof(float), SP_ARENA) : -1;
+  }
   bool available(const _odla_value* v) const {
     return v->kind != _odla_value::TEMP || vs_[v->index].main >= 0;
   }
@@ -754,14 +831,34 @@ void Planner::run() {
   // Outputs: row-major, declared element type.
   for (_odla_value* ov : comp_->outputs) {
     const DType want = dtype_from_odla(ov->etype);
-    int t = get(ov, L_ROWMAJOR, FORM_FLOAT);
+    const VState& os = vs_[ov->index];
+    int t = -1;
     bool converted = false;
+    // a channels-last result leaves in one launch that changes layout and type together
+    if (!calib_ && dtype_is_float(want) && ov->shape.rank == 4 && os.main >= 0 && T(os.main).layout == L_NHWC &&
+        dtype_is_float(T(os.main).dt) && !T(os.main).quant && os.slot[L_ROWMAJOR][FORM_FLOAT] < 0 && storage_dtype(ov) == T(os.main).dt) {
+      const int src = os.main;
+      LayoutParams lp;
+      lp.N = (int)ov->shape.d[0]; lp.C = (int)ov->shape.d[1]; lp.HW = (int)(ov->shape.d[2] * ov->shape.d[3]);
+      lp.cs = T(src).cs;
+      lp.src_dt = T(src).dt;
+      lp.dst_dt = want;
+      t = new_tensor(want, L_ROWMAJOR, ov->shape, 0, SP_ARENA);
+      const Ref a = ref(src), b = ref(t);
+      emit("to_nchw:" + ov->name, {src}, {t}, [=](const ExecEnv& e, hipStream_t st) {
+        LayoutParams p = lp; p.src = a(e); p.dst = b(e);
+        return launch_nhwc_to_nchw(p, st);
+      }, kWrites16);
+      converted = true;
+    } else {
+      t = get(ov, L_ROWMAJOR, FORM_FLOAT);
+    }
     if (T(t).dt != want) {
       const int dst = new_tensor(want, L_ROWMAJOR, ov->shape, 0, SP_ARENA);
       const int64_t n = ov->shape.numel();
       const DType sdt = T(t).dt;
       const Ref a = ref(t), b = ref(dst);
-      emit("out.cast:" + ov->name, {t}, {dst}, [=](const ExecEnv& e, hipStream_t st) { return launch_cast(a(e), sdt, b(e), want, n, st); });
+      emit("out.cast:" + ov->name, {t}, {dst}, [=](const ExecEnv& e, hipStream_t st) { return launch_cast(a(e), sdt, b(e), want, n, st); }, kWrites16);
       t = dst;
       converted = true;
     }
@@ -772,24 +869,32 @@ void Planner::run() {
     io.tensor = root(t);
     io.offset = T(t).alias_off;
     io.bytes = (size_t)ov->shape.numel() * dtype_size(want);
-    // The conversion to the declared type is the only step that touches its result, and it
-    // writes exactly the result's elements: it can write the caller's device buffer directly.
-    if (converted && !calib_ && io.tensor == t && io.offset == 0) {
-      io.in_place_ok = true;
-      T(t).ext_slot = (int)(plan_->inputs.size() + plan_->outputs.size());
-    }
     plan_->outputs.push_back(io);
   }
-  // Arguments whose staging tensor only layout conversions read: the conversion can read the
-  // caller's device buffer, and the copy into the arena is skipped.
+  // Results that launches write exactly and none reads can be written in the caller's device
+  // buffer directly (a tensor behind two outputs, or one that is also an argument, stays here).
+  for (size_t k = 0; k < plan_->outputs.size(); ++k) {
+    Plan::IO& io = plan_->outputs[k];
+    bool ok = !calib_ && io.offset == 0 && T(io.tensor).space == SP_ARENA && T(io.tensor).bytes == io.bytes &&
+              written_.count(io.tensor) && !read_.count(io.tensor) && !arena_only_.count(io.tensor);
+    for (size_t j = 0; j < plan_->outputs.size(); ++j) ok = ok && (j == k || plan_->outputs[j].tensor != io.tensor);
+    for (const Plan::IO& in : plan_->inputs) ok = ok && root(in.tensor) != io.tensor;
+    if (ok) {
+      io.in_place_ok = true;
+      T(io.tensor).ext_slot = (int)(plan_->inputs.size() + k);
+    }
+  }
+  // Arguments whose staging tensor launches read exactly: they can read the caller's device
+  // buffer, and the copy into the arena is skipped.
   for (size_t k = 0; k < plan_->inputs.size(); ++k) {
     Plan::IO& io = plan_->inputs[k];
     const int r = root(io.tensor);
-    bool ok = !calib_ && r == io.tensor && T(r).space == SP_ARENA && T(r).last_step >= 0 && !arena_only_.count(r);
+    bool ok = !calib_ && r == io.tensor && T(r).space == SP_ARENA && T(r).last_step >= 0 && !arena_only_.count(r) && !written_.count(r);
     for (const Plan::IO& o : plan_->outputs) ok = ok && root(o.tensor) != r;
     for (const auto& ft : plan_->final_tensor) ok = ok && root(ft.second) != r;
     if (ok) {
       io.in_place_ok = true;
+      io.align16 = aligned_only_.count(r) != 0;
       T(r).ext_slot = (int)k;
     }
   }
@@ -1537,7 +1642,8 @@ void Planner::lower_conv(int ni) {
 
   int ty;
   if (cl) ty = new_tensor(odt, L_ROWMAJOR, outv->shape, 0, SP_ARENA);
-  else ty = new_tensor(odt, L_NHWC, outv->shape, (int)O, SP_ARENA);
+  else ty = channels_last_result(outv, odt);
+  if (!cl) ip.ycs = T(ty).cs;
 
   if (runtime_bias) {
     // bias supplied at run time: read it as fp32 from its staging tensor
@@ -2163,6 +2269,7 @@ void Planner::lower_binary(int ni) {
       return v->shape == os && s.main >= 0 && T(s.main).layout == L_NHWC;
     };
     if (nhwc_main(a) || nhwc_main(b)) lay = L_NHWC;
+    else if (a->shape == os && b->shape == os && feeds_channels_last(outv)) lay = L_NHWC;
   }
   auto operand = [&](const _odla_value* v, const Shape& aligned) -> int {
     // full-shape rank-4 operands follow the output layout; broadcast operands stay row-major
@@ -2172,6 +2279,26 @@ void Planner::lower_binary(int ni) {
   };
   int ta = operand(a, sa), tb = operand(b, sb);
   int ocs = 0;
+  if (lay == L_NHWC && a->shape == os && b->shape == os && T(ta).dt == dt && T(tb).dt == dt && os.numel() < (1ll << 31)) {
+    // pixels of any pitch, into the slice of a Concat where the result has one
+    const int slice = concat_slice(outv, dt);
+    if (slice >= 0 || T(ta).cs != os.d[1] || T(tb).cs != os.d[1]) {
+      const int ty = slice >= 0 ? slice : new_tensor(dt, L_NHWC, os, (int)os.d[1], SP_ARENA);
+      ChannelRowsParams rp;
+      rp.dt = dt;
+      rp.rows = os.d[0] * os.d[2] * os.d[3];
+      rp.C = (int)os.d[1]; rp.xcs = T(ta).cs; rp.rcs = T(tb).cs; rp.ycs = T(ty).cs;
+      rp.op = (BinKind)n.i[0];
+      rp.act = act; rp.act_a = act_a; rp.act_b = act_b;
+      const Ref ra = ref(ta), rb = ref(tb), ry = ref(ty);
+      emit("binary:" + outv->name, {ta, tb}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
+        ChannelRowsParams p = rp; p.x = ra(e); p.r = rb(e); p.y = ry(e);
+        return launch_channel_rows(p, st);
+      });
+      set_main(outv, ty);
+      return;
+    }
+  }
   if (lay == L_NHWC) {
     ocs = (int)os.d[1];
     if ((a->shape == os && T(ta).cs != ocs) || (b->shape == os && T(tb).cs != ocs)) {
@@ -2250,7 +2377,7 @@ void Planner::lower_binary(int ni) {
   emit("binary:" + outv->name, {ta, tb}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
     BinaryParams p = bp; p.a = ra(e); p.b = rb(e); p.y = ry(e);
     return launch_binary(p, st);
-  });
+  }, kReads16 | kWrites16);
   set_main(outv, ty);
 }
 
@@ -2335,16 +2462,31 @@ void Planner::lower_unary(int ni) {
   if (s.main >= 0 && !T(s.main).quant) lay = T(s.main).layout;
   else if (x->shape.rank == 4 && s.slot[L_NHWC][FORM_FLOAT] >= 0) lay = L_NHWC;
   else if (s.main >= 0 && T(s.main).quant) lay = T(s.main).layout;
+  if (lay == L_ROWMAJOR && x->shape.rank == 4 && feeds_channels_last(n.out)) lay = L_NHWC;
   const int tx = get(x, lay, FORM_FLOAT);
   const PTensor px = T(tx);
-  const int ty = new_tensor(px.dt, px.layout, n.out->shape, px.cs, SP_ARENA);
+  const int slice = px.layout == L_NHWC && !px.quant ? concat_slice(n.out, px.dt) : -1;
+  const int ty = slice >= 0 ? slice : new_tensor(px.dt, px.layout, n.out->shape, px.cs, SP_ARENA);
   const int64_t ne = px.phys_elems();
   const float fa = n.f[0], fb = n.f[1];
   const DType dt = px.dt;
   const Ref a = ref(tx), b = ref(ty);
+  if (slice >= 0) {
+    ChannelRowsParams rp;
+    rp.dt = dt;
+    rp.rows = x->shape.d[0] * x->shape.d[2] * x->shape.d[3];
+    rp.C = (int)x->shape.d[1]; rp.xcs = px.cs; rp.ycs = T(ty).cs;
+    rp.act = act; rp.act_a = fa; rp.act_b = fb;
+    emit("unary:" + n.out->name, {tx}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
+      ChannelRowsParams p = rp; p.x = a(e); p.y = b(e);
+      return launch_channel_rows(p, st);
+    });
+    set_main(n.out, ty);
+    return;
+  }
   emit(std::string("unary:") + n.out->name, {tx}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
     return launch_unary(a(e), b(e), dt, ne, act, fa, fb, st);
-  });
+  }, kReads16 | kWrites16);
   set_main(n.out, ty);
 }
 
@@ -2769,9 +2911,9 @@ void Planner::lower_batchnorm(int ni) {
   const VState& s = vs_[x->index];
   Layout lay = L_ROWMAJOR;
   if (cf && xs.rank == 4 && s.main >= 0 && T(s.main).layout == L_NHWC) lay = L_NHWC;
+  if (cf && lay == L_ROWMAJOR && feeds_channels_last(n.out)) lay = L_NHWC;
   const int tx = get(x, lay, FORM_FLOAT);
   const PTensor px = T(tx);
-  const int ty = new_tensor(px.dt, px.layout, n.out->shape, px.cs, SP_ARENA);
   int64_t inner;
   int channels;
   if (lay == L_NHWC) { inner = 1; channels = px.cs; }
@@ -2821,6 +2963,26 @@ void Planner::lower_batchnorm(int ni) {
   }
   const int64_t ne = px.phys_elems();
   const DType dt = px.dt;
+  if (inner == 1 && ne < (1ll << 31)) {
+    // channel innermost: the launch takes the activation behind it along
+    _odla_value* outv = n.out;
+    ChannelRowsParams rp;
+    take_activation(&outv, &rp.act, &rp.act_a, &rp.act_b);
+    const bool dense = lay == L_NHWC && px.cs == (int)C;
+    const int ty = dense ? channels_last_result(outv, dt) : new_tensor(dt, px.layout, outv->shape, px.cs, SP_ARENA);
+    rp.dt = dt;
+    rp.rows = ne / channels;
+    rp.C = channels; rp.xcs = channels;
+    rp.ycs = dense ? T(ty).cs : channels;
+    const Ref a = ref(tx), b = ref(ty), rs = ref(tscale), rt = ref(tshift);
+    emit("bn:" + outv->name, {tx, tscale, tshift}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
+      ChannelRowsParams p = rp; p.x = a(e); p.y = b(e); p.scale = (const float*)rs(e); p.shift = (const float*)rt(e);
+      return launch_channel_rows(p, st);
+    });
+    set_main(outv, ty);
+    return;
+  }
+  const int ty = new_tensor(dt, px.layout, n.out->shape, px.cs, SP_ARENA);
   const Ref a = ref(tx), b = ref(ty), rs = ref(tscale), rt = ref(tshift);
   emit("bn:" + n.out->name, {tx, tscale, tshift}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
     return launch_channel_affine(a(e), b(e), dt, ne, inner, channels, (const float*)rs(e), (const float*)rt(e), st);
@@ -2863,7 +3025,7 @@ void Planner::lower_layernorm(int ni) {
   emit("layernorm:" + n.out->name, {tx}, {ty, t2}, [=](const ExecEnv& e, hipStream_t st) {
     return launch_layernorm(a(e), b(e), dt, rows, len, hg ? (const float*)rg(e) : nullptr,
                             hb ? (const float*)rb(e) : nullptr, eps, st, dual ? b2(e) : nullptr, dt2);
-  });
+  }, kWrites16);
   set_main(n.out, ty);
   if (dual) vs_[n.out->index].slot[L_ROWMAJOR][FORM_OPERAND] = t2;
 }
@@ -2899,7 +3061,8 @@ void Planner::lower_pool(int ni) {
   pp.count_include_pad = n.i[10] != 0;
   int ty;
   if (cl) ty = new_tensor(px.dt, L_ROWMAJOR, os, 0, SP_ARENA);
-  else ty = new_tensor(px.dt, L_NHWC, os, pp.C, SP_ARENA);
+  else ty = q8 ? new_tensor(px.dt, L_NHWC, os, pp.C, SP_ARENA) : channels_last_result(n.out, px.dt);
+  if (!cl) pp.ycs = T(ty).cs;
   if (q8) set_quant(ty, true, px.qscale, px.qzp);
   const Ref a = ref(tx), b = ref(ty);
   emit(std::string(is_max ? "maxpool:" : "avgpool:") + n.out->name, {tx}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
@@ -2951,9 +3114,12 @@ void Planner::lower_reduce(int ni) {
       ty = new_tensor(px.dt, L_ROWMAJOR, n.out->shape, 0, SP_ARENA);
       const Ref b = ref(ty);
       const DType dt = px.dt;
-      emit("reduce:" + n.out->name, {s.main}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
-        return launch_reduce(a(e), b(e), dt, dt, outer, len, inner, kind, st, eps);
-      });
+      const int tws = reduce_scratch(dt, outer, len, inner);
+      const bool hw = tws >= 0;
+      const Ref w = ref(hw ? tws : ty);
+      emit("reduce:" + n.out->name, {s.main}, {ty, tws}, [=](const ExecEnv& e, hipStream_t st) {
+        return launch_reduce(a(e), b(e), dt, dt, outer, len, inner, kind, st, eps, hw ? (float*)w(e) : nullptr);
+      }, kWrites16);
     }
     set_main(n.out, ty);
     return;
@@ -3004,10 +3170,12 @@ void Planner::lower_reduce(int ni) {
     outer = xs.numel() / len;
   }
   const int ty = new_tensor(dt, L_ROWMAJOR, n.out->shape, 0, SP_ARENA);
-  const Ref a = ref(tx), b = ref(ty);
-  emit("reduce:" + n.out->name, {tx}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
-    return launch_reduce(a(e), b(e), dt, dt, outer, len, inner, kind, st, eps);
-  });
+  const int tws = reduce_scratch(dt, outer, len, inner);
+  const bool hw = tws >= 0;
+  const Ref a = ref(tx), b = ref(ty), w = ref(hw ? tws : ty);
+  emit("reduce:" + n.out->name, {tx}, {ty, tws}, [=](const ExecEnv& e, hipStream_t st) {
+    return launch_reduce(a(e), b(e), dt, dt, outer, len, inner, kind, st, eps, hw ? (float*)w(e) : nullptr);
+  }, kWrites16);
   set_main(n.out, ty);
 }
 
@@ -3065,7 +3233,7 @@ void Planner::lower_softmax(int ni) {
   const bool has_add = tadd >= 0;
   emit("softmax:" + n.out->name, {tx, tadd}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
     return launch_softmax(a(e), b(e), dt, odt, outer, len, inner, logsm, st, has_add ? m(e) : nullptr, add_div);
-  });
+  }, kWrites16);
   set_main(n.out, ty);
 }
 
@@ -3107,10 +3275,12 @@ void Planner::lower_concat(int ni) {
   for (_odla_value* v : n.in) tin.push_back(get(v, lay, FORM_FLOAT));
   const DType dt = T(tin[0]).dt;
   const int es = dtype_size(dt);
-  const int ty = new_tensor(dt, lay, os, nhwc ? (int)os.d[1] : 0, SP_ARENA);
+  const auto placed = concat_dst_.find(ni);   // (some parts are stored in the result already)
+  const int ty = placed != concat_dst_.end() ? placed->second : new_tensor(dt, lay, os, nhwc ? (int)os.d[1] : 0, SP_ARENA);
   int64_t off = 0;
   for (size_t k = 0; k < n.in.size(); ++k) {
     const PTensor pi = T(tin[k]);
+    if (root(tin[k]) == root(ty)) { off += n.in[k]->shape.d[1]; continue; }
     if (pi.dt != dt) fail(ODLA_UNSUPPORTED_DATATYPE, "odla_Concat of mixed storage types");
     const Shape& is = n.in[k]->shape;
     StridedCopyParams cp;
@@ -3265,11 +3435,14 @@ void Planner::lower_resize(int ni) {
   const PTensor px = T(tx);
   const Shape& xs = x->shape;
   const Shape& os = n.out->shape;
-  const int ty = new_tensor(px.dt, L_NHWC, os, px.cs, SP_ARENA);
+  const bool linear = n.i[0] == ODLA_LINEAR;
+  const int slice = linear || px.quant ? -1 : concat_slice(n.out, px.dt);
+  const int ty = slice >= 0 ? slice : new_tensor(px.dt, L_NHWC, os, px.cs, SP_ARENA);
   const int es = dtype_size(px.dt);
   const int N = (int)xs.d[0], H = (int)xs.d[2], W = (int)xs.d[3], cs = px.cs, Ho = (int)os.d[2], Wo = (int)os.d[3];
+  const int ycs = T(ty).cs, C = slice >= 0 ? (int)xs.d[1] : cs;
   const Ref a = ref(tx), b = ref(ty);
-  if (n.i[0] == ODLA_LINEAR) {
+  if (linear) {
     const DType dt = px.dt;
     if (!dtype_is_float(dt)) fail(ODLA_UNSUPPORTED_DATATYPE, "linear odla_Resize of a non-float value ('%s')", n.out->name.c_str());
     emit("resize.linear:" + n.out->name, {tx}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
@@ -3277,7 +3450,7 @@ void Planner::lower_resize(int ni) {
     });
   } else {
     emit("resize:" + n.out->name, {tx}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
-      return launch_resize_nearest_nhwc(a(e), b(e), es, N, H, W, cs, Ho, Wo, st);
+      return launch_resize_nearest_nhwc(a(e), b(e), es, N, H, W, C, cs, ycs, Ho, Wo, st);
     });
   }
   set_main(n.out, ty);
