@@ -336,37 +336,55 @@ struct BinaryParams {
 hipError_t launch_binary(const BinaryParams& p, hipStream_t stream);
 
 // A connected group of float unary / binary operators run as one launch.
-// Every thread evaluates the whole group for one point of the iteration space
+// Every thread evaluates the whole group for points of the iteration space
 // dims[0..3]: threads enumerate (dims[0], dims[1], pieces of dims[2], dims[3])
 // with dims[3] fastest and walk their piece of dims[2] themselves, so that the
 // planner can give stores a unit stride across threads and loads a unit stride
 // along a thread's walk.
 // The group is a short program over per-thread registers: loads and stores go
-// through views (base pointer, element offset, one element stride per dim; a
-// stride of 0 broadcasts), all of storage type `dt`; arithmetic is fp32.
+// through views (element offset, one element stride per dim; a stride of 0
+// broadcasts), all of storage type `dt`; arithmetic is fp32.  Its sections: the
+// first n_once_loads loads do not depend on dims[2] and run once per walk; the
+// next n_loads instructions are loads as well; the next n_once do not depend on
+// dims[2] either.
 enum FusedOp : int { FOP_LOAD = 0, FOP_UNARY, FOP_BINARY, FOP_STORE };
-struct FusedView {
-  const void* base = nullptr;   // stores cast the const away
-  int64_t off = 0;
-  int64_t st[4] = {0, 0, 0, 0};
-};
+struct FusedView { int64_t off = 0; int64_t st[4] = {0, 0, 0, 0}; };
 struct FusedInstr {
-  int op = FOP_LOAD;   // FusedOp
-  int dst = 0;         // register written (FOP_STORE: view index)
-  int a = 0, b = 0;    // registers read (FOP_LOAD: a = view index; FOP_BINARY: -1 = the immediate fa)
-  int kind = 0;        // ActKind / BinKind
+  uint8_t op = FOP_LOAD;      // FusedOp
+  uint8_t kind = 0;           // ActKind / BinKind
+  int8_t dst = 0;             // register written (FOP_STORE: view index)
+  int8_t a = 0, b = 0;        // registers read (FOP_LOAD: a = view index; FOP_BINARY: -1 = the immediate fa)
+  uint8_t pad[3] = {0, 0, 0};
   float fa = 0.f, fb = 0.f;   // FOP_UNARY: the activation's parameters
 };
 constexpr int kFusedMaxRegs = 32, kFusedMaxViews = 24, kFusedMaxInstr = 64;
-struct FusedParams {
-  DType dt = DT_F32;
-  int n_instr = 0;
+// One group as the kernel reads it (in device memory, the same for every execution).
+struct FusedGroup {
+  int n_instr = 0, n_once_loads = 0, n_loads = 0, n_once = 0, n_views = 0;
+  int points = 1;      // points of dims[2] a thread takes at once: 1, 2, 4 or 8 (set by fused_prepare)
   int64_t dims[4] = {1, 1, 1, 1};
   int64_t walk = 0;    // points of dims[2] per thread (0: all of them); short walks give more threads
+  unsigned magic[3] = {0, 0, 0};
+  int shift[3] = {0, 0, 0};
   FusedView view[kFusedMaxViews];
   FusedInstr prog[kFusedMaxInstr];
 };
-hipError_t launch_fused_eltwise(const FusedParams& p, hipStream_t stream);
+// Checks a group and sets `points`; *blocks: the workgroups it takes, *lds_bytes: its registers,
+// *wide: its offsets need 64 bits.
+bool fused_prepare(FusedGroup* g, int* blocks, size_t* lds_bytes, bool* wide);
+// One launch of up to kFusedMaxGroups groups that do not depend on each other.
+constexpr int kFusedMaxGroups = 8, kFusedMaxBases = 72;
+struct FusedLaunch {
+  DType dt = DT_F32;
+  int n_groups = 0;
+  bool wide = false;
+  size_t lds_bytes = 0;
+  int block0[kFusedMaxGroups + 1] = {0};   // first workgroup of a group; behind the last: the grid
+  int view0[kFusedMaxGroups + 1] = {0};    // a group's first view in base[]
+  const FusedGroup* group[kFusedMaxGroups] = {nullptr};
+  const void* base[kFusedMaxBases] = {nullptr};   // per view (stores cast the const away)
+};
+hipError_t launch_fused_eltwise(const FusedLaunch& l, hipStream_t stream);
 
 // Typed element-wise operators with broadcast (row-major operands, up to 6
 // collapsed dims, one element stride per dim and operand, 0 where it

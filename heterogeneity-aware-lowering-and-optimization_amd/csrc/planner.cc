@@ -154,8 +154,8 @@ class Planner {
     plan_->tensors.push_back(t);
     return (int)plan_->tensors.size() - 1;
   }
-  // by root tensor: some launch relies on the arena for it; needs a 16-byte aligned base; reads it; writes it
-  std::unordered_set<int> arena_only_, aligned_only_, read_, written_;
+  // by root tensor: some launch relies on the arena for it; needs a 16-byte aligned base; writes it
+  std::unordered_set<int> arena_only_, aligned_only_, written_;
   // The 8-bit convolution steps, kept so that a plain 1x1 layer over the result of one can ride in
   // its launch (lower_conv; igemm_stream_q8_fusable decides).
   struct FuseProducer {
@@ -193,7 +193,7 @@ class Planner {
   //   kReads16      the same from 16-byte aligned bases
   //   kWrites16     it writes exactly the elements of its results, at 16-byte aligned bases
   // A source that is an argument's staging tensor may then be the caller's own device buffer, and
-  // so may a result that no launch reads.
+  // so may a result (which later launches may read, if they do it exactly too).
   enum : unsigned { kReadsAny = 1, kReads16 = 2, kWrites16 = 4 };
   void emit(const std::string& name, std::initializer_list<int> reads, std::initializer_list<int> writes,
             std::function<hipError_t(const ExecEnv&, hipStream_t)> fn, unsigned exact = 0) {
@@ -205,19 +205,22 @@ class Planner {
       plan_->init_steps.push_back({name, std::move(fn)});
       return;
     }
-    const int idx = (int)plan_->steps.size();
-    auto touch = [&](int t) {
+    touch((int)plan_->steps.size(), reads, writes, exact);
+    plan_->steps.push_back({name, std::move(fn)});
+  }
+  // Step `idx` reads and writes these tensors.
+  void touch(const int idx, const std::vector<int>& reads, const std::vector<int>& writes, unsigned exact) {
+    auto use = [&](int t) {
       if (t < 0) return;
       PTensor& p = T(root(t));
       if (p.space != SP_ARENA) return;
       if (idx < p.def_step) p.def_step = idx;
       if (idx > p.last_step) p.last_step = idx;
     };
-    for (int t : reads) touch(t);
-    for (int t : writes) touch(t);
+    for (int t : reads) use(t);
+    for (int t : writes) use(t);
     for (int t : reads) {
       if (t < 0) continue;
-      read_.insert(root(t));
       if (!(exact & (kReadsAny | kReads16))) arena_only_.insert(root(t));
       if (!(exact & kReadsAny)) aligned_only_.insert(root(t));
     }
@@ -226,7 +229,6 @@ class Planner {
       written_.insert(root(t));
       if (!(exact & kWrites16)) arena_only_.insert(root(t));
     }
-    plan_->steps.push_back({name, std::move(fn)});
   }
 
   // -------------------------------------------------------------- constants
@@ -335,7 +337,7 @@ class Planner {
   int get(const _odla_value* v, Layout want, Form form = FORM_FLOAT, int cvec = 0) {
     if (form == FORM_OPERAND && (!acc_mode_ || dtype_from_odla(v->etype) != DT_F32)) form = FORM_FLOAT;
     VState& s = vs_[v->index];
-    if (s.main < 0) materialize_source(v);
+    if (s.main < 0 && !settle(v)) materialize_source(v);
     if (want == L_NHWC && v->shape.rank != 4) fail(ODLA_INTERNAL_LOGIC_ERR, "channels-last form requested for rank-%d value", v->shape.rank);
     int& slot = s.slot[want][form];
     if (slot >= 0 && (want != L_NHWC || cvec <= 1 || T(slot).cs % cvec == 0)) return slot;
@@ -583,6 +585,27 @@ class Planner {
     plan_->tensors.push_back(t);
     return (int)plan_->tensors.size() - 1;
   }
+  // Where the row-major result `v` of an element-wise group belongs if its only reader is a Concat:
+  // the Concat's result (or -1), the offset of this part in it and its strides over the dims of `v`.
+  std::unordered_set<int> placed_;   // parts (by value index) that are stored in their Concat's result
+  int concat_part(const _odla_value* v, DType dt, int64_t* off, int64_t* st) {
+    if (calib_ || comp_->opts.int8 || v->is_output || v->shape.rank > 3 || consumers_[v->index].size() != 1) return -1;
+    const int ci = consumers_[v->index][0];
+    const Node& c = comp_->nodes[ci];
+    if (c.op != OP_CONCAT || c.absorbed || c.out->shape.rank != v->shape.rank || storage_dtype(c.out) != dt) return -1;
+    for (const _odla_value* part : c.in) if (storage_dtype(part) != dt) return -1;
+    int64_t acc = 1;
+    for (int i = v->shape.rank - 1; i >= 0; --i) { st[i] = acc; acc *= c.out->shape.d[i]; }
+    *off = 0;
+    for (const _odla_value* part : c.in) {
+      if (part == v) break;
+      *off += part->shape.d[(int)c.i[0]] * st[(int)c.i[0]];
+    }
+    auto it = concat_dst_.find(ci);
+    if (it == concat_dst_.end()) it = concat_dst_.emplace(ci, new_tensor(dt, L_ROWMAJOR, c.out->shape, 0, SP_ARENA)).first;
+    placed_.insert(v->index);
+    return it->second;
+  }
   // A channels-last result: its Concat slice, or a tensor of its own.
   int channels_last_result(const _odla_value* v, DType dt) {
     const int s = concat_slice(v, dt);
@@ -606,7 +629,72 @@ class Planner {
     return n > 1 ? raw_buffer((size_t)(outer * n * inner) * sizeof(float), SP_ARENA) : -1;
   }
   bool available(const _odla_value* v) const {
-    return v->kind != _odla_value::TEMP || vs_[v->index].main >= 0;
+    return v->kind != _odla_value::TEMP || vs_[v->index].main >= 0 || strided_.count(v->index) != 0;
+  }
+  // The launches of element-wise groups so far (later groups may join one).
+  struct FusedStep { int step = 0, n_ops = 0; FusedGroup model; FusedLaunch launch; std::vector<Ref> groups, bases; };
+  std::vector<std::shared_ptr<FusedStep>> fused_steps_;
+  // A Transpose (and Reshapes behind it) whose readers all look like members of element-wise groups
+  // stays a description of where its elements lie: extents and source strides, outermost first, of
+  // the row-major walk over the value (a Reshape leaves them as they are).  The group then loads
+  // straight from the source; settle() makes the value for any reader that wants it as a tensor.
+  struct Strided { int tensor = -1; std::vector<std::pair<int64_t, int64_t>> walk; };
+  std::unordered_map<int, Strided> strided_;   // by value index
+  bool read_by_groups(const _odla_value* v, int depth = 0) const {
+    if (calib_ || comp_->opts.int8 || v->is_output || depth > 4 || !dtype_is_float(storage_dtype(v)) || consumers_[v->index].empty()) return false;
+    for (int ci : consumers_[v->index]) {
+      const Node& c = comp_->nodes[ci];
+      if (c.op == OP_RESHAPE && !c.absorbed) {
+        if (!read_by_groups(c.out, depth + 1)) return false;
+      } else if (!fuse_candidate(ci) && !fuse_slice_seed(ci)) {
+        return false;
+      }
+    }
+    return true;
+  }
+  bool settle(const _odla_value* v) {
+    auto it = strided_.find(v->index);
+    if (it == strided_.end()) return false;
+    const Strided sv = it->second;
+    strided_.erase(it);
+    const int ty = new_tensor(T(sv.tensor).dt, L_ROWMAJOR, v->shape, 0, SP_ARENA);
+    StridedCopyParams cp;
+    cp.elem_size = dtype_size(T(sv.tensor).dt);
+    cp.rank = (int)sv.walk.size();
+    int64_t sy = 1;
+    for (int i = cp.rank - 1; i >= 0; --i) {
+      cp.dims[i] = sv.walk[i].first;
+      cp.sx[i] = sv.walk[i].second;
+      cp.sy[i] = sy;
+      sy *= cp.dims[i];
+    }
+    strided_copy_step("transpose:" + v->name, sv.tensor, ty, cp);
+    set_main(v, ty);
+    return true;
+  }
+  // The walk of a strided value cut at the dims of `sh`: per dim its extents and strides, outermost first.
+  static bool cut_walk(const Strided& sv, const Shape& sh, std::vector<std::pair<int64_t, int64_t>>* per_dim) {
+    std::vector<std::pair<int64_t, int64_t>> left = sv.walk;
+    for (int i = sh.rank - 1; i >= 0; --i) {
+      per_dim[i].clear();
+      int64_t need = sh.d[i];
+      while (need > 1) {
+        if (left.empty()) return false;
+        auto& f = left.back();
+        if (need % f.first == 0) {
+          per_dim[i].insert(per_dim[i].begin(), f);
+          need /= f.first;
+          left.pop_back();
+        } else if (f.first % need == 0) {
+          per_dim[i].insert(per_dim[i].begin(), {need, f.second});
+          f = {f.first / need, f.second * need};
+          need = 1;
+        } else {
+          return false;
+        }
+      }
+    }
+    return true;
   }
 
   // ------------------------------------------------------------------ nodes
@@ -833,7 +921,6 @@ void Planner::run() {
     const DType want = dtype_from_odla(ov->etype);
     const VState& os = vs_[ov->index];
     int t = -1;
-    bool converted = false;
     // a channels-last result leaves in one launch that changes layout and type together
     if (!calib_ && dtype_is_float(want) && ov->shape.rank == 4 && os.main >= 0 && T(os.main).layout == L_NHWC &&
         dtype_is_float(T(os.main).dt) && !T(os.main).quant && os.slot[L_ROWMAJOR][FORM_FLOAT] < 0 && storage_dtype(ov) == T(os.main).dt) {
@@ -849,7 +936,6 @@ void Planner::run() {
         LayoutParams p = lp; p.src = a(e); p.dst = b(e);
         return launch_nhwc_to_nchw(p, st);
       }, kWrites16);
-      converted = true;
     } else {
       t = get(ov, L_ROWMAJOR, FORM_FLOAT);
     }
@@ -860,7 +946,6 @@ void Planner::run() {
       const Ref a = ref(t), b = ref(dst);
       emit("out.cast:" + ov->name, {t}, {dst}, [=](const ExecEnv& e, hipStream_t st) { return launch_cast(a(e), sdt, b(e), want, n, st); }, kWrites16);
       t = dst;
-      converted = true;
     }
     PTensor& p = T(root(t));
     if (p.space == SP_ARENA) { p.pinned = true; p.last_step = 1 << 30; }
@@ -871,12 +956,12 @@ void Planner::run() {
     io.bytes = (size_t)ov->shape.numel() * dtype_size(want);
     plan_->outputs.push_back(io);
   }
-  // Results that launches write exactly and none reads can be written in the caller's device
+  // Results that launches write and read exactly can be written in the caller's device
   // buffer directly (a tensor behind two outputs, or one that is also an argument, stays here).
   for (size_t k = 0; k < plan_->outputs.size(); ++k) {
     Plan::IO& io = plan_->outputs[k];
     bool ok = !calib_ && io.offset == 0 && T(io.tensor).space == SP_ARENA && T(io.tensor).bytes == io.bytes &&
-              written_.count(io.tensor) && !read_.count(io.tensor) && !arena_only_.count(io.tensor);
+              written_.count(io.tensor) && !arena_only_.count(io.tensor);
     for (size_t j = 0; j < plan_->outputs.size(); ++j) ok = ok && (j == k || plan_->outputs[j].tensor != io.tensor);
     for (const Plan::IO& in : plan_->inputs) ok = ok && root(in.tensor) != io.tensor;
     if (ok) {
@@ -1238,7 +1323,7 @@ int Planner::strided_copy_step(const std::string& name, int src, int dst, const 
   emit(name, {src}, {dst}, [=](const ExecEnv& e, hipStream_t st) {
     StridedCopyParams p = cp; p.x = a(e); p.y = b(e);
     return launch_strided_copy(p, st);
-  });
+  }, kReads16 | kWrites16);
   return dst;
 }
 
@@ -2625,7 +2710,7 @@ bool Planner::lower_fused_group(int seed, int from) {
   };
 
   // ---- program over virtual registers
-  struct View { int tensor = -1; const _odla_value* value = nullptr; int64_t off = 0; int64_t st[3] = {0, 0, 0}; bool store = false; };
+  struct View { int tensor = -1; const _odla_value* value = nullptr; int64_t off = 0; int64_t st[4] = {0, 0, 0, 0}; bool store = false; };
   std::vector<View> views;
   struct VI { int op, dst, a, b, kind; float fa, fb; };
   std::vector<VI> prog;
@@ -2678,6 +2763,67 @@ bool Planner::lower_fused_group(int seed, int from) {
       prog.push_back({FOP_BINARY, dst, src[0], src[1], (int)n.i[0], src[0] < 0 ? imm[0] : imm[1], 0.f});
     }
   }
+  // ---- loads that follow a Transpose to its source (see Strided): strides over the dims of S, one of
+  // which may be walked as two (`split_dim`, whose inner part has split_n points)
+  struct Source { const _odla_value* x = nullptr; const Node* slice = nullptr; bool strided = false; int64_t off = 0, st[3] = {0, 0, 0}, inner_st = 0; };
+  std::vector<Source> sources;
+  int split_dim = -1, unit_dim = R - 1;
+  int64_t split_n = 1;
+  bool any_strided = false, all_along = true;   // all_along: every load of all of S runs along unit_dim
+  for (const PendingLoad& l : loads) {
+    Source src;
+    src.x = l.v;
+    auto sl = slice_of.find(l.v);
+    if (sl != slice_of.end() && std::find(slices.begin(), slices.end(), sl->second) != slices.end()) {
+      src.slice = &comp_->nodes[sl->second];
+      src.x = src.slice->in[0];
+    }
+    auto sv = strided_.find(src.x->index);
+    if (sv != strided_.end()) {
+      std::vector<std::pair<int64_t, int64_t>> per_dim[ODLA_MAX_DIMENSION];
+      const int r = src.x->shape.rank;
+      bool ok = cut_walk(sv->second, src.x->shape, per_dim);
+      const Shape pal = padded(l.aligned);
+      const Shape& own = l.v->shape;
+      int to = 0, sd = -1;
+      int64_t sn = 1;
+      for (int i = 0; ok && i < r; ++i) {
+        const int64_t begin = src.slice ? src.slice->iv[i] : 0, step = src.slice ? src.slice->iv[2 * r + i] : 1;
+        if (per_dim[i].size() == 1) src.off += begin * per_dim[i][0].second;
+        if (own.d[i] == 1) { ok = per_dim[i].size() <= 1 || (begin == 0 && step == 1); continue; }
+        while (to < R && pal.d[to] == 1) ++to;
+        if (to >= R || pal.d[to] != own.d[i]) { ok = false; break; }
+        if (per_dim[i].size() == 2) {
+          ok = sd < 0 && begin == 0 && step == 1 && own.d[i] == src.x->shape.d[i];
+          sd = to;
+          sn = per_dim[i][1].first;
+          src.st[to] = per_dim[i][0].second;
+          src.inner_st = per_dim[i][1].second;
+        } else {
+          ok = per_dim[i].size() == 1;
+          if (ok) src.st[to] = per_dim[i][0].second * step;
+        }
+        ++to;
+      }
+      if (ok && sd >= 0 && split_dim >= 0) ok = sd == split_dim && sn == split_n;
+      if (ok) {
+        if (sd >= 0) { split_dim = sd; split_n = sn; }
+        src.strided = any_strided = true;
+        if (pal == S)
+          for (int i = 0; i < R; ++i)
+            if (S.d[i] > 1 && (i == sd ? src.inner_st : src.st[i]) == 1) unit_dim = i;
+      } else {
+        src.off = 0;
+        for (int i = 0; i < 3; ++i) src.st[i] = 0;
+      }
+    }
+    sources.push_back(src);
+  }
+  for (size_t k = 0; any_strided && k < loads.size(); ++k) {
+    if (!(padded(loads[k].aligned) == S)) continue;
+    const Source& src = sources[k];
+    all_along = all_along && (src.strided ? (unit_dim == split_dim && src.inner_st != 0 ? src.inner_st : src.st[unit_dim]) == 1 : unit_dim == R - 1);
+  }
   // ---- results that leave the group: plain, through a Concat, through a Transpose
   struct Sink { int node; const _odla_value* src; int kind; /* 0 plain, 1 concat part, 2 transpose */ int part; };
   std::vector<Sink> sinks;
@@ -2709,9 +2855,10 @@ bool Planner::lower_fused_group(int seed, int from) {
       }
       // A Transpose that moves the innermost dim turns the group's stores into single
       // elements a row apart; beyond a few million elements the tiled copy
-      // behind a plain store is several times faster than that.
+      // behind a plain store is several times faster than that - unless the loads
+      // come from in front of a Transpose that did the opposite.
       if (cn.op == OP_TRANSPOSE && !cn.absorbed && full && storage_dtype(cn.out) == dt && (int)cn.iv.size() == R &&
-          (cn.iv[R - 1] == R - 1 || S.numel() <= kTransposeSinkMax)) {
+          (cn.iv[R - 1] == R - 1 || S.numel() <= kTransposeSinkMax || (any_strided && all_along && cn.iv[R - 1] == unit_dim))) {
         if (std::find(sink_nodes.begin(), sink_nodes.end(), c) == sink_nodes.end()) {
           sink_nodes.push_back(c);
           sinks.push_back({c, v, 2, 0});
@@ -2726,45 +2873,86 @@ bool Planner::lower_fused_group(int seed, int from) {
     }
   }
   if (sinks.empty()) return give_up();
+  // (the same for the loads: a large group whose stores run along another dim than its strided
+  //  loads reads what the tiled copy made)
+  if (any_strided && S.numel() > kTransposeSinkMax) {
+    bool along = all_along;
+    for (const Sink& sk : sinks) along = along && (sk.kind == 2 ? (int)comp_->nodes[sk.node].iv[R - 1] : R - 1) == unit_dim;
+    if (!along) {
+      // (a Transpose that was accepted for the loads' sake needs them strided: leave the group alone)
+      for (const Sink& sk : sinks)
+        if (sk.kind == 2 && comp_->nodes[sk.node].iv[R - 1] != R - 1) return give_up();
+      for (Source& src : sources) src.strided = false;
+      split_dim = -1;
+      split_n = 1;
+    }
+  }
   if ((int)(loads.size() + sinks.size()) > kFusedMaxViews || (int)(prog.size() + sinks.size()) > kFusedMaxInstr) return give_up();
 
-  // ---- physical registers: a register is free again after its last reader
-  std::vector<int> last_use((size_t)n_vregs, -1);
-  for (size_t k = 0; k < prog.size(); ++k) {
-    if (prog[k].op != FOP_LOAD && prog[k].a >= 0) last_use[prog[k].a] = (int)k;
-    if (prog[k].op == FOP_BINARY && prog[k].b >= 0) last_use[prog[k].b] = (int)k;
-  }
-  for (const Sink& sk : sinks) last_use[reg_of.at(sk.src)] = (int)prog.size();   // stores come last
-  std::vector<int> phys((size_t)n_vregs, -1);
-  {
+  // ---- physical registers: a register is free again after its last reader.  Results that are made
+  // once per walk (`once`, by virtual register) keep theirs: what else the program does runs again
+  // and again behind them.  Returns the number of registers, 0 if there are not enough.
+  std::vector<int> phys;
+  auto allocate = [&](const std::vector<VI>& code, const std::vector<char>& once) -> int {
+    std::vector<int> last_use((size_t)n_vregs, -1);
+    for (size_t k = 0; k < code.size(); ++k) {
+      if (code[k].op != FOP_LOAD && code[k].a >= 0) last_use[code[k].a] = (int)k;
+      if (code[k].op == FOP_BINARY && code[k].b >= 0) last_use[code[k].b] = (int)k;
+    }
+    for (size_t v = 0; v < once.size(); ++v) if (once[v]) last_use[v] = (int)code.size();
+    for (const Sink& sk : sinks) last_use[reg_of.at(sk.src)] = (int)code.size();   // stores come last
+    phys.assign((size_t)n_vregs, -1);
+    int most = 0;
     std::vector<int> free_regs;
     for (int i = kFusedMaxRegs - 1; i >= 0; --i) free_regs.push_back(i);
-    for (size_t k = 0; k < prog.size(); ++k) {
-      VI& in = prog[k];
+    for (size_t k = 0; k < code.size(); ++k) {
+      const VI& in = code[k];
       const int va = in.op != FOP_LOAD ? in.a : -1, vb = in.op == FOP_BINARY ? in.b : -1;
       // operands read before the result is written: a register freed here may take the result
       if (va >= 0 && last_use[va] == (int)k) free_regs.push_back(phys[va]);
       if (vb >= 0 && vb != va && last_use[vb] == (int)k) free_regs.push_back(phys[vb]);
-      if (free_regs.empty()) return give_up();
-      phys[in.dst] = free_regs.back();
-      free_regs.pop_back();
+      if (free_regs.empty()) return 0;
+      auto low = std::min_element(free_regs.begin(), free_regs.end());   // (the registers used are the lowest ones)
+      phys[in.dst] = *low;
+      free_regs.erase(low);
+      most = std::max(most, phys[in.dst] + 1);
       if (last_use[in.dst] < 0) free_regs.push_back(phys[in.dst]);   // never read: reusable at once
     }
-  }
+    return most;
+  };
+  const int plain_regs = allocate(prog, std::vector<char>());
+  if (plain_regs == 0) return give_up();
 
   // ---- from here on the plan changes: nothing below gives up
   // outside operands (conversion steps, if any, are emitted here, before the group)
-  FusedParams fp;
-  fp.dt = dt;
+  FusedGroup fp;
   std::vector<int> read_tensors, write_tensors;
   std::vector<int64_t> in_main_stride;   // per load: used to pick the iteration order
-  for (const PendingLoad& l : loads) {
+  // strides of a view over the axes of the walk: the dims of S, `split_dim` as two of them
+  std::vector<int64_t> axes;
+  for (int i = 0; i < R; ++i) {
+    if (i == split_dim) { axes.push_back(S.d[i] / split_n); axes.push_back(split_n); } else axes.push_back(S.d[i]);
+  }
+  const int A = (int)axes.size();
+  auto on_axes = [&](View* vw, const int64_t* st) {
+    int a = 0;
+    for (int i = 0; i < R; ++i) {
+      if (i == split_dim) { vw->st[a++] = st[i] * split_n; vw->st[a++] = st[i]; } else vw->st[a++] = st[i];
+    }
+  };
+  for (size_t k = 0; k < loads.size(); ++k) {
+    const PendingLoad& l = loads[k];
+    const Source& src = sources[k];
     View vw;
-    auto sl = slice_of.find(l.v);
     const Shape pal = padded(l.aligned);
-    if (sl != slice_of.end() && std::find(slices.begin(), slices.end(), sl->second) != slices.end()) {
-      const Node& sn = comp_->nodes[sl->second];
-      const _odla_value* x = sn.in[0];
+    if (src.strided) {
+      vw.tensor = strided_.at(src.x->index).tensor;
+      vw.off = src.off;
+      on_axes(&vw, src.st);
+      if (src.inner_st != 0) { vw.st[split_dim] = src.st[split_dim]; vw.st[split_dim + 1] = src.inner_st; }
+    } else if (src.slice != nullptr) {
+      const Node& sn = *src.slice;
+      const _odla_value* x = src.x;
       const int r = x->shape.rank;
       vw.tensor = get(x, L_ROWMAJOR, FORM_FLOAT);
       // strides of the slice's own dims, then mapped through the aligned shape (which only adds 1-dims)
@@ -2776,16 +2964,20 @@ bool Planner::lower_fused_group(int seed, int from) {
         acc *= x->shape.d[i];
       }
       // walk the non-1 dims of the slice result and of the aligned shape together
+      int64_t st[3] = {0, 0, 0};
       int oi = 0;
       for (int i = 0; i < R; ++i) {
         if (pal.d[i] == 1) continue;
         while (oi < r && sn.out->shape.d[oi] == 1) ++oi;
-        vw.st[i] = own_st[oi++];
+        st[i] = own_st[oi++];
       }
+      on_axes(&vw, st);
     } else {
       vw.tensor = get(l.v, L_ROWMAJOR, FORM_FLOAT);
+      int64_t st[3] = {0, 0, 0};
       int64_t acc = 1;
-      for (int i = R - 1; i >= 0; --i) { vw.st[i] = pal.d[i] == 1 ? 0 : acc; acc *= pal.d[i]; }
+      for (int i = R - 1; i >= 0; --i) { st[i] = pal.d[i] == 1 ? 0 : acc; acc *= pal.d[i]; }
+      on_axes(&vw, st);
     }
     if (T(vw.tensor).dt != dt) fail(ODLA_UNSUPPORTED_DATATYPE, "mixed storage types in the element-wise group at '%s'", comp_->nodes[seed].out->name.c_str());
     vw.value = l.v;
@@ -2793,70 +2985,78 @@ bool Planner::lower_fused_group(int seed, int from) {
     read_tensors.push_back(vw.tensor);
   }
   const size_t n_loads = views.size();
-  std::unordered_map<int, int> sink_tensor;   // sink node -> its result tensor
+  struct SinkDst { int tensor = -1; int64_t off = 0, st[3] = {0, 0, 0}; };
+  std::unordered_map<int, SinkDst> sink_dst;   // by sink node
   std::vector<std::pair<_odla_value*, int>> results;
-  auto row_major = [&](const Shape& sh, int64_t* st) { int64_t acc = 1; for (int i = sh.rank - 1; i >= 0; --i) { st[i] = acc; acc *= sh.d[i]; } };
   for (const Sink& sk : sinks) {
     const Node& sn = comp_->nodes[sk.node];
     View vw;
     vw.store = true;
     vw.value = sk.src;
-    int64_t st[ODLA_MAX_DIMENSION] = {0};
-    if (sk.kind == 0) {
-      vw.tensor = new_tensor(dt, L_ROWMAJOR, sk.src->shape, 0, SP_ARENA);
-      results.push_back({sn.out, vw.tensor});
-      row_major(S, st);
-      for (int i = 0; i < R; ++i) vw.st[i] = st[i];
-    } else {
-      auto it = sink_tensor.find(sk.node);
-      if (it == sink_tensor.end()) {
-        const int t = new_tensor(dt, L_ROWMAJOR, sn.out->shape, 0, SP_ARENA);
-        it = sink_tensor.emplace(sk.node, t).first;
-        results.push_back({sn.out, t});
+    // the result: a tensor of its own, or this value's part of a Concat over several groups
+    auto it = sink_dst.find(sk.node);
+    if (it == sink_dst.end()) {
+      SinkDst d;
+      const Shape& os = sn.out->shape;
+      d.tensor = concat_part(sn.out, dt, &d.off, d.st);
+      if (d.tensor < 0) {
+        d.off = 0;
+        int64_t acc = 1;
+        for (int i = os.rank - 1; i >= 0; --i) { d.st[i] = acc; acc *= os.d[i]; }
+        d.tensor = new_tensor(dt, L_ROWMAJOR, os, 0, SP_ARENA);
+        results.push_back({sn.out, d.tensor});
       }
-      vw.tensor = it->second;
-      row_major(sn.out->shape, st);
+      it = sink_dst.emplace(sk.node, d).first;
+    }
+    const SinkDst& d = it->second;
+    vw.tensor = d.tensor;
+    vw.off = d.off;
+    int64_t st[3] = {0, 0, 0};
+    if (sk.kind == 2) {
+      for (int i = 0; i < R; ++i) st[(int)sn.iv[i]] = d.st[i];   // result dim i walks source dim perm[i]
+    } else {
+      const int lead = R - sn.out->shape.rank;   // (a plain result may have fewer dims, all of S's others being 1)
+      for (int i = lead; i < R; ++i) st[i] = d.st[i - lead];
       if (sk.kind == 1) {
         const int axis = (int)sn.i[0];
-        int64_t before = 0;
-        for (int k = 0; k < sk.part; ++k) before += sn.in[k]->shape.d[axis];
-        vw.off = before * st[axis];
-        for (int i = 0; i < R; ++i) vw.st[i] = st[i];
-      } else {
-        for (int i = 0; i < R; ++i) vw.st[(int)sn.iv[i]] = st[i];   // result dim i walks source dim perm[i]
+        for (int k = 0; k < sk.part; ++k) vw.off += sn.in[k]->shape.d[axis] * d.st[axis];
       }
     }
+    on_axes(&vw, st);
     views.push_back(vw);
     if (std::find(write_tensors.begin(), write_tensors.end(), vw.tensor) == write_tensors.end()) write_tensors.push_back(vw.tensor);
   }
 
   // ---- iteration order: stores contiguous across threads, loads along a thread's walk
-  int d3 = R - 1, d2 = -1;
+  int d3 = A - 1, d2 = -1;
+  bool spare = false, placed_only = false;
   {
     const View& mo = views[n_loads];
     int64_t best = 0;
-    for (int i = 0; i < R; ++i)
-      if (S.d[i] > 1 && mo.st[i] > 0 && (best == 0 || mo.st[i] < best)) { best = mo.st[i]; d3 = i; }
+    for (int i = 0; i < A; ++i)
+      if (axes[i] > 1 && mo.st[i] > 0 && (best == 0 || mo.st[i] < best)) { best = mo.st[i]; d3 = i; }
     int64_t most = -1;
     const View* mi = nullptr;
     for (size_t k = 0; k < n_loads; ++k) {
       int64_t elems = 1;
-      for (int i = 0; i < R; ++i) if (views[k].st[i] != 0) elems *= S.d[i];
+      for (int i = 0; i < A; ++i) if (views[k].st[i] != 0) elems *= axes[i];
       if (elems > most) { most = elems; mi = &views[k]; }
     }
     if (mi != nullptr && mi->st[d3] != 1)
-      for (int i = 0; i < R; ++i) if (i != d3 && S.d[i] > 1 && mi->st[i] == 1) d2 = i;
-    // no such dim: with points to spare, a thread still takes four per decoded instruction,
-    // along the longest other dim
-    if (d2 < 0 && S.numel() >= (int64_t)4 * 256 * 2048)
-      for (int i = 0; i < R; ++i) if (i != d3 && S.d[i] >= 4 && (d2 < 0 || S.d[i] > S.d[d2])) d2 = i;
+      for (int i = 0; i < A; ++i) if (i != d3 && axes[i] > 1 && mi->st[i] == 1) d2 = i;
+    // no such dim: with points to spare (four for every thread of one workgroup per CU), a thread still takes four per decoded instruction,
+    // along the longest other dim (a fourth axis takes this place anyhow)
+    spare = S.numel() >= (int64_t)4 * 256 * 256;
+    placed_only = d2 < 0 && !spare;
+    if (d2 < 0 && (A == 4 || spare))
+      for (int i = 0; i < A; ++i) if (i != d3 && (axes[i] >= 4 || A == 4) && (d2 < 0 || axes[i] > axes[d2])) d2 = i;
   }
   int order[4] = {-1, -1, d2, d3};
   {
     int slot = 1;
-    for (int i = R - 1; i >= 0; --i) if (i != d2 && i != d3) order[slot--] = i;
+    for (int i = A - 1; i >= 0; --i) if (i != d2 && i != d3) order[slot--] = i;
   }
-  for (int k = 0; k < 4; ++k) fp.dims[k] = order[k] < 0 ? 1 : S.d[order[k]];
+  for (int k = 0; k < 4; ++k) fp.dims[k] = order[k] < 0 ? 1 : axes[order[k]];
   {
     // every step of a walk waits for its loads: keep walks short until the chip has
     // a few resident threads per lane (256 CUs x 2048 threads x 2)
@@ -2864,36 +3064,106 @@ bool Planner::lower_fused_group(int seed, int from) {
     const int64_t want = 256 * 2048 * 2;
     int64_t w = fp.dims[2] * base / want;
     fp.walk = std::min<int64_t>(fp.dims[2], std::max<int64_t>(4, w / 4 * 4));   // whole groups of four points
+    if (placed_only) fp.walk = 1;
   }
+  fp.n_views = (int)views.size();
   for (size_t k = 0; k < views.size(); ++k) {
     fp.view[k].off = views[k].off;
     for (int q = 0; q < 4; ++q) fp.view[k].st[q] = order[q] < 0 ? 0 : views[k].st[order[q]];
   }
+  // ---- instruction order: what the walk does not change first, then the loads, unless the
+  // registers that this holds would halve the points a thread takes at once (32 registers between them)
+  {
+    std::vector<VI> code;
+    std::vector<char> once((size_t)n_vregs, 0);
+    const int w2 = order[2];
+    for (const VI& in : prog)
+      if (in.op == FOP_LOAD && (w2 < 0 || views[in.a].st[w2] == 0)) { once[in.dst] = 1; code.push_back(in); }
+    fp.n_once_loads = (int)code.size();
+    for (const VI& in : prog) if (in.op == FOP_LOAD && !once[in.dst]) code.push_back(in);
+    fp.n_loads = (int)code.size() - fp.n_once_loads;
+    for (const VI& in : prog)
+      if (in.op != FOP_LOAD && (in.a < 0 || once[in.a]) && (in.op == FOP_UNARY || in.b < 0 || once[in.b])) { once[in.dst] = 1; code.push_back(in); }
+    fp.n_once = (int)code.size() - fp.n_once_loads - fp.n_loads;
+    for (const VI& in : prog) if (in.op != FOP_LOAD && !once[in.dst]) code.push_back(in);
+    auto points = [&](int regs) { return fp.walk >= 8 && regs * 8 <= 32 ? 8 : fp.walk >= 4 && regs * 4 <= 32 ? 4 : (fp.walk >= 2 && regs * 2 <= 32 ? 2 : 1); };
+    const int regs = allocate(code, once);
+    if (regs > 0 && points(regs) >= points(plain_regs)) {
+      prog = code;
+    } else {
+      fp.n_once_loads = fp.n_once = fp.n_loads = 0;
+      allocate(prog, std::vector<char>());
+    }
+  }
   int ni = 0;
   for (const VI& in : prog) {
     FusedInstr& o = fp.prog[ni++];
-    o.op = in.op; o.kind = in.kind; o.fa = in.fa; o.fb = in.fb;
-    o.dst = phys[in.dst];
-    o.a = in.op == FOP_LOAD ? in.a : (in.a < 0 ? -1 : phys[in.a]);
-    o.b = in.op == FOP_BINARY ? (in.b < 0 ? -1 : phys[in.b]) : 0;
+    o.op = (uint8_t)in.op; o.kind = (uint8_t)in.kind; o.fa = in.fa; o.fb = in.fb;
+    o.dst = (int8_t)phys[in.dst];
+    o.a = (int8_t)(in.op == FOP_LOAD ? in.a : (in.a < 0 ? -1 : phys[in.a]));
+    o.b = (int8_t)(in.op == FOP_BINARY ? (in.b < 0 ? -1 : phys[in.b]) : 0);
   }
   for (size_t k = 0; k < sinks.size(); ++k) {
     FusedInstr& o = fp.prog[ni++];
     o.op = FOP_STORE;
-    o.dst = (int)(n_loads + k);
-    o.a = phys[reg_of.at(sinks[k].src)];
+    o.dst = (int8_t)(n_loads + k);
+    o.a = (int8_t)phys[reg_of.at(sinks[k].src)];
   }
   fp.n_instr = ni;
 
-  std::vector<Ref> refs;
-  for (const View& vw : views) refs.push_back(ref(vw.tensor));
-  std::vector<int64_t> elem_off;
+  int blocks = 0;
+  size_t lds = 0;
+  bool wide = false;
+  if (!fused_prepare(&fp, &blocks, &lds, &wide)) fail(ODLA_INTERNAL_LOGIC_ERR, "element-wise group at '%s'", comp_->nodes[seed].out->name.c_str());
+  std::vector<uint8_t> raw(sizeof(FusedGroup));
+  memcpy(raw.data(), &fp, sizeof(FusedGroup));
+  Shape gs;
+  gs.rank = 1;
+  gs.d[0] = (int64_t)raw.size();
+  const Ref rg = ref(const_from_host(DT_U8, gs, nullptr, &raw));
   const std::string name = "fused:" + comp_->nodes[members.back()].out->name + "(" + std::to_string(members.size()) + ")";
-  emit_lists(name, read_tensors, write_tensors, [=](const ExecEnv& e, hipStream_t st) {
-    FusedParams p = fp;
-    for (size_t k = 0; k < refs.size(); ++k) p.view[k].base = refs[k](e);
-    return launch_fused_eltwise(p, st);
-  });
+  // A group that repeats the program of an earlier one (the decode of another head) and reads
+  // nothing made since goes into its launch: each is a short launch that hides none of its latency.
+  FusedStep* join = nullptr;
+  for (auto& f : fused_steps_) {
+    const FusedLaunch& l = f->launch;
+    bool ok = l.dt == dt && f->n_ops == (int)members.size() && l.n_groups < kFusedMaxGroups && l.view0[l.n_groups] + fp.n_views <= kFusedMaxBases &&
+              f->model.n_instr == fp.n_instr && f->model.n_views == fp.n_views;
+    for (int k = 0; ok && k < fp.n_instr; ++k) {
+      const FusedInstr &x = f->model.prog[k], &y = fp.prog[k];
+      ok = x.op == y.op && x.kind == y.kind && x.dst == y.dst && x.a == y.a && x.b == y.b;
+    }
+    for (int t : read_tensors) ok = ok && (T(root(t)).space != SP_ARENA || T(root(t)).def_step < f->step);
+    if (ok) join = f.get();
+  }
+  auto add = [&](FusedStep* f) {
+    FusedLaunch& l = f->launch;
+    const int k = l.n_groups++;
+    l.block0[k + 1] = l.block0[k] + blocks;
+    l.view0[k + 1] = l.view0[k] + fp.n_views;
+    l.lds_bytes = std::max(l.lds_bytes, lds);
+    l.wide = l.wide || wide;
+    f->groups.push_back(rg);
+    for (const View& vw : views) f->bases.push_back(ref(vw.tensor));
+  };
+  if (join != nullptr) {
+    add(join);
+    touch(join->step, read_tensors, write_tensors, kReads16 | kWrites16);
+  } else {
+    auto f = std::make_shared<FusedStep>();
+    f->step = (int)plan_->steps.size();
+    f->n_ops = (int)members.size();
+    f->model = fp;
+    f->launch.dt = dt;
+    add(f.get());
+    fused_steps_.push_back(f);
+    emit_lists(name, read_tensors, write_tensors, [f](const ExecEnv& e, hipStream_t st) {
+      FusedLaunch l = f->launch;
+      for (size_t k = 0; k < f->groups.size(); ++k) l.group[k] = (const FusedGroup*)f->groups[k](e);
+      for (size_t k = 0; k < f->bases.size(); ++k) l.base[k] = f->bases[k](e);
+      return launch_fused_eltwise(l, st);
+    }, kReads16 | kWrites16);
+  }
   for (int j : members) comp_->nodes[j].absorbed = true;
   for (int j : slices) comp_->nodes[j].absorbed = true;
   for (int j : sink_nodes) comp_->nodes[j].absorbed = true;
@@ -3272,15 +3542,20 @@ void Planner::lower_concat(int ni) {
   }
   const Layout lay = nhwc ? L_NHWC : L_ROWMAJOR;
   std::vector<int> tin;
-  for (_odla_value* v : n.in) tin.push_back(get(v, lay, FORM_FLOAT));
+  const auto placed = concat_dst_.find(ni);   // (some parts are stored in the result already)
+  for (_odla_value* v : n.in) tin.push_back(placed_.count(v->index) ? placed->second : get(v, lay, FORM_FLOAT));
   const DType dt = T(tin[0]).dt;
   const int es = dtype_size(dt);
-  const auto placed = concat_dst_.find(ni);   // (some parts are stored in the result already)
   const int ty = placed != concat_dst_.end() ? placed->second : new_tensor(dt, lay, os, nhwc ? (int)os.d[1] : 0, SP_ARENA);
   int64_t off = 0;
   for (size_t k = 0; k < n.in.size(); ++k) {
     const PTensor pi = T(tin[k]);
-    if (root(tin[k]) == root(ty)) { off += n.in[k]->shape.d[1]; continue; }
+    if (root(tin[k]) == root(ty)) {   // (stored there by the launch that made it)
+      int64_t inner = 1;
+      if (!nhwc) for (int i = axis + 1; i < os.rank; ++i) inner *= os.d[i];
+      off += n.in[k]->shape.d[axis] * inner;
+      continue;
+    }
     if (pi.dt != dt) fail(ODLA_UNSUPPORTED_DATATYPE, "odla_Concat of mixed storage types");
     const Shape& is = n.in[k]->shape;
     StridedCopyParams cp;
@@ -3335,7 +3610,7 @@ void Planner::lower_gather(int ni) {
   const Ref a = ref(tx), ri = ref(ti), b = ref(ty);
   emit("gather:" + n.out->name, {tx, ti}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
     return launch_gather_rows(a(e), ri(e), idt, b(e), outer, n_src, n_idx, row_bytes, st);
-  });
+  }, kReads16 | kWrites16);
   set_main(n.out, ty);
 }
 
@@ -3417,6 +3692,14 @@ void Planner::lower_reshape(int ni) {
   Node& n = comp_->nodes[ni];
   const _odla_value* x = n.in[0];
   const VState& s = vs_[x->index];
+  {
+    auto it = strided_.find(x->index);
+    if (it != strided_.end() && read_by_groups(n.out)) {
+      const Strided sv = it->second;
+      strided_[n.out->index] = sv;
+      return;
+    }
+  }
   // keep 8-bit data 8-bit through a reshape when it is already row-major
   int tx;
   if (s.main >= 0 && T(s.main).quant && s.slot[L_ROWMAJOR][FORM_QUANT] >= 0 && qentry(n.out) != nullptr)
@@ -3606,12 +3889,25 @@ void Planner::lower_transpose(int ni) {
   }
   const int tx = get_moved(x, L_ROWMAJOR);
   const DType dt = T(tx).dt;
-  const int ty = new_tensor(dt, L_ROWMAJOR, os, 0, SP_ARENA);
   int64_t xstr[ODLA_MAX_DIMENSION];
   {
     int64_t acc = 1;
     for (int i = r - 1; i >= 0; --i) { xstr[i] = acc; acc *= xs.d[i]; }
   }
+  if (dt == storage_dtype(n.out) && read_by_groups(n.out)) {
+    Strided sv;
+    sv.tensor = tx;
+    for (int i = 0; i < r; ++i) {
+      const int64_t e = os.d[i], st = xstr[n.iv[i]];
+      if (e == 1) continue;
+      if (!sv.walk.empty() && sv.walk.back().second == e * st) sv.walk.back() = {sv.walk.back().first * e, st};
+      else sv.walk.push_back({e, st});
+    }
+    if (sv.walk.empty()) sv.walk.push_back({1, 1});
+    strided_[n.out->index] = sv;
+    return;
+  }
+  const int ty = new_tensor(dt, L_ROWMAJOR, os, 0, SP_ARENA);
   StridedCopyParams cp;
   cp.elem_size = dtype_size(dt);
   cp.rank = r;
@@ -3684,7 +3980,7 @@ void Planner::lower_nms(int ni) {
   const Ref rb = ref(tb), rs = ref(ts), rw = ref(tw), ry = ref(ty);
   emit("nms:" + n.out->name, {tb, ts, tw}, {ty, tw}, [=](const ExecEnv& e, hipStream_t st) {
     return launch_nms(rb(e), bdt, rs(e), sdt, N, C, B, max_out, iou, thr, (int32_t*)ry(e), rw(e), st, e.image_base);
-  });
+  }, kReads16 | kWrites16);
   if (dtype_from_odla(n.out->etype) == DT_I64) {
     const int t64 = new_tensor(DT_I64, L_ROWMAJOR, o32, 0, SP_ARENA);
     const int64_t ne = o32.numel();
