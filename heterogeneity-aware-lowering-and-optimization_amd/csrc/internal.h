@@ -183,6 +183,9 @@ struct Plan {
     // device buffer can be written in place
     bool in_place_ok = false;
     bool align16 = false;    // ... at a 16-byte aligned address
+    // arguments: the one launch that reads the tensor reads every element once;
+    // results: no launch reads the tensor.  Page-locked host memory then serves as well as device memory.
+    bool host_ok = false;
   };
   std::vector<IO> inputs, outputs;
   std::unordered_map<const _odla_value*, int> final_tensor;  // for odla_GetValueData
@@ -267,6 +270,10 @@ struct _odla_context {
   std::vector<const char*> graph_ext;   // the caller's buffers the captured launches read / write in place
   std::vector<const char*> last_ext;    // those of the last execution (odla_GetValueData finds results there)
   int capture_streak = 0;               // executions in a row that had to capture for new buffers
+  // Page-locked room through which executions that wait pass small pageable arguments and results
+  // (see host_stage); made on first use, one per context.
+  char* host_stage = nullptr;
+  bool host_stage_failed = false;
   bool in_place_off = false;            // the caller binds new buffers every time: copy instead
   // Graphs captured for other sets of argument buffers (a caller that alternates between a
   // few device buffers replays instead of capturing again); bounded, oldest dropped first.

@@ -156,6 +156,7 @@ class Planner {
   }
   // by root tensor: some launch relies on the arena for it; needs a 16-byte aligned base; writes it
   std::unordered_set<int> arena_only_, aligned_only_, written_;
+  std::unordered_map<int, int> reads_;   // by root tensor: passes over it (2 for a launch that may read it several times)
   // The 8-bit convolution steps, kept so that a plain 1x1 layer over the result of one can ride in
   // its launch (lower_conv; igemm_stream_q8_fusable decides).
   struct FuseProducer {
@@ -192,9 +193,10 @@ class Planner {
   //                 conversions launch_nchw_to_nhwc / launch_nchw_to_s2d test it themselves)
   //   kReads16      the same from 16-byte aligned bases
   //   kWrites16     it writes exactly the elements of its results, at 16-byte aligned bases
+  //   kReadsOnce    with one of the first two: it reads every element of its sources once
   // A source that is an argument's staging tensor may then be the caller's own device buffer, and
   // so may a result (which later launches may read, if they do it exactly too).
-  enum : unsigned { kReadsAny = 1, kReads16 = 2, kWrites16 = 4 };
+  enum : unsigned { kReadsAny = 1, kReads16 = 2, kWrites16 = 4, kReadsOnce = 8 };
   void emit(const std::string& name, std::initializer_list<int> reads, std::initializer_list<int> writes,
             std::function<hipError_t(const ExecEnv&, hipStream_t)> fn, unsigned exact = 0) {
     emit_lists(name, std::vector<int>(reads), std::vector<int>(writes), std::move(fn), exact);
@@ -223,6 +225,7 @@ class Planner {
       if (t < 0) continue;
       if (!(exact & (kReadsAny | kReads16))) arena_only_.insert(root(t));
       if (!(exact & kReadsAny)) aligned_only_.insert(root(t));
+      reads_[root(t)] += exact & kReadsOnce ? 1 : 2;
     }
     for (int t : writes) {
       if (t < 0) continue;
@@ -448,7 +451,7 @@ class Planner {
         emit("to_nhwc:" + v->name, {from}, {dst}, [=](const ExecEnv& e, hipStream_t st) {
           LayoutParams p = lp; p.src = a(e); p.dst = b(e);
           return launch_nchw_to_nhwc(p, st);
-        }, kReadsAny);
+        }, kReadsAny | kReadsOnce);
         return dst;
       } else {
         lp.cs = s2.cs;
@@ -489,7 +492,7 @@ class Planner {
       });
     } else if (src.dt != fdt) {
       const DType sdt = src.dt, ddt = fdt;
-      emit("cast:" + v->name, {have}, {dst}, [=](const ExecEnv& e, hipStream_t st) { return launch_cast(a(e), sdt, b(e), ddt, n, st); }, kReads16 | kWrites16);
+      emit("cast:" + v->name, {have}, {dst}, [=](const ExecEnv& e, hipStream_t st) { return launch_cast(a(e), sdt, b(e), ddt, n, st); }, kReads16 | kWrites16 | kReadsOnce);
     } else {
       fail(ODLA_INTERNAL_LOGIC_ERR, "no conversion needed for '%s'", v->name.c_str());
     }
@@ -966,6 +969,7 @@ void Planner::run() {
     for (const Plan::IO& in : plan_->inputs) ok = ok && root(in.tensor) != io.tensor;
     if (ok) {
       io.in_place_ok = true;
+      io.host_ok = reads_.count(io.tensor) == 0;
       T(io.tensor).ext_slot = (int)(plan_->inputs.size() + k);
     }
   }
@@ -979,6 +983,7 @@ void Planner::run() {
     for (const auto& ft : plan_->final_tensor) ok = ok && root(ft.second) != r;
     if (ok) {
       io.in_place_ok = true;
+      io.host_ok = reads_[r] == 1;
       io.align16 = aligned_only_.count(r) != 0;
       T(r).ext_slot = (int)k;
     }
@@ -1385,6 +1390,8 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
   const Ref rx = ref(tx), rw = ref(tw), ry = ref(ty);
   const Ref rb = ref(tb >= 0 ? tb : tx), rr = ref(tr >= 0 ? tr : tx);
   const bool hb = tb >= 0, hr = tr >= 0;
+  // (one wavefront per row: whole 16-byte pieces of its row, once, and single elements of the result)
+  const unsigned exact = !hr && T(tw).space == SP_CONST && ip.ycs == Kout_total && gemm_rowdot_shape(ip) ? kReads16 | kReadsOnce | kWrites16 : 0u;
   emit(name, {tx, tw, tr}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
     IgemmParams p = ip;
     p.x = rx(e); p.w = rw(e); p.y = ry(e);
@@ -1392,7 +1399,7 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
     p.residual = hr ? rr(e) : nullptr;
     p.w_frag = hf ? rf(e) : nullptr;
     return launch_igemm(p, st);
-  });
+  }, exact);
 }
 
 // ---------------------------------------------------------------- Conv ----
@@ -1510,7 +1517,7 @@ void Planner::lower_conv(int ni) {
       emit("to_s2d:" + x->name, {from}, {tx_s2d}, [=](const ExecEnv& e, hipStream_t st) {
         S2dParams p = sp; p.src = a(e); p.dst = b(e);
         return launch_nchw_to_s2d(p, st);
-      }, /*exact_reader=*/true);
+      }, kReadsAny | kReadsOnce);
       C = C2; Cg = C2; H = H2; W = W2; R = R2; S = S2;
       str_h = str_w = 1;
       pad_t = -dy0; pad_l = -dx0;

@@ -706,7 +706,7 @@ class Session:
         """Shape of a value at the batch this session runs at."""
         s = ValueShape()
         _check(self.L.odla_GetRuntimeShape(self.ctx, h, ctypes.byref(s)), "odla_GetRuntimeShape")
-        return tuple(s.dims[i] for i in range(s.size))
+        return tuple(s.dims[:s.size])
 
     def run(self, feeds):
         """feeds: name -> numpy array.  Returns name -> numpy array."""
@@ -715,12 +715,12 @@ class Session:
             a = np.ascontiguousarray(feeds[name], dtype=dt)
             assert tuple(a.shape) == self.runtime_shape(h), (name, a.shape, self.runtime_shape(h))
             keep.append(a)
-            _check(self.L.odla_BindToArgument(h, a.ctypes.data_as(ctypes.c_void_p), self.ctx), "odla_BindToArgument")
+            _check(self.L.odla_BindToArgument(h, a.ctypes.data, self.ctx), "odla_BindToArgument")
         outs = {}
         for name, (h, shape, dt) in self.b.outs.items():
             o = np.empty(self.runtime_shape(h), dt)
             outs[name] = o
-            _check(self.L.odla_BindToOutput(h, o.ctypes.data_as(ctypes.c_void_p), self.ctx), "odla_BindToOutput")
+            _check(self.L.odla_BindToOutput(h, o.ctypes.data, self.ctx), "odla_BindToOutput")
         _check(self.L.odla_ExecuteComputation(self.b.comp, self.ctx, ODLA_COMPUTE_INFERENCE, None), "odla_ExecuteComputation")
         return outs
 
