@@ -29,10 +29,16 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
 }
 // Round to nearest even; NaN stays NaN.
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+#if defined(__HIP_DEVICE_COMPILE__)
+  // one instruction for eight of integer arithmetic.  (By hand: a plain conversion of two
+  // neighbouring values is not accepted by the compiler without packed fp32 operations.)
+  uint32_t r;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %1" : "=v"(r) : "v"(f));
+  return (uint16_t)r;
+#else
+  (void)f;
+  return 0;
+#endif
 }
 __device__ __forceinline__ float f16_to_f32(uint16_t h) {
   _Float16 v;
@@ -63,6 +69,22 @@ template <> struct Store<bf16_t> {
   __device__ static __forceinline__ float ld(const bf16_t* p) { return bf16_to_f32(p->bits); }
   __device__ static __forceinline__ void st(bf16_t* p, float v) { p->bits = f32_to_bf16(v); }
 };
+
+// Two neighbouring 2-byte elements from floats.
+template <typename T> __device__ __forceinline__ unsigned pack2(float a, float b);
+template <> __device__ __forceinline__ unsigned pack2<f16_t>(float a, float b) {
+  return (unsigned)f32_to_f16(a) | (unsigned)f32_to_f16(b) << 16;
+}
+template <> __device__ __forceinline__ unsigned pack2<bf16_t>(float a, float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t r;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+#else
+  (void)a; (void)b;
+  return 0;
+#endif
+}
 
 // 16-byte vector of T viewed as floats.
 template <typename T> struct Vec16 {

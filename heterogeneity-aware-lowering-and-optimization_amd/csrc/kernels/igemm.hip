@@ -1263,6 +1263,12 @@ hipError_t launch_igemm(const IgemmParams& p_in, hipStream_t stream) {
     if (p.in_dt != DT_I8 || p.out_dt != DT_I8 || p.w_frag == nullptr || !(epi_vec & 2)) return hipErrorInvalidValue;
     return launch_igemm_stream_q8(p, stream);
   }
+  if (p.ln) {
+    if (!igemm_slim_ln_ok(p, p.w_frag != nullptr) || !aligned16(p.ln_x) || !aligned16(p.ln_y) || !aligned16(p.ln_g) || !aligned16(p.ln_b) ||
+        !aligned16(p.ln_y2) || p.ln_x == nullptr || p.ln_y == nullptr)
+      return hipErrorInvalidValue;
+    return launch_igemm_slim(p, epi_vec, igemm_slim_variant(p, p.w_frag != nullptr), stream);
+  }
   if (gemm_rowdot_shape(p)) return launch_gemm_rowdot(p, stream);
   if (p.row_softmax != 0) return hipErrorInvalidValue;   // (no other kernel finishes with a Softmax)
   if (const int big = igemm_big_variant(p)) return launch_igemm_big(p, epi_vec, big, stream);

@@ -10,6 +10,19 @@
 
 namespace ohip {
 
+// Kernel arguments are scalar loads that miss every cache in a fresh launch (some 0.5 us each), and
+// the compiler puts each next to its first use, one behind the other.  A launch of a few
+// microseconds names those it needs here, at its start: they are then requested together.
+template <typename... A>
+__device__ __forceinline__ void fetch_args(const A... a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  (..., [](const auto v) __attribute__((always_inline)) { asm volatile("" ::"s"(v)); }(a));
+#else
+  ((void)a, ...);
+#endif
+}
+
+
 // Element offset of result row m / column n / problem z (see IgemmParams::y_rdiv, y_zdiv).
 __device__ __forceinline__ int64_t y_row_off(const IgemmParams& p, const int m) {
   if (p.y_rdiv > 0) {

@@ -156,6 +156,17 @@ struct IgemmParams {
   void* f_y = nullptr;
   int f_kout = 0, f_ycs = 0, f_wf_chunks = 0;
   float f_q_add = 0.f, f_q_lo = 0.f;
+  // A LayerNorm over the C channels of every pixel in front of the product (igemm_slim_ln_ok says
+  // where): rows of ln_dt at ln_x, C elements apart, are normalised, become the operand (x is not
+  // read) and leave as ln_y (ln_dt) and, where asked for, as ln_y2 (in_dt).
+  bool ln = false;
+  DType ln_dt = DT_F32;
+  const void* ln_x = nullptr;
+  const float* ln_g = nullptr;   // scale and offset per channel, or null
+  const float* ln_b = nullptr;
+  float ln_eps = 0.f;
+  void* ln_y = nullptr;
+  void* ln_y2 = nullptr;
 };
 hipError_t launch_igemm(const IgemmParams& p, hipStream_t stream);
 // Name of the kernel variant launch_igemm would pick (for reports); small_tiles = false: of the
@@ -177,6 +188,8 @@ hipError_t launch_igemm_big(const IgemmParams& p, int epi_vec, int variant, hipS
 // the weights exist in fragment order; us: the estimated time in us, beside the launch itself.
 int igemm_slim_variant(const IgemmParams& p, bool frag, float* us = nullptr);
 hipError_t launch_igemm_slim(const IgemmParams& p, int epi_vec, int variant, hipStream_t stream);
+// Whether that kernel also takes a LayerNorm in front of the product (p.ln and p.ln_dt filled in).
+bool igemm_slim_ln_ok(const IgemmParams& p, bool frag);
 hipError_t launch_igemm_mid(const IgemmParams& p, int epi_vec, hipStream_t stream);
 
 // Streaming kernel for 8-bit 1x1 filters over short pixel rows (igemm_stream.hip):

@@ -166,6 +166,14 @@ class Planner {
     int tx = -1, tw = -1, ty = -1, tb = -1, tm = -1, tr = -1, tf = -1;
   };
   std::unordered_map<const _odla_value*, FuseProducer> fuse_prods_;   // by result value
+  // The last LayerNorm step: a product of few rows that follows it at once computes it itself (finish_igemm).
+  struct LastNorm {
+    int step = -1;
+    int tx = -1, ty = -1, t2 = -1, tg = -1, tb = -1;
+    int64_t len = 0;
+    float eps = 0.f;
+    DType dt = DT_F32;
+  } last_norm_;
   int root(int t) const {
     while (plan_->tensors[t].alias_of >= 0) t = plan_->tensors[t].alias_of;
     return t;
@@ -1387,6 +1395,35 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
   const bool hf = tf >= 0;
   log_igemm_choice(name, ip, hf, tr >= 0);
   const Ref rf = ref(hf ? tf : tx);
+  // the rows were normalised by the step right in front of this one: a launch of few rows takes that along
+  const LastNorm ln = last_norm_;
+  if (ln.step >= 0 && ln.step + 1 == (int)plan_->steps.size() && !in_init_ && T(tx).alias_off == 0 &&
+      (root(tx) == ln.ty || root(tx) == ln.t2) && ip.C == ln.len && ip.xcs == ln.len &&
+      (ln.tg < 0 || T(ln.tg).space == SP_CONST) && (ln.tb < 0 || T(ln.tb).space == SP_CONST)) {
+    IgemmParams q = ip;
+    q.ln = true;
+    q.ln_dt = ln.dt;
+    q.ln_eps = ln.eps;
+    if (igemm_slim_ln_ok(q, hf)) {
+      plan_->steps.pop_back();   // (its tensors keep their lifetimes: this step takes its number)
+      const bool hb = tb >= 0, hr = tr >= 0, hg = ln.tg >= 0, ho = ln.tb >= 0, h2 = ln.t2 >= 0;
+      const Ref rx = ref(ln.tx), rw = ref(tw), ry = ref(ty), rb = ref(hb ? tb : tx), rr = ref(hr ? tr : tx);
+      const Ref rg = ref(hg ? ln.tg : tx), ro = ref(ho ? ln.tb : tx), rn = ref(ln.ty), r2 = ref(h2 ? ln.t2 : tx);
+      emit("layernorm+" + name, {ln.tx, tw, tr}, {ty, ln.ty, ln.t2}, [=](const ExecEnv& e, hipStream_t st) {
+        IgemmParams p = q;
+        p.x = p.ln_x = rx(e); p.w = rw(e); p.y = ry(e);
+        p.bias = hb ? rb(e) : nullptr;
+        p.residual = hr ? rr(e) : nullptr;
+        p.w_frag = hf ? rf(e) : nullptr;
+        p.ln_g = hg ? (const float*)rg(e) : nullptr;
+        p.ln_b = ho ? (const float*)ro(e) : nullptr;
+        p.ln_y = rn(e);
+        p.ln_y2 = h2 ? r2(e) : nullptr;
+        return launch_igemm(p, st);
+      });
+      return;
+    }
+  }
   const Ref rx = ref(tx), rw = ref(tw), ry = ref(ty);
   const Ref rb = ref(tb >= 0 ? tb : tx), rr = ref(tr >= 0 ? tr : tx);
   const bool hb = tb >= 0, hr = tr >= 0;
@@ -3303,6 +3340,7 @@ void Planner::lower_layernorm(int ni) {
     return launch_layernorm(a(e), b(e), dt, rows, len, hg ? (const float*)rg(e) : nullptr,
                             hb ? (const float*)rb(e) : nullptr, eps, st, dual ? b2(e) : nullptr, dt2);
   }, kWrites16);
+  if (!calib_ && !in_init_) last_norm_ = {(int)plan_->steps.size() - 1, tx, ty, t2, tg, tb, len, eps, dt};
   set_main(n.out, ty);
   if (dual) vs_[n.out->index].slot[L_ROWMAJOR][FORM_OPERAND] = t2;
 }
