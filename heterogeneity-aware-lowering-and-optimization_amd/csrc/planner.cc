@@ -166,9 +166,10 @@ class Planner {
     int tx = -1, tw = -1, ty = -1, tb = -1, tm = -1, tr = -1, tf = -1;
   };
   std::unordered_map<const _odla_value*, FuseProducer> fuse_prods_;   // by result value
-  // The last LayerNorm step: a product of few rows that follows it at once computes it itself (finish_igemm).
+  // The LayerNorm whose launch is the last step of the plan (ty < 0: the last step is something
+  // else; every emitted step clears it): a product of few rows that comes next computes it itself
+  // in place of that step (finish_igemm).
   struct LastNorm {
-    int step = -1;
     int tx = -1, ty = -1, t2 = -1, tg = -1, tb = -1;
     int64_t len = 0;
     float eps = 0.f;
@@ -217,6 +218,7 @@ class Planner {
     }
     touch((int)plan_->steps.size(), reads, writes, exact);
     plan_->steps.push_back({name, std::move(fn)});
+    last_norm_ = LastNorm();
   }
   // Step `idx` reads and writes these tensors.
   void touch(const int idx, const std::vector<int>& reads, const std::vector<int>& writes, unsigned exact) {
@@ -1397,7 +1399,7 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
   const Ref rf = ref(hf ? tf : tx);
   // the rows were normalised by the step right in front of this one: a launch of few rows takes that along
   const LastNorm ln = last_norm_;
-  if (ln.step >= 0 && ln.step + 1 == (int)plan_->steps.size() && !in_init_ && T(tx).alias_off == 0 &&
+  if (ln.ty >= 0 && !in_init_ && T(tx).alias_off == 0 &&
       (root(tx) == ln.ty || root(tx) == ln.t2) && ip.C == ln.len && ip.xcs == ln.len &&
       (ln.tg < 0 || T(ln.tg).space == SP_CONST) && (ln.tb < 0 || T(ln.tb).space == SP_CONST)) {
     IgemmParams q = ip;
@@ -3340,7 +3342,7 @@ void Planner::lower_layernorm(int ni) {
     return launch_layernorm(a(e), b(e), dt, rows, len, hg ? (const float*)rg(e) : nullptr,
                             hb ? (const float*)rb(e) : nullptr, eps, st, dual ? b2(e) : nullptr, dt2);
   }, kWrites16);
-  if (!calib_ && !in_init_) last_norm_ = {(int)plan_->steps.size() - 1, tx, ty, t2, tg, tb, len, eps, dt};
+  if (!calib_ && !in_init_) last_norm_ = {tx, ty, t2, tg, tb, len, eps, dt};
   set_main(n.out, ty);
   if (dual) vs_[n.out->index].slot[L_ROWMAJOR][FORM_OPERAND] = t2;
 }

@@ -42,3 +42,50 @@ def test_layernorm_rides_in_the_product(rows, c, affine, mode):
     for name in want:
         err = np.abs(got[name] - want[name]).max() / np.abs(want[name]).max()
         assert err <= TOL[mode], (name, err)
+
+
+def forms(rows, c):
+    """Graphs in which the product with the LayerNorm in its launch is not the rows' only reader."""
+    r = np.random.default_rng(rows * c)
+    w = {n: (r.standard_normal((c, n)) * c ** -0.5).astype(np.float32) for n in (c, 256, 72)}
+    norm = lambda b, t, name: b.layernorm(t, 1, 1e-5, name=name)
+    mm = lambda b, t, n, name: b.gemm(t, b.const(name + ".w", w[n]), None, False, False, 1.0, 0.0, name=name)
+
+    def two_widths(b):
+        h = norm(b, b.arg("x", (rows, c)), "h")
+        b.output(mm(b, h, c, "q"), "q")
+        b.output(mm(b, h, 256, "k"), "k")
+
+    def three_widths_and_the_rows(b):
+        h = norm(b, b.arg("x", (rows, c)), "h")
+        b.output(b.gelu(mm(b, h, c, "q"), False, name="act"), "q")
+        b.output(mm(b, h, 256, "k"), "k")
+        b.output(mm(b, h, 72, "v"), "v")
+        b.output(h, "rows")
+
+    return {f.__name__: f for f in (two_widths, three_widths_and_the_rows)}
+
+
+@pytest.mark.parametrize("mode", list(KW))
+@pytest.mark.parametrize("rows,c", [(1, 768), (41, 768), (17, 512)])
+@pytest.mark.parametrize("form", list(forms(1, 64)))
+def test_other_readers_of_the_rows(form, rows, c, mode):
+    """Two inputs through one context: what the second leaves is not what the first left."""
+    announce("readers of layernorm rows: %s %d x %d %s" % (form, rows, c, mode))
+    build = forms(rows, c)[form]
+    feeds = [{"x": (np.random.default_rng(s).standard_normal((rows, c)) * (1 + s)).astype(np.float32)} for s in (0, 1)]
+    hb = entry.load().odla.HipBuilder(**KW[mode])
+    try:
+        build(hb)
+        s = hb.session()
+        try:
+            got = [s.run(f) for f in feeds]
+        finally:
+            s.close()
+    finally:
+        hb.destroy()
+    for f, g in zip(feeds, got):
+        want = run_ref(build, f)
+        for name in want:
+            err = np.abs(g[name] - want[name]).max() / np.abs(want[name]).max()
+            assert err <= TOL[mode], (name, err)
