@@ -27,18 +27,14 @@ struct f16_t { uint16_t bits; };
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
   return __uint_as_float(((uint32_t)b) << 16);
 }
-// Round to nearest even; NaN stays NaN.
+// Round to nearest even; NaN stays NaN.  v_cvt_pk_bf16_f32: one instruction for eight of integer
+// arithmetic.  A conversion the compiler knows, not inline assembly: behind that it takes the
+// epilogues with the transcendental activations for too large to unroll, and their accumulators
+// go to scratch memory (up to 576 bytes per lane of the 256 x 256 tile).  What the compiler does
+// not accept without packed fp32 operations is the conversion of two values it has just negated
+// as a pair: unary_kernel turns sign bits instead.
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  // one instruction for eight of integer arithmetic.  (By hand: a plain conversion of two
-  // neighbouring values is not accepted by the compiler without packed fp32 operations.)
-  uint32_t r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %1" : "=v"(r) : "v"(f));
-  return (uint16_t)r;
-#else
-  (void)f;
-  return 0;
-#endif
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
 }
 __device__ __forceinline__ float f16_to_f32(uint16_t h) {
   _Float16 v;
@@ -76,14 +72,9 @@ template <> __device__ __forceinline__ unsigned pack2<f16_t>(float a, float b) {
   return (unsigned)f32_to_f16(a) | (unsigned)f32_to_f16(b) << 16;
 }
 template <> __device__ __forceinline__ unsigned pack2<bf16_t>(float a, float b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-#else
-  (void)a; (void)b;
-  return 0;
-#endif
+  typedef float floatx2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((floatx2){a, b}, bf16x2));
 }
 
 // 16-byte vector of T viewed as floats.

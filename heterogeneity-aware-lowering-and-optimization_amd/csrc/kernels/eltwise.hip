@@ -44,8 +44,12 @@ unary_kernel(const T* __restrict__ x, T* __restrict__ y, int64_t n, ActKind act,
   for (int u = 0; u < U; ++u) {
     const int64_t i = base + u * kThreads;
     if (i < nvec) {
+      if constexpr (KIND == ACT_NEG) {   // (sign bits, a word at a time: see f32_to_bf16)
+        v[u].raw ^= sizeof(T) == 4 ? 0x80000000u : 0x80008000u;
+      } else {
 #pragma unroll
-      for (int e = 0; e < V; ++e) v[u].set(e, apply_act(v[u].get(e), kind, a, b));
+        for (int e = 0; e < V; ++e) v[u].set(e, apply_act(v[u].get(e), kind, a, b));
+      }
       out_store(v[u], y + i * V);
     }
   }

@@ -427,3 +427,17 @@ def test_quantize_dequantize_sweep():
             b.output(b.dequantize(q, scale, zp, axis, name="d", zp_dtype=zp.dtype), "d")
 
         check(build, {"x": X}, tag=tag, modes=("fp32",))
+
+
+@pytest.mark.parametrize("mode", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("n", [1, 7, 8, 255, 8 * 256 * 4 + 3])
+def test_negation_turns_the_sign_bit_only(n, mode):
+    """Exact, zeros, infinities and subnormals included (whole vectors and the elements behind them)."""
+    announce("neg %d %s" % (n, mode))
+    x = np.resize(np.array([0.0, -0.0, 1.5, -2.0, np.inf, -np.inf, 2.0 ** -24, -3.0, np.nan], np.float32), n)
+
+    def build(b):
+        b.output(b.neg(b.arg("x", (n,)), name="y"), "y")
+    got = run_hip(build, {"x": x}, **{"fp32": {}, "fp16": {"fp16": True}, "bf16": {"bf16": "performance"}}[mode])["y"]
+    nan = np.isnan(x)
+    assert np.isnan(got[nan]).all() and (got.view(np.uint32)[~nan] == (-x).view(np.uint32)[~nan]).all()

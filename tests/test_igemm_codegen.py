@@ -2,7 +2,7 @@
 speed rely on and that a compiler change could silently break:
 
   * no igemm kernel uses scratch memory (spilled accumulators cost an order of
-    magnitude);
+    magnitude), and no kernel of the built library keeps an array there;
   * in igemm_wreg_kernel the weight fragments are requested by inline assembly
     into registers the compiler knows nothing about while the request is in
     flight: each fragment keeps one register quad, and between the pipeline
@@ -54,6 +54,27 @@ def test_no_scratch(compiled):
         scratch = int(re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b).group(1))
         assert scratch == 0, (name, scratch)
     assert seen >= 40
+
+
+def test_no_array_in_scratch(tmp_path):
+    """All kernels of the built library, by the metadata of their code objects.  (A value or two
+    of a thread that waits out a loop is not an array: 16 bytes.)"""
+    tools = "/opt/rocm/llvm/bin/"
+    if not os.path.exists(tools + "llvm-objdump"):
+        pytest.skip("llvm-objdump not available")
+    lib = shutil.copy(os.path.join(entry.PKG_DIR, "libodla_hip.so"), tmp_path)
+    subprocess.run([tools + "llvm-objdump", "--offloading", lib], cwd=tmp_path, check=True, capture_output=True)
+    seen = 0
+    for f in sorted(os.listdir(tmp_path)):
+        if not f.endswith("gfx950"):
+            continue
+        notes = subprocess.run([tools + "llvm-readelf", "--notes", f], cwd=tmp_path, check=True, capture_output=True, text=True).stdout
+        kernels = re.findall(r"\.name: +(_Z\w+)\n(?:.*\n)*? +\.private_segment_fixed_size: (\d+)", notes)
+        assert len(kernels) == notes.count(".private_segment_fixed_size:"), f
+        for name, scratch in kernels:
+            seen += 1
+            assert int(scratch) <= 16, (name, scratch)
+    assert seen >= 500
 
 
 def kernel_bodies(asm, prefix):
