@@ -1397,10 +1397,12 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
   const bool hf = tf >= 0;
   log_igemm_choice(name, ip, hf, tr >= 0);
   const Ref rf = ref(hf ? tf : tx);
-  // the rows were normalised by the step right in front of this one: a launch of few rows takes that along
+  // The rows were normalised by the step right in front of this one: a launch of few rows takes that
+  // along.  Not one that reads the rows as anything but its left operand (residual, weights): the
+  // workgroups that write them are not ordered before the others.
   const LastNorm ln = last_norm_;
-  if (ln.ty >= 0 && !in_init_ && T(tx).alias_off == 0 &&
-      (root(tx) == ln.ty || root(tx) == ln.t2) && ip.C == ln.len && ip.xcs == ln.len &&
+  auto normalised = [&](const int t) { return t >= 0 && (root(t) == ln.ty || root(t) == ln.t2); };
+  if (ln.ty >= 0 && !in_init_ && T(tx).alias_off == 0 && normalised(tx) && !normalised(tr) && !normalised(tw) && ip.C == ln.len && ip.xcs == ln.len &&
       (ln.tg < 0 || T(ln.tg).space == SP_CONST) && (ln.tb < 0 || T(ln.tb).space == SP_CONST)) {
     IgemmParams q = ip;
     q.ln = true;

@@ -63,7 +63,23 @@ def forms(rows, c):
         b.output(mm(b, h, 72, "v"), "v")
         b.output(h, "rows")
 
-    return {f.__name__: f for f in (two_widths, three_widths_and_the_rows)}
+    def residual(b):
+        h = norm(b, b.arg("x", (rows, c)), "h")
+        b.output(b.add(mm(b, h, c, "p"), h, name="y"), "y")
+
+    def addend_of_a_view(b):
+        h = b.reshape(norm(b, b.arg("x", (rows, c)), "h"), (1, rows, c), name="v")
+        b.output(b.gemm(h, b.const("p.w", w[c]), h, False, False, 1.0, 1.0, name="y"), "y")
+
+    def residual_in_front_of_the_norm(b):
+        x = b.arg("x", (rows, c))
+        b.output(b.add(mm(b, norm(b, x, "h"), c, "p"), x, name="y"), "y")
+
+    def outer_product(b):
+        h = norm(b, b.arg("x", (rows, c)), "h")
+        b.output(b.gemm(h, h, None, False, True, 1.0, 0.0, name="y"), "y")
+
+    return {f.__name__: f for f in (two_widths, three_widths_and_the_rows, residual, addend_of_a_view, residual_in_front_of_the_norm, outer_product)}
 
 
 @pytest.mark.parametrize("mode", list(KW))

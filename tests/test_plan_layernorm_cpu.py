@@ -58,3 +58,52 @@ def test_every_product_over_the_rows_has_its_launch(odla, widths, mode):
     norm = [i for i, s in enumerate(steps) if "layernorm" in s][0]
     for i in range(len(widths)):
         assert position(steps, "p%d" % i) >= norm, steps
+
+
+# products that read the normalised rows a second time, as their residual or their right operand
+def residual(b, rows):
+    h = b.layernorm(b.arg("x", (rows, 768)), 1, 1e-5, name="h")
+    b.output(b.add(product(b, h, "p", 768, 768), h, name="y"), "y")
+
+
+def addend(b, rows):
+    h = b.layernorm(b.arg("x", (rows, 768)), 1, 1e-5, name="h")
+    b.output(b.gemm(h, weight(b, "p.w", 768, 768), h, False, False, 1.0, 1.0, name="y"), "y")
+
+
+def residual_view(b, rows):
+    h = b.layernorm(b.arg("x", (rows, 768)), 1, 1e-5, name="h")
+    v = b.reshape(h, (1, rows, 768), name="v")
+    b.output(b.add(product(b, v, "p", 768, 768), v, name="y"), "y")
+
+
+def residual_behind_activation(b, rows):
+    h = b.layernorm(b.arg("x", (rows, 768)), 1, 1e-5, name="h")
+    b.output(b.add(b.relu(product(b, h, "p", 768, 768), name="r"), h, name="y"), "y")
+
+
+def outer_product(b, rows):
+    h = b.layernorm(b.arg("x", (rows, 768)), 1, 1e-5, name="h")
+    b.output(b.gemm(h, h, None, False, True, 1.0, 0.0, name="y"), "y")
+
+
+TWICE = [residual, addend, residual_view, residual_behind_activation, outer_product]
+
+
+@pytest.mark.parametrize("mode", list(MODES))
+@pytest.mark.parametrize("rows", [1, 41])
+@pytest.mark.parametrize("build", TWICE, ids=lambda f: f.__name__)
+def test_rows_read_twice_are_written_by_a_launch_in_front(odla, build, rows, mode):
+    steps = steps_of(odla, lambda b: build(b, rows), **MODES[mode])
+    assert [s for s in steps if "layernorm" in s] == ["layernorm:h"], steps
+    assert steps.index("layernorm:h") < position(steps, "y"), steps
+
+
+@pytest.mark.parametrize("mode", list(MODES))
+def test_residual_of_the_rows_in_front_of_the_norm_still_rides(odla, mode):
+    def build(b):
+        x = b.arg("x", (41, 768))
+        h = b.layernorm(x, 1, 1e-5, name="h")
+        b.output(b.add(product(b, h, "p", 768, 768), x, name="y"), "y")
+
+    assert "layernorm+gemm:y" in steps_of(odla, build, **MODES[mode])
