@@ -390,20 +390,30 @@ transpose2d_kernel(const E* __restrict__ x, E* __restrict__ y, int batch, int ro
 }
 
 // Nearest resize: a workgroup row (grid.y) is one result row, whose source row is found once; x
-// covers the row's units (cv per pixel; pitches xv / yv in units).  Divisions by magic pairs.
+// covers the row's units (cv per pixel; pitches xv / yv in units).  I: the type that the rows, the
+// units of a row and the source column's numerator (wo * W) are counted in; 32-bit ones are divided
+// by magic pairs, 64-bit ones (signals of tens of thousands of points) by division.
 struct ResizeDiv { unsigned cv_magic, wo_magic; int cv_shift, wo_shift; };
-template <typename E>
+template <typename E, typename I>
 __global__ void __launch_bounds__(kThreads)
-resize_nearest_kernel(const E* __restrict__ x, E* __restrict__ y, int rows, int H, int W, int cv, int xv, int yv, int Ho, int Wo,
+resize_nearest_kernel(const E* __restrict__ x, E* __restrict__ y, I rows, int H, int W, int cv, int xv, int yv, int Ho, int Wo,
                       ResizeDiv d) {
-  for (int row = blockIdx.y; row < rows; row += gridDim.y) {
-    const int n = row / Ho, ho = row - n * Ho;
+  for (I row = blockIdx.y; row < rows; row += gridDim.y) {
+    const I n = row / Ho;
+    const int ho = (int)(row - n * Ho);
     const int hi = (int)(((int64_t)ho * H) / Ho);
     const E* src = x + ((int64_t)n * H + hi) * W * xv;
     E* dst = y + (int64_t)row * Wo * yv;
-    for (int j = blockIdx.x * kThreads + threadIdx.x; j < Wo * cv; j += gridDim.x * kThreads) {
-      const int wo = fast_div(j, d.cv_magic, d.cv_shift), c = j - wo * cv;
-      const int wi = fast_div(wo * W, d.wo_magic, d.wo_shift);
+    for (I j = blockIdx.x * kThreads + threadIdx.x; j < (I)Wo * cv; j += gridDim.x * kThreads) {
+      int wo, wi;
+      if constexpr (sizeof(I) == 4) {
+        wo = fast_div(j, d.cv_magic, d.cv_shift);
+        wi = fast_div(wo * W, d.wo_magic, d.wo_shift);
+      } else {
+        wo = (int)(j / cv);
+        wi = (int)(((int64_t)wo * W) / Wo);
+      }
+      const int c = (int)(j - (I)wo * cv);
       dst[(int64_t)wo * yv + c] = src[(int64_t)wi * xv + c];
     }
   }
@@ -809,11 +819,11 @@ hipError_t launch_transpose2d(const void* x, void* y, int elem_size, int batch, 
 hipError_t launch_resize_nearest_nhwc(const void* x, void* y, int elem_size, int N, int H, int W, int C, int cs, int ycs,
                                       int Ho, int Wo, hipStream_t stream) {
   if (!x || !y || N <= 0 || H <= 0 || W <= 0 || C <= 0 || cs < C || ycs < C || Ho <= 0 || Wo <= 0) return hipErrorInvalidValue;
-  if ((int64_t)N * Ho >= (1ll << 31) || (int64_t)Wo * C >= (1ll << 31) || (int64_t)Wo * W >= (1ll << 31)) return hipErrorInvalidValue;
   const int64_t bytes = (int64_t)C * elem_size;
   const bool v16 = bytes % 16 == 0 && (int64_t)cs * elem_size % 16 == 0 && (int64_t)ycs * elem_size % 16 == 0 &&
                    ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0;
-  if (v16 && cs == C && Ho % H == 0 && Wo % W == 0 && (int64_t)N * H < (1ll << 31) && (int64_t)W * (bytes / 16) < (1ll << 31)) {
+  constexpr int64_t kFar = 1ll << 30;   // 32-bit counters below it hold a whole grid's step more
+  if (v16 && cs == C && Ho % H == 0 && Wo % W == 0 && (int64_t)N * H < kFar && (int64_t)W * (bytes / 16) < kFar) {
     // (nearest: source index floor(o * in / out) = o / factor)
     const int cv = (int)(bytes / 16);
     const int64_t rows = (int64_t)N * H;
@@ -828,10 +838,19 @@ hipError_t launch_resize_nearest_nhwc(const void* x, void* y, int elem_size, int
   ResizeDiv d;
   div_magic(cv, &d.cv_magic, &d.cv_shift);
   div_magic(Wo, &d.wo_magic, &d.wo_shift);
-  const int rows = N * Ho;
-  const int64_t pieces = ((int64_t)Wo * cv + kThreads - 1) / kThreads;
+  const int64_t rows = (int64_t)N * Ho, units = (int64_t)Wo * cv;
+  const bool near = rows < kFar && units < kFar && (int64_t)Wo * W < kFar;
+  const int64_t pieces = (units + kThreads - 1) / kThreads;
   const dim3 grid((unsigned)(pieces < 64 ? pieces : 64), (unsigned)(rows < 65535 ? rows : 65535));
-#define RESIZE_GO(E_) hipLaunchKernelGGL(resize_nearest_kernel<E_>, grid, dim3(kThreads), 0, stream, (const E_*)x, (E_*)y, rows, H, W, cv, cs / unit, ycs / unit, Ho, Wo, d)
+#define RESIZE_GO(E_)                                                                                                             \
+  do {                                                                                                                            \
+    if (near)                                                                                                                     \
+      hipLaunchKernelGGL((resize_nearest_kernel<E_, int>), grid, dim3(kThreads), 0, stream, (const E_*)x, (E_*)y, (int)rows, H, W, \
+                         cv, cs / unit, ycs / unit, Ho, Wo, d);                                                                   \
+    else                                                                                                                          \
+      hipLaunchKernelGGL((resize_nearest_kernel<E_, int64_t>), grid, dim3(kThreads), 0, stream, (const E_*)x, (E_*)y, rows, H, W,  \
+                         cv, cs / unit, ycs / unit, Ho, Wo, d);                                                                   \
+  } while (0)
   if (v16) RESIZE_GO(b16);
   else if (elem_size == 1) RESIZE_GO(uint8_t);
   else if (elem_size == 2) RESIZE_GO(uint16_t);
