@@ -91,19 +91,13 @@ __global__ void __launch_bounds__(kThreads) pool2d_vec_kernel(PoolParams p) {
   }
 }
 
-// Scalar-channel fallback (C not a multiple of the vector width).
-template <typename T, bool IS_MAX>
+// Scalar-channel fallback (C not a multiple of the vector width): a thread per position and channel
+// of an image.  FAR: an image of more elements than 32 bits count, all images in one run of indices.
+template <typename T, bool IS_MAX, bool FAR>
 __global__ void __launch_bounds__(kThreads) pool2d_scalar_kernel(PoolParams p) {
   const T* x = reinterpret_cast<const T*>(p.x);
   T* y = reinterpret_cast<T*>(p.y);
-  const int i = blockIdx.x * kThreads + threadIdx.x;   // position and channel within an image
-  const int row_units = p.Wo * p.C;
-  if (i >= p.Ho * row_units) return;
-  const int ho = fast_div(i, p.row_magic, p.row_shift);
-  const int rem = i - ho * row_units;
-  const int wo = fast_div(rem, p.cv_magic, p.cv_shift);
-  const int c = rem - wo * p.C;
-  for (int n = blockIdx.y; n < p.N; n += gridDim.y) {
+  auto at = [&](const int n, const int ho, const int wo, const int c) __attribute__((always_inline)) {
     const int h0 = ho * p.sh - p.ph, w0 = wo * p.sw - p.pw;
     float acc = IS_MAX ? -INFINITY : 0.f;
     int cnt = 0;
@@ -120,6 +114,23 @@ __global__ void __launch_bounds__(kThreads) pool2d_scalar_kernel(PoolParams p) {
     }
     if (!IS_MAX) acc /= (float)(p.count_include_pad ? p.kh * p.kw : (cnt > 0 ? cnt : 1));
     Store<T>::st(y + (((int64_t)n * p.Ho + ho) * p.Wo + wo) * p.ycs + c, acc);
+  };
+  if constexpr (FAR) {
+    const int64_t total = (int64_t)p.N * p.Ho * p.Wo * p.C;
+    for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < total; i += (int64_t)gridDim.x * kThreads) {
+      const int c = (int)(i % p.C);
+      int64_t t = i / p.C;
+      const int wo = (int)(t % p.Wo); t /= p.Wo;
+      at((int)(t / p.Ho), (int)(t % p.Ho), wo, c);
+    }
+  } else {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    const int row_units = p.Wo * p.C;
+    if (i >= p.Ho * row_units) return;
+    const int ho = fast_div(i, p.row_magic, p.row_shift);
+    const int rem = i - ho * row_units;
+    const int wo = fast_div(rem, p.cv_magic, p.cv_shift);
+    for (int n = blockIdx.y; n < p.N; n += gridDim.y) at(n, ho, wo, rem - wo * p.C);
   }
 }
 
@@ -917,12 +928,18 @@ hipError_t launch_pool2d(const PoolParams& p_in, hipStream_t stream) {
 #undef POOL_LAUNCH
   } else {
     const int64_t per_image = (int64_t)p.Ho * p.Wo * p.C;
-    if (per_image >= (1ll << 31)) return hipErrorInvalidValue;
+#define POOL_SCALAR(MAX_, FAR_, GRID_) \
+  FLOAT_DISPATCH(p.dt, hipLaunchKernelGGL((pool2d_scalar_kernel<T, MAX_, FAR_>), GRID_, dim3(kThreads), 0, stream, p))
+    if (per_image >= (1ll << 31)) {
+      const dim3 grid((unsigned)grid_for((int64_t)p.N * per_image, kThreads));
+      if (p.is_max) { POOL_SCALAR(true, true, grid); } else { POOL_SCALAR(false, true, grid); }
+      return hipGetLastError();
+    }
     div_magic(p.Wo * p.C, &p.row_magic, &p.row_shift);
     div_magic(p.C, &p.cv_magic, &p.cv_shift);
     const dim3 grid((unsigned)((per_image + kThreads - 1) / kThreads), (unsigned)(p.N < 65535 ? p.N : 65535));
-    if (p.is_max) { FLOAT_DISPATCH(p.dt, hipLaunchKernelGGL((pool2d_scalar_kernel<T, true>), grid, dim3(kThreads), 0, stream, p)); }
-    else { FLOAT_DISPATCH(p.dt, hipLaunchKernelGGL((pool2d_scalar_kernel<T, false>), grid, dim3(kThreads), 0, stream, p)); }
+    if (p.is_max) { POOL_SCALAR(true, false, grid); } else { POOL_SCALAR(false, false, grid); }
+#undef POOL_SCALAR
   }
   return hipGetLastError();
 }
