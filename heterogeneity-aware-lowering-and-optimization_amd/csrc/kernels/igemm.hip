@@ -21,6 +21,7 @@
 // the exact k permutation inside one MFMA is irrelevant to the result.
 #include "igemm_common.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -1189,7 +1190,44 @@ const char* igemm_variant_name(const IgemmParams& p, const bool small_tiles) {
   return choose_variant(p).name;
 }
 
+namespace {
+
+constexpr int kMaxBatch = 65535;   // a grid's limit in z
+
+// More problems than one grid holds: launches of whole groups of y_zdiv (or, of a longer group, of
+// pieces).  32768 strides of any size keep every base as aligned as the first.
+hipError_t launch_in_parts(const IgemmParams& all, hipStream_t stream) {
+  if (all.x == nullptr || all.w == nullptr || all.y == nullptr || all.f_y != nullptr || all.ln) return hipErrorInvalidValue;
+  const int es = dtype_size(all.in_dt), oes = dtype_size(all.out_dt), bias_es = 4;
+  auto at = [](const void* base, const int64_t bytes) { return base == nullptr ? nullptr : static_cast<const char*>(base) + bytes; };
+  for (int z = 0; z < all.batch;) {
+    int n = std::min(all.batch - z, 32768);
+    int64_t y = z * all.y_bs;
+    if (all.y_zdiv > 0) {
+      const int u = z / all.y_zdiv, v = z - u * all.y_zdiv;
+      if (v == 0 && n >= all.y_zdiv) n -= n % all.y_zdiv;
+      else n = std::min(n, all.y_zdiv - v);
+      y = u * all.y_bs_hi + v * all.y_bs;
+    }
+    IgemmParams p = all;
+    p.batch = n;
+    p.x = at(all.x, z * all.x_bs * es);
+    p.w = at(all.w, z * all.w_bs * es);
+    p.w_frag = at(all.w_frag, (int64_t)z * all.wf_tiles * all.wf_chunks * 1024);
+    p.y = const_cast<char*>(at(all.y, y * oes));
+    p.bias = at(all.bias, z * all.bias_bs * bias_es);
+    p.residual = at(all.residual, z * all.r_bs * oes);
+    const hipError_t e = launch_igemm(p, stream);
+    if (e != hipSuccess) return e;
+    z += n;
+  }
+  return hipSuccess;
+}
+
+}  // namespace
+
 hipError_t launch_igemm(const IgemmParams& p_in, hipStream_t stream) {
+  if (p_in.batch > kMaxBatch) return launch_in_parts(p_in, stream);
   IgemmParams p = p_in;
   if (p.Ho > 0 && p.Wo > 0) {
     div_magic(p.Ho * p.Wo, &p.howo_magic, &p.howo_shift);
