@@ -4,9 +4,9 @@
 // What bounds such a launch is not bandwidth or the matrix cores but one workgroup's chain of
 // K stages (128-pixel x 128-channel tiles: ResNet-50's last 3x3 layer at one image is four
 // workgroups of 72 stages, 32 us) on a mostly idle chip.  Here
-//   - the output tile is small (16 .. 64 pixels x 16 .. 64 channels, 16x16 MFMA blocks), so that
+//   - the output tile is small (16 x 16 or 32 x 32 pixels x channels, 16x16 MFMA blocks), so that
 //     a layer of 49 pixels x 512 channels is 128 workgroups instead of four;
-//   - the wavefronts of a workgroup (4 .. 16) all own the SAME tile and split K: each walks a
+//   - the wavefronts of a workgroup (16 or 8 of them) all own the SAME tile and split K: each walks a
 //     contiguous share of the 64-byte K steps, so the chain is a few steps long and its loads
 //     are all in flight together;
 //   - both operands go straight from global memory into MFMA registers (16 bytes per lane; the
@@ -26,7 +26,6 @@
 // launches less.
 #include "igemm_common.h"
 
-#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 
@@ -517,7 +516,6 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
 // ---------------------------------------------------------------------------
 namespace {
 
-
 template <typename TIn, typename Epi, int MB, int NB, int NW>
 hipError_t launch_tile(const IgemmParams& p, const int epi_vec, SlimArgs a, const int mode, hipStream_t stream) {
   const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
@@ -527,19 +525,8 @@ hipError_t launch_tile(const IgemmParams& p, const int epi_vec, SlimArgs a, cons
   a.tiles_n = (int)tn;
   constexpr size_t lds = (size_t)NW * MB * 16 * (NB * 16 + 4) * 4;
   const dim3 grid((unsigned)(tm * tn), 1, (unsigned)p.batch), block(NW * 64);
-#define SLIM_LAUNCH(MODE_)                                                                                            \
-  do {                                                                                                                \
-    if constexpr (lds > 65536) {                                                                                      \
-      static bool ready = false; /* (repeating the call is harmless: no lock) */                                      \
-      if (!ready) {                                                                                                   \
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&igemm_slim_kernel<TIn, Epi, MB, NB, NW, MODE_>), \
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
-        if (e != hipSuccess) return e;                                                                                \
-        ready = true;                                                                                                 \
-      }                                                                                                               \
-    }                                                                                                                 \
-    hipLaunchKernelGGL((igemm_slim_kernel<TIn, Epi, MB, NB, NW, MODE_>), grid, block, lds, stream, p, epi_vec, a);    \
-  } while (0)
+  static_assert(lds <= 65536, "more than a launch may ask for by itself");
+#define SLIM_LAUNCH(MODE_) hipLaunchKernelGGL((igemm_slim_kernel<TIn, Epi, MB, NB, NW, MODE_>), grid, block, lds, stream, p, epi_vec, a)
   if constexpr (std::is_same<TIn, f16_t>::value || std::is_same<TIn, bf16_t>::value) {
     if (mode == SLIM_LN32) { SLIM_LAUNCH(SLIM_LN32); return hipGetLastError(); }
   }
