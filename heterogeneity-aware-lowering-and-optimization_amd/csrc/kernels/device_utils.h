@@ -9,6 +9,7 @@
 #include <stdint.h>
 
 #include "kernels.h"
+#include "lds_limit.h"
 
 namespace ohip {
 

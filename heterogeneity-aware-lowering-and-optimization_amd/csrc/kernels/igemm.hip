@@ -1002,13 +1002,9 @@ hipError_t launch_wreg(const IgemmParams& p, int epi_vec, hipStream_t stream) {
       return hipGetLastError();
     }
     if (wreg_k_groups(p, tiles * p.batch) == 2) {
-      static bool ready = false;   // (repeating the call is harmless: no lock)
-      if (!ready) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&igemm_wreg_kernel<TIn, Epi, 1, 2>),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * ring + mul));
-        if (e != hipSuccess) return e;
-        ready = true;
-      }
+      static LdsLimit limit;
+      const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_wreg_kernel<TIn, Epi, 1, 2>), (int)(2 * ring + mul));
+      if (e != hipSuccess) return e;
       hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 1, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(512),
                          2 * ring + mul, stream, p, epi_vec);
       return hipGetLastError();

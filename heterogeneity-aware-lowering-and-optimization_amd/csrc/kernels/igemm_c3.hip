@@ -397,13 +397,10 @@ hipError_t launch_c3(const IgemmParams& p, const int epi_vec, const C3Geom& g, h
   // (more than the 64 KiB a kernel may use without asking)
 #define C3_CASE(NKK, WS, NJ)                                                                                            \
   if (g.nkk == NKK && g.ws == WS && g.nj == NJ) {                                                                       \
-    static bool ready = false; /* (repeating the call is harmless: no lock) */                                          \
-    if (!ready) {                                                                                                       \
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&igemm_c3_kernel<TIn, Epi, NKK, WS, NJ>), \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, c3_main_bytes(NKK, WS, 2) + 512); \
-      if (e != hipSuccess) return e;                                                                                    \
-      ready = true;                                                                                                     \
-    }                                                                                                                   \
+    static LdsLimit limit;                                                                                              \
+    const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_c3_kernel<TIn, Epi, NKK, WS, NJ>),            \
+                                     c3_main_bytes(NKK, WS, 2) + 512);                                                  \
+    if (e != hipSuccess) return e;                                                                                      \
     hipLaunchKernelGGL((igemm_c3_kernel<TIn, Epi, NKK, WS, NJ>), grid, block, lds, stream, p, epi_vec, g);             \
     return hipGetLastError();                                                                                           \
   }

@@ -547,26 +547,18 @@ static hipError_t launch_stream_q8_rows(const IgemmParams& p, hipStream_t stream
   const int epi_vec = 3;   // rows and bases are 16-byte aligned (stream_q8_ready)
 #define ROWS_CASE(NKK_, NG_)                                                                                         \
   if (nkk == NKK_ && ng == NG_) {                                                                                    \
-    static bool attr_set = false;                                                                                   \
-    if (!attr_set) {                                                                                                \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&igemm_stream_q8_rows_kernel<NKK_, NG_, 4>), \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);                    \
-      if (e != hipSuccess) return e;                                                                                \
-      attr_set = true;                                                                                              \
-    }                                                                                                               \
+    static LdsLimit limit;                                                                                             \
+    const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_stream_q8_rows_kernel<NKK_, NG_, 4>), 96 * 1024); \
+    if (e != hipSuccess) return e;                                                                                     \
     hipLaunchKernelGGL((igemm_stream_q8_rows_kernel<NKK_, NG_, 4>), dim3((unsigned)grid, (unsigned)nsplit), dim3(4 * 64), lds, stream, \
                        p, (int)groups, epi_vec);                                                                    \
     return hipGetLastError();                                                                                       \
   }
 #define FUSED_CASE(NF_, NW_)                                                                                          \
   if (nf == NF_) {                                                                                                    \
-    static bool attr_set = false;                                                                                    \
-    if (!attr_set) {                                                                                                 \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&igemm_stream_q8_rows_kernel<2, 2, NW_, NF_>), \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);                    \
-      if (e != hipSuccess) return e;                                                                                 \
-      attr_set = true;                                                                                               \
-    }                                                                                                                \
+    static LdsLimit limit;                                                                                             \
+    const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_stream_q8_rows_kernel<2, 2, NW_, NF_>), 144 * 1024); \
+    if (e != hipSuccess) return e;                                                                                     \
     hipLaunchKernelGGL((igemm_stream_q8_rows_kernel<2, 2, NW_, NF_>), dim3((unsigned)grid, 1u), dim3(NW_ * 64), lds, stream, p, \
                        (int)groups, epi_vec);                                                                        \
     return hipGetLastError();                                                                                        \
@@ -620,13 +612,9 @@ hipError_t launch_igemm_stream_q8(const IgemmParams& p, hipStream_t stream) {
   if (grid > groups) grid = groups;
 #define STREAM_CASE(NKK_, NS_, NW_)                                                                                 \
   if (nkk == NKK_ && ns == NS_) {                                                                          \
-    static bool attr_set = false;                                                                                   \
-    if (!attr_set) {                                                                                                \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&igemm_stream_q8_kernel<NKK_, NS_, NW_>),   \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, kStreamMaxLds);               \
-      if (e != hipSuccess) return e;                                                                                \
-      attr_set = true;                                                                                              \
-    }                                                                                                               \
+    static LdsLimit limit;                                                                                             \
+    const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_stream_q8_kernel<NKK_, NS_, NW_>), kStreamMaxLds); \
+    if (e != hipSuccess) return e;                                                                                     \
     hipLaunchKernelGGL((igemm_stream_q8_kernel<NKK_, NS_, NW_>), dim3((unsigned)grid, (unsigned)nsplit), dim3(NW_ * 64), lds, stream, \
                        p, (int)groups);                                                                             \
     return hipGetLastError();                                                                                       \

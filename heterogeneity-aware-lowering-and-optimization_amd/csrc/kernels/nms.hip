@@ -463,13 +463,9 @@ static hipError_t launch_nms_kernel(const void* boxes, const float* best, int N,
   // slot), then boxes and flags in their place (16 + 1 B per slot): up to 8192 candidates
   const int lds_slots = (int)(bpad < 8192 ? bpad : 8192);
   const size_t lds_bytes = (size_t)lds_slots * 17;
-  static bool lds_limit_raised = false;  // (benign if two threads both do it)
-  if (!lds_limit_raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(nms_kernel<TB>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            8192 * 17) != hipSuccess)
-      return hipErrorInvalidValue;
-    lds_limit_raised = true;
-  }
+  static LdsLimit limit;
+  const hipError_t e = limit.raise(reinterpret_cast<const void*>(nms_kernel<TB>), 8192 * 17);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(nms_kernel<TB>, dim3(N), dim3(kNmsThreads), lds_bytes, stream, (const TB*)boxes, best, B, max_out,
                      iou_thr, masks, out, keys, cls, sup, bpad, lds_slots, image_base);
   return hipGetLastError();
