@@ -591,6 +591,7 @@ constexpr float kSlimMargin = 0.88f, kSlimMarginFull = 0.7f;
 
 int igemm_slim_variant(const IgemmParams& p, const bool frag, float* us) {
   if (us != nullptr) *us = 0.f;
+  if (p.slim >= 0) return p.slim;
   if (p.f_y != nullptr || p.row_softmax != 0 || p.fixed_order) return 0;
   // what the kernels' addressing assumes: 32-bit offsets inside an image, no column of K behind the packed rows
   const int es = dtype_size(p.in_dt);

@@ -127,6 +127,9 @@ struct IgemmParams {
   // fp32 sums of an 8-bit plan keep one order whatever the number of rows (an image's results do
   // not depend on its batch, bit for bit): no small-tile kernel.
   bool fixed_order = false;
+  // The small-tile kernel of this launch as igemm_slim_variant gave it when the plan was made (what
+  // the plan relies on then holds whatever the environment says later); -1: the launch asks itself.
+  int slim = -1;
   // Softmax (1) or LogSoftmax (2) over the Kout columns of every result row, behind bias and
   // activation: only the one-wavefront-per-row kernel computes it (gemm_rowdot_shape).
   int row_softmax = 0;

@@ -1395,6 +1395,7 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
   ip.stream_out = T(ty).bytes >= stream_out_bytes();
   const int tf = make_wfrag(name, &ip, tw);
   const bool hf = tf >= 0;
+  ip.slim = igemm_slim_variant(ip, hf);
   log_igemm_choice(name, ip, hf, tr >= 0);
   const Ref rf = ref(hf ? tf : tx);
   // The rows were normalised by the step right in front of this one: a launch of few rows takes that
@@ -1655,6 +1656,7 @@ void Planner::lower_conv(int ni) {
     ip.stream_out = T(ty).bytes >= stream_out_bytes();
     const int tf = make_wfrag("conv.i8:" + outv->name, &ip, tw);
     const bool hf = tf >= 0;
+    ip.slim = igemm_slim_variant(ip, hf);
     log_igemm_choice("conv.i8:" + outv->name, ip, hf, tr >= 0);
     const Ref rf = ref(hf ? tf : tx);
     const Ref rx = ref(tx), rw = ref(tw), ry = ref(ty), rb = ref(tb), rm = ref(tm), rr = ref(tr >= 0 ? tr : tx);

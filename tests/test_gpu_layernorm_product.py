@@ -105,3 +105,26 @@ def test_other_readers_of_the_rows(form, rows, c, mode):
         for name in want:
             err = np.abs(g[name] - want[name]).max() / np.abs(want[name]).max()
             assert err <= TOL[mode], (name, err)
+
+
+@pytest.mark.parametrize("mode", ["fp32", "bf16"])
+def test_a_plan_outlives_its_tuning_environment(mode, monkeypatch):
+    """Launches that are made anew on every execution keep the kernels of the plan."""
+    announce("plan and environment %s" % mode)
+    monkeypatch.setenv("ODLA_HIP_GRAPH_MIN_STEPS", "1000")
+    build = forms(41, 768)["three_widths_and_the_rows"]
+    feeds = {"x": np.random.default_rng(5).standard_normal((41, 768)).astype(np.float32)}
+    hb = entry.load().odla.HipBuilder(**KW[mode])
+    try:
+        build(hb)
+        s = hb.session()
+        try:
+            first = s.run(feeds)
+            monkeypatch.setenv("ODLA_HIP_IGEMM_TILE", "128x64")
+            second = s.run(feeds)
+        finally:
+            s.close()
+    finally:
+        hb.destroy()
+    for name in first:
+        assert np.array_equal(first[name], second[name]), name
