@@ -767,8 +767,13 @@ class Planner {
     ip.w_frag = has_wfrag ? &dummy : nullptr;
     ip.residual = has_residual ? &dummy : nullptr;
     OHIP_DEBUG("%s: kernel %s", name.c_str(), igemm_variant_name(ip));
-    if (igemm_slim_variant(ip, has_wfrag) > 0)
-      OHIP_DEBUG("%s: the small tile is estimated to beat kernel %s", name.c_str(), igemm_variant_name(ip, false));
+    const int small = igemm_slim_variant(ip, has_wfrag);
+    ip.slim = -1;
+    float us = 0.f;
+    igemm_slim_variant(ip, has_wfrag, &us);
+    OHIP_DEBUG("%s: %lld rows x %d columns x %d, %lld stages of 128 bytes; small tile%s chosen, best estimated at %.1f us, else kernel %s", name.c_str(),
+               (long long)ip.N * ip.Ho * ip.Wo, ip.Kout, ip.batch, ((long long)ip.R * ip.S * ip.C * dtype_size(ip.in_dt) + 127) / 128,
+               small > 0 ? "" : " not", us, igemm_variant_name(ip, false));
   }
   // A value whose only use is Reshape -> [B, S, heads, d] -> Transpose (0, 2, 1, 3): the
   // GEMM that computes it can store [B, heads, S, d] directly (IgemmParams::y_rdiv).
