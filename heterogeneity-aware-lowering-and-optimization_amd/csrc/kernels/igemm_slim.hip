@@ -568,14 +568,16 @@ hipError_t launch_slim(const IgemmParams& p, const int epi_vec, const int varian
 // Which kernel a launch gets, by an estimate of its time in us (beside the launch itself):
 //   c0 + c1 * chain + c2 * tiles / 256 + c3 * tiles * stages / 256
 // chain: K stages of 128 bytes that one wavefront walks; tiles: of the kernel's own size.  The
-// coefficients are a least-squares fit to some 1300 launches (ResNet-50 at 1 .. 48 images in
-// three types, BERT-base at 1 .. 64 sequences, YOLOv3 at 1 .. 16 images) of which each kernel's
-// fit saw those where it came within a factor of two of the best (three for the 128 x 128 row,
-// which stands for all kernels of igemm.hip and its siblings); rms errors 10 .. 20 %.  Chosen
-// by these estimates the launches take 3 % more than with the best kernel for each, and as much
-// as a fifth of what the 128 x 128 tiles take: ResNet-50 fp16, sums of the launches of a step,
-// 1 / 4 / 16 images 0.63 / 0.66 / 0.75 -> 0.18 / 0.28 / 0.51 ms, fp32 at 4 images 3.6 -> 0.75 ms,
-// BERT-base fp32 at 2 x 128 tokens 5.0 -> 1.2 ms.
+// coefficients are a least-squares fit to launches of ResNet-50 at 1 .. 48 images in three types,
+// BERT-base at 1 .. 64 sequences and YOLOv3 at 1 .. 16 images, of which each kernel's fit saw those
+// where it came within a factor of two of the best (three for the 128 x 128 row, which stands for
+// all kernels of igemm.hip and its siblings).  A kernel trace of 2225 such launches, each with
+// every kernel that can compute it: estimate + 2.1 us (what a duration holds of the launch itself)
+// is off by 8 .. 20 % rms per kernel and type, and the launches as chosen take 2.5 % more than with
+// the best kernel for each (20 % in one network: BERT-base bf16 at 8 x 128 tokens).  Sums of the
+// launches of a step with the wide kernels alone and as chosen: ResNet-50 fp16 at 1 / 4 / 16
+// images 0.74 / 0.77 / 0.85 -> 0.30 / 0.40 / 0.64 ms, fp32 at 4 images 3.7 -> 0.83 ms, BERT-base
+// fp32 at 2 x 128 tokens 4.8 -> 1.05 ms.
 namespace {
 struct SlimCost { float fix, chain, tile, work; };
 struct SlimCosts { SlimCost wide, k16, k8, mid; };

@@ -32,7 +32,8 @@ template <> __device__ __forceinline__ void st_from_float<int8_t>(int8_t* p, flo
 // row leave one compute unit whole.  Reads: 64 consecutive positions of a channel per wavefront.
 // VEC: 16-byte stores of consecutive channels (the pitch and the base allow them); the tile's
 // pitch of 65 words puts the lanes' reads (eight channel groups x eight positions) in 64 different
-// banks.  [64, 96, 75 x 75] fp32 -> fp16: cast and tiles of 32 channels 33 + 49 us -> 47 us.
+// banks.  [64, 96, 75 x 75] fp32 -> fp16: cast and tiles of 32 channels 33 + 49 us -> 47 us
+// (69 us as the first pass of a chain whose tensors are in no cache).
 template <typename TS, typename TD, bool VEC>
 __global__ void __launch_bounds__(kThreads) nchw_to_nhwc_tiled(LayoutParams p, float fill) {
   __shared__ float tile[TC * (THW + 1)];
@@ -168,7 +169,8 @@ __global__ void __launch_bounds__(kThreads) nchw_to_nhwc_rows16(LayoutParams p, 
 
 // src [N][HW][cs] -> dst [N][C][HW], the way back of nchw_to_nhwc_tiled: VEC 16-byte loads of
 // consecutive channels, stores of 64 consecutive positions of a channel per wavefront.
-// [64, 192, 75 x 75] fp16 -> fp32: tiles of 32 channels and a cast 133 + 70 us -> 97 us.
+// [64, 192, 75 x 75] fp16 -> fp32: tiles of 32 channels and a cast 133 + 70 us -> 97 us
+// (102 us as the last pass of such a chain).
 template <typename TS, typename TD, bool VEC>
 __global__ void __launch_bounds__(kThreads) nhwc_to_nchw_tiled(LayoutParams p) {
   __shared__ float tile[TC * (THW + 1)];
