@@ -17,6 +17,16 @@
 // served; weights are read from the fragment-ordered copy where one exists, from the packed
 // rows otherwise.
 //
+// Where a launch's 4 .. 9 us go (clock stamps, chains of captured launches): 1.3 us between the
+// last store of a launch and the first instruction of the next, 0.4 - 0.6 us arguments and
+// addresses, 0.6 us the last store, 0.2 - 0.5 us the start of all workgroups, and the rest is the
+// K loop, which is its round trips to memory and, from some 100 KB per workgroup on, the 64 bytes
+// per clock of a compute unit's L1.  Hence all requests of up to 2 U steps at once, with nothing
+// behind a request that waits for it: as two or four steps at a time, with the select of padding
+// lanes right behind each request (a wait), 14 x 14 maps of one image took 6.3 (3x3 256 -> 256) and
+// 5.1 us (1x1 1024 -> 256) with the 16-wide tile, and take 6.0 and 4.5; ResNet-50 fp16 at one image
+// 316 -> 302 us, fp32 at four images from host arrays 973 -> 853 us, BERT-base bf16 at 1 x 41 tokens 400 -> 389 us.
+//
 // A LayerNorm in front of a product of so few rows is a launch of 4 us for 60 KB, beside a
 // product that reads every row whole in each of its workgroups anyway: SLIM_LN takes it along.
 // A wavefront holds its share of K of the 16 or 32 rows in registers (at most three steps), the
@@ -67,6 +77,8 @@ template <> struct Mma16<int8_t> {
 struct SlimArgs {
   int tiles_m = 0, tiles_n = 0;
   int m_fast = 0;        // neighbouring workgroups share channels (1) or pixels (0)
+  int t_div = 1, t_shift = 0;   // division of a workgroup's number by the tiles of the fast direction
+  unsigned t_magic = 0;
   int steps = 0;         // 64-byte K steps, the last one possibly partial
   int cvec = 1;          // 16-byte vectors per tap
   unsigned cv_magic = 0, s_magic = 0;
@@ -79,6 +91,24 @@ enum SlimMode { SLIM_ROW = 0, SLIM_TAP = 1, SLIM_ANY = 2,
                 SLIM_LN32 = 4 }; // ... rows of floats under a 2-byte operand
 constexpr int kSlimLnSteps = 3;   // K steps of a wavefront it can hold
 
+// 16 bytes at byte `off` of a buffer; zero where off is kNoByte.  (A lane without a pixel or behind
+// the end of K needs no select on the loaded value then: such a select is a wait for the value, and
+// the compiler puts it next to the request.)
+constexpr unsigned kNoByte = 0xffffffffu;
+#if defined(__HIP_DEVICE_COMPILE__)  // (the builtins are unknown to the host pass, which only needs the launch stub)
+using SlimBuf = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ SlimBuf slim_buf(const unsigned char* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(base), 0, 0x7fffffff, 0x00020000);
+}
+__device__ __forceinline__ uintx4 slim_load(const SlimBuf b, const unsigned off, const unsigned soff) {
+  return __builtin_bit_cast(uintx4, __builtin_amdgcn_raw_buffer_load_b128(b, (int)off, (int)soff, 0));
+}
+#else
+using SlimBuf = const unsigned char*;
+__device__ __forceinline__ SlimBuf slim_buf(const unsigned char* base) { return base; }
+__device__ __forceinline__ uintx4 slim_load(const SlimBuf, const unsigned, const unsigned) { return uintx4{0, 0, 0, 0}; }
+#endif
+
 template <typename TIn, typename Epi, int MB, int NB, int NW, int MODE>
 __global__ void __launch_bounds__(NW * 64, 4)
 igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
@@ -89,14 +119,14 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
   constexpr int ES = sizeof(TIn);
   constexpr int BM = MB * 16, BN = NB * 16;
   constexpr int PITCH = BN + 4;             // words per pixel of a partial tile
-  constexpr int U = MB + NB <= 2 ? 4 : 2;   // K steps requested together
+  constexpr int U = MB + NB <= 2 ? 5 : ES == 1 && MODE == SLIM_ANY ? 1 : MODE == SLIM_ANY || (ES == 1 && MODE == SLIM_TAP) ? 2 : 3;   // K steps of a batch; two batches are in flight
   constexpr int REGION = BM * PITCH * 4;    // bytes of a wavefront's partial tile
   constexpr int UNITS = BM * BN / 4;        // (pixel, four channels) pairs of the tile
   constexpr int UPT = (UNITS + NW * 64 - 1) / (NW * 64);
   static_assert(UNITS % 64 == 0, "whole wavefronts in the epilogue");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   fetch_args(p.x, p.w, p.w_frag, p.wf_chunks, p.wf_tiles, p.N, p.H, p.W, p.C, p.xcs, p.Ho, p.Wo, p.sh, p.sw, p.ph, p.pw, p.howo_magic,
-             p.howo_shift, p.wo_magic, p.wo_shift, p.x_bs, a.tiles_m, a.tiles_n, a.m_fast, a.steps, a.cvec, p.Kout, p.w_bs, p.w_rs, p.w_rows);
+             p.howo_shift, p.wo_magic, p.wo_shift, p.x_bs, a.tiles_m, a.tiles_n, a.m_fast, a.t_div, a.t_shift, a.t_magic, a.steps, a.cvec, p.Kout, p.w_bs, p.w_rs, p.w_rows);
   if constexpr (MODE == SLIM_LN || MODE == SLIM_LN32) fetch_args(p.ln_x, p.ln_g, p.ln_b, p.ln_y, p.ln_eps);
   fetch_args(p.bias, p.residual, p.y, p.ycs, p.rcs, p.y_bs, p.y_rdiv, p.y_zdiv, p.alpha, p.act, p.act_a, p.act_b, epi_vec);
 
@@ -110,34 +140,51 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
     const int per = (a.tiles_m * a.tiles_n) >> 3;   // (gridDim is a load of its own)
     if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
   }
-  const int tile_m = a.m_fast ? bid % a.tiles_m : bid / a.tiles_n;
-  const int tile_n = a.m_fast ? bid / a.tiles_m : bid % a.tiles_n;
+  const int outer = fast_div(bid, a.t_magic, a.t_shift), inner = bid - outer * a.t_div;
+  const int tile_m = a.m_fast ? inner : outer;
+  const int tile_n = a.m_fast ? outer : inner;
   const int z = blockIdx.z;
 
-  const unsigned char* x = reinterpret_cast<const unsigned char*>(reinterpret_cast<const TIn*>(p.x) + (int64_t)z * p.x_bs);
+  // ---- this wavefront's share of the K steps ----
+  const int per = a.steps / NW, extra = a.steps - per * NW;
+  const int k0 = wave * per + (wave < extra ? wave : extra);
+  const int k1 = k0 + per + (wave < extra ? 1 : 0);
+  const int kvecs = p.R * p.S * a.cvec;          // valid 16-byte vectors of K
 
-  // ---- weights: lane base address and bytes per 64 bytes of K ----
-  const unsigned char* w_ptr[NB];
+  // ---- weights: scalar base, a lane's bytes from there, bytes per 64 bytes of K ----
+  SlimBuf w_buf[NB];
+  unsigned w_off[NB];
   const bool frag = p.w_frag != nullptr;
   const int w_step = frag ? 2048 : 64;
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
-    int n = tile_n * BN + j * 16 + l16;
+    const int n0 = tile_n * BN + j * 16;
+    const unsigned char* base;
     if (frag) {
-      int t = n >> 5;
+      int t = n0 >> 5;
       t = t < p.wf_tiles ? t : p.wf_tiles - 1;   // surplus channels are computed and never stored
-      w_ptr[j] = reinterpret_cast<const unsigned char*>(p.w_frag) +
-                 (((int64_t)z * p.wf_tiles + t) * p.wf_chunks + (g >> 1)) * 1024 + ((g & 1) * 32 + (n & 31)) * 16;
+      base = reinterpret_cast<const unsigned char*>(p.w_frag) + ((int64_t)z * p.wf_tiles + t) * p.wf_chunks * 1024;
+      w_off[j] = (unsigned)((g >> 1) * 1024 + ((g & 1) * 32 + ((n0 + l16) & 31)) * 16);
     } else {
-      n = n < p.w_rows ? n : p.w_rows - 1;
-      w_ptr[j] = reinterpret_cast<const unsigned char*>(reinterpret_cast<const TIn*>(p.w) + (int64_t)z * p.w_bs + (int64_t)n * p.w_rs) + g * 16;
+      const int r0 = n0 < p.w_rows ? n0 : p.w_rows - 1, r = n0 + l16 < p.w_rows ? n0 + l16 : p.w_rows - 1;
+      base = reinterpret_cast<const unsigned char*>(reinterpret_cast<const TIn*>(p.w) + (int64_t)z * p.w_bs + (int64_t)r0 * p.w_rs);
+      w_off[j] = (unsigned)((r - r0) * p.w_rs * ES + g * 16);
     }
+    w_buf[j] = slim_buf(base);
   }
+  auto load_w = [&](const int k, uintx4 (&W)[NB]) __attribute__((always_inline)) {
+    // (packed rows end at w_cols: the last step may reach behind them)
+    const bool in = MODE == SLIM_TAP || k * 4 + g < kvecs;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) W[j] = slim_load(w_buf[j], in ? w_off[j] : kNoByte, (unsigned)(k * w_step));
+  };
 
-  // ---- pixels: lane base address at tap (0, 0), channel 0 ----
-  const unsigned char* a_ptr[MB];
-  int a_hi[MB], a_wi[MB];
+  // ---- pixels: scalar base (the tile's first image), a lane's bytes from there at tap (0, 0), channel 0 ----
   const int HoWo = p.Ho * p.Wo;
+  const int img_bytes = p.H * p.W * p.xcs * ES;
+  const int img0 = fast_div(tile_m * BM, p.howo_magic, p.howo_shift);
+  const SlimBuf x_buf = slim_buf(reinterpret_cast<const unsigned char*>(reinterpret_cast<const TIn*>(p.x) + (int64_t)z * p.x_bs) + (int64_t)img0 * img_bytes);
+  int a_off[MB], a_hi[MB], a_wi[MB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
     int m = tile_m * BM + i * 16 + l16;
@@ -148,16 +195,8 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
     const int wo = rem - ho * p.Wo;
     a_hi[i] = ho * p.sh - p.ph;
     a_wi[i] = wo * p.sw - p.pw;
-    a_ptr[i] = x + (((int64_t)n_img * p.H + a_hi[i]) * p.W + a_wi[i]) * p.xcs * ES + (MODE == SLIM_ANY ? 0 : g * 16);
+    a_off[i] = (n_img - img0) * img_bytes + (a_hi[i] * p.W + a_wi[i]) * p.xcs * ES + (MODE == SLIM_ANY ? 0 : g * 16);
   }
-  const unsigned f = (unsigned)(p.a_fill & 0xff) * 0x01010101u;
-  const uintx4 fillv = {f, f, f, f}, zerov = {0u, 0u, 0u, 0u};
-
-  // ---- this wavefront's share of the K steps ----
-  const int per = a.steps / NW, extra = a.steps - per * NW;
-  const int k0 = wave * per + (wave < extra ? wave : extra);
-  const int k1 = k0 + per + (wave < extra ? 1 : 0);
-  const int kvecs = p.R * p.S * a.cvec;          // valid 16-byte vectors of K
 
   // walk of SLIM_TAP: wavefront-uniform tap and step inside the tap
   int kc = 0, kr = 0, ks = 0;
@@ -168,32 +207,26 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
     kr = fast_div(tap, a.s_magic, a.s_shift);
     ks = tap - kr * p.S;
   }
-
-  auto load = [&](const int k, uintx4 (&A)[MB], uintx4 (&W)[NB]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      if (!frag && MODE != SLIM_TAP) {
-        // (packed rows end at w_cols: the last step may reach behind them)
-        const bool in = k * 4 + g < kvecs;
-        const uintx4 v = *reinterpret_cast<const uintx4*>(w_ptr[j] + (in ? (int64_t)k * 64 : (int64_t)0));
-        W[j] = in ? v : zerov;
-      } else {
-        W[j] = *reinterpret_cast<const uintx4*>(w_ptr[j] + (int64_t)k * w_step);
-      }
-    }
+  // Padding taps of 8-bit operands hold the stored byte of the value 0, which no load returns by
+  // itself: those lanes keep a mask for the select at the use.
+  constexpr bool kFill = ES == 1 && MODE != SLIM_ROW;
+  const unsigned f = (unsigned)(p.a_fill & 0xff) * 0x01010101u;
+  auto load_a = [&](const int k, uintx4 (&A)[MB], bool (&okv)[MB]) __attribute__((always_inline)) {
     if constexpr (MODE == SLIM_ROW) {
       const bool in = k * 4 + g < kvecs;
 #pragma unroll
-      for (int i = 0; i < MB; ++i) {
-        const uintx4 v = *reinterpret_cast<const uintx4*>(a_ptr[i] + (in ? k * 64 : -g * 16));
-        A[i] = in ? v : zerov;
-      }
+      for (int i = 0; i < MB; ++i) A[i] = slim_load(x_buf, in ? (unsigned)(a_off[i] + k * 64) : kNoByte, 0u);
     } else {
       int hoff, woff, coff;
       bool in = true;
       if constexpr (MODE == SLIM_TAP) {
         hoff = kr * p.dh; woff = ks * p.dw; coff = kc * 64;
-        if (++kc == cps) { kc = 0; if (++ks == p.S) { ks = 0; ++kr; } }
+        const int tap_end = ++kc == cps ? 1 : 0;
+        kc = tap_end ? 0 : kc;
+        ks += tap_end;
+        const int row_end = ks == p.S ? 1 : 0;
+        ks = row_end ? 0 : ks;
+        kr += row_end;
       } else {
         const int kv = k * 4 + g;
         in = kv < kvecs;
@@ -205,9 +238,8 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
 #pragma unroll
       for (int i = 0; i < MB; ++i) {
         const bool ok = in && (unsigned)(a_hi[i] + hoff) < (unsigned)p.H && (unsigned)(a_wi[i] + woff) < (unsigned)p.W;
-        const unsigned char* src = ok ? a_ptr[i] + off : x;
-        const uintx4 v = *reinterpret_cast<const uintx4*>(src);
-        A[i] = ok ? v : fillv;
+        A[i] = slim_load(x_buf, ok ? (unsigned)(a_off[i] + off) : kNoByte, 0u);
+        if constexpr (kFill) okv[i] = ok;
       }
     }
   };
@@ -222,6 +254,55 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
     for (int i = 0; i < MB; ++i)
 #pragma unroll
       for (int j = 0; j < NB; ++j) acc[i][j] = Mma16<TIn>::run(W[j], A[i], acc[i][j]);
+  };
+  // U steps at once: requested together, multiplied together
+  struct Batch {
+    uintx4 A[U][MB], W[U][NB];
+    bool ok[U][MB];
+  };
+  auto load = [&](const int at, auto count, Batch& b) __attribute__((always_inline)) {
+    constexpr int n = decltype(count)::value;
+#pragma unroll
+    for (int u = 0; u < n; ++u) { load_w(at + u, b.W[u]); load_a(at + u, b.A[u], b.ok[u]); }
+  };
+  auto use = [&](auto count, Batch& b) __attribute__((always_inline)) {
+    constexpr int n = decltype(count)::value;
+#pragma unroll
+    for (int u = 0; u < n; ++u) {
+      if constexpr (kFill) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          asm volatile("" : "+v"(b.A[u][i]));   // the select belongs here, not to the request
+          b.A[u][i] = b.ok[u][i] ? b.A[u][i] : uintx4{f, f, f, f};
+        }
+      }
+      mul(b.A[u], b.W[u]);
+    }
+  };
+
+  // ---- operands of the epilogue: requested behind the first batch, so that they travel with it ----
+  const AccE* bias = p.bias ? reinterpret_cast<const AccE*>(p.bias) + (int64_t)z * p.bias_bs : nullptr;
+  TOut* ybase = reinterpret_cast<TOut*>(p.y) + (EpiTraits<Epi>::quant ? (int64_t)z * p.y_bs : y_batch_off(p, z));
+  const TOut* rbase = p.residual ? reinterpret_cast<const TOut*>(p.residual) + (int64_t)z * p.r_bs : nullptr;
+  constexpr bool kQ8 = std::is_same<Epi, EpiQuant<0>>::value;
+  const bool wide = (epi_vec & 1) != 0;
+  // raw: a conversion here would be a wait for the request here
+  uintx4 b_raw[UPT], m_raw[UPT];
+  typename std::conditional<sizeof(TOut) == 4, uintx4, typename std::conditional<sizeof(TOut) == 2, uintx2, unsigned>::type>::type r_raw[UPT];
+  const bool q_wide = EpiTraits<Epi>::quant && p.qmul != nullptr && (reinterpret_cast<uintptr_t>(p.qmul) & 15u) == 0;
+  auto fetch_epi = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < UPT; ++t) {
+      const int u = tid + t * NW * 64;
+      const int m = tile_m * BM + u / (BN / 4), n = tile_n * BN + (u % (BN / 4)) * 4;
+      if (u < UNITS && m < M && wide && n + 4 <= p.Kout) {
+        if (bias != nullptr) b_raw[t] = *reinterpret_cast<const uintx4*>(bias + n);
+        if (rbase != nullptr) __builtin_memcpy(&r_raw[t], __builtin_assume_aligned(rbase + (int64_t)m * p.rcs + n, sizeof(TOut) * 4), sizeof(TOut) * 4);
+        if constexpr (EpiTraits<Epi>::quant) {
+          if (q_wide) m_raw[t] = *reinterpret_cast<const uintx4*>(p.qmul + n);
+        }
+      }
+    }
   };
 
   if constexpr (MODE == SLIM_LN || MODE == SLIM_LN32) {
@@ -273,8 +354,7 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
 #pragma unroll
     for (int u = 0; u < LU; ++u) {
       const int k = u < cnt ? k0 + u : k1 - 1;
-#pragma unroll
-      for (int j = 0; j < NB; ++j) W[u][j] = *reinterpret_cast<const uintx4*>(w_ptr[j] + (int64_t)k * w_step);
+      load_w(k, W[u]);
     }
 #pragma unroll
     for (int r = 0; r < GBR; ++r) {
@@ -324,6 +404,7 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
       }
     }
     row_sums(1, rstd);
+    if constexpr (MB == 1) fetch_epi();   // (at 32 rows there are no registers for them here)
 #pragma unroll
     for (int i = 0; i < MB; ++i) rstd[i] = 1.0f / sqrtf(rstd[i] / (float)p.C + p.ln_eps);
     const bool writes = tile_n == 0 && z == 0;
@@ -360,98 +441,48 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
       }
       mul(A, W[u]);
     }
+    if constexpr (MB > 1) fetch_epi();
   } else {
-    uintx4 A0[U][MB], W0[U][NB], A1[U][MB], W1[U][NB];
-    int k = k0;
-    const bool first = k + U <= k1;
-    if (first) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) load(k + u, A0[u], W0[u]);
-      k += U;
-      // two batches in turn: the next one is requested before the current one is used
-      for (; k + 2 * U <= k1; k += 2 * U) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) load(k + u, A1[u], W1[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) mul(A0[u], W0[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) load(k + U + u, A0[u], W0[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) mul(A1[u], W1[u]);
+    // Straight-line code for every number of steps up to 2 U: all of them are in flight together.
+    // Longer shares: a full batch and what fills none first, then full batches in turn, the next one
+    // requested before the one in hand is multiplied.  (Requests in conditional code cannot be
+    // counted: the compiler would wait for all of them at every use.)
+    constexpr std::integral_constant<int, U> full{};
+    Batch b0, b1;
+    const int n = k1 - k0, batches = n / U, rest = n - batches * U;
+    if (batches == 0) {
+      static_for<U>([&](auto r) __attribute__((always_inline)) {   // (no steps: the epilogue's operands all the same)
+        if (rest != decltype(r)::value) return;
+        load(k0, r, b0);
+        fetch_epi();
+        use(r, b0);
+      });
+    } else {
+      static_for<U>([&](auto r) __attribute__((always_inline)) {
+        if (rest != decltype(r)::value) return;
+        load(k0, r, b0);
+        load(k0 + decltype(r)::value, full, b1);
+        fetch_epi();
+        use(r, b0);
+      });
+      int k = k0 + rest;   // b1 holds the batch at k
+      for (; k + 3 * U <= k1; k += 2 * U) {
+        load(k + U, full, b0);
+        use(full, b1);
+        load(k + 2 * U, full, b1);
+        use(full, b0);
+      }
+      if (k + 2 * U <= k1) {
+        load(k + U, full, b0);
+        use(full, b1);
+        use(full, b0);
+      } else {
+        use(full, b1);
       }
     }
-    // fewer than 2 U steps are left beside the batch in hand
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (k + u < k1) load(k + u, A1[u], W1[u]);
-    if (first) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) mul(A0[u], W0[u]);
-    }
-#pragma unroll
-    for (int u = 0; u + 1 < U; ++u)
-      if (k + U + u < k1) load(k + U + u, A0[u], W0[u]);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (k + u < k1) mul(A1[u], W1[u]);
-#pragma unroll
-    for (int u = 0; u + 1 < U; ++u)
-      if (k + U + u < k1) mul(A0[u], W0[u]);
   }
 
   unsigned char* mine = smem + wave * REGION;
-  // ---- operands of the epilogue, requested ahead of the barrier ----
-  const AccE* bias = p.bias ? reinterpret_cast<const AccE*>(p.bias) + (int64_t)z * p.bias_bs : nullptr;
-  TOut* ybase = reinterpret_cast<TOut*>(p.y) + (EpiTraits<Epi>::quant ? (int64_t)z * p.y_bs : y_batch_off(p, z));
-  const TOut* rbase = p.residual ? reinterpret_cast<const TOut*>(p.residual) + (int64_t)z * p.r_bs : nullptr;
-  constexpr bool kQ8 = std::is_same<Epi, EpiQuant<0>>::value;
-  const bool wide = (epi_vec & 1) != 0;
-  AccE b4[UPT][4];
-  float m4[UPT][4], r4[UPT][4];
-  unsigned rq[UPT];
-#pragma unroll
-  for (int t = 0; t < UPT; ++t) {
-    const int u = tid + t * NW * 64;
-    const int m = tile_m * BM + u / (BN / 4), n = tile_n * BN + (u % (BN / 4)) * 4;
-    rq[t] = 0u;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { b4[t][e] = 0; m4[t][e] = 0.f; r4[t][e] = 0.f; }
-    if (u < UNITS && m < M && n < p.Kout) {
-      if (wide && n + 4 <= p.Kout) {
-        if (bias != nullptr) __builtin_memcpy(b4[t], __builtin_assume_aligned(bias + n, 16), 16);
-        if (rbase != nullptr) {
-          const TOut* r = rbase + (int64_t)m * p.rcs + n;
-          if constexpr (kQ8) rq[t] = *reinterpret_cast<const unsigned*>(r);
-          else if constexpr (sizeof(TOut) == 4) __builtin_memcpy(r4[t], __builtin_assume_aligned(r, 16), 16);
-          else {
-            const uintx2 v = *reinterpret_cast<const uintx2*>(r);
-            const TOut* e4 = reinterpret_cast<const TOut*>(&v);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) r4[t][e] = Store<TOut>::ld(e4 + e);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if (n + e >= p.Kout) break;
-          if (bias != nullptr) b4[t][e] = bias[n + e];
-          if (rbase != nullptr) {
-            if constexpr (kQ8) rq[t] |= (unsigned)(uint8_t)rbase[(int64_t)m * p.rcs + n + e] << (8 * e);
-            else if constexpr (sizeof(TOut) == 4) r4[t][e] = (float)rbase[(int64_t)m * p.rcs + n + e];
-            else r4[t][e] = Store<TOut>::ld(rbase + (int64_t)m * p.rcs + n + e);
-          }
-        }
-      }
-      if constexpr (EpiTraits<Epi>::quant) {
-        if (p.qmul != nullptr) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < p.Kout) m4[t][e] = p.qmul[n + e];
-        }
-      }
-    }
-  }
-
   // ---- partial tiles through LDS ----
 #pragma unroll
   for (int i = 0; i < MB; ++i)
@@ -469,10 +500,47 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
 #pragma unroll
     for (int w = 1; w < NW; ++w) s += *reinterpret_cast<const accx4*>(smem + w * REGION + (pix * PITCH + c) * 4);
     const bool vec = wide && n + 4 <= p.Kout;
+    AccE b4[4] = {0, 0, 0, 0};
+    float m4[4] = {0.f, 0.f, 0.f, 0.f}, r4[4] = {0.f, 0.f, 0.f, 0.f};
+    unsigned rq = 0u;
+    if (vec) {
+      if (bias != nullptr) __builtin_memcpy(b4, &b_raw[t], 16);
+      if (rbase != nullptr) {
+        if constexpr (kQ8) rq = r_raw[t];
+        else {
+          TOut e4[4];
+          __builtin_memcpy(e4, &r_raw[t], sizeof(e4));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (sizeof(TOut) == 4) r4[e] = (float)e4[e];
+            else r4[e] = Store<TOut>::ld(e4 + e);
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= p.Kout) break;
+        if (bias != nullptr) b4[e] = bias[n + e];
+        if (rbase != nullptr) {
+          if constexpr (kQ8) rq |= (unsigned)(uint8_t)rbase[(int64_t)m * p.rcs + n + e] << (8 * e);
+          else if constexpr (sizeof(TOut) == 4) r4[e] = (float)rbase[(int64_t)m * p.rcs + n + e];
+          else r4[e] = Store<TOut>::ld(rbase + (int64_t)m * p.rcs + n + e);
+        }
+      }
+    }
+    if constexpr (EpiTraits<Epi>::quant) {
+      if (vec && q_wide) __builtin_memcpy(m4, &m_raw[t], 16);
+      else if (p.qmul != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < p.Kout) m4[e] = p.qmul[n + e];
+      }
+    }
     if constexpr (kQ8) {
-      const floatx4 mq = {m4[t][0], m4[t][1], m4[t][2], m4[t][3]};
-      const int a0 = s.x + b4[t][0], a1 = s.y + b4[t][1], a2 = s.z + b4[t][2], a3 = s.w + b4[t][3];
-      const unsigned w = rbase != nullptr ? requant4<true>(a0, a1, a2, a3, mq, rq[t], p) : requant4<false>(a0, a1, a2, a3, mq, 0u, p);
+      const floatx4 mq = {m4[0], m4[1], m4[2], m4[3]};
+      const int a0 = s.x + b4[0], a1 = s.y + b4[1], a2 = s.z + b4[2], a3 = s.w + b4[3];
+      const unsigned w = rbase != nullptr ? requant4<true>(a0, a1, a2, a3, mq, rq, p) : requant4<false>(a0, a1, a2, a3, mq, 0u, p);
       int8_t* y = ybase + (int64_t)m * p.ycs + n;
       if (vec) *reinterpret_cast<unsigned*>(y) = w;
       else {
@@ -485,17 +553,17 @@ igemm_slim_kernel(const IgemmParams p, const int epi_vec, const SlimArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if (n + e >= p.Kout) break;
-        const int v = s[e] + b4[t][e];
+        const int v = s[e] + b4[e];
         if constexpr (std::is_same<TOut, int>::value) y[e] = v;
-        else y[e] = epi_act((float)v * m4[t][e] + r4[t][e], p.act, p.act_a, p.act_b);
+        else y[e] = epi_act((float)v * m4[e] + r4[e], p.act, p.act_a, p.act_b);
       }
     } else {
       float v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(s[e], p.alpha, b4[t][e]);
+      for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(s[e], p.alpha, b4[e]);
       if (p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += r4[t][e];
+      for (int e = 0; e < 4; ++e) v[e] += r4[e];
       if (!p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
       TOut* y = ybase + y_row_off(p, m) + y_col_off(p, n);
       if (vec) {
@@ -523,6 +591,8 @@ hipError_t launch_tile(const IgemmParams& p, const int epi_vec, SlimArgs a, cons
   if (tm * tn <= 0 || tm * tn > 0x7fffffff || p.batch > 65535) return hipErrorInvalidValue;
   a.tiles_m = (int)tm;
   a.tiles_n = (int)tn;
+  a.t_div = a.m_fast ? a.tiles_m : a.tiles_n;
+  div_magic(a.t_div, &a.t_magic, &a.t_shift);
   constexpr size_t lds = (size_t)NW * MB * 16 * (NB * 16 + 4) * 4;
   const dim3 grid((unsigned)(tm * tn), 1, (unsigned)p.batch), block(NW * 64);
   static_assert(lds <= 65536, "more than a launch may ask for by itself");
@@ -573,15 +643,16 @@ hipError_t launch_slim(const IgemmParams& p, const int epi_vec, const int varian
 // where it came within a factor of two of the best (three for the 128 x 128 row, which stands for
 // all kernels of igemm.hip and its siblings).  A kernel trace of 2225 such launches, each with
 // every kernel that can compute it: estimate + 2.1 us (what a duration holds of the launch itself)
-// is off by 8 .. 20 % rms per kernel and type, and the launches as chosen take 2.5 % more than with
-// the best kernel for each (20 % in one network: BERT-base bf16 at 8 x 128 tokens).  Sums of the
+// is off by 8 .. 20 % rms per kernel and type, and the launches as chosen take 1.8 % more than with
+// the best kernel for each (16 % in one network: BERT-base bf16 at 8 x 128 tokens).  Sums of the
 // launches of a step with the wide kernels alone and as chosen: ResNet-50 fp16 at 1 / 4 / 16
-// images 0.74 / 0.77 / 0.85 -> 0.30 / 0.40 / 0.64 ms, fp32 at 4 images 3.7 -> 0.83 ms, BERT-base
-// fp32 at 2 x 128 tokens 4.8 -> 1.05 ms.
+// images 0.74 / 0.77 / 0.85 -> 0.28 / 0.39 / 0.64 ms, fp32 at 4 images 3.7 -> 0.72 ms, BERT-base
+// fp32 at 2 x 128 tokens 4.8 -> 0.96 ms.  (8-bit coefficients: refitted to the K loop of all requests
+// at once; refitting the others as well gave 1.2 %, and BERT-base bf16 at 1 x 41 tokens 389 -> 399 us.)
 namespace {
 struct SlimCost { float fix, chain, tile, work; };
 struct SlimCosts { SlimCost wide, k16, k8, mid; };
-constexpr SlimCosts kCost1 = {{4.3f, .37f, .98f, .117f}, {.05f, .62f, 2.27f, .056f}, {.73f, .88f, .82f, .108f}, {1.74f, .18f, 1.06f, .16f}};
+constexpr SlimCosts kCost1 = {{4.9f, .37f, 1.4f, .044f}, {0.f, .49f, 2.05f, .045f}, {.66f, 1.04f, .86f, .083f}, {1.28f, .275f, 1.76f, .045f}};
 constexpr SlimCosts kCost2 = {{4.4f, .42f, 1.0f, .42f}, {.05f, .62f, 2.27f, .056f}, {.73f, .88f, .82f, .108f}, {1.74f, .18f, 1.06f, .16f}};
 constexpr SlimCosts kCost4 = {{1.8f, 2.05f, 6.9f, .144f}, {0.f, .59f, 2.07f, .075f}, {1.14f, .93f, 1.15f, .19f}, {2.5f, .344f, 1.78f, .42f}};
 // How much faster than the 128 x 128 tiles the choice has to be.  (0.85 .. 1 cost the same over
@@ -596,8 +667,10 @@ int igemm_slim_variant(const IgemmParams& p, const bool frag, float* us) {
   if (p.slim >= 0) return p.slim;
   if (p.f_y != nullptr || p.row_softmax != 0 || p.fixed_order) return 0;
   // what the kernels' addressing assumes: 32-bit offsets inside an image, no column of K behind the packed rows
+  // (a tile of 32 pixels touches at most 32 images; weights: 32 rows of the fragment copy, 16 packed ones)
   const int es = dtype_size(p.in_dt);
-  if (es == 0 || (int64_t)p.H * p.W * p.xcs * es >= (1ll << 31) || (int64_t)p.R * p.S * p.C > p.w_cols) return 0;
+  if (es == 0 || (int64_t)(p.N < 32 ? p.N : 32) * p.H * p.W * p.xcs * es >= (1ll << 31) || (int64_t)p.R * p.S * p.C > p.w_cols) return 0;
+  if ((int64_t)p.w_rs * es >= (1ll << 25)) return 0;
   if (const char* force = getenv("ODLA_HIP_IGEMM_TILE")) {  // tuning aid: "slim1", "slim2", "mid"
     if (strncmp(force, "slim", 4) == 0 && force[4] >= '1' && force[4] <= '2') return force[4] - '0';
     if (strcmp(force, "mid") == 0) return frag ? 3 : 0;
