@@ -402,6 +402,58 @@ struct FusedLaunch {
 };
 hipError_t launch_fused_eltwise(const FusedLaunch& l, hipStream_t stream);
 
+// A chain of row-major operators that work within one plane (image, channel) - affine maps per
+// channel, activations, same-shape binary operators, pools, nearest resizes, plane means - as one
+// launch (plane_group.hip): a workgroup takes `planes` neighbouring planes of an image and runs the
+// instructions on them; values that a later window reads stay in LDS, arguments are read and
+// results written once.
+constexpr int kPlaneMaxInst = 12, kPlaneMaxExt = 10, kPlaneMaxAffine = 4;
+enum PlaneKind : int { PLANE_POINT = 0, PLANE_POOL, PLANE_RESIZE };
+struct PlaneInst {
+  int kind = PLANE_POINT;
+  // Operands: an LDS buffer (element offset) or an outside tensor (index); results: LDS, an outside
+  // tensor, the mean over the plane to an outside tensor.  -1: none.
+  int a = -1, a_ext = -1, b = -1, b_ext = -1, dst = -1, dst_ext = -1, mean_ext = -1;
+  int affine = -1;                 // POINT: x * scale[c] + shift[c] with this pair of vectors
+  int bin = -1;                    // POINT: BinKind with operand b
+  ActKind act = ACT_NONE;
+  float act_a = 0.f, act_b = 0.f;
+  int H = 0, W = 0, Ho = 0, Wo = 0;   // planes of operand a and of the result
+  int kh = 1, kw = 1, sh = 1, sw = 1, ph = 0, pw = 0;
+  int is_max = 0, count_pad = 0;
+  int barrier = 0;                 // the workgroup meets in front of this instruction
+  // filled in by plane_prepare
+  int window = 0;                  // POOL: which compile-time window
+  float inv = 0.f;                 // POOL, mean over full windows: 1 / count where that is exact (else 0)
+  int div = 0;                     // ... the count where every window has the same (else 0)
+  float hw_inv = 0.f, rq_inv = 0.f, q_inv = 0.f, ho_inv = 0.f, wo_inv = 0.f;   // reciprocals for divisions below 2^20
+};
+struct PlaneExt {
+  DType dt = DT_F32;
+  int64_t img = 0, off = 0;        // elements between images; in front of channel 0
+  int hw = 0;                      // elements of a plane
+  int stream = 0;                  // a result that no launch reads: non-temporal stores
+};
+struct PlaneGroup {
+  DType dt = DT_F32;               // type of the values in LDS (every result is rounded to it)
+  int N = 0, C = 0, planes = 1, chunks = 1, threads = 256, lds_bytes = 0;
+  unsigned chunk_magic = 0;
+  int chunk_shift = 0;
+  int n_inst = 0;
+  PlaneInst inst[kPlaneMaxInst];
+  PlaneExt ext[kPlaneMaxExt];
+};
+struct PlaneLaunch {
+  PlaneGroup g;
+  void* ext[kPlaneMaxExt] = {nullptr};
+  const float* scale[kPlaneMaxAffine] = {nullptr};
+  const float* shift[kPlaneMaxAffine] = {nullptr};
+};
+constexpr int kPlaneLdsMax = 159 * 1024;   // (a little is static)
+bool plane_act_ok(ActKind a);   // the activations its instructions take
+void plane_prepare(PlaneGroup* g);
+hipError_t launch_plane_group(const PlaneLaunch& l, hipStream_t stream);
+
 // Typed element-wise operators with broadcast (row-major operands, up to 6
 // collapsed dims, one element stride per dim and operand, 0 where it
 // broadcasts).  EW_ADD .. EW_SQDIFF: y has the operands' type `dt` (float types

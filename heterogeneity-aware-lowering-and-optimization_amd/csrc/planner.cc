@@ -15,6 +15,7 @@
 //   * memory: constants are packed once into one device pool; temporaries get
 //     offsets in one arena by liveness (first fit over step intervals).
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <unordered_set>
@@ -739,6 +740,8 @@ class Planner {
   void lower_postprocess(int ni);
   void lower_axisop(int ni);
   bool lower_fused_group(int seed, int from);
+  bool plane_candidate(const Node& n) const;
+  bool lower_plane_group(int seed);
   bool fuse_slice_seed(int ni) const;
   bool fuse_candidate(int ni) const;
   bool gemm_epilogue(int ni, Epilogue* ep);
@@ -925,6 +928,7 @@ void Planner::run() {
       if (fuse_slice_seed((int)ni) && lower_fused_group(consumers_[comp_->nodes[ni].out->index][0], (int)ni) &&
           comp_->nodes[ni].absorbed)
         continue;
+      if (plane_candidate(comp_->nodes[ni]) && lower_plane_group((int)ni)) continue;
     }
     lower((int)ni);
     if (calib_) {
@@ -3223,6 +3227,376 @@ bool Planner::lower_fused_group(int seed, int from) {
   for (int j : slices) comp_->nodes[j].absorbed = true;
   for (int j : sink_nodes) comp_->nodes[j].absorbed = true;
   for (auto& rv : results) set_main(rv.first, rv.second);
+  return true;
+}
+
+// ------------------------------------------------- plane group fusion ----
+// Row-major rank-4 values that no convolution touches: operators that stay within one plane (image,
+// channel) run as one launch with the values of a plane in LDS (plane_group.hip), where the
+// channels-last kernels would need a layout change at either end and a pass over memory each.  The
+// group grows from its first operator over everything that is connected with it and whose outside
+// operands are there already; results are stored row-major, a graph result in its declared type, a
+// part of a Concat (all of whose parts the group makes) in its place.
+bool Planner::plane_candidate(const Node& n) const {
+  if (n.absorbed || n.out == nullptr || !dtype_is_float(storage_dtype(n.out)) || dtype_from_odla(n.out->etype) != DT_F32) return false;
+  const _odla_value* x = n.in.empty() ? nullptr : n.in[0];
+  if (x == nullptr || x->shape.rank != 4 || dtype_from_odla(x->etype) != DT_F32) return false;
+  const Shape &xs = x->shape, &os = n.out->shape;
+  for (int i = 0; i < 4; ++i) if (xs.d[i] <= 0) return false;
+  switch (n.op) {
+    case OP_BATCHNORM:
+      for (int i = 1; i <= 4; ++i)
+        if (n.in[i] && n.in[i]->kind != _odla_value::CONSTANT) return false;
+      return n.i[0] != ODLA_CHANNELS_LAST && xs.d[2] * xs.d[3] >= 4;
+    case OP_UNARY: return os == xs && plane_act_ok((ActKind)n.i[0]);
+    case OP_BINARY:
+      return os == xs && n.in[1] != nullptr && n.in[1]->shape == xs && n.i[0] >= BIN_ADD && n.i[0] <= BIN_MIN &&
+             dtype_from_odla(n.in[1]->etype) == DT_F32;
+    case OP_POOL: return n.i[0] != ODLA_CHANNELS_LAST && os.rank == 4 && os.numel() > 0 && os.d[2] * os.d[3] < (1 << 20);
+    case OP_RESIZE:   // (source positions are quotients of products below 2^20)
+      return n.i[0] != ODLA_LINEAR && os.rank == 4 && os.d[0] == xs.d[0] && os.d[1] == xs.d[1] && os.numel() > 0 &&
+             os.d[2] * os.d[3] < (1 << 20) && os.d[2] * xs.d[2] < (1 << 20) && (os.d[3] + 4) * xs.d[3] < (1 << 20);
+    case OP_REDUCE: return (ReduceKind)n.i[0] == RED_MEAN && n.iv.size() == 2 && n.iv[0] == 2 && n.iv[1] == 3;
+    case OP_CONCAT: return n.i[0] == 1 && os.rank == 4;
+    default: return false;
+  }
+}
+
+bool Planner::lower_plane_group(int seed) {
+  const Node& first = comp_->nodes[seed];
+  if (first.op == OP_CONCAT || first.op == OP_REDUCE) return false;
+  const int64_t N = first.in[0]->shape.d[0], C = first.in[0]->shape.d[1];
+  if (N * C > 0x7fffffff) return false;
+  auto planes_of = [&](const _odla_value* v) { return v->shape.rank == 4 && v->shape.d[0] == N && v->shape.d[1] == C; };
+  // outside operands: float tensors that lie row-major, arguments in their declared type
+  auto source = [&](const _odla_value* v) -> int {
+    if (v->kind == _odla_value::CONSTANT || !planes_of(v)) return -1;
+    const VState& s = vs_[v->index];
+    const int row = s.slot[L_ROWMAJOR][FORM_FLOAT];
+    if (row >= 0) return T(row).quant || T(row).dt != cdt_ || (s.main >= 0 && T(s.main).layout == L_NHWC) ? -1 : row;
+    return v->kind == _odla_value::ARG && s.main >= 0 && T(s.main).layout == L_ROWMAJOR && T(s.main).dt == DT_F32 && s.slot[L_NHWC][FORM_FLOAT] < 0 ? s.main : -1;
+  };
+
+  // ---- members, in order
+  std::vector<int> members;
+  std::unordered_map<const _odla_value*, int> made;      // value -> member node
+  std::unordered_set<const _odla_value*> outside;
+  std::unordered_set<int> in_group;
+  const int scan_end = std::min((int)comp_->nodes.size(), seed + 256);
+  for (int j = seed; j < scan_end; ++j) {
+    const Node& n = comp_->nodes[j];
+    if (n.absorbed || !plane_candidate(n)) continue;
+    const size_t data = n.op == OP_BINARY ? 2 : n.op == OP_CONCAT ? n.in.size() : 1;
+    bool ok = true, joined = j == seed;
+    for (size_t k = 0; k < data && ok; ++k) {
+      const _odla_value* v = n.in[k];
+      auto m = made.find(v);
+      if (m != made.end()) {
+        const int op = comp_->nodes[m->second].op;
+        ok = op != OP_CONCAT && op != OP_REDUCE && planes_of(v);
+        joined = true;
+      } else {
+        ok = n.op != OP_CONCAT && source(v) >= 0;
+        joined = joined || outside.count(v);
+      }
+    }
+    if (!ok || !joined) continue;
+    if (n.op == OP_CONCAT) {   // every part once, and with no other place it has to go to
+      std::unordered_set<const _odla_value*> parts(n.in.begin(), n.in.end());
+      if (parts.size() != n.in.size()) continue;
+    }
+    for (size_t k = 0; k < data; ++k) if (!made.count(n.in[k])) outside.insert(n.in[k]);
+    members.push_back(j);
+    in_group.insert(j);
+    made[n.out] = j;
+  }
+  bool windows = false;
+  for (int j : members) windows = windows || comp_->nodes[j].op == OP_POOL || comp_->nodes[j].op == OP_RESIZE;
+  if (members.size() < 2 || !windows) return false;
+  // results that leave the group for an operator that works channels-last stay with that layout
+  auto wants_channels_last = [&](const _odla_value* v) {
+    for (int ci : consumers_[v->index]) {
+      if (in_group.count(ci)) continue;
+      const Node& c = comp_->nodes[ci];
+      if (c.op == OP_CONV || c.op == OP_POOL || c.op == OP_RESIZE || c.op == OP_CONCAT) return true;
+      if ((c.op == OP_UNARY || c.op == OP_BINARY || c.op == OP_BATCHNORM) && feeds_channels_last(c.out)) return true;
+    }
+    return false;
+  };
+  for (int j : members) if (wants_channels_last(comp_->nodes[j].out)) return false;
+
+  for (int j : members)
+    for (const _odla_value* v : comp_->nodes[j].in)
+      if (v != nullptr && v->shape.rank == 4 && v->shape.d[2] * v->shape.d[3] >= (1 << 20)) return false;
+
+  // ---- instructions
+  // (a group that turns out not to fit leaves no tensors behind)
+  const size_t tensors0 = plan_->tensors.size(), blobs0 = plan_->blobs.size(), const0 = plan_->const_bytes;
+  auto give_up = [&]() {
+    plan_->tensors.resize(tensors0);
+    plan_->blobs.resize(blobs0);
+    plan_->const_bytes = const0;
+    return false;
+  };
+  struct Val { int inst = -1, last = -1, lds = -1; int64_t hw = 0; };   // made by / last read by instruction
+  PlaneLaunch L;
+  PlaneGroup& g = L.g;
+  g.dt = cdt_;
+  g.N = (int)N;
+  g.C = (int)C;
+  std::vector<PlaneInst> prog;
+  std::vector<Val> bufs;                                       // LDS buffers
+  std::vector<std::array<int, 3>> uses;                        // per instruction: buffers a, b, dst
+  std::vector<int> ext_tensor;
+  std::vector<std::pair<int, int>> affine;                     // scale and shift tensors
+  std::vector<char> ext_written;
+  std::unordered_map<const _odla_value*, int> buf_of;          // value -> LDS buffer
+  std::unordered_map<const _odla_value*, int> ext_of;          // outside operand -> index
+  std::vector<std::pair<_odla_value*, int>> results;           // value -> tensor
+  auto add_ext = [&](int tensor, int64_t img, int64_t off, int64_t hw, bool written, bool stream = false) {
+    const int k = (int)ext_tensor.size();
+    if (k < kPlaneMaxExt) { g.ext[k].dt = T(tensor).dt; g.ext[k].img = img; g.ext[k].off = off; g.ext[k].hw = (int)hw; g.ext[k].stream = written && stream; }
+    ext_tensor.push_back(tensor);
+    ext_written.push_back(written ? 1 : 0);
+    return k;
+  };
+  auto plane = [](const _odla_value* v) { return v->shape.d[2] * v->shape.d[3]; };
+  auto push = [&](const PlaneInst& I, int a, int b, int dst) {
+    prog.push_back(I);
+    uses.push_back({a, b, dst});
+    const int at = (int)prog.size() - 1;
+    for (int u : {a, b}) if (u >= 0) bufs[u].last = at;
+    if (dst >= 0) { bufs[dst].inst = at; bufs[dst].last = at; }
+    return at;
+  };
+  auto new_buf = [&](const _odla_value* v) {
+    Val b;
+    b.hw = plane(v);
+    bufs.push_back(b);
+    return buf_of[v] = (int)bufs.size() - 1;
+  };
+  auto outside_index = [&](const _odla_value* v) {
+    auto it = ext_of.find(v);
+    if (it != ext_of.end()) return it->second;
+    return ext_of[v] = add_ext(source(v), C * plane(v), 0, plane(v), false);
+  };
+  auto set_dims = [&](PlaneInst* I, const _odla_value* x, const _odla_value* y) {
+    I->H = (int)x->shape.d[2]; I->W = (int)x->shape.d[3]; I->Ho = (int)y->shape.d[2]; I->Wo = (int)y->shape.d[3];
+  };
+  // an operand of an element-wise instruction / of a window (which needs it in LDS)
+  auto point_operand = [&](const _odla_value* v, int* buf, int* ext) {
+    auto it = buf_of.find(v);
+    if (it != buf_of.end()) *buf = it->second;
+    else *ext = outside_index(v);
+  };
+  auto window_operand = [&](const _odla_value* v) {
+    auto it = buf_of.find(v);
+    if (it != buf_of.end()) return it->second;
+    PlaneInst I;
+    I.a_ext = outside_index(v);
+    set_dims(&I, v, v);
+    const int b = new_buf(v);
+    push(I, -1, -1, b);
+    return b;
+  };
+  std::unordered_set<int> folded;
+  std::unordered_map<int, int> concat_tensor;   // Concat member -> its result
+  auto leaves = [&](const _odla_value* v) {
+    if (v->is_output) return true;
+    for (int ci : consumers_[v->index]) if (!in_group.count(ci)) return true;
+    return false;
+  };
+  auto only_output = [&](const _odla_value* v) {
+    bool read = false;
+    for (int ci : consumers_[v->index]) read = read || !in_group.count(ci);
+    return v->is_output && !read;
+  };
+  auto outer_tensor = [&](_odla_value* v) {   // where a value goes that leaves the group
+    return new_tensor(only_output(v) ? DT_F32 : cdt_, L_ROWMAJOR, v->shape, 0, SP_ARENA);
+  };
+  for (int j : members) {
+    if (folded.count(j)) continue;
+    Node& n = comp_->nodes[j];
+    if (n.op == OP_CONCAT) continue;   // (a place its parts are stored to)
+    _odla_value* out = n.out;
+    PlaneInst I;
+    set_dims(&I, n.in[0], n.op == OP_REDUCE ? n.in[0] : out);
+    int a = -1, b = -1;
+    if (n.op == OP_REDUCE || n.op == OP_POOL || n.op == OP_RESIZE) {
+      a = window_operand(n.in[0]);
+      I.kind = n.op == OP_RESIZE ? PLANE_RESIZE : PLANE_POOL;
+      if (n.op == OP_POOL) {
+        I.is_max = n.i[1] != 0;
+        I.kh = (int)n.i[2]; I.kw = (int)n.i[3]; I.sh = (int)n.i[4]; I.sw = (int)n.i[5];
+        I.ph = (int)n.i[6]; I.pw = (int)n.i[7];
+        I.count_pad = n.i[10] != 0;
+        // a pool whose only reader is the mean over its planes is not stored
+        if (!out->is_output && consumers_[out->index].size() == 1) {
+          const int ci = consumers_[out->index][0];
+          if (in_group.count(ci) && comp_->nodes[ci].op == OP_REDUCE) {
+            folded.insert(ci);
+            out = comp_->nodes[ci].out;
+            const int t = outer_tensor(out);
+            I.mean_ext = add_ext(t, C, 0, 1, true);
+            results.push_back({out, t});
+            push(I, a, -1, -1);
+            continue;
+          }
+        }
+      }
+      if (n.op == OP_REDUCE) {   // (a pool of one element)
+        const int t = outer_tensor(out);
+        I.mean_ext = add_ext(t, C, 0, 1, true);
+        results.push_back({out, t});
+        push(I, a, -1, -1);
+        continue;
+      }
+    } else {
+      point_operand(n.in[0], &a, &I.a_ext);
+      if (n.op == OP_BATCHNORM) {
+        std::vector<float> sc, sh;
+        bn_params_host(n, C, &sc, &sh);
+        I.affine = (int)affine.size();
+        const int ts = const_vector<float>(DT_F32, sc);
+        affine.push_back({ts, const_vector<float>(DT_F32, sh)});
+      } else if (n.op == OP_BINARY) {
+        I.bin = (int)n.i[0];
+        point_operand(n.in[1], &b, &I.b_ext);
+      } else {
+        I.act = (ActKind)n.i[0];
+        I.act_a = n.f[0];
+        I.act_b = n.f[1];
+      }
+      // the activation behind it comes along
+      if (n.op != OP_UNARY && !out->is_output && consumers_[out->index].size() == 1) {
+        const int ci = consumers_[out->index][0];
+        const Node& nx = comp_->nodes[ci];
+        if (in_group.count(ci) && nx.op == OP_UNARY) {
+          folded.insert(ci);
+          I.act = (ActKind)nx.i[0];
+          I.act_a = nx.f[0];
+          I.act_b = nx.f[1];
+          out = nx.out;
+        }
+      }
+    }
+    // where the result goes: LDS for readers in the group, tensors for everyone else
+    bool inner = false;
+    std::vector<int> places;
+    for (int ci : consumers_[out->index]) {
+      if (!in_group.count(ci)) continue;
+      const Node& c = comp_->nodes[ci];
+      if (c.op != OP_CONCAT) { inner = true; continue; }
+      auto it = concat_tensor.find(ci);
+      if (it == concat_tensor.end()) {
+        it = concat_tensor.emplace(ci, outer_tensor(c.out)).first;
+        results.push_back({c.out, it->second});
+      }
+      int64_t off = 0;
+      for (const _odla_value* part : c.in) {
+        if (part == out) break;
+        off += part->shape.d[1];
+      }
+      places.push_back(add_ext(it->second, c.out->shape.d[1] * plane(out), off * plane(out), plane(out), true, only_output(c.out)));
+    }
+    if (leaves(out)) {
+      const int t = outer_tensor(out);
+      places.push_back(add_ext(t, C * plane(out), 0, plane(out), true, only_output(out)));
+      results.push_back({out, t});
+    }
+    if (!places.empty()) I.dst_ext = places[0];
+    const int dst = inner || places.size() > 1 ? new_buf(out) : -1;
+    push(I, a, b, dst);
+    for (size_t k = 1; k < places.size(); ++k) {   // (a second place: a copy from LDS)
+      PlaneInst cp;
+      set_dims(&cp, out, out);
+      cp.dst_ext = places[k];
+      push(cp, dst, -1, -1);
+    }
+  }
+  if ((int)prog.size() > kPlaneMaxInst || (int)ext_tensor.size() > kPlaneMaxExt || (int)affine.size() > kPlaneMaxAffine) return give_up();
+
+  // ---- LDS: first fit over the buffers' lifetimes, for a number of planes
+  int64_t largest = 1;
+  for (const PlaneInst& I : prog) largest = std::max({largest, (int64_t)I.H * I.W, (int64_t)I.Ho * I.Wo});
+  const int es = dtype_size(cdt_);
+  auto place_bufs = [&](int64_t P) -> int64_t {
+    int64_t top = 0;
+    for (size_t i = 0; i < bufs.size(); ++i) {
+      const int64_t size = (P * bufs[i].hw + 7) / 8 * 8;
+      int64_t at = 0;
+      for (bool moved = true; moved;) {
+        moved = false;
+        for (size_t k = 0; k < i; ++k) {
+          if (bufs[k].last < bufs[i].inst || bufs[i].last < bufs[k].inst) continue;
+          const int64_t ks = (P * bufs[k].hw + 7) / 8 * 8;
+          if (at < bufs[k].lds + ks && bufs[k].lds < at + size) { at = bufs[k].lds + ks; moved = true; }
+        }
+      }
+      if (at + size > (1 << 24)) return -1;
+      bufs[i].lds = (int)at;
+      top = std::max(top, at + size);
+    }
+    return top * es;
+  };
+  // As many planes as make some 8 K elements, at most 20 KiB of LDS (eight workgroups per compute
+  // unit) where there are several, and workgroups enough for the chip.
+  int64_t P = std::max<int64_t>(1, std::min<int64_t>(C, 8192 / largest));
+  while (P > 1 && (N * ((C + P - 1) / P) < 1024 || place_bufs(P) > 20 * 1024)) --P;
+  const int64_t lds = place_bufs(P);
+  if (lds < 0 || lds > kPlaneLdsMax) return give_up();
+  g.chunks = (int)((C + P - 1) / P);
+  g.planes = (int)((C + g.chunks - 1) / g.chunks);
+  g.chunks = (int)((C + g.planes - 1) / g.planes);
+  g.lds_bytes = (int)place_bufs(g.planes);
+  if (N * g.chunks > 0x7fffffff) return give_up();
+  g.threads = g.lds_bytes <= 20 * 1024 ? 256 : g.lds_bytes <= 40 * 1024 ? 512 : 1024;
+
+  // ---- barriers: a window reads what other threads wrote; a buffer's place may have had readers
+  struct Touch { int64_t lo, hi; bool point, write; };
+  std::vector<Touch> open;   // since the last barrier
+  for (size_t i = 0; i < prog.size(); ++i) {
+    PlaneInst& I = prog[i];
+    const bool point = I.kind == PLANE_POINT;
+    auto range = [&](int b, bool write) { return Touch{bufs[b].lds, bufs[b].lds + g.planes * bufs[b].hw, point, write}; };
+    std::vector<Touch> now;
+    if (uses[i][0] >= 0) { I.a = bufs[uses[i][0]].lds; now.push_back(range(uses[i][0], false)); }
+    if (uses[i][1] >= 0) { I.b = bufs[uses[i][1]].lds; now.push_back(range(uses[i][1], false)); }
+    if (uses[i][2] >= 0) { I.dst = bufs[uses[i][2]].lds; now.push_back(range(uses[i][2], true)); }
+    for (const Touch& t : now)
+      for (const Touch& o : open) {
+        if (t.hi <= o.lo || o.hi <= t.lo || !(t.write || o.write)) continue;
+        // element-wise instructions that see a buffer at the same place give an element to one thread
+        if (!(t.point && o.point && t.lo == o.lo && t.hi == o.hi)) I.barrier = 1;
+      }
+    if (I.barrier) open.clear();
+    open.insert(open.end(), now.begin(), now.end());
+    g.inst[i] = I;
+  }
+  g.n_inst = (int)prog.size();
+  plane_prepare(&g);
+
+  // ---- the launch
+  std::vector<int> rd, wr;
+  std::vector<Ref> ext, sc, sh;
+  for (size_t k = 0; k < ext_tensor.size(); ++k) {
+    ext.push_back(ref(ext_tensor[k]));
+    (ext_written[k] ? wr : rd).push_back(ext_tensor[k]);
+  }
+  for (auto& a : affine) {
+    sc.push_back(ref(a.first));
+    sh.push_back(ref(a.second));
+    rd.push_back(a.first);
+    rd.push_back(a.second);
+  }
+  emit_lists("planes(" + std::to_string(members.size()) + "):" + first.out->name, rd, wr, [=](const ExecEnv& e, hipStream_t st) {
+    PlaneLaunch l = L;
+    for (size_t k = 0; k < ext.size(); ++k) l.ext[k] = ext[k](e);
+    for (size_t k = 0; k < sc.size(); ++k) { l.scale[k] = (const float*)sc[k](e); l.shift[k] = (const float*)sh[k](e); }
+    return launch_plane_group(l, st);
+  }, kReads16 | kWrites16);
+  for (int j : members) comp_->nodes[j].absorbed = true;
+  for (auto& r : results) set_main(r.first, r.second);
   return true;
 }
 
