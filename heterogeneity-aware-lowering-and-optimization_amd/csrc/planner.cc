@@ -3117,10 +3117,11 @@ bool Planner::lower_fused_group(int seed, int from) {
   }
   for (int k = 0; k < 4; ++k) fp.dims[k] = order[k] < 0 ? 1 : axes[order[k]];
   {
-    // every step of a walk waits for its loads: keep walks short until the chip has
-    // a few resident threads per lane (256 CUs x 2048 threads x 2)
+    // every step of a walk waits for its loads: keep walks short until the chip has a thread for
+    // every place (256 CUs x 2048); longer ones repeat what the walk does not change less often
+    // (class scores of 16 images behind their objectness: 8 -> 16 points, 2 us of 90)
     const int64_t base = fp.dims[0] * fp.dims[1] * fp.dims[3];
-    const int64_t want = 256 * 2048 * 2;
+    const int64_t want = 256 * 2048;
     int64_t w = fp.dims[2] * base / want;
     fp.walk = std::min<int64_t>(fp.dims[2], std::max<int64_t>(4, w / 4 * 4));   // whole groups of four points
     if (placed_only) fp.walk = 1;
@@ -3181,19 +3182,24 @@ bool Planner::lower_fused_group(int seed, int from) {
   gs.d[0] = (int64_t)raw.size();
   const Ref rg = ref(const_from_host(DT_U8, gs, nullptr, &raw));
   const std::string name = "fused:" + comp_->nodes[members.back()].out->name + "(" + std::to_string(members.size()) + ")";
-  // A group that repeats the program of an earlier one (the decode of another head) and reads
-  // nothing made since goes into its launch: each is a short launch that hides none of its latency.
+  // A group that reads nothing made since an earlier one goes into its launch, if it repeats that
+  // one's program (the decode of another head: each is a short launch that hides none of its latency)
+  // or brings a workgroup for every compute unit (the class scores beside the boxes): its traffic then
+  // runs beside the chain of the other.  Box decode and class scores of 16 images: 13 + 42 us as two
+  // launches, 45 us as one.  With the LDS of its hungriest group up to 32 KiB a compute unit still
+  // holds five workgroups.
   FusedStep* join = nullptr;
   for (auto& f : fused_steps_) {
     const FusedLaunch& l = f->launch;
-    bool ok = l.dt == dt && f->n_ops == (int)members.size() && l.n_groups < kFusedMaxGroups && l.view0[l.n_groups] + fp.n_views <= kFusedMaxBases &&
-              f->model.n_instr == fp.n_instr && f->model.n_views == fp.n_views;
-    for (int k = 0; ok && k < fp.n_instr; ++k) {
+    bool same = f->n_ops == (int)members.size() && f->model.n_instr == fp.n_instr && f->model.n_views == fp.n_views;
+    for (int k = 0; same && k < fp.n_instr; ++k) {
       const FusedInstr &x = f->model.prog[k], &y = fp.prog[k];
-      ok = x.op == y.op && x.kind == y.kind && x.dst == y.dst && x.a == y.a && x.b == y.b;
+      same = x.op == y.op && x.kind == y.kind && x.dst == y.dst && x.a == y.a && x.b == y.b;
     }
+    bool ok = l.dt == dt && l.n_groups < kFusedMaxGroups && l.view0[l.n_groups] + fp.n_views <= kFusedMaxBases &&
+              (same || (blocks >= 256 && std::max(lds, l.lds_bytes) <= 32 * 1024));
     for (int t : read_tensors) ok = ok && (T(root(t)).space != SP_ARENA || T(root(t)).def_step < f->step);
-    if (ok) join = f.get();
+    if (ok) { join = f.get(); if (same) break; }
   }
   auto add = [&](FusedStep* f) {
     FusedLaunch& l = f->launch;

@@ -89,3 +89,18 @@ def test_nms_block_edges(n, boxes, classes, max_out, span):
     got, want = run_both(build, {"boxes": bx, "scores": sc})
     assert np.array_equal(got["y"], want["y"])
     assert np.array_equal(got["all"], want["all"])
+
+
+@pytest.mark.parametrize("mode", ["fp32", "fp16"])
+def test_scores_that_fill_the_chip_share_the_launch_of_the_boxes(mode):
+    """Groups of different programs in one launch (a workgroup per compute unit and more of class
+    scores), with heads below and above that size."""
+    sizes, classes, n = (9, 5000, 700), 80, 3
+    announce("decode in one launch, %s" % mode)
+    r = np.random.default_rng(5)
+    feeds = {"h%d" % i: r.standard_normal((n, 3 * (5 + classes), g)).astype(np.float32) for i, g in enumerate(sizes)}
+    build = lambda b: decode(b, n, sizes, classes)
+    got, steps = run_with_steps(build, feeds, fp16=(mode == "fp16"))
+    check(got, run_ref(build, feeds), 1e-5 if mode == "fp32" else 2e-2)
+    if mode == "fp32":
+        assert len(fused(steps)) <= 2, steps
