@@ -6,6 +6,7 @@
 
 #include "device_utils.h"
 
+#include <cstddef>
 #include <type_traits>
 
 namespace ohip {
@@ -21,6 +22,15 @@ __device__ __forceinline__ void fetch_args(const A... a) {
   ((void)a, ...);
 #endif
 }
+
+// An argument that is named late, where there are no scalar registers to hold it until then: its
+// cache line is requested with the others and the value dropped (the later load then takes some 50 ns).
+#define WARM_ARG(p, member)                                                                                             \
+  do {                                                                                                                  \
+    const unsigned w_ = ((const __attribute__((address_space(4))) unsigned*)__builtin_amdgcn_kernarg_segment_ptr())     \
+        [offsetof(IgemmParams, member) / 4];   /* (the parameters are the kernel's first argument) */                   \
+    asm volatile("" ::"s"(w_));                                                                                         \
+  } while (0)
 
 
 // Element offset of result row m / column n / problem z (see IgemmParams::y_rdiv, y_zdiv).

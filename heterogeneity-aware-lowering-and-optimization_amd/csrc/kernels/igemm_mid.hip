@@ -7,8 +7,15 @@
 // ring of four, three stages ahead.  Per stage a wavefront issues four requests and eight
 // fragment reads for four MFMA steps; fragments are read one stage ahead of their MFMAs, so that
 // neither the request nor the LDS latency is on the chain.
-// (Measured and left out: two K groups of four wavefronts with a ring each, and a ring of eight;
-//  where they help - tens of tiles with a long K - the K-split workgroups of igemm_slim.hip do.)
+// (Measured and left out: two K groups of four wavefronts with a ring each; eight wavefronts that
+//  take half of every stage each, 3x3 256 -> 256 on 13 maps of 15 x 15 8.8 -> 8.7 us and 1x1 layers 4 %
+//  slower; a ring of eight, which only long runs of K over 1x1 filters gain from.)
+// A launch here is 4 - 12 us, of which the K loop is a third to two thirds (clock stamps): what the
+// epilogue needs is requested before the K loop, its arithmetic runs where the accumulators are, and
+// the arguments are fetched together.  With the shared epilogue behind the loop (bias, multipliers
+// and residual one round trip after the other, results through LDS) and arguments loaded where they
+// are named, 8-bit layers of 13 images took: 3x3 256 -> 256 at 15 x 15 9.9 us, 8.8 now; 1x1
+// 256 -> 1024 with a residual 12 us, 8.9 now; ResNet-50 int8 on 13 images of 237 x 237 532 -> 502 us.
 #include "igemm_common.h"
 
 #include <cstdlib>
@@ -19,10 +26,201 @@ namespace ohip {
 struct MidArgs {
   int tiles_m = 0, tiles_n = 0;
   int m_fast = 0;        // neighbouring workgroups share channels (1) or pixels (0)
+  int t_div = 1, t_shift = 0;   // division of a workgroup's number by the tiles of the fast direction
+  unsigned t_magic = 0;
   int stages = 0;        // 128-byte K stages
   int cvec = 1;          // 16-byte vectors per tap
   unsigned cv_magic = 0, s_magic = 0;
   int cv_shift = 0, s_shift = 0;
+};
+
+// What happens to a wavefront's 32 x 32 block behind the K loop.  A lane holds pixel l32 and four
+// quads of channels, q * 8 + lg * 4 + (0 .. 3).  Its operands are requested before the K loop, the
+// arithmetic runs on the quads as they lie in the accumulators, and results (and residuals) of 1
+// and 2 bytes trade pieces with the other half of the wavefront (v_permlane32_swap), so that a lane
+// moves 16 bytes of a row and nothing passes through LDS: no staging, no barrier, no round trip to
+// memory between the last product and the store.
+__device__ __forceinline__ void swap_halves(unsigned& lo, unsigned& hi) {   // lo of the upper half <-> hi of the lower half
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto r = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
+  lo = r[0];
+  hi = r[1];
+#endif
+}
+template <typename TIn, typename Epi>
+struct MidEpilogue {
+  using AccE = typename Epi::AccE;
+  using TOut = typename EpiTraits<Epi>::TOut;
+  using Acc = typename Mma<TIn>::Acc;
+  static constexpr bool kQ8 = std::is_same<Epi, EpiQuant<0>>::value;
+  static constexpr int OS = sizeof(TOut);
+  uintx4 b[4], m[4], r[OS == 4 ? 4 : OS == 2 ? 2 : 1];
+  int row, n0, lg;
+  bool live, wide;                          // the row exists; whole pieces only (for the whole wavefront)
+  const AccE* bias;
+  TOut* y;
+  const TOut* res;
+
+  __device__ __forceinline__ void fetch(const IgemmParams& p, const int epi_vec, const int z, const int m_row, const int M, const int n_first, const int lane_group) {
+    row = m_row < M ? m_row : M - 1;
+    n0 = n_first;
+    lg = lane_group;
+    live = m_row < M;
+    bias = p.bias ? reinterpret_cast<const AccE*>(p.bias) + (int64_t)z * p.bias_bs : nullptr;
+    y = reinterpret_cast<TOut*>(p.y) + (EpiTraits<Epi>::quant ? (int64_t)z * p.y_bs : y_batch_off(p, z));
+    res = p.residual ? reinterpret_cast<const TOut*>(p.residual) + (int64_t)z * p.r_bs + (int64_t)row * p.rcs : nullptr;
+    // (multipliers are read four at a time: rows of whole blocks and an aligned table)
+    wide = (epi_vec & (kQ8 ? 2 : 1)) != 0 && n0 + 32 <= p.Kout &&
+           (!kQ8 || ((reinterpret_cast<uintptr_t>(p.qmul) | reinterpret_cast<uintptr_t>(bias)) & 15u) == 0);
+    if (!wide) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = n0 + q * 8 + lg * 4;
+      if (bias != nullptr) b[q] = *reinterpret_cast<const uintx4*>(bias + c);
+      if constexpr (kQ8) m[q] = *reinterpret_cast<const uintx4*>(p.qmul + c);
+    }
+    if (res != nullptr) {   // (a cache line is several pieces: plain loads, the L1 keeps it between them)
+#pragma unroll
+      for (int k = 0; k < (int)(sizeof(r) / 16); ++k) r[k] = *reinterpret_cast<const uintx4*>(res + piece(k));
+    }
+  }
+  // first channel of a lane's k-th piece
+  __device__ __forceinline__ int piece(const int k) const {
+    return n0 + (OS == 4 ? k * 8 + lg * 4 : OS == 2 ? k * 16 + lg * 8 : lg * 16);
+  }
+
+  __device__ __forceinline__ void finish(const IgemmParams& p, const Acc& acc) {
+    if (!wide) {
+      narrow(p, acc);
+      return;
+    }
+    if constexpr (kQ8) {
+      unsigned d[4];   // quads 0, 2, 1, 3
+      __builtin_memcpy(d, &r[0], 16);
+      swap_halves(d[0], d[1]);
+      swap_halves(d[2], d[3]);
+      unsigned w[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const intx4 bi = bias != nullptr ? __builtin_bit_cast(intx4, b[q]) : intx4{0, 0, 0, 0};
+        const floatx4 mq = __builtin_bit_cast(floatx4, m[q]);
+        const int a0 = acc[q * 4] + bi.x, a1 = acc[q * 4 + 1] + bi.y, a2 = acc[q * 4 + 2] + bi.z, a3 = acc[q * 4 + 3] + bi.w;
+        w[q] = res != nullptr ? requant4<true>(a0, a1, a2, a3, mq, d[(q & 1) * 2 + (q >> 1)], p) : requant4<false>(a0, a1, a2, a3, mq, 0u, p);
+      }
+      swap_halves(w[0], w[2]);
+      swap_halves(w[1], w[3]);
+      if (live) store_row16(y + (int64_t)row * p.ycs + piece(0), uintx4{w[0], w[2], w[1], w[3]}, true, 16, p.stream_out);
+    } else if constexpr (!EpiTraits<Epi>::quant) {
+      TOut* yr = y + y_row_off(p, row);
+      unsigned o[8];
+      unsigned rd[8];   // quad by quad
+      if constexpr (OS == 2) {
+        if (res != nullptr) {
+          __builtin_memcpy(rd, r, 32);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) { swap_halves(rd[k * 4], rd[k * 4 + 2]); swap_halves(rd[k * 4 + 1], rd[k * 4 + 3]); }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v[4];
+        const floatx4 bf = bias != nullptr ? __builtin_bit_cast(floatx4, b[q]) : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[q * 4 + e], p.alpha, bf[e]);
+        if (p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+        if (res != nullptr) {
+          if constexpr (OS == 4) {
+            const floatx4 rf = __builtin_bit_cast(floatx4, r[q]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += rf[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const TOut t = {(uint16_t)(rd[q * 2 + (e >> 1)] >> (16 * (e & 1)))};
+              v[e] += Store<TOut>::ld(&t);
+            }
+          }
+        }
+        if (!p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+        if constexpr (OS == 4) {
+          if (live) *reinterpret_cast<floatx4*>(yr + y_col_off(p, piece(q))) = floatx4{v[0], v[1], v[2], v[3]};
+        } else {
+          o[q * 2] = pack2<TOut>(v[0], v[1]);
+          o[q * 2 + 1] = pack2<TOut>(v[2], v[3]);
+        }
+      }
+      if constexpr (OS == 2) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          swap_halves(o[k * 4], o[k * 4 + 2]);
+          swap_halves(o[k * 4 + 1], o[k * 4 + 3]);
+          const uintx4 w = {o[k * 4], o[k * 4 + 1], o[k * 4 + 2], o[k * 4 + 3]};
+          if (live) {
+            TOut* d = yr + y_col_off(p, piece(k));
+            if (p.stream_out) __builtin_nontemporal_store(w, reinterpret_cast<uintx4*>(d));
+            else *reinterpret_cast<uintx4*>(d) = w;
+          }
+        }
+      }
+    }
+  }
+
+  // element by element: blocks that reach past the last channel, rows that allow no vectors
+  __device__ __forceinline__ void narrow(const IgemmParams& p, const Acc& acc) {
+    if (!live) return;
+    TOut* yr = y + (EpiTraits<Epi>::quant ? (int64_t)row * p.ycs : y_row_off(p, row));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[4], mul[4], rv[4];
+      AccE t[4];
+      unsigned rq = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int c = n0 + q * 8 + lg * 4 + e;
+        const bool in = c < p.Kout;
+        t[e] = bias != nullptr && in ? bias[c] : (AccE)0;
+        mul[e] = rv[e] = 0.f;
+        if constexpr (EpiTraits<Epi>::quant) mul[e] = p.qmul != nullptr && in ? p.qmul[c] : 0.f;
+        if (res != nullptr && in) {
+          if constexpr (kQ8) rq |= (unsigned)(uint8_t)res[c] << (8 * e);
+          else if constexpr (OS == 4) rv[e] = (float)res[c];
+          else rv[e] = Store<TOut>::ld(res + c);
+        }
+      }
+      if constexpr (kQ8) {
+        const floatx4 mq = {mul[0], mul[1], mul[2], mul[3]};
+        const int a0 = acc[q * 4] + t[0], a1 = acc[q * 4 + 1] + t[1], a2 = acc[q * 4 + 2] + t[2], a3 = acc[q * 4 + 3] + t[3];
+        const unsigned w = res != nullptr ? requant4<true>(a0, a1, a2, a3, mq, rq, p) : requant4<false>(a0, a1, a2, a3, mq, 0u, p);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = n0 + q * 8 + lg * 4 + e;
+          if (c < p.Kout) yr[c] = (int8_t)(w >> (8 * e));
+        }
+      } else if constexpr (EpiTraits<Epi>::quant) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = n0 + q * 8 + lg * 4 + e, s = acc[q * 4 + e] + t[e];
+          if (c >= p.Kout) continue;
+          if constexpr (std::is_same<TOut, int>::value) yr[c] = s;
+          else yr[c] = epi_act((float)s * mul[e] + rv[e], p.act, p.act_a, p.act_b);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[q * 4 + e], p.alpha, t[e]);
+        if (p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += rv[e];
+        if (!p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = n0 + q * 8 + lg * 4 + e;
+          if (c >= p.Kout) continue;
+          if constexpr (OS == 4) yr[y_col_off(p, c)] = v[e];
+          else Store<TOut>::st(yr + y_col_off(p, c), v[e]);
+        }
+      }
+    }
+  }
 };
 
 // How K maps to taps: one contiguous run per pixel (1x1 filters without padding) / a stage inside
@@ -37,6 +235,12 @@ igemm_mid_kernel(const IgemmParams p, const int epi_vec, const MidArgs a) {
   constexpr int NBUF = 4, BUF = 16384;
   using Acc = typename Mma<TIn>::Acc;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];   // NBUF * BUF
+  fetch_args(p.x, p.w_frag, p.wf_chunks, p.wf_tiles, p.N, p.H, p.W, p.xcs, p.Ho, p.Wo, p.R, p.S, p.sh, p.sw, p.ph, p.pw, p.dh, p.dw, p.howo_magic,
+             p.howo_shift, p.wo_magic, p.wo_shift, p.x_bs, p.batch, a.tiles_m, a.tiles_n, a.m_fast, a.t_div, a.t_magic, a.t_shift, a.stages, a.cvec);
+  fetch_args(p.bias, p.residual, p.y, p.ycs, p.rcs, p.y_bs, p.r_bs, p.bias_bs, p.y_rdiv, p.y_zdiv, p.alpha, p.act, p.act_a, p.act_b, p.Kout, p.qmul, epi_vec);
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (EpiTraits<Epi>::quant) { WARM_ARG(p, q_add); WARM_ARG(p, r_add); }
+#endif
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -45,11 +249,12 @@ igemm_mid_kernel(const IgemmParams p, const int epi_vec, const MidArgs a) {
   // workgroups that share operands stay on one XCD (they are dealt round-robin)
   int bid = blockIdx.x;
   {
-    const int per = gridDim.x >> 3;
+    const int per = (a.tiles_m * a.tiles_n) >> 3;   // (gridDim is a load of its own)
     if (bid < (per << 3)) bid = (bid & 7) * per + (bid >> 3);
   }
-  const int tile_m = a.m_fast ? bid % a.tiles_m : bid / a.tiles_n;
-  const int tile_n = a.m_fast ? bid / a.tiles_m : bid % a.tiles_n;
+  const int outer = fast_div(bid, a.t_magic, a.t_shift), inner = bid - outer * a.t_div;
+  const int tile_m = a.m_fast ? inner : outer;
+  const int tile_n = a.m_fast ? outer : inner;
   const int z = blockIdx.z;
   const unsigned char* x = reinterpret_cast<const unsigned char*>(reinterpret_cast<const TIn*>(p.x) + (int64_t)z * p.x_bs);
 
@@ -85,10 +290,9 @@ igemm_mid_kernel(const IgemmParams p, const int epi_vec, const MidArgs a) {
     a_off[i] = (unsigned)off;
     a_mask[i] = 0u;
     if constexpr (MODE == MID_TAP) {                // one validity bit per tap
-      int t = 0;
-      for (int r = 0; r < p.R; ++r)
-        for (int q = 0; q < p.S; ++q, ++t)
-          if ((unsigned)(a_hi[i] + r * p.dh) < (unsigned)p.H && (unsigned)(a_wi[i] + q * p.dw) < (unsigned)p.W) a_mask[i] |= 1u << t;
+      unsigned cols = 0u;                           // ... of one filter row, then where the rows are inside
+      for (int q = 0; q < p.S; ++q) cols |= (unsigned)((unsigned)(a_wi[i] + q * p.dw) < (unsigned)p.W) << q;
+      for (int r = 0; r < p.R; ++r) a_mask[i] |= (unsigned)(a_hi[i] + r * p.dh) < (unsigned)p.H ? cols << (r * p.S) : 0u;
     }
   }
   const int kvecs = p.R * p.S * a.cvec;
@@ -149,10 +353,9 @@ igemm_mid_kernel(const IgemmParams p, const int epi_vec, const MidArgs a) {
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[0][0][e] = 0;
   const int wm = wave & 1, wn = wave >> 1;
-  if constexpr (EpiTraits<Epi>::quant) {
-    // (consumed right here: older than every request the K loop counts)
-    acc_init_bias_vec<1, 1>(p, z, tile_n * BN + wn * 32, lg, acc);
-  }
+  // the epilogue's operands: older than every request the K loop counts, so nothing waits for them
+  MidEpilogue<TIn, Epi> epi;
+  epi.fetch(p, epi_vec, z, tile_m * BM + wm * 32 + l32, M, tile_n * BN + wn * 32, lg);
 
   // fragments: row l32 of the quadrant, chunk 2 * kk + lg in its swizzled slot; weights lane-major
   const int sw = (l32 >> 1) & 7;
@@ -207,10 +410,9 @@ igemm_mid_kernel(const IgemmParams p, const int epi_vec, const MidArgs a) {
       frags(std::integral_constant<int, (b + 1) % NBUF>{}, fa[(b + 1) & 1], fw[(b + 1) & 1]);
     });
   }
-  // the ring becomes the staging area: no direct-to-LDS write may still be in flight
+  // (no request may be in flight when the workgroup ends: its LDS is another's then)
   arrive(std::integral_constant<int, 0>{});
-
-  igemm_epilogue<TIn, Epi, BM, BN, 32, 32>(p, epi_vec, acc, smem, tile_m, tile_n, z, M, wave, lane);
+  epi.finish(p, acc[0][0]);
 }
 
 // ---------------------------------------------------------------------------
@@ -234,6 +436,8 @@ hipError_t launch_mid(const IgemmParams& p, const int epi_vec, hipStream_t strea
   a.tiles_n = (int)tn;
   // one XCD keeps the larger operand's tiles
   a.m_fast = M < p.Kout;
+  a.t_div = a.m_fast ? a.tiles_m : a.tiles_n;
+  div_magic(a.t_div, &a.t_magic, &a.t_shift);
   const dim3 grid((unsigned)(tm * tn), 1, (unsigned)p.batch);
   const bool row = p.R == 1 && p.S == 1 && p.ph == 0 && p.pw == 0 && (int64_t)(p.Ho - 1) * p.sh < p.H && (int64_t)(p.Wo - 1) * p.sw < p.W;
   // (the row form keeps 32-bit byte offsets from the start of the problem's pixels)

@@ -652,13 +652,19 @@ hipError_t launch_slim(const IgemmParams& p, const int epi_vec, const int varian
 namespace {
 struct SlimCost { float fix, chain, tile, work; };
 struct SlimCosts { SlimCost wide, k16, k8, mid; };
-constexpr SlimCosts kCost1 = {{4.9f, .37f, 1.4f, .044f}, {0.f, .49f, 2.05f, .045f}, {.66f, 1.04f, .86f, .083f}, {1.28f, .275f, 1.76f, .045f}};
+constexpr SlimCosts kCost1 = {{4.9f, .37f, 1.4f, .044f}, {0.f, .49f, 2.05f, .045f}, {.66f, 1.04f, .86f, .083f}, {.79f, .25f, 1.49f, .054f}};
 constexpr SlimCosts kCost2 = {{4.4f, .42f, 1.0f, .42f}, {.05f, .62f, 2.27f, .056f}, {.73f, .88f, .82f, .108f}, {1.74f, .18f, 1.06f, .16f}};
 constexpr SlimCosts kCost4 = {{1.8f, 2.05f, 6.9f, .144f}, {0.f, .59f, 2.07f, .075f}, {1.14f, .93f, 1.15f, .19f}, {2.5f, .344f, 1.78f, .42f}};
 // How much faster than the 128 x 128 tiles the choice has to be.  (0.85 .. 1 cost the same over
-// all launches.)  More than two 64 x 64 tiles per compute unit: 0.7 - they ask the L2s for twice
-// the bytes per operation, which a launch that runs beside this one (the other half of a batch)
-// feels: YOLOv3 at 16 images in two halves 2.27 -> 2.34 ms with 0.88 there.
+// all launches.)  2-byte types with more than two 64 x 64 tiles per compute unit: 0.7 - they ask the
+// L2s for twice the bytes per operation, which a launch that runs beside this one (the other half of
+// a batch) feels: YOLOv3 at 16 images in two halves 2.27 -> 2.34 ms with 0.88 there.  (8-bit layers
+// of that size are bound by their results: 1 against 0.7 there takes 427 instead of 449 us for the
+// launches of ResNet-50 on 13 images.)
+// A transcendental activation in the epilogue of the wide tiles (64 elements per thread behind the
+// K loop, where the 64 x 64 tiles have 16): kWideRich + kWideRichTile * tiles / 256 more; GELU behind
+// 1024 x 768 x 3072 takes 21.9 us there and 14.8 with the 64 x 64 tiles.
+constexpr float kWideRich = 4.f, kWideRichTile = 1.5f;
 constexpr float kSlimMargin = 0.88f, kSlimMarginFull = 0.7f;
 }  // namespace
 
@@ -693,8 +699,11 @@ int igemm_slim_variant(const IgemmParams& p, const bool frag, float* us) {
   if (frag && t3 < t) { v = 3; t = t3; }
   if (us != nullptr) *us = t;
   const int64_t tiles64 = ((M + 63) / 64) * (((int64_t)p.Kout + 63) / 64) * p.batch;
-  const float margin = v == 3 && es < 4 && tiles64 > 512 ? kSlimMarginFull : kSlimMargin;
-  return t < margin * cost(c.wide, 128, 1) ? v : 0;
+  const float margin = v == 3 && es == 2 && tiles64 > 512 ? kSlimMarginFull : kSlimMargin;
+  float wide = cost(c.wide, 128, 1);
+  if (es == 2 && (p.act == ACT_GELU_ERF || p.act == ACT_GELU_TANH || p.act == ACT_SIGMOID || p.act == ACT_TANH))
+    wide += kWideRich + kWideRichTile * (float)((M + 127) / 128) * (float)((p.Kout + 127) / 128) * (float)p.batch / 256.f;
+  return t < margin * wide ? v : 0;
 }
 
 // A product that runs here, of whole rows that the wavefronts of a workgroup can hold.
