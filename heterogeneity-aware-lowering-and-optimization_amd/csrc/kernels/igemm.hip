@@ -254,10 +254,12 @@ igemm_kernel(const IgemmParams p, const int epi_vec) {
 // before the epilogue, which the first group runs alone.  For layers with fewer tiles than
 // compute units (13 x 13 feature maps at batch 16): their time is the latency chain of the K
 // stages of one workgroup, and two chains of half the length run side by side.
-template <typename TIn, typename Epi, int NJ, int KS = 1>
+//
+// kDirect: the epilogue of float results, see wreg_direct.
+template <typename TIn, typename Epi, int kDirect, int NJ, int KS = 1>
 // NJ = 1: three wavefronts per SIMD: at most 168 registers (two with the
-// transcendental activations in the epilogue, which need more)
-__global__ void __launch_bounds__(256 * KS, (EpiTraits<Epi>::rich || NJ == 2) ? 2 : 3)
+// transcendental activations in the epilogue by rows, which need more)
+__global__ void __launch_bounds__(256 * KS, ((EpiTraits<Epi>::rich && kDirect == 0) || kDirect == 2 || NJ == 2) ? 2 : 3)
 igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
   constexpr int BM = 128, BN = 128 * NJ, WM = 128, NW = 4;
   constexpr int NWF = 4 * NJ;  // weight fragments of a wavefront per K stage
@@ -280,6 +282,8 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
   static_assert(KS == 1 || (KS == 2 && NJ == 1), "two K groups with one slice per wavefront only");
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];   // RING_BYTES (+ NJ * 512 for the multipliers)
 
+  fetch_args(p.x, p.w_frag, p.wf_chunks, p.wf_tiles, p.N, p.H, p.W, p.C, p.xcs, p.Ho, p.Wo, p.Kout, p.R, p.S, p.sh, p.sw, p.ph, p.pw, p.dh,
+             p.dw, p.howo_magic, p.howo_shift, p.wo_magic, p.wo_shift, p.batch, p.x_bs);
   const int tid = threadIdx.x;
   const int M = p.N * p.Ho * p.Wo;
   const int tiles_n = (p.Kout + BN - 1) / BN;
@@ -368,6 +372,19 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
 #define IGEMM_WWAIT(N, dst) (void)(dst)
 #define IGEMM_WDRAIN8(a, b) (void)(a), (void)(b)
 #endif
+  BlockOperands<TIn, Epi, true> ops;
+  BlockResult<TIn, Epi, true, kDirect == 2> res[TM];
+  auto fetch_epi = [&]() __attribute__((always_inline)) {
+    int n0 = tile_n * BN + wave_u * 32;
+    n0 = n0 < p.Kout ? n0 : p.Kout - 32;
+    ops.fetch(p, epi_vec, z, n0, lg);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) res[i].fetch(p, ops, tile_m * BM + i * 32 + l32, M);
+  };
+  if constexpr (kDirect == 2) {
+    fetch_epi();
+    __builtin_amdgcn_sched_barrier(0);
+  }
   // fragment kk of slice j sits at position kk * NJ + j: the order of use
   uintx4 w0[NWF], w1[NWF];
   auto wload = [&](uintx4& dst, const unsigned char* ptr, const int kk) __attribute__((always_inline)) {
@@ -631,10 +648,28 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
     // (a wavefront that has ended no longer counts at the workgroup's barriers)
     if (kg_u == 1) return;
   }
+  if constexpr (kDirect != 0) {
+    if (tile_n * BN + wave_u * 32 >= p.Kout) return;
+    if constexpr (kDirect == 1) fetch_epi();
+    // (one branch per tile, not per quad: the code of one activation runs straight through)
+    auto all = [&](auto act) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < NJ; ++j)
-    igemm_epilogue_rows128<TIn, Epi>(p, epi_vec, acc[j], smem, tile_m, tile_n * NJ + j, z, M, wave, lane,
-                                     kMulLds ? reinterpret_cast<const float*>(smem + RING_BYTES) + j * 128 : nullptr);
+      for (int i = 0; i < TM; ++i) res[i].template finish<decltype(act)::value>(p, ops, acc[0][i][0]);
+    };
+    if constexpr (EpiTraits<Epi>::rich) {
+      if (p.act == ACT_GELU_ERF) all(std::integral_constant<int, ACT_GELU_ERF>{});
+      else if (p.act == ACT_GELU_TANH) all(std::integral_constant<int, ACT_GELU_TANH>{});
+      else if (p.act == ACT_SIGMOID) all(std::integral_constant<int, ACT_SIGMOID>{});
+      else all(std::integral_constant<int, ACT_TANH>{});
+    } else {
+      all(std::integral_constant<int, -1>{});
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      igemm_epilogue_rows128<TIn, Epi>(p, epi_vec, acc[j], smem, tile_m, tile_n * NJ + j, z, M, wave, lane,
+                                       kMulLds ? reinterpret_cast<const float*>(smem + RING_BYTES) + j * 128 : nullptr);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -983,6 +1018,23 @@ int wreg_k_groups(const IgemmParams& p, const int64_t workgroups) {
   return legal && stages >= 24 && workgroups <= 180 ? 2 : 1;
 }
 
+// Epilogue of the weights-in-registers kernel for float results: 0 = by rows, 1 = in the accumulator
+// layout, 2 = the same with the residual requested ahead of the K loop (two workgroups per compute
+// unit: the residual's registers).  In the accumulator layout a tile's tail has no staging, no barrier
+// and, with an activation, one branch per tile (bf16, chains of launches, us by rows -> so: 4096 x 3072
+// x 768 GELU 29.4 -> 26.6, 8192 rows 50.3 -> 45.9, 16384 rows 90.5 -> 84.4; ReLU 26.6 -> 25.0;
+// 4096 x 2304 x 768 24.5 -> 23.1; with a residual 4096 x 768 x 768 15.9 -> 14.7, K = 3072 34.5 -> 33.0).
+// Its stores cover 32-byte pieces of rows: results of 200 MB go either way (28 x 28 x 512 at batch 256,
+// K = 512, 149 -> 158 us; 56 x 56, K = 128, 73 -> 67), results of 100 MB are faster (125 -> 122).  Reading
+// a residual in pieces needs the whole K loop to hide behind: with more workgroups than are resident at
+// once, 14 x 14 x 1024 at batch 256, 61 -> 84 us.
+int wreg_direct(const IgemmParams& p, const int epi_vec, const int64_t workgroups, const bool rich) {
+  if (p.Kout % 32 != 0 || (epi_vec & 1) == 0 || p.stream_out) return 0;
+  if (p.residual != nullptr) return !rich && workgroups <= 512 ? 2 : 0;
+  const int64_t bytes = (int64_t)p.N * p.Ho * p.Wo * p.Kout * p.batch * dtype_size(p.out_dt);
+  return bytes <= ((int64_t)128 << 20) ? 1 : 0;
+}
+
 template <typename TIn, typename Epi>
 hipError_t launch_wreg(const IgemmParams& p, int epi_vec, hipStream_t stream) {
   const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
@@ -997,20 +1049,35 @@ hipError_t launch_wreg(const IgemmParams& p, int epi_vec, hipStream_t stream) {
   constexpr size_t mul = std::is_same<Epi, EpiQuant<0>>::value ? 512 : 0;
   if constexpr (!EpiTraits<Epi>::rich) {
     if (nj == 2) {
-      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256),
+      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 0, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256),
                          ring + 2 * mul, stream, p, epi_vec);
       return hipGetLastError();
     }
     if (wreg_k_groups(p, tiles * p.batch) == 2) {
       static LdsLimit limit;
-      const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_wreg_kernel<TIn, Epi, 1, 2>), (int)(2 * ring + mul));
+      const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_wreg_kernel<TIn, Epi, 0, 1, 2>), (int)(2 * ring + mul));
       if (e != hipSuccess) return e;
-      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 1, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(512),
+      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 0, 1, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(512),
                          2 * ring + mul, stream, p, epi_vec);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 1>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), ring + mul,
+  if constexpr (!EpiTraits<Epi>::quant) {
+    const int direct = wreg_direct(p, epi_vec, tiles * p.batch, EpiTraits<Epi>::rich);
+    if constexpr (!EpiTraits<Epi>::rich) {
+      if (direct == 2) {
+        hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 2, 1>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), ring,
+                           stream, p, epi_vec);
+        return hipGetLastError();
+      }
+    }
+    if (direct == 1) {
+      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 1, 1>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), ring,
+                         stream, p, epi_vec);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 0, 1>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), ring + mul,
                      stream, p, epi_vec);
   return hipGetLastError();
 }

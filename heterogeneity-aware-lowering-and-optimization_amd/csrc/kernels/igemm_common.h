@@ -560,6 +560,225 @@ __device__ __forceinline__ void igemm_epilogue_q8(const IgemmParams& p, const in
   }
 }
 
+// Epilogue of a wavefront's 32 x 32 blocks that does not leave the accumulator layout.  A lane holds,
+// per block, pixel l32 and four quads of channels, q * 8 + lg * 4 + (0 .. 3): the arithmetic runs on
+// the quads, and results (and residuals) of 1 and 2 bytes trade pieces with the other half of the
+// wavefront (v_permlane32_swap), so that a lane moves 16 bytes of a row and nothing passes through
+// LDS - no staging, no barrier, and every operand can be requested long before it is used.  A store
+// instruction covers 32 bytes of each of 32 rows, which the L2 merges: right where a launch is a chain
+// of latencies; results that stream past the caches want whole rows (igemm_epilogue).
+// BlockOperands: what all blocks of the same channels share; BlockResult: one block.
+__device__ __forceinline__ void swap_halves(unsigned& lo, unsigned& hi) {   // lo of the upper half <-> hi of the lower half
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto r = __builtin_amdgcn_permlane32_swap(lo, hi, false, false);
+  lo = r[0];
+  hi = r[1];
+#endif
+}
+// kWhole: the launcher has seen to it that every block is whole and every row takes vectors.
+template <typename TIn, typename Epi, bool kWhole = false>
+struct BlockOperands {
+  using AccE = typename Epi::AccE;
+  using TOut = typename EpiTraits<Epi>::TOut;
+  using Acc = typename Mma<TIn>::Acc;
+  static constexpr bool kQ8 = std::is_same<Epi, EpiQuant<0>>::value;
+  static constexpr int OS = sizeof(TOut);
+  uintx4 b[4], m[4];
+  int n0, lg;
+  bool wide;                                // whole pieces only (the same for the whole wavefront)
+  const AccE* bias;
+  TOut* y;
+  const TOut* res;
+
+  // (kBias false: the accumulators hold it already)
+  template <bool kBias = true>
+  __device__ __forceinline__ void fetch(const IgemmParams& p, const int epi_vec, const int z, const int n_first, const int lane_group) {
+    n0 = n_first;
+    lg = lane_group;
+    bias = kBias && p.bias ? reinterpret_cast<const AccE*>(p.bias) + (int64_t)z * p.bias_bs : nullptr;
+    y = reinterpret_cast<TOut*>(p.y) + (EpiTraits<Epi>::quant ? (int64_t)z * p.y_bs : y_batch_off(p, z));
+    res = p.residual ? reinterpret_cast<const TOut*>(p.residual) + (int64_t)z * p.r_bs : nullptr;
+    // (multipliers are read four at a time: rows of whole blocks and an aligned table)
+    wide = kWhole || (epi_vec & (kQ8 ? 2 : 1)) != 0 && n0 + 32 <= p.Kout &&
+           (!kQ8 || ((reinterpret_cast<uintptr_t>(p.qmul) | reinterpret_cast<uintptr_t>(bias)) & 15u) == 0);
+    if (!wide) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = n0 + q * 8 + lg * 4;
+      if (bias != nullptr) b[q] = *reinterpret_cast<const uintx4*>(bias + c);
+      if constexpr (kQ8) m[q] = *reinterpret_cast<const uintx4*>(p.qmul + c);
+    }
+  }
+  // first channel of a lane's k-th piece
+  __device__ __forceinline__ int piece(const int k) const {
+    return n0 + (OS == 4 ? k * 8 + lg * 4 : OS == 2 ? k * 16 + lg * 8 : lg * 16);
+  }
+};
+
+// (kRes false: the launcher knows of no residual)
+template <typename TIn, typename Epi, bool kWhole = false, bool kRes = true>
+struct BlockResult {
+  using Shared = BlockOperands<TIn, Epi, kWhole>;
+  using AccE = typename Shared::AccE;
+  using TOut = typename Shared::TOut;
+  using Acc = typename Shared::Acc;
+  static constexpr bool kQ8 = Shared::kQ8;
+  static constexpr int OS = Shared::OS;
+  uintx4 r[OS == 4 ? 4 : OS == 2 ? 2 : 1];
+  int row;
+  bool live;                                // the row exists
+
+  __device__ __forceinline__ void fetch(const IgemmParams& p, const Shared& s, const int m_row, const int M) {
+    row = m_row < M ? m_row : M - 1;
+    live = m_row < M;
+    if (!kRes || (!kWhole && !s.wide) || s.res == nullptr) return;
+    // (a cache line is several pieces: plain loads, the L1 keeps it between them)
+    const TOut* rr = s.res + (int64_t)row * p.rcs;
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(r) / 16); ++k) r[k] = *reinterpret_cast<const uintx4*>(rr + s.piece(k));
+  }
+
+  // kAct: the activation where the caller has branched on it already, -1: p.act
+  template <int kAct = -1>
+  __device__ __forceinline__ void finish(const IgemmParams& p, const Shared& s, const Acc& acc) {
+    const ActKind act = kAct >= 0 ? (ActKind)kAct : p.act;
+    if constexpr (!kWhole) {
+      if (!s.wide) {
+        narrow(p, s, acc);
+        return;
+      }
+    }
+    const bool has_bias = s.bias != nullptr, has_res = kRes && s.res != nullptr;
+    if constexpr (kQ8) {
+      unsigned d[4];   // quads 0, 2, 1, 3
+      __builtin_memcpy(d, &r[0], 16);
+      swap_halves(d[0], d[1]);
+      swap_halves(d[2], d[3]);
+      unsigned w[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const intx4 bi = has_bias ? __builtin_bit_cast(intx4, s.b[q]) : intx4{0, 0, 0, 0};
+        const floatx4 mq = __builtin_bit_cast(floatx4, s.m[q]);
+        const int a0 = acc[q * 4] + bi.x, a1 = acc[q * 4 + 1] + bi.y, a2 = acc[q * 4 + 2] + bi.z, a3 = acc[q * 4 + 3] + bi.w;
+        w[q] = has_res ? requant4<true>(a0, a1, a2, a3, mq, d[(q & 1) * 2 + (q >> 1)], p) : requant4<false>(a0, a1, a2, a3, mq, 0u, p);
+      }
+      swap_halves(w[0], w[2]);
+      swap_halves(w[1], w[3]);
+      if (live) store_row16(s.y + (int64_t)row * p.ycs + s.piece(0), uintx4{w[0], w[2], w[1], w[3]}, true, 16, p.stream_out);
+    } else if constexpr (!EpiTraits<Epi>::quant) {
+      TOut* yr = s.y + y_row_off(p, row);
+      unsigned o[8];
+      unsigned rd[8];   // quad by quad
+      if constexpr (OS == 2) {
+        if (has_res) {
+          __builtin_memcpy(rd, r, 32);
+#pragma unroll
+          for (int k = 0; k < 2; ++k) { swap_halves(rd[k * 4], rd[k * 4 + 2]); swap_halves(rd[k * 4 + 1], rd[k * 4 + 3]); }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float v[4];
+        const floatx4 bf = has_bias ? __builtin_bit_cast(floatx4, s.b[q]) : floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[q * 4 + e], p.alpha, bf[e]);
+        if (kRes && p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, act, p.act_a, p.act_b);
+        if (has_res) {
+          if constexpr (OS == 4) {
+            const floatx4 rf = __builtin_bit_cast(floatx4, r[q]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += rf[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const TOut t = {(uint16_t)(rd[q * 2 + (e >> 1)] >> (16 * (e & 1)))};
+              v[e] += Store<TOut>::ld(&t);
+            }
+          }
+        }
+        if (!kRes || !p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, act, p.act_a, p.act_b);
+        if constexpr (OS == 4) {
+          if (live) *reinterpret_cast<floatx4*>(yr + y_col_off(p, s.piece(q))) = floatx4{v[0], v[1], v[2], v[3]};
+        } else {
+          o[q * 2] = pack2<TOut>(v[0], v[1]);
+          o[q * 2 + 1] = pack2<TOut>(v[2], v[3]);
+        }
+      }
+      if constexpr (OS == 2) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          swap_halves(o[k * 4], o[k * 4 + 2]);
+          swap_halves(o[k * 4 + 1], o[k * 4 + 3]);
+          const uintx4 w = {o[k * 4], o[k * 4 + 1], o[k * 4 + 2], o[k * 4 + 3]};
+          if (live) {
+            TOut* d = yr + y_col_off(p, s.piece(k));
+            if (p.stream_out) __builtin_nontemporal_store(w, reinterpret_cast<uintx4*>(d));
+            else *reinterpret_cast<uintx4*>(d) = w;
+          }
+        }
+      }
+    }
+  }
+
+  // element by element: blocks that reach past the last channel, rows that allow no vectors
+  __device__ __forceinline__ void narrow(const IgemmParams& p, const Shared& s, const Acc& acc) {
+    if (!live) return;
+    const TOut* res = s.res != nullptr ? s.res + (int64_t)row * p.rcs : nullptr;
+    TOut* yr = s.y + (EpiTraits<Epi>::quant ? (int64_t)row * p.ycs : y_row_off(p, row));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[4], mul[4], rv[4];
+      AccE t[4];
+      unsigned rq = 0u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int c = s.n0 + q * 8 + s.lg * 4 + e;
+        const bool in = c < p.Kout;
+        t[e] = s.bias != nullptr && in ? s.bias[c] : (AccE)0;
+        mul[e] = rv[e] = 0.f;
+        if constexpr (EpiTraits<Epi>::quant) mul[e] = p.qmul != nullptr && in ? p.qmul[c] : 0.f;
+        if (res != nullptr && in) {
+          if constexpr (kQ8) rq |= (unsigned)(uint8_t)res[c] << (8 * e);
+          else if constexpr (OS == 4) rv[e] = (float)res[c];
+          else rv[e] = Store<TOut>::ld(res + c);
+        }
+      }
+      if constexpr (kQ8) {
+        const floatx4 mq = {mul[0], mul[1], mul[2], mul[3]};
+        const int a0 = acc[q * 4] + t[0], a1 = acc[q * 4 + 1] + t[1], a2 = acc[q * 4 + 2] + t[2], a3 = acc[q * 4 + 3] + t[3];
+        const unsigned w = res != nullptr ? requant4<true>(a0, a1, a2, a3, mq, rq, p) : requant4<false>(a0, a1, a2, a3, mq, 0u, p);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = s.n0 + q * 8 + s.lg * 4 + e;
+          if (c < p.Kout) yr[c] = (int8_t)(w >> (8 * e));
+        }
+      } else if constexpr (EpiTraits<Epi>::quant) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = s.n0 + q * 8 + s.lg * 4 + e, sum = acc[q * 4 + e] + t[e];
+          if (c >= p.Kout) continue;
+          if constexpr (std::is_same<TOut, int>::value) yr[c] = sum;
+          else yr[c] = epi_act((float)sum * mul[e] + rv[e], p.act, p.act_a, p.act_b);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[q * 4 + e], p.alpha, t[e]);
+        if (p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += rv[e];
+        if (!p.res_after_act) epi_act_n<EpiTraits<Epi>::rich>(v, p.act, p.act_a, p.act_b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = s.n0 + q * 8 + s.lg * 4 + e;
+          if (c >= p.Kout) continue;
+          if constexpr (OS == 4) yr[y_col_off(p, c)] = v[e];
+          else Store<TOut>::st(yr + y_col_off(p, c), v[e]);
+        }
+      }
+    }
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Epilogue shared by the kernels below: each wavefront parks one 32-pixel slice
 // of its accumulators in LDS (pixel-major, fp32 / int32), then every lane picks
