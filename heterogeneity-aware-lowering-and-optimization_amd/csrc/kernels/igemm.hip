@@ -222,7 +222,7 @@ igemm_kernel(const IgemmParams p, const int epi_vec) {
 // load rate, and one K stage of register prefetch does not cover the latency of
 // the gathered pixel loads, so a kernel that stages both operands through
 // registers into LDS is bound by exactly those two things.  Here
-//   - only the 128-pixel tile goes through LDS, written by direct-to-LDS global
+//   - only the pixel tile (96 or 128 pixels) goes through LDS, written by direct-to-LDS global
 //     loads (no registers, no LDS store instructions) into a ring of three
 //     buffers, two K stages ahead of its use, one barrier per stage;
 //   - the four wavefronts split the 128 output channels; each reads its
@@ -255,26 +255,26 @@ igemm_kernel(const IgemmParams p, const int epi_vec) {
 // compute units (13 x 13 feature maps at batch 16): their time is the latency chain of the K
 // stages of one workgroup, and two chains of half the length run side by side.
 //
-// kDirect: the epilogue of float results, see wreg_direct.
-template <typename TIn, typename Epi, int kDirect, int NJ, int KS = 1>
+// TM: rows of a tile in 32s, 3 or 4 (wreg_rows32).  kDirect: the epilogue of float results (wreg_direct).
+template <typename TIn, typename Epi, int TM, int kDirect, int NJ, int KS = 1>
 // NJ = 1: three wavefronts per SIMD: at most 168 registers (two with the
 // transcendental activations in the epilogue by rows, which need more)
 __global__ void __launch_bounds__(256 * KS, ((EpiTraits<Epi>::rich && kDirect == 0) || kDirect == 2 || NJ == 2) ? 2 : 3)
 igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
-  constexpr int BM = 128, BN = 128 * NJ, WM = 128, NW = 4;
+  constexpr int BM = 32 * TM, BN = 128 * NJ;
   constexpr int NWF = 4 * NJ;  // weight fragments of a wavefront per K stage
   constexpr int ES = sizeof(TIn);
   constexpr int BKB = 128, BK = BKB / ES;
-  constexpr int VEC = 16 / ES, A_IT = 4;
-  constexpr int TM = WM / 32;
-  constexpr int BUF_BYTES = BM * BKB;  // 16 KiB
+  constexpr int VEC = 16 / ES, A_IT = TM;   // (a request of the workgroup covers 32 rows)
+  constexpr int BUF_BYTES = BM * BKB;  // 12 or 16 KiB
   constexpr int NBUF = 3;
   constexpr int EPI_BYTES = 2 * 32 * (128 + 4) * 4;
   static_assert(NBUF * BUF_BYTES >= EPI_BYTES, "staging area must fit in the pixel buffers");
   using Acc = typename Mma<TIn>::Acc;
-  // s_waitcnt immediates (vmcnt only; expcnt / lgkmcnt left at their maxima):
-  // vmcnt(0), and vmcnt(2 * NWF + 4) = 12 / 20 for the wait at the top of a stage
-  constexpr int kWaitVm0 = 0x0f70, kWaitVmStage = NJ == 1 ? 0x0f7c : 0x4f74;
+  // s_waitcnt immediates (vmcnt only; expcnt / lgkmcnt left at their maxima): nothing in flight, and what
+  // is in flight behind a stage's pixels: its fragments and the operations of the stage between
+  constexpr int kVmStage = 2 * NWF + A_IT;
+  constexpr int kWaitVm0 = 0x0f70, kWaitVmStage = 0x0f70 | (kVmStage & 15) | (kVmStage >> 4 << 14);
 
   // (8-bit results: the multipliers of the tile's channels wait behind the pixel rings)
   constexpr bool kMulLds = std::is_same<Epi, EpiQuant<0>>::value;
@@ -360,7 +360,7 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
     else                                                                                                                  \
       asm volatile("global_load_dwordx4 %0, %1, off offset:" #OFF : "+v"(dst) : "v"(ptr) : "memory");                     \
   } while (0)
-#define IGEMM_WWAIT(N, dst) asm volatile("s_waitcnt vmcnt(" #N ")" : "+v"(dst) : : "memory")
+#define IGEMM_WWAIT(N, dst) asm volatile("s_waitcnt vmcnt(%1)" : "+v"(dst) : "n"(N) : "memory")
 #define IGEMM_WDRAIN8(a, b)                                                                                    \
   asm volatile("s_waitcnt vmcnt(0)"                                                                            \
                : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(b[0]), "+v"(b[1]), "+v"(b[2]), "+v"(b[3]) \
@@ -382,7 +382,7 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
     for (int i = 0; i < TM; ++i) res[i].fetch(p, ops, tile_m * BM + i * 32 + l32, M);
   };
   if constexpr (kDirect == 2) {
-    fetch_epi();
+    if (kg_u == 0) fetch_epi();   // (of two K groups the first finishes the tile)
     __builtin_amdgcn_sched_barrier(0);
   }
   // fragment kk of slice j sits at position kk * NJ + j: the order of use
@@ -535,7 +535,7 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
     // the pixel vectors of this stage have landed (mine), and everyone's have
     // (a bare barrier: the fence of __syncthreads would also wait for the
     // requests of the stages still in flight).  Behind them in flight: this
-    // stage's NWF fragments and the 4 + NWF operations of the stage between.
+    // stage's NWF fragments and the A_IT + NWF operations of the stage between.
     if (kt < 2) __builtin_amdgcn_s_waitcnt(kWaitVm0);
     else __builtin_amdgcn_s_waitcnt(kWaitVmStage);
     __builtin_amdgcn_sched_barrier(0);
@@ -564,11 +564,10 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
         const int k = kk * NJ + j;
         __builtin_amdgcn_sched_barrier(0);
         // In flight behind wc[k] (requested two stages ago at this position):
-        // NWF-1-k fragments of that stage, 4 + NWF operations of the stage
-        // between, the 4 pixel requests above and k fragments of this stage:
-        // always 2 * NWF + 7.
-        if constexpr (NJ == 1) IGEMM_WWAIT(15, wc[k]);
-        else IGEMM_WWAIT(23, wc[k]);
+        // NWF-1-k fragments of that stage, A_IT + NWF operations of the stage
+        // between, the A_IT pixel requests above and k fragments of this stage:
+        // whatever k, the operations of two stages but one.
+        IGEMM_WWAIT(2 * (A_IT + NWF) - 1, wc[k]);
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[j][i][0] = Mma<TIn>::run(wc[k], fa[kk & 1][i], acc[j][i][0]);
         __builtin_amdgcn_sched_barrier(0);
@@ -624,7 +623,7 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
     };
-    V4* red = reinterpret_cast<V4*>(smem) + (wave_u * 16) * 64 + lane;
+    V4* red = reinterpret_cast<V4*>(smem) + (wave_u * 4 * TM) * 64 + lane;
     lds_barrier();
     if (kg_u == 1) {
 #pragma unroll
@@ -667,7 +666,7 @@ igemm_wreg_kernel(const IgemmParams p, const int epi_vec) {
   } else {
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
-      igemm_epilogue_rows128<TIn, Epi>(p, epi_vec, acc[j], smem, tile_m, tile_n * NJ + j, z, M, wave, lane,
+      igemm_epilogue_rows128<TIn, Epi, TM>(p, epi_vec, acc[j], smem, tile_m, tile_n * NJ + j, z, M, wave, lane,
                                        kMulLds ? reinterpret_cast<const float*>(smem + RING_BYTES) + j * 128 : nullptr);
   }
 }
@@ -996,11 +995,32 @@ int wreg_slices(const IgemmParams& p) {
   return 1;
 }
 
+// Rows of the weights-in-registers kernel's tile, in 32s (one slice per wavefront): 96 where the
+// busiest compute unit then has at least 5 % fewer rows to do, 128 otherwise.  A workgroup that has
+// a compute unit to itself needs 545 ns for a stage of 128 rows and 440 ns for one of 96 (2-byte
+// operands; latencies and the LDS reads of four wavefronts, which nothing else covers), two need 650
+// and 550, three 950 and 780.  Measured, us at 128 -> at 96 rows: as many workgroups per unit either
+// way, bf16 3072 x 768 x 768 14.5 -> 12.3, 1536 x 3072 x 768 GELU 18.6 -> 16.5, 6144 x 768 x 3072
+// 47.3 -> 37.6, 3x3 256 -> 512 over 26 x 26 at batch 16 40.3 -> 33.2 (int8 27.7 -> 23.1); four and five
+// (14 x 14, 256 -> 1024, batch 64) 23.8 -> 22.2; one and two (4096 x 768 x 3072) 33.0 -> 36.5; six and
+// nine (8192 x 3072 x 768) 44.3 -> 49.6.
+int wreg_rows32(const IgemmParams& p) {
+  if (const char* force = getenv("ODLA_HIP_WREG_ROWS")) {  // tuning aid
+    const int v = atoi(force);
+    if (v == 96 || v == 128) return v / 32;
+  }
+  const int64_t M = (int64_t)p.N * p.Ho * p.Wo, columns = (int64_t)((p.Kout + 127) / 128) * p.batch;
+  const int64_t per4 = ((M + 127) / 128 * columns + 255) / 256, per3 = ((M + 95) / 96 * columns + 255) / 256;
+  return per3 * 3 * 20 <= per4 * 4 * 19 ? 3 : 4;
+}
+
 // K groups of the weights-in-registers kernel (one slice per wavefront): two where the launch has
-// far fewer workgroups than the chip has compute units and the K loop is long enough to be worth
-// splitting (an even number of stages, at least 24: measured on YOLOv3 at batch 16, 72 stages
-// 53 -> 46 us, 16 stages unchanged, 8 stages 14.6 -> 16 .. 21 us).
-int wreg_k_groups(const IgemmParams& p, const int64_t workgroups) {
+// no more workgroups than the chip has compute units and the K loop is long enough to be worth
+// splitting (an even number of stages).  96 rows: 16 stages 13.5 -> 13.1 us (13 x 13, 1024 -> 512,
+// batch 16, fp16), 24 stages 15.5 -> 14.4, 48 stages 27.4 -> 23.9 (3072 x 768 x 3072), 72 stages
+// 38.8 -> 34.0; 12 stages 12.3 -> 12.6, 8 stages 9.9 -> 10.2 (int8).  128 rows: 72 stages 53 -> 46 us,
+// 16 stages unchanged, 8 stages 14.6 -> 16 .. 21 us.
+int wreg_k_groups(const IgemmParams& p, const int rows32, const int64_t workgroups) {
   const int64_t stages = (int64_t)p.wf_chunks / 4;
   const bool legal = stages % 2 == 0 && stages >= 4;
   if (const char* force = getenv("ODLA_HIP_WREG_KSPLIT")) {  // tuning aid: 0 = never, 2 = wherever legal
@@ -1011,11 +1031,12 @@ int wreg_k_groups(const IgemmParams& p, const int64_t workgroups) {
   // (fp32 layers keep one summation chain per result: their parity bound is relative to single
   //  results, which a second chain's rounding can exceed where a sum nearly cancels)
   if (p.in_dt == DT_F32) return 1;
-  // (at most 180 workgroups: a workgroup of this form takes a compute unit's LDS for itself, and
+  // (128 rows, at most 180 workgroups: a workgroup of this form takes a compute unit's LDS for itself, and
   //  when two half-batch copies of a plan run side by side the other copy's launch wants the
   //  units this one leaves - BERT-base halves of 32 sequences, 192 workgroups of 48 stages,
-  //  2.36 -> 2.43 ms per step with it)
-  return legal && stages >= 24 && workgroups <= 180 ? 2 : 1;
+  //  2.36 -> 2.43 ms per step with it; of 96 rows, where a launch alone gains three times as much,
+  //  up to one workgroup per unit)
+  return legal && (rows32 == 3 ? stages >= 16 && workgroups <= 256 : stages >= 24 && workgroups <= 180) ? 2 : 1;
 }
 
 // Epilogue of the weights-in-registers kernel for float results: 0 = by rows, 1 = in the accumulator
@@ -1035,51 +1056,58 @@ int wreg_direct(const IgemmParams& p, const int epi_vec, const int64_t workgroup
   return bytes <= ((int64_t)128 << 20) ? 1 : 0;
 }
 
+template <typename TIn, typename Epi, int TM>
+hipError_t launch_wreg_rows(const IgemmParams& p, const int epi_vec, hipStream_t stream) {
+  const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
+  const int64_t tiles = ((M + 32 * TM - 1) / (32 * TM)) * ((p.Kout + 127) / 128), workgroups = tiles * p.batch;
+  if (tiles <= 0 || tiles > 0x7fffffff) return hipErrorInvalidValue;
+  // pixel ring and, for 8-bit results, the tile's multipliers
+  constexpr int ring = 3 * 32 * TM * 128, mul = std::is_same<Epi, EpiQuant<0>>::value ? 512 : 0;
+  constexpr bool rich = EpiTraits<Epi>::rich;
+  const dim3 grid((unsigned)tiles, 1, (unsigned)p.batch);
+  const int direct = EpiTraits<Epi>::quant ? 0 : wreg_direct(p, epi_vec, workgroups, rich);
+  auto launch = [&](auto kind, auto k_groups) {
+    constexpr int kDirect = decltype(kind)::value, KS = decltype(k_groups)::value, lds = KS * ring + mul;
+    if constexpr (lds > 64 * 1024) {
+      static LdsLimit limit;
+      const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_wreg_kernel<TIn, Epi, TM, kDirect, 1, KS>), lds);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, TM, kDirect, 1, KS>), grid, dim3(256 * KS), lds, stream, p, epi_vec);
+    return hipGetLastError();
+  };
+  auto with_groups = [&](auto k_groups) {
+    if constexpr (!EpiTraits<Epi>::quant) {
+      if constexpr (!rich) {
+        if (direct == 2) return launch(std::integral_constant<int, 2>{}, k_groups);
+      }
+      if (direct == 1) return launch(std::integral_constant<int, 1>{}, k_groups);
+    }
+    return launch(std::integral_constant<int, 0>{}, k_groups);
+  };
+  if constexpr (!rich) {
+    if (wreg_k_groups(p, TM, workgroups) == 2) return with_groups(std::integral_constant<int, 2>{});
+  }
+  return with_groups(std::integral_constant<int, 1>{});
+}
+
 template <typename TIn, typename Epi>
 hipError_t launch_wreg(const IgemmParams& p, int epi_vec, hipStream_t stream) {
   const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
   // what the kernel's tap walk assumes: whole K stages per tap, one mask bit per tap
   if (p.C % (128 / (int)sizeof(TIn)) != 0 || p.R * p.S > 32) return hipErrorInvalidValue;
   // (the transcendental epilogues do not fit beside twice the accumulators)
-  const int nj = EpiTraits<Epi>::rich ? 1 : wreg_slices(p);
-  const int64_t tiles = ((M + 127) / 128) * ((p.Kout + 128 * nj - 1) / (128 * nj));
-  if (tiles <= 0 || tiles > 0x7fffffff) return hipErrorInvalidValue;
-  // pixel ring(s) and, for 8-bit results, the tile's multipliers
-  constexpr size_t ring = 3 * 128 * 128;
-  constexpr size_t mul = std::is_same<Epi, EpiQuant<0>>::value ? 512 : 0;
   if constexpr (!EpiTraits<Epi>::rich) {
-    if (nj == 2) {
-      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 0, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256),
-                         ring + 2 * mul, stream, p, epi_vec);
-      return hipGetLastError();
-    }
-    if (wreg_k_groups(p, tiles * p.batch) == 2) {
-      static LdsLimit limit;
-      const hipError_t e = limit.raise(reinterpret_cast<const void*>(&igemm_wreg_kernel<TIn, Epi, 0, 1, 2>), (int)(2 * ring + mul));
-      if (e != hipSuccess) return e;
-      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 0, 1, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(512),
-                         2 * ring + mul, stream, p, epi_vec);
+    if (wreg_slices(p) == 2) {
+      const int64_t tiles = ((M + 127) / 128) * ((p.Kout + 255) / 256);
+      if (tiles <= 0 || tiles > 0x7fffffff) return hipErrorInvalidValue;
+      constexpr size_t lds = 3 * 128 * 128 + (std::is_same<Epi, EpiQuant<0>>::value ? 1024 : 0);
+      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 4, 0, 2>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), lds, stream,
+                         p, epi_vec);
       return hipGetLastError();
     }
   }
-  if constexpr (!EpiTraits<Epi>::quant) {
-    const int direct = wreg_direct(p, epi_vec, tiles * p.batch, EpiTraits<Epi>::rich);
-    if constexpr (!EpiTraits<Epi>::rich) {
-      if (direct == 2) {
-        hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 2, 1>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), ring,
-                           stream, p, epi_vec);
-        return hipGetLastError();
-      }
-    }
-    if (direct == 1) {
-      hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 1, 1>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), ring,
-                         stream, p, epi_vec);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((igemm_wreg_kernel<TIn, Epi, 0, 1>), dim3((unsigned)tiles, 1, (unsigned)p.batch), dim3(256), ring + mul,
-                     stream, p, epi_vec);
-  return hipGetLastError();
+  return wreg_rows32(p) == 3 ? launch_wreg_rows<TIn, Epi, 3>(p, epi_vec, stream) : launch_wreg_rows<TIn, Epi, 4>(p, epi_vec, stream);
 }
 
 // 1x1 filters with at most one K stage and no padding: the streaming variant.
@@ -1244,10 +1272,10 @@ const char* igemm_variant_name(const IgemmParams& p, const bool small_tiles) {
   if (p.w_frag != nullptr && taps_shape(p).nkk > 0) return "128x64t";
   if (p.w_frag != nullptr && wreg_shape(p)) {
     const bool rich = p.act == ACT_GELU_ERF || p.act == ACT_GELU_TANH || p.act == ACT_SIGMOID || p.act == ACT_TANH;
-    const int nj = rich ? 1 : wreg_slices(p);
+    const int rows32 = wreg_rows32(p);   // (tiles of 96 rows go by the same names)
     const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
-    const int64_t tiles = ((M + 127) / 128) * ((p.Kout + 128 * nj - 1) / (128 * nj));
-    if (!rich && nj == 1 && wreg_k_groups(p, tiles * p.batch) == 2) return "128x128w2k";   // two K groups per workgroup
+    const int64_t tiles = ((M + 32 * rows32 - 1) / (32 * rows32)) * ((p.Kout + 127) / 128);
+    if (!rich && wreg_slices(p) == 1 && wreg_k_groups(p, rows32, tiles * p.batch) == 2) return "128x128w2k";   // two K groups per workgroup
     return "128x128w";
   }
   return choose_variant(p).name;

@@ -1,4 +1,4 @@
-"""The 128 x 128 tile's epilogue in the accumulator layout: rows past the last one, 32-channel blocks
+"""The 128-channel tiles of 96 and 128 rows and their epilogue in the accumulator layout: rows past the last one, 32-channel blocks
 past the last channel, every activation it branches on, a residual requested ahead of the K loop,
 results addressed as attention heads, and the borders that keep the epilogue by rows."""
 import math
@@ -6,6 +6,7 @@ import math
 import numpy as np
 import pytest
 
+import test_gpu_int8 as q8
 from test_gpu_taps_kernel import run_logged
 from util import announce, run_both
 
@@ -21,12 +22,14 @@ def tolerance(mode, k, want):
     return 1.13 * 5 * (2 * EPS[mode] + 2.0 ** -24 * np.sqrt(k)) + 2 * EPS[mode] * np.max(np.abs(want)) + 4e-7
 
 
+@pytest.mark.parametrize("rows", ["96", "128"])
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("act", ["none", "relu", "gelu", "sigmoid", "tanh"])
-def test_ragged_tiles(mode, act, monkeypatch):
+def test_ragged_tiles(rows, mode, act, monkeypatch):
+    monkeypatch.setenv("ODLA_HIP_WREG_ROWS", rows)
     monkeypatch.setenv("ODLA_HIP_IGEMM_TILE", "wreg")
     r = np.random.default_rng(5)
-    for m, n, k in ((1, 32, 64), (127, 96, 128), (129, 160, 192), (300, 128, 64), (200, 100, 128)):
+    for m, n, k in ((1, 32, 64), (95, 96, 128), (97, 64, 64), (129, 160, 192), (300, 128, 64), (200, 100, 128)):
         announce("tile epilogue %s %s %s" % (mode, act, (m, n, k)))
         x = r.standard_normal((m, k)).astype(np.float32)
         w, bias = (r.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32), r.standard_normal((n,)).astype(np.float32)
@@ -40,11 +43,15 @@ def test_ragged_tiles(mode, act, monkeypatch):
         assert np.max(np.abs(got["o"] - want["o"])) <= tolerance(mode, k, want["o"]), (m, n, k)
 
 
+@pytest.mark.parametrize("rows,groups", [("96", "0"), ("96", "2"), ("128", "0"), ("128", "2")])
 @pytest.mark.parametrize("mode", MODES)
-def test_residual_and_activation_in_either_order(mode, monkeypatch):
+def test_residual_and_activation_in_either_order(mode, rows, groups, monkeypatch):
+    """One K group and two (an even number of stages; an odd one keeps one)."""
+    monkeypatch.setenv("ODLA_HIP_WREG_ROWS", rows)
+    monkeypatch.setenv("ODLA_HIP_WREG_KSPLIT", groups)
     monkeypatch.setenv("ODLA_HIP_IGEMM_TILE", "wreg")
     r = np.random.default_rng(6)
-    for m, n, k in ((1, 32, 64), (127, 96, 128), (257, 224, 192), (130, 100, 128)):
+    for m, n, k in ((1, 32, 256), (95, 96, 512), (193, 224, 192), (130, 100, 1024)):
         announce("tile epilogue %s residual %s" % (mode, (m, n, k)))
         x, res = r.standard_normal((m, k)).astype(np.float32), r.standard_normal((m, n)).astype(np.float32)
         w, bias = (r.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32), r.standard_normal((n,)).astype(np.float32)
@@ -77,6 +84,16 @@ def test_residual_on_either_side_of_the_resident_workgroups(batch, monkeypatch):
 
     got, want = run_both(build, {"x": x, "res": res}, fp16=True)
     assert np.max(np.abs(got["o"] - want["o"])) <= tolerance("fp16", 64, want["o"])
+
+
+@pytest.mark.parametrize("dims", [(1, 128, 8, 8, 64), (3, 128, 9, 7, 96), (2, 512, 5, 5, 160), (2, 256, 7, 7, 256)])
+@pytest.mark.parametrize("groups", ["0", "2"])
+def test_8bit_residual_block_in_tiles_of_96_rows(dims, groups, odla, ref, monkeypatch):
+    """Bit-equal to the oracle."""
+    monkeypatch.setenv("ODLA_HIP_IGEMM_TILE", "wreg")
+    monkeypatch.setenv("ODLA_HIP_WREG_ROWS", "96")
+    monkeypatch.setenv("ODLA_HIP_WREG_KSPLIT", groups)
+    q8.test_q8_residual_fused_equals_unfused_equals_oracle(dims, 0, odla, ref, monkeypatch)
 
 
 @pytest.mark.parametrize("mode", ["fp16", "bf16", "bf16acc"])
