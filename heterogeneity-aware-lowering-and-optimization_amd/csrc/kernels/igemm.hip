@@ -779,16 +779,14 @@ igemm_lean_kernel(const IgemmParams p, const int epi_vec, const int tiles_per_wg
 template <typename TIn, typename Epi, int NKK, int VPT, int NJ>
 __global__ void __launch_bounds__(256, 2)
 igemm_taps_kernel(const IgemmParams p, const int epi_vec, const int tiles_per_wg) {
-  // NJ = 2: four wavefronts on four 32-pixel blocks, 64 channels each; NJ = 1 (K rows too
-  // long to keep 64 channels of weights in registers): two blocks, two channel halves
-  constexpr int BM = NJ == 2 ? 128 : 64, BN = 64, WN = 32 * NJ;
+  // four wavefronts on four 32-pixel blocks, 64 channels each or (NJ = 1) 32
+  constexpr int BM = 128, BN = 32 * NJ, WN = 32 * NJ;
   using Acc = typename Mma<TIn>::Acc;
   __shared__ __attribute__((aligned(16))) unsigned char smem[4 * 32 * (64 + 4) * 4];
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int l32 = lane & 31, lg = lane >> 5;
-  const int wm = wave % (BM / 32), wn = wave / (BM / 32);
   const int M = p.N * p.Ho * p.Wo;
   const int tiles_m = (M + BM - 1) / BM;
   const int tiles_n = (p.Kout + BN - 1) / BN;
@@ -805,7 +803,7 @@ igemm_taps_kernel(const IgemmParams p, const int epi_vec, const int tiles_per_wg
   uintx4 w[NJ][NKK];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
-    int wtile = tile_n * 2 + wn * NJ + j;
+    int wtile = tile_n * NJ + j;
     wtile = wtile < p.wf_tiles ? wtile : p.wf_tiles - 1;  // a surplus slice computes channels that are never stored
 #pragma unroll
     for (int kk = 0; kk < NKK; ++kk) w[j][kk] = wf[((int64_t)wtile * p.wf_chunks + kk) * 64];
@@ -821,10 +819,10 @@ igemm_taps_kernel(const IgemmParams p, const int epi_vec, const int tiles_per_wg
     for (int e = 0; e < 16; ++e) acc0[0][j][e] = 0;
   IgemmParams pe = p;   // the epilogue's view: no bias left to add
   if constexpr (EpiTraits<Epi>::quant) {
-    acc_init_bias_vec<1, NJ>(p, 0, tile_n * BN + wn * WN, lg, acc0);
+    acc_init_bias_vec<1, NJ>(p, 0, tile_n * BN, lg, acc0);
     constexpr int TILE = 32 * (WN + 16);
     float* mtile = reinterpret_cast<float*>(smem + wave * (2 * TILE + WN * 4) + 2 * TILE);
-    if (lane < WN / 4) *reinterpret_cast<floatx4*>(mtile + lane * 4) = load_qmul4(p.qmul, tile_n * BN + wn * WN + lane * 4, p.Kout);
+    if (lane < WN / 4) *reinterpret_cast<floatx4*>(mtile + lane * 4) = load_qmul4(p.qmul, tile_n * BN + lane * 4, p.Kout);
   } else {
     if (p.bias != nullptr) {
       const float* bias = reinterpret_cast<const float*>(p.bias);
@@ -835,7 +833,7 @@ igemm_taps_kernel(const IgemmParams p, const int epi_vec, const int tiles_per_wg
         for (int q = 0; q < 4; ++q)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const int c = tile_n * BN + wn * WN + j * 32 + q * 8 + lg * 4 + r;
+            const int c = tile_n * BN + j * 32 + q * 8 + lg * 4 + r;
             acc0[0][j][q * 4 + r] = p.alpha == 1.0f ? bias[c < last ? c : last] : 0.f;
           }
       if (p.alpha == 1.0f) pe.bias = nullptr;   // (a scaled accumulator keeps its bias in the epilogue)
@@ -856,7 +854,7 @@ igemm_taps_kernel(const IgemmParams p, const int epi_vec, const int tiles_per_wg
   uintx4 a[NKK];
   unsigned okmask = 0;   // bit kk: this lane's unit of K step kk is real data
   auto load_a = [&](const int tile_m) {
-    int m = tile_m * BM + wm * 32 + l32;
+    int m = tile_m * BM + wave * 32 + l32;
     m = m < M ? m : M - 1;
     const int n_img = fast_div(m, p.howo_magic, p.howo_shift);
     const int rem = m - n_img * HoWo;
@@ -1154,8 +1152,10 @@ hipError_t launch_lean(const IgemmParams& p, int epi_vec, hipStream_t stream) {
 // and vectors per tap, or {0, 0}.
 struct TapsShape { int nkk, vpt; };
 TapsShape taps_shape(const IgemmParams& p) {
+  bool forced = false;
   if (const char* force = getenv("ODLA_HIP_IGEMM_TILE")) {  // tuning aid
     if (strcmp(force, "taps") != 0 && force[0] != 0) return {0, 0};
+    forced = force[0] != 0;
   }
   const int es = dtype_size(p.in_dt);
   if (p.in_dt != DT_F16 && p.in_dt != DT_BF16 && p.in_dt != DT_I8) return {0, 0};
@@ -1179,7 +1179,11 @@ TapsShape taps_shape(const IgemmParams& p) {
   // 256: 159 -> 122 us).  The 2-byte forms of the same layers request twice the bytes per
   // pixel from the vector-memory pipeline, which then bounds them (215 -> 288 us), and stay
   // on the two-operand kernel.
-  const bool built = vpt == 1 && nkk == 8 && es == 1;
+  // Nine taps of one 2-byte vector into at most 32 channels (a detector's first layer) write twice as
+  // much per requested byte: 416 x 416 at batch 16, 3 -> 32 channels, fp16, 110 -> 74 us (2.4 TB/s
+  // written), from 2048 tiles on, where workgroups walk several.
+  const bool nine = vpt == 1 && nkk == 5 && es == 2 && p.Kout <= 32 && (forced || (int64_t)p.N * p.Ho * p.Wo >= (128 << 11));
+  const bool built = (vpt == 1 && nkk == 8 && es == 1) || nine;
   return built ? TapsShape{nkk, vpt} : TapsShape{0, 0};
 }
 
@@ -1187,7 +1191,8 @@ template <typename TIn, typename Epi>
 hipError_t launch_taps(const IgemmParams& p, int epi_vec, hipStream_t stream) {
   const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
   const TapsShape ts = taps_shape(p);
-  const int64_t tiles_m = (M + 127) / 128, tiles_n = (p.Kout + 63) / 64;
+  const bool narrow = ts.nkk == 5;
+  const int64_t tiles_m = (M + 127) / 128, tiles_n = narrow ? (p.Kout + 31) / 32 : (p.Kout + 63) / 64;
   // several pixel tiles per workgroup (the weights are fetched once for all of them),
   // as long as the chip keeps eight workgroups per compute unit
   int tpw = 1;
@@ -1199,8 +1204,12 @@ hipError_t launch_taps(const IgemmParams& p, int epi_vec, hipStream_t stream) {
   const int64_t wgs = ((tiles_m + tpw - 1) / tpw) * tiles_n;
   if (wgs <= 0 || wgs > 0x7fffffff) return hipErrorInvalidValue;
   const dim3 grid((unsigned)wgs), block(256);
-  if (ts.vpt == 1) hipLaunchKernelGGL((igemm_taps_kernel<TIn, Epi, 8, 1, 2>), grid, block, 0, stream, p, epi_vec, tpw);
-  else hipLaunchKernelGGL((igemm_taps_kernel<TIn, Epi, 2, 4, 2>), grid, block, 0, stream, p, epi_vec, tpw);
+  if constexpr (sizeof(TIn) == 2) {
+    hipLaunchKernelGGL((igemm_taps_kernel<TIn, Epi, 5, 1, 1>), grid, block, 0, stream, p, epi_vec, tpw);
+  } else {
+    if (ts.vpt == 1) hipLaunchKernelGGL((igemm_taps_kernel<TIn, Epi, 8, 1, 2>), grid, block, 0, stream, p, epi_vec, tpw);
+    else hipLaunchKernelGGL((igemm_taps_kernel<TIn, Epi, 2, 4, 2>), grid, block, 0, stream, p, epi_vec, tpw);
+  }
   return hipGetLastError();
 }
 
@@ -1224,7 +1233,10 @@ hipError_t dispatch(const IgemmParams& p, int epi_vec, hipStream_t s) {
   if constexpr (std::is_same<TIn, f16_t>::value || std::is_same<TIn, bf16_t>::value) {
     if (p.w_frag != nullptr && lean_steps(p) > 0) return launch_lean<TIn, Epi>(p, epi_vec, s);
   }
-  // (the streaming 1x1 kernel and the short-tap kernel are built for 8-bit layers with 8-bit results)
+  if constexpr (std::is_same<Epi, EpiFloat<TIn, false>>::value && sizeof(TIn) == 2) {
+    if (p.w_frag != nullptr && taps_shape(p).nkk > 0) return launch_taps<TIn, Epi>(p, epi_vec, s);
+  }
+  // (the streaming 1x1 kernel is built for 8-bit layers with 8-bit results)
   if constexpr (std::is_same<Epi, EpiQuant<0>>::value) {
     if (p.w_frag != nullptr && (epi_vec & 2) && igemm_stream_q8_geometry(p)) return launch_igemm_stream_q8(p, s);
     if (p.w_frag != nullptr && taps_shape(p).nkk > 0) return launch_taps<TIn, Epi>(p, epi_vec, s);

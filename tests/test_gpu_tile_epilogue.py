@@ -116,6 +116,29 @@ def test_projection_into_heads(mode, monkeypatch):
         assert np.max(np.abs(got["o"] - want["o"])) <= tolerance(mode, h, want["o"]), (bs, s, heads, d)
 
 
+@pytest.mark.parametrize("mode", ["fp16", "bf16"])
+@pytest.mark.parametrize("tiles", ["", "1", "3"])
+def test_nine_taps_of_one_vector(mode, tiles, monkeypatch):
+    """3 x 3 filters over three channels (one 16-byte vector) in the short-tap kernel, at most 32 results."""
+    monkeypatch.setenv("ODLA_HIP_IGEMM_TILE", "taps")
+    if tiles:
+        monkeypatch.setenv("ODLA_HIP_LEAN_TILES", tiles)
+    r = np.random.default_rng(9)
+    for n, h, w_, o, stride, pad in ((1, 5, 5, 32, 1, 1), (2, 31, 29, 32, 1, 1), (3, 26, 27, 17, 2, 1), (1, 40, 33, 8, 1, 0), (2, 3, 3, 32, 1, 2)):
+        announce("nine taps %s %s" % (mode, (n, h, w_, o, stride, pad)))
+        x = r.standard_normal((n, 3, h, w_)).astype(np.float32)
+        w = (r.standard_normal((o, 3, 3, 3)) / np.sqrt(27)).astype(np.float32)
+        bias = r.standard_normal((o,)).astype(np.float32)
+
+        def build(b):
+            y = b.conv(b.arg("x", x.shape), b.const("w", w), b.const("b", bias), (stride, stride), (pad,) * 4, (1, 1), 1, name="c")
+            b.output(b.leaky_relu(y, 0.1, name="o"), "o")
+
+        (got, want), seen = run_logged(lambda: run_both(build, {"x": x}, **MODES[mode]))
+        assert any(s.endswith("kernel 128x64t") for s in seen) or stride == 2, [s for s in seen if "kernel" in s]
+        assert np.max(np.abs(got["o"] - want["o"])) <= tolerance(mode, 27, want["o"]), (n, h, w_, o, stride, pad)
+
+
 def test_gelu_over_its_range():
     """Against the exact function in 64 bits; infinities and NaN as x (1 + erf(x / sqrt 2)) / 2 has them."""
     special = np.array([np.inf, -np.inf, np.nan, 0.0, -0.0, 1e-30, -1e-30, 3e38, -3e38, 1e10, -1e10, 5.65, -5.65], np.float32)
