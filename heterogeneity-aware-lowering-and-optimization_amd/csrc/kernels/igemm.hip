@@ -994,14 +994,16 @@ int wreg_slices(const IgemmParams& p) {
 }
 
 // Rows of the weights-in-registers kernel's tile, in 32s (one slice per wavefront): 96 where the
-// busiest compute unit then has at least 5 % fewer rows to do, 128 otherwise.  A workgroup that has
+// busiest compute unit then gets as many workgroups (which takes at most three, all resident: the
+// launch is one round either way, of shorter workgroups), 128 otherwise.  A workgroup that has
 // a compute unit to itself needs 545 ns for a stage of 128 rows and 440 ns for one of 96 (2-byte
 // operands; latencies and the LDS reads of four wavefronts, which nothing else covers), two need 650
-// and 550, three 950 and 780.  Measured, us at 128 -> at 96 rows: as many workgroups per unit either
-// way, bf16 3072 x 768 x 768 14.5 -> 12.3, 1536 x 3072 x 768 GELU 18.6 -> 16.5, 6144 x 768 x 3072
-// 47.3 -> 37.6, 3x3 256 -> 512 over 26 x 26 at batch 16 40.3 -> 33.2 (int8 27.7 -> 23.1); four and five
-// (14 x 14, 256 -> 1024, batch 64) 23.8 -> 22.2; one and two (4096 x 768 x 3072) 33.0 -> 36.5; six and
-// nine (8192 x 3072 x 768) 44.3 -> 49.6.
+// and 550, three 950 and 780.  Measured, us at 128 -> at 96 rows: as many workgroups per unit,
+// bf16 3072 x 768 x 768 14.5 -> 12.3, 1536 x 3072 x 768 GELU 18.6 -> 16.5, 6144 x 768 x 3072
+// 47.3 -> 37.6, 3x3 256 -> 512 over 26 x 26 at batch 16 40.3 -> 33.2 (int8 27.7 -> 23.1); one and two
+// (4096 x 768 x 3072) 33.0 -> 36.5; six and nine (8192 x 3072 x 768) 44.3 -> 49.6.  Four and five gain
+// 1 to 7 % alone (14 x 14, 256 -> 1024, batch 64, 23.8 -> 22.2) but ask for a third more weight
+// traffic, which two half-batch copies of a plan that run side by side do not have to spare.
 int wreg_rows32(const IgemmParams& p) {
   if (const char* force = getenv("ODLA_HIP_WREG_ROWS")) {  // tuning aid
     const int v = atoi(force);
@@ -1009,7 +1011,7 @@ int wreg_rows32(const IgemmParams& p) {
   }
   const int64_t M = (int64_t)p.N * p.Ho * p.Wo, columns = (int64_t)((p.Kout + 127) / 128) * p.batch;
   const int64_t per4 = ((M + 127) / 128 * columns + 255) / 256, per3 = ((M + 95) / 96 * columns + 255) / 256;
-  return per3 * 3 * 20 <= per4 * 4 * 19 ? 3 : 4;
+  return per3 == per4 ? 3 : 4;
 }
 
 // K groups of the weights-in-registers kernel (one slice per wavefront): two where the launch has
@@ -1043,15 +1045,16 @@ int wreg_k_groups(const IgemmParams& p, const int rows32, const int64_t workgrou
 // and, with an activation, one branch per tile (bf16, chains of launches, us by rows -> so: 4096 x 3072
 // x 768 GELU 29.4 -> 26.6, 8192 rows 50.3 -> 45.9, 16384 rows 90.5 -> 84.4; ReLU 26.6 -> 25.0;
 // 4096 x 2304 x 768 24.5 -> 23.1; with a residual 4096 x 768 x 768 15.9 -> 14.7, K = 3072 34.5 -> 33.0).
-// Its stores cover 32-byte pieces of rows: results of 200 MB go either way (28 x 28 x 512 at batch 256,
-// K = 512, 149 -> 158 us; 56 x 56, K = 128, 73 -> 67), results of 100 MB are faster (125 -> 122).  Reading
+// Its stores cover 32-byte pieces of rows, which costs a little where many rounds of workgroups keep the
+// memory busy anyway: ResNet-50 in fp16 at batch 256, results of 25 MB 59 -> 56, of 51 MB 65.2 -> 65.9, of
+// 103 MB 80.7 -> 83.9; with a transcendental activation 100 MB still gain (above).  Reading
 // a residual in pieces needs the whole K loop to hide behind: with more workgroups than are resident at
 // once, 14 x 14 x 1024 at batch 256, 61 -> 84 us.
 int wreg_direct(const IgemmParams& p, const int epi_vec, const int64_t workgroups, const bool rich) {
   if (p.Kout % 32 != 0 || (epi_vec & 1) == 0 || p.stream_out) return 0;
   if (p.residual != nullptr) return !rich && workgroups <= 512 ? 2 : 0;
   const int64_t bytes = (int64_t)p.N * p.Ho * p.Wo * p.Kout * p.batch * dtype_size(p.out_dt);
-  return bytes <= ((int64_t)128 << 20) ? 1 : 0;
+  return bytes <= ((int64_t)(rich ? 128 : 48) << 20) ? 1 : 0;
 }
 
 template <typename TIn, typename Epi, int TM>
