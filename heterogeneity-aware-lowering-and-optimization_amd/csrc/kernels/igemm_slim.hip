@@ -661,10 +661,6 @@ constexpr SlimCosts kCost4 = {{1.8f, 2.05f, 6.9f, .144f}, {0.f, .59f, 2.07f, .07
 // a batch) feels: YOLOv3 at 16 images in two halves 2.27 -> 2.34 ms with 0.88 there.  (8-bit layers
 // of that size are bound by their results: 1 against 0.7 there takes 427 instead of 449 us for the
 // launches of ResNet-50 on 13 images.)
-// A transcendental activation in the epilogue of the wide tiles (64 elements per thread behind the
-// K loop, where the 64 x 64 tiles have 16): kWideRich + kWideRichTile * tiles / 256 more; GELU behind
-// 1024 x 768 x 3072 takes 21.9 us there and 14.8 with the 64 x 64 tiles.
-constexpr float kWideRich = 4.f, kWideRichTile = 1.5f;
 constexpr float kSlimMargin = 0.88f, kSlimMarginFull = 0.7f;
 }  // namespace
 
@@ -683,7 +679,7 @@ int igemm_slim_variant(const IgemmParams& p, const bool frag, float* us) {
     if (force[0] != 0) return 0;
   }
   // (a tuning aid of another kernel asks for that kernel)
-  for (const char* aid : {"ODLA_HIP_WREG_SLICES", "ODLA_HIP_WREG_KSPLIT", "ODLA_HIP_C3_MIN_FILL", "ODLA_HIP_C3_BC", "ODLA_HIP_C3_SLICES",
+  for (const char* aid : {"ODLA_HIP_WREG_SLICES", "ODLA_HIP_WREG_KSPLIT", "ODLA_HIP_WREG_ROWS", "ODLA_HIP_C3_MIN_FILL", "ODLA_HIP_C3_BC", "ODLA_HIP_C3_SLICES",
                           "ODLA_HIP_LEAN_TILES", "ODLA_HIP_STREAM_WGS"})
     if (getenv(aid) != nullptr) return 0;
   const SlimCosts& c = es == 1 ? kCost1 : es == 2 ? kCost2 : kCost4;
@@ -700,10 +696,7 @@ int igemm_slim_variant(const IgemmParams& p, const bool frag, float* us) {
   if (us != nullptr) *us = t;
   const int64_t tiles64 = ((M + 63) / 64) * (((int64_t)p.Kout + 63) / 64) * p.batch;
   const float margin = v == 3 && es == 2 && tiles64 > 512 ? kSlimMarginFull : kSlimMargin;
-  float wide = cost(c.wide, 128, 1);
-  if (es == 2 && (p.act == ACT_GELU_ERF || p.act == ACT_GELU_TANH || p.act == ACT_SIGMOID || p.act == ACT_TANH))
-    wide += kWideRich + kWideRichTile * (float)((M + 127) / 128) * (float)((p.Kout + 127) / 128) * (float)p.batch / 256.f;
-  return t < margin * wide ? v : 0;
+  return t < margin * cost(c.wide, 128, 1) ? v : 0;
 }
 
 // A product that runs here, of whole rows that the wavefronts of a workgroup can hold.
