@@ -158,6 +158,7 @@ class Planner {
   // by root tensor: some launch relies on the arena for it; needs a 16-byte aligned base; writes it
   std::unordered_set<int> arena_only_, aligned_only_, written_;
   std::unordered_map<int, int> reads_;   // by root tensor: passes over it (2 for a launch that may read it several times)
+  std::unordered_map<int, int> last_write_;   // by root tensor: the last step so far that writes it (a Concat's result has several)
   // The 8-bit convolution steps, kept so that a plain 1x1 layer over the result of one can ride in
   // its launch (lower_conv; igemm_stream_q8_fusable decides).
   struct FuseProducer {
@@ -241,6 +242,8 @@ class Planner {
     for (int t : writes) {
       if (t < 0) continue;
       written_.insert(root(t));
+      int& last = last_write_.emplace(root(t), idx).first->second;
+      if (idx > last) last = idx;
       if (!(exact & kWrites16)) arena_only_.insert(root(t));
     }
   }
@@ -1696,14 +1699,7 @@ void Planner::lower_conv(int ni) {
         p.f_wfrag = rf(e); p.f_bias = rb(e); p.f_qmul = (const float*)rm(e); p.f_y = ry(e);
         return launch_igemm(p, st);
       };
-      {  // the second result is written by that step
-        PTensor& yt = T(root(ty));
-        if (yt.space == SP_ARENA) {
-          if (fp.step < yt.def_step) yt.def_step = fp.step;
-          if (fp.step > yt.last_step) yt.last_step = fp.step;
-        }
-        arena_only_.insert(root(ty));
-      }
+      touch(fp.step, {}, {ty}, 0);   // (the second result is written by that step)
       set_main(outv, ty);
       return;
     }
@@ -3182,8 +3178,8 @@ bool Planner::lower_fused_group(int seed, int from) {
   gs.d[0] = (int64_t)raw.size();
   const Ref rg = ref(const_from_host(DT_U8, gs, nullptr, &raw));
   const std::string name = "fused:" + comp_->nodes[members.back()].out->name + "(" + std::to_string(members.size()) + ")";
-  // A group that reads nothing made since an earlier one goes into its launch, if it repeats that
-  // one's program (the decode of another head: each is a short launch that hides none of its latency)
+  // A group whose operands were finished before an earlier one goes into its launch (every writer of
+  // them, not the first one: the parts of a Concat arrive by several launches), if it repeats that one's program (the decode of another head: each is a short launch that hides none of its latency)
   // or brings a workgroup for every compute unit (the class scores beside the boxes): its traffic then
   // runs beside the chain of the other.  Box decode and class scores of 16 images: 13 + 42 us as two
   // launches, 45 us as one.  With the LDS of its hungriest group up to 32 KiB a compute unit still
@@ -3198,7 +3194,10 @@ bool Planner::lower_fused_group(int seed, int from) {
     }
     bool ok = l.dt == dt && l.n_groups < kFusedMaxGroups && l.view0[l.n_groups] + fp.n_views <= kFusedMaxBases &&
               (same || (blocks >= 256 && std::max(lds, l.lds_bytes) <= 32 * 1024));
-    for (int t : read_tensors) ok = ok && (T(root(t)).space != SP_ARENA || T(root(t)).def_step < f->step);
+    for (int t : read_tensors) {
+      const auto w = last_write_.find(root(t));
+      ok = ok && (w == last_write_.end() || w->second < f->step);
+    }
     if (ok) { join = f.get(); if (same) break; }
   }
   auto add = [&](FusedStep* f) {
