@@ -479,7 +479,8 @@ void plane_prepare(PlaneGroup* g) {
     I.ho_inv = 1.0f / (float)I.Ho;
     I.wo_inv = 1.0f / (float)I.Wo;
     if (I.kind != PLANE_POOL) continue;
-    const int ks = I.kh == I.kw && I.sh == I.sw ? I.kh * 10 + I.sh : 0;
+    // (size and step as one number, for those that have a compiled window: single digits only)
+    const int ks = I.kh == I.kw && I.sh == I.sw && I.kh <= 3 && I.sh <= 2 ? I.kh * 10 + I.sh : 0;
     const bool full = I.ph == 0 && I.pw == 0 && (I.Ho - 1) * I.sh + I.kh <= I.H && (I.Wo - 1) * I.sw + I.kw <= I.W;
     const bool overlap = I.ph < I.kh && I.pw < I.kw && (I.Ho - 1) * I.sh - I.ph < I.H && (I.Wo - 1) * I.sw - I.pw < I.W;
     I.window = I.is_max ? (!overlap ? 8 : ks == 22 ? 5 : ks == 32 ? 6 : ks == 31 ? 7 : 8)

@@ -53,6 +53,23 @@ def test_windows(kind, window, step, pad, mode):
 
 
 @pytest.mark.parametrize("mode", KW)
+@pytest.mark.parametrize("kind", ["max", "avg"])
+@pytest.mark.parametrize("window,step", [(1, 11), (1, 12), (1, 22), (2, 11), (2, 12)])
+def test_steps_beyond_ten(kind, window, step, mode):
+    """Small windows with steps whose digits, behind the window's, are those of a compiled window."""
+    for n, c, h, w in ((1, 3, 48, 48), (2, 5, 36, 91)):
+        announce("plane steps %s %s %d %d %s" % (mode, kind, window, step, (n, c, h, w)))
+
+        def build(b):
+            pool = b.maxpool if kind == "max" else b.avgpool
+            y = pool(b.leaky_relu(b.arg("x", (n, c, h, w)), 0.25, name="a"), (window,) * 2, (step,) * 2, (0,) * 4, name="p")
+            b.output(y, "pool")
+            b.output(b.reduce_mean(y, (2, 3), True, name="m"), "mean")
+
+        check(build, {"x": image(n, c, h, w)}, mode, 1)
+
+
+@pytest.mark.parametrize("mode", KW)
 def test_places_and_shapes(mode):
     """A value that is a result, a part of two Concats and read by a window; resizes up, down and to odd sizes."""
     for n, c, h, w in ((1, 3, 5, 4), (2, 6, 13, 9), (1, 16, 40, 31), (2, 65, 7, 7)):
