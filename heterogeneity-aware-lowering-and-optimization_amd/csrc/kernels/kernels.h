@@ -452,6 +452,7 @@ struct PlaneLaunch {
 constexpr int kPlaneLdsMax = 159 * 1024;   // (a little is static)
 bool plane_act_ok(ActKind a);   // the activations its instructions take
 void plane_prepare(PlaneGroup* g);
+float plane_group_us(const PlaneGroup& g);   // an estimate of its launch (behind plane_prepare)
 hipError_t launch_plane_group(const PlaneLaunch& l, hipStream_t stream);
 
 // Typed element-wise operators with broadcast (row-major operands, up to 6

@@ -492,6 +492,30 @@ void plane_prepare(PlaneGroup* g) {
   }
 }
 
+// What a launch takes, in microseconds: the longer of the instructions of one workgroup that has a
+// compute unit to itself, of all workgroups of a unit at the rate their threads share, and of the traffic.
+// A step is four elements of every thread.  Fitted to 230 calls that are one chain (1 .. 6144 planes of
+// 14 x 14 .. 280 x 280, fp16 and fp32): two thirds of them within 20 %.
+float plane_group_us(const PlaneGroup& g) {
+  const float full = (float)g.threads / 1024.f, alone = 0.55f + 0.45f * full;   // (few wavefronts hide less, but share less)
+  float chain = 0.f, shared = 0.f, bytes = 0.f;
+  for (int i = 0; i < g.n_inst; ++i) {
+    const PlaneInst& I = g.inst[i];
+    const float units = (float)g.planes * (I.kind == PLANE_POINT ? (float)I.Ho * I.Wo / 4.f : (float)I.Ho * ((I.Wo + 3) / 4));
+    const float steps = units / (float)g.threads;
+    const bool loop = I.kind == PLANE_POOL && I.window >= 8;   // a window that is not compiled: a chain of reads, tap after tap
+    const float us = loop ? 0.25f * (float)I.kh * (float)I.kw
+                          : I.kind == PLANE_POOL ? 0.2f + 0.12f * (float)I.kh * (float)I.kw
+                                                 : I.kind == PLANE_RESIZE ? 0.47f : 0.55f + (I.act == ACT_SIGMOID || I.act == ACT_TANH ? 0.9f : 0.f);
+    chain += 0.3f + (loop ? ceilf(steps) * us : steps * us * alone);
+    shared += steps * us * full * (loop ? 1.f : 0.7f);
+    for (int x : {I.a_ext, I.b_ext, I.dst_ext})
+      if (x >= 0) bytes += (float)g.N * (float)g.C * (float)g.ext[x].hw * (g.ext[x].dt == DT_F32 ? 4.f : 2.f);
+  }
+  const float per_unit = ceilf((float)g.N * (float)g.chunks / 256.f);
+  return 2.f + fmaxf(fmaxf(chain, shared * per_unit), bytes / 3.5e6f);
+}
+
 hipError_t launch_plane_group(const PlaneLaunch& l, hipStream_t stream) {
   const PlaneGroup& g = l.g;
   if (g.n_inst <= 0 || g.n_inst > kPlaneMaxInst || g.N <= 0 || g.C <= 0 || g.planes <= 0 || g.threads < 64 || g.threads > 1024 ||

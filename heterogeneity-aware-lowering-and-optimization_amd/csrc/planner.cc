@@ -3581,6 +3581,48 @@ bool Planner::lower_plane_group(int seed) {
   g.n_inst = (int)prog.size();
   plane_prepare(&g);
 
+  // ---- worth it?  Few large planes leave most of the chip idle for as long as one workgroup takes,
+  // and windows without compiled code are slow in LDS; the separate launches spread both.  Their side of
+  // the estimate: 3.4 us for a launch of an operator and 2.4 for a conversion (a layout change, or
+  // a cast where one channel needs none), their traffic, and 10 us for a plan that only they make long
+  // enough to be replayed from a graph.  us per call, separate -> one launch: [1,4,280,280] fp16 ReLU -
+  // MaxPool 2x2 26 -> 29, [1,64,280,280] 32 -> 30; BatchNorm - Sigmoid - AveragePool - add on
+  // [1,4,195,195] 40 -> 42, [1,4,230,230] 43 -> 52, [1,32,230,230] 63 -> 53; AveragePool 7x7 on
+  // [1,64,75,75] 39 -> 88, [64,96,75,75] 307 -> 377, [1,64,28,28] 39 -> 28.
+  {
+    const bool converts = C > 1 || cdt_ != DT_F32;
+    const double conversion = C > 1 ? 2.4 : 1.2;
+    double us = 0.0, bytes = 0.0;
+    int launches = 0, others = 0;
+    for (int j : members) {
+      const Node& n = comp_->nodes[j];
+      if (n.op == OP_CONCAT || (n.op == OP_UNARY && folded.count(j))) continue;
+      ++launches;
+      us += 3.4;
+      for (int k = 0; k < (n.op == OP_BINARY ? 2 : 1); ++k) bytes += (double)n.in[k]->shape.numel() * es;
+      bytes += (double)n.out->shape.numel() * es;
+    }
+    for (const PlaneInst& I : prog) {
+      if (I.kind == PLANE_POINT && (I.act == ACT_SIGMOID || I.act == ACT_TANH)) us += 2.0;
+      if (I.kind == PLANE_POOL && g.inst[&I - prog.data()].window >= 8) us += 0.1 * I.kh * I.kw;
+    }
+    std::unordered_set<int> converted;   // (a Concat is one conversion of all its parts)
+    for (size_t k = 0; converts && k < ext_tensor.size(); ++k) {
+      if (g.ext[k].hw == 1) continue;
+      bytes += (double)N * C * g.ext[k].hw * (4 + es);
+      if (!converted.insert(ext_tensor[k]).second) continue;
+      ++launches;
+      us += conversion;
+    }
+    for (const Node& n : comp_->nodes) others += n.absorbed || n.op == OP_RESHAPE ? 0 : 1;
+    others -= (int)members.size();
+    if (launches + others >= 6 && 1 + others < 6) us += 10.0;
+    us += bytes / (bytes < 256e6 ? 4e6 : 3.2e6);
+    const double mine = plane_group_us(g);
+    OHIP_DEBUG("planes(%d):%s: %.1f us as one launch, %.1f us as %d", (int)members.size(), first.out->name.c_str(), mine, us, launches);
+    if (mine > us) return give_up();
+  }
+
   // ---- the launch
   std::vector<int> rd, wr;
   std::vector<Ref> ext, sc, sh;
