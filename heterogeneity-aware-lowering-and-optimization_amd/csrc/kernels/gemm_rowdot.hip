@@ -7,15 +7,10 @@
 // reduction.  fp32 only (the summation order differs from the tiled kernels': within the
 // fp32 bound, as theirs differ among themselves).  With every column of a row in one wavefront
 // a Softmax / LogSoftmax over the columns is a few more instructions (IgemmParams::row_softmax).
-// kAct: the activations are 10 KB of code between the sums and the Softmax, through which a launch
-// without one (every classifier head) jumps, one instruction fetch from cold lines behind the other;
-// its own instance is 1.6 .. 3.8 KB of straight code.  mnist, 64 digits from host arrays: 26.9 us per
-// call with the activations in the way, 26.3 without (and 26.4 when GELU was 52 bytes shorter).
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
 #include <cstring>
-#include <type_traits>
 
 #include "device_utils.h"
 #include "kernels.h"
@@ -23,7 +18,7 @@
 namespace ohip {
 namespace {
 
-template <int NB, bool kAct>
+template <int NB>
 __global__ __launch_bounds__(64) void gemm_rowdot_kernel(const IgemmParams p) {
   const int m = blockIdx.x, lane = threadIdx.x;
   const float* x = reinterpret_cast<const float*>(p.x) + (int64_t)m * p.xcs;
@@ -55,7 +50,7 @@ __global__ __launch_bounds__(64) void gemm_rowdot_kernel(const IgemmParams p) {
   const bool col = lane < p.Kout;
   const float b = col && p.bias ? reinterpret_cast<const float*>(p.bias)[lane] : 0.f;
   float v = __builtin_fmaf(mine, p.alpha, b);
-  if constexpr (kAct) v = apply_act(v, p.act, p.act_a, p.act_b);
+  v = apply_act(v, p.act, p.act_a, p.act_b);
   if (p.row_softmax != 0) {
     // (wavefront-uniform)  the row's columns sit in lanes 0 .. Kout-1: maximum, exponentials and
     // their sum across the wavefront, the arithmetic of the stand-alone Softmax launch
@@ -93,14 +88,10 @@ hipError_t launch_gemm_rowdot(const IgemmParams& p, hipStream_t stream) {
   if (!gemm_rowdot_shape(p) || p.x == nullptr || p.w == nullptr || p.y == nullptr || !al16(p.x) || !al16(p.w))
     return hipErrorInvalidValue;
   const dim3 grid((unsigned)((int64_t)p.N * p.Ho * p.Wo)), block(64);
-  auto launch = [&](auto act) {
-    constexpr bool kAct = decltype(act)::value;
-    if (p.Kout <= 4) hipLaunchKernelGGL((gemm_rowdot_kernel<4, kAct>), grid, block, 0, stream, p);
-    else if (p.Kout <= 8) hipLaunchKernelGGL((gemm_rowdot_kernel<8, kAct>), grid, block, 0, stream, p);
-    else hipLaunchKernelGGL((gemm_rowdot_kernel<16, kAct>), grid, block, 0, stream, p);
-    return hipGetLastError();
-  };
-  return p.act == ACT_NONE ? launch(std::false_type{}) : launch(std::true_type{});
+  if (p.Kout <= 4) hipLaunchKernelGGL(gemm_rowdot_kernel<4>, grid, block, 0, stream, p);
+  else if (p.Kout <= 8) hipLaunchKernelGGL(gemm_rowdot_kernel<8>, grid, block, 0, stream, p);
+  else hipLaunchKernelGGL(gemm_rowdot_kernel<16>, grid, block, 0, stream, p);
+  return hipGetLastError();
 }
 
 }  // namespace ohip
