@@ -117,9 +117,9 @@ __device__ __forceinline__ uintx4 pack8_rne(const float (&v)[8]) {
 }
 
 // x * Phi(x) with Phi from erfc(|x| / sqrt 2) = 2^(|x| q(|x|)), q a polynomial of degree 9 fitted to
-// log2(erfc(t)) / t on t = [0, 4] and scaled to |x|.  Beyond, |x| q goes on falling (below -26.9 for
-// every |x| > 5.65, without a bound towards infinity): Phi is 0 or 1 there to the last bit of a float,
-// and nothing needs clamping.  No branch, sixteen instructions - this runs in a GEMM epilogue, where
+// log2(erfc(t)) / t on t = [0, 4] and scaled to |x|.  Beyond, |x| q goes on falling (below -25.8 for
+// every |x| > 5.65, without a bound towards infinity): erfc / 2 is less than 2^-26.8 there, under half of the
+// last bit of 1, so that Phi is 0 or 1 to a float, and nothing needs clamping.  No branch, sixteen instructions - this runs in a GEMM epilogue, where
 // the matrix cores wait for it - and no cancellation for negative x: against the exact function,
 // absolute error below 4e-7 and, down to x = -5.65, relative error below 4e-6 (the float formula
 // 0.5 x (1 + erff(x / sqrt 2)) loses all relative accuracy in the negative tail, where 1 + erff cancels).

@@ -1047,7 +1047,10 @@ int wreg_k_groups(const IgemmParams& p, const int rows32, const int64_t workgrou
 // 4096 x 2304 x 768 24.5 -> 23.1; with a residual 4096 x 768 x 768 15.9 -> 14.7, K = 3072 34.5 -> 33.0).
 // Its stores cover 32-byte pieces of rows, which costs a little where many rounds of workgroups keep the
 // memory busy anyway: ResNet-50 in fp16 at batch 256, results of 25 MB 59 -> 56, of 51 MB 65.2 -> 65.9, of
-// 103 MB 80.7 -> 83.9; with a transcendental activation 100 MB still gain (above).  Reading
+// 103 MB 80.7 -> 83.9; with a transcendental activation 100 MB still gain (above).  The line of 48 MB lies where
+// the first layers lose, which are those of few columns: 1x1 into 256 channels, fp16, results of 35 MB (128 -> 256 over
+// 104 x 104) 40.6 -> 36.2, 51 MB (512 -> 256, 1024 -> 256 over 28 x 28) 51.0 -> 48.9 and 86.5 -> 89.3, 77 MB 75 -> 79, 103 MB 93 -> 98.6;
+// 256 -> 1024 over 14 x 14 would gain at every size: 26 MB 22.9 -> 20.5, 51 MB 34.1 -> 30.0, 103 MB 55.7 -> 50.4.  Reading
 // a residual in pieces needs the whole K loop to hide behind: with more workgroups than are resident at
 // once, 14 x 14 x 1024 at batch 256, 61 -> 84 us.
 int wreg_direct(const IgemmParams& p, const int epi_vec, const int64_t workgroups, const bool rich) {
@@ -1184,7 +1187,9 @@ TapsShape taps_shape(const IgemmParams& p) {
   // on the two-operand kernel.
   // Nine taps of one 2-byte vector into at most 32 channels (a detector's first layer) write twice as
   // much per requested byte: 416 x 416 at batch 16, 3 -> 32 channels, fp16, 110 -> 74 us (2.4 TB/s
-  // written), from 2048 tiles on, where workgroups walk several.
+  // written), from 2048 tiles on, where workgroups walk several.  (At 2, 4 and 8 images 21.8 -> 19.6, 32.7 -> 25.2,
+  // 57.9 -> 39.6; 512 x 512 alone 19.4 -> 17.3, into 16 channels 16.7 -> 14.9.  Below the line it is ahead too, of smaller
+  // launches: 416 x 416 15.1 -> 13.9, 256 x 256 7.7 -> 6.5, 181 x 181 6.9 -> 5.2, and behind at 128 x 128, 4.8 -> 5.2.)
   const bool nine = vpt == 1 && nkk == 5 && es == 2 && p.Kout <= 32 && (forced || (int64_t)p.N * p.Ho * p.Wo >= (128 << 11));
   const bool built = (vpt == 1 && nkk == 8 && es == 1) || nine;
   return built ? TapsShape{nkk, vpt} : TapsShape{0, 0};
@@ -1248,6 +1253,33 @@ hipError_t dispatch(const IgemmParams& p, int epi_vec, hipStream_t s) {
   return dispatch_tiles<TIn, Epi>(p, epi_vec, s);
 }
 
+// Eight consecutive output elements are accessed as one vector (16 bytes, or
+// 8 bytes for 8-bit output, two 16-byte vectors for 4-byte output) when rows
+// and base pointers are aligned accordingly.
+int epilogue_vectors(const IgemmParams& p) {
+  const int oes = dtype_size(p.out_dt);
+  const int64_t vbytes = oes == 1 ? 8 : 16;
+  auto rows_ok = [&](const void* ptr, int64_t cs, int64_t bs) {
+    return ((cs * oes) % vbytes == 0) && ((bs * oes) % vbytes == 0) &&
+           ((reinterpret_cast<uintptr_t>(ptr) % (uintptr_t)vbytes) == 0);
+  };
+  int epi_vec = rows_ok(p.y, p.ycs, p.y_bs);
+  if (p.y_rdiv > 0) epi_vec = epi_vec && rows_ok(p.y, p.y_rlo, p.y_rhi) && rows_ok(p.y, p.y_chi, p.y_chi);
+  if (p.y_zdiv > 0) epi_vec = epi_vec && rows_ok(p.y, p.ycs, p.y_bs_hi);
+  if (p.residual != nullptr) epi_vec = epi_vec && rows_ok(p.residual, p.rcs, p.r_bs);
+  if (p.bias != nullptr) epi_vec = epi_vec && ((reinterpret_cast<uintptr_t>(p.bias) % 16) == 0) && (p.bias_bs % 4 == 0);
+  if (oes == 1) {
+    // bit 2: 8-bit rows allow 16-byte accesses (the requantising epilogue moves 16 channels per lane)
+    auto rows16 = [&](const void* ptr, int64_t cs, int64_t bs) {
+      return cs % 16 == 0 && bs % 16 == 0 && (reinterpret_cast<uintptr_t>(ptr) % 16u) == 0;
+    };
+    bool ok16 = rows16(p.y, p.ycs, p.y_bs);
+    if (p.residual != nullptr) ok16 = ok16 && rows16(p.residual, p.rcs, p.r_bs);
+    if (ok16) epi_vec |= 2;
+  }
+  return epi_vec;
+}
+
 }  // namespace
 
 bool igemm_wants_wfrag(const IgemmParams& p) {
@@ -1285,14 +1317,8 @@ const char* igemm_variant_name(const IgemmParams& p, const bool small_tiles) {
   if (p.w_frag != nullptr && igemm_stream_q8_geometry(p)) return "stream";
   if (p.w_frag != nullptr && lean_steps(p) > 0) return "128x128s";
   if (p.w_frag != nullptr && taps_shape(p).nkk > 0) return "128x64t";
-  if (p.w_frag != nullptr && wreg_shape(p)) {
-    const bool rich = p.act == ACT_GELU_ERF || p.act == ACT_GELU_TANH || p.act == ACT_SIGMOID || p.act == ACT_TANH;
-    const int rows32 = wreg_rows32(p);   // (tiles of 96 rows go by the same names)
-    const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
-    const int64_t tiles = ((M + 32 * rows32 - 1) / (32 * rows32)) * ((p.Kout + 127) / 128);
-    if (!rich && wreg_slices(p) == 1 && wreg_k_groups(p, rows32, tiles * p.batch) == 2) return "128x128w2k";   // two K groups per workgroup
-    return "128x128w";
-  }
+  // (two K groups per workgroup or one; igemm_wreg_form tells the rest)
+  if (p.w_frag != nullptr && wreg_shape(p)) return igemm_wreg_form(p).groups == 2 ? "128x128w2k" : "128x128w";
   return choose_variant(p).name;
 }
 
@@ -1331,6 +1357,16 @@ hipError_t launch_in_parts(const IgemmParams& all, hipStream_t stream) {
 }
 
 }  // namespace
+
+WregForm igemm_wreg_form(const IgemmParams& p) {
+  const bool rich = p.act == ACT_GELU_ERF || p.act == ACT_GELU_TANH || p.act == ACT_SIGMOID || p.act == ACT_TANH;
+  if (!rich && wreg_slices(p) == 2) return {128, 2, 1, 0};
+  const int rows32 = wreg_rows32(p);
+  const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
+  const int64_t workgroups = ((M + 32 * rows32 - 1) / (32 * rows32)) * ((p.Kout + 127) / 128) * p.batch;
+  return {32 * rows32, 1, rich ? 1 : wreg_k_groups(p, rows32, workgroups),
+          p.in_dt == DT_I8 ? 0 : wreg_direct(p, epilogue_vectors(p), workgroups, rich)};
+}
 
 hipError_t launch_igemm(const IgemmParams& p_in, hipStream_t stream) {
   if (p_in.batch > kMaxBatch) return launch_in_parts(p_in, stream);
@@ -1378,30 +1414,7 @@ hipError_t launch_igemm(const IgemmParams& p_in, hipStream_t stream) {
       (int64_t)(p.Wo - 1) * p.sw + (int64_t)(p.S - 1) * p.dw >= (1ll << 30) || p.ph >= (1 << 30) || p.pw >= (1 << 30))
     return hipErrorInvalidValue;
 
-  const int oes = dtype_size(p.out_dt);
-  // Eight consecutive output elements are accessed as one vector (16 bytes, or
-  // 8 bytes for 8-bit output, two 16-byte vectors for 4-byte output) when rows
-  // and base pointers are aligned accordingly.
-  const int64_t vbytes = oes == 1 ? 8 : 16;
-  auto rows_ok = [&](const void* ptr, int64_t cs, int64_t bs) {
-    return ((cs * oes) % vbytes == 0) && ((bs * oes) % vbytes == 0) &&
-           ((reinterpret_cast<uintptr_t>(ptr) % (uintptr_t)vbytes) == 0);
-  };
-  int epi_vec = rows_ok(p.y, p.ycs, p.y_bs);
-  if (p.y_rdiv > 0) epi_vec = epi_vec && rows_ok(p.y, p.y_rlo, p.y_rhi) && rows_ok(p.y, p.y_chi, p.y_chi);
-  if (p.y_zdiv > 0) epi_vec = epi_vec && rows_ok(p.y, p.ycs, p.y_bs_hi);
-  if (p.residual != nullptr) epi_vec = epi_vec && rows_ok(p.residual, p.rcs, p.r_bs);
-  if (p.bias != nullptr) epi_vec = epi_vec && ((reinterpret_cast<uintptr_t>(p.bias) % 16) == 0) && (p.bias_bs % 4 == 0);
-  if (oes == 1) {
-    // bit 2: 8-bit rows allow 16-byte accesses (the requantising epilogue moves 16 channels per lane)
-    auto rows16 = [&](const void* ptr, int64_t cs, int64_t bs) {
-      return cs % 16 == 0 && bs % 16 == 0 && (reinterpret_cast<uintptr_t>(ptr) % 16u) == 0;
-    };
-    bool ok16 = rows16(p.y, p.ycs, p.y_bs);
-    if (p.residual != nullptr) ok16 = ok16 && rows16(p.residual, p.rcs, p.r_bs);
-    if (ok16) epi_vec |= 2;
-  }
-
+  const int epi_vec = epilogue_vectors(p);
   if (p.f_y != nullptr) {
     // a second layer rides in this launch: only the streaming row kernel computes it
     if (p.in_dt != DT_I8 || p.out_dt != DT_I8 || p.w_frag == nullptr || !(epi_vec & 2)) return hipErrorInvalidValue;

@@ -175,6 +175,10 @@ hipError_t launch_igemm(const IgemmParams& p, hipStream_t stream);
 // Name of the kernel variant launch_igemm would pick (for reports); small_tiles = false: of the
 // variant it would pick without the small-tile kernels.
 const char* igemm_variant_name(const IgemmParams& p, bool small_tiles = true);
+// How the weights-in-registers kernel ("128x128w..") runs the launch: rows of a tile, channel slices of a wavefront,
+// K groups, and its epilogue (0 = by rows, 1 = in the accumulator layout, 2 = the same with the residual ahead of the K loop).
+struct WregForm { int rows, slices, groups, epilogue; };
+WregForm igemm_wreg_form(const IgemmParams& p);
 
 // Products with at most 16 output columns, a long reduction and few rows (gemm_rowdot.hip): one
 // wavefront per output row.  Whether the shape qualifies, and the launch (launch_igemm uses both).
@@ -435,7 +439,9 @@ struct PlaneExt {
   int stream = 0;                  // a result that no launch reads: non-temporal stores
 };
 struct PlaneGroup {
-  DType dt = DT_F32;               // type of the values in LDS (every result is rounded to it)
+  // Type of the values in LDS: what an instruction reads of another one's result is rounded to it.
+  // (A result that leaves the plan as fp32 is stored as it was computed, one rounding less.)
+  DType dt = DT_F32;
   int N = 0, C = 0, planes = 1, chunks = 1, threads = 256, lds_bytes = 0;
   unsigned chunk_magic = 0;
   int chunk_shift = 0;

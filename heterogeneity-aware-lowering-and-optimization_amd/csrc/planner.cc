@@ -769,10 +769,17 @@ class Planner {
   // Debug-level log line "<launch>: kernel <variant>" (the device pointers that the
   // choice looks at are replaced by stand-ins: only their presence matters).
   void log_igemm_choice(const std::string& name, IgemmParams ip, bool has_wfrag, bool has_residual) {
-    static int dummy;
+    alignas(16) static int dummy;
     ip.w_frag = has_wfrag ? &dummy : nullptr;
     ip.residual = has_residual ? &dummy : nullptr;
-    OHIP_DEBUG("%s: kernel %s", name.c_str(), igemm_variant_name(ip));
+    const char* kernel = igemm_variant_name(ip);
+    OHIP_DEBUG("%s: kernel %s", name.c_str(), kernel);
+    if (strncmp(kernel, "128x128w", 8) == 0) {
+      static const char* const kEpilogue[] = {"by rows", "in the accumulator layout", "in the accumulator layout, residual ahead"};
+      const WregForm f = igemm_wreg_form(ip);
+      OHIP_DEBUG("%s: tiles of %d rows, %d x 32 channels a wavefront, %d K group%s, results %s", name.c_str(), f.rows, f.slices, f.groups,
+                 f.groups > 1 ? "s" : "", kEpilogue[f.epilogue]);
+    }
     const int small = igemm_slim_variant(ip, has_wfrag);
     ip.slim = -1;
     float us = 0.f;

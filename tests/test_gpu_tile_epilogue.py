@@ -22,6 +22,10 @@ def tolerance(mode, k, want):
     return 1.13 * 5 * (2 * EPS[mode] + 2.0 ** -24 * np.sqrt(k)) + 2 * EPS[mode] * np.max(np.abs(want)) + 4e-7
 
 
+def tile_forms(seen):
+    return [s for s in seen if ": tiles of " in s]
+
+
 @pytest.mark.parametrize("rows", ["96", "128"])
 @pytest.mark.parametrize("mode", MODES)
 @pytest.mark.parametrize("act", ["none", "relu", "gelu", "sigmoid", "tanh"])
@@ -40,6 +44,8 @@ def test_ragged_tiles(rows, mode, act, monkeypatch):
 
         (got, want), seen = run_logged(lambda: run_both(build, {"x": x}, **MODES[mode]))
         assert any("kernel 128x128w" in s for s in seen), [s for s in seen if "kernel" in s]
+        form = tile_forms(seen)
+        assert form and all("tiles of %s rows" % rows in s and ("accumulator" in s) == (n % 32 == 0) for s in form), form
         assert np.max(np.abs(got["o"] - want["o"])) <= tolerance(mode, k, want["o"]), (m, n, k)
 
 
@@ -65,6 +71,10 @@ def test_residual_and_activation_in_either_order(mode, rows, groups, monkeypatch
 
         (got, want), seen = run_logged(lambda: run_both(build, {"x": x, "res": res}, **MODES[mode]))
         assert any("kernel 128x128w" in s for s in seen), [s for s in seen if "kernel" in s]
+        form = tile_forms(seen)
+        stages = k * (4 if mode == "fp32" else 2) // 128
+        assert form and all("tiles of %s rows" % rows in s and ("residual ahead" in s) == (n % 32 == 0) and
+                            ("2 K groups" in s) == (groups == "2" and stages % 2 == 0) for s in form), form
         for key in want:
             assert np.max(np.abs(got[key] - want[key])) <= tolerance(mode, k, want[key]), (m, n, k, key)
 
@@ -82,7 +92,9 @@ def test_residual_on_either_side_of_the_resident_workgroups(batch, monkeypatch):
         y = b.conv(b.arg("x", x.shape), b.const("w", w), name="c")
         b.output(b.relu(b.add(y, b.arg("res", res.shape), name="a"), name="o"), "o")
 
-    got, want = run_both(build, {"x": x, "res": res}, fp16=True)
+    (got, want), seen = run_logged(lambda: run_both(build, {"x": x, "res": res}, fp16=True))
+    form = tile_forms(seen)
+    assert form and all(s.endswith("residual ahead" if batch == 8 else "results by rows") for s in form), form
     assert np.max(np.abs(got["o"] - want["o"])) <= tolerance("fp16", 64, want["o"])
 
 
