@@ -643,12 +643,13 @@ hipError_t launch_slim(const IgemmParams& p, const int epi_vec, const int varian
 // where it came within a factor of two of the best (three for the 128 x 128 row, which stands for
 // all kernels of igemm.hip and its siblings).  A kernel trace of 2225 such launches, each with
 // every kernel that can compute it: estimate + 2.1 us (what a duration holds of the launch itself)
-// is off by 8 .. 20 % rms per kernel and type, and the launches as chosen take 1.8 % more than with
-// the best kernel for each (16 % in one network: BERT-base bf16 at 8 x 128 tokens).  Sums of the
+// is off by 8 .. 24 % rms per kernel and type, and the launches as chosen take 2.8 % more than with
+// the best kernel for each (16 % in one network: ResNet-50 int8 at one image).  Sums of the
 // launches of a step with the wide kernels alone and as chosen: ResNet-50 fp16 at 1 / 4 / 16
-// images 0.74 / 0.77 / 0.85 -> 0.28 / 0.39 / 0.64 ms, fp32 at 4 images 3.7 -> 0.72 ms, BERT-base
-// fp32 at 2 x 128 tokens 4.8 -> 0.96 ms.  (8-bit coefficients: refitted to the K loop of all requests
-// at once; refitting the others as well gave 1.2 %, and BERT-base bf16 at 1 x 41 tokens 389 -> 399 us.)
+// images 0.62 / 0.65 / 0.77 -> 0.28 / 0.38 / 0.63 ms, fp32 at 4 images 2.9 -> 0.72 ms, BERT-base
+// fp32 at 2 x 128 tokens 3.7 -> 0.96 ms.  (8-bit coefficients: refitted to the K loop of all requests
+// at once.  The 2- and 4-byte ones are older and estimate four of eight kernels 13 .. 19 % too long; refitting them
+// too gave 1.2 % over all launches, and BERT-base bf16 at 1 x 41 tokens 389 -> 399 us.)
 namespace {
 struct SlimCost { float fix, chain, tile, work; };
 struct SlimCosts { SlimCost wide, k16, k8, mid; };
