@@ -518,6 +518,8 @@ float plane_group_us(const PlaneGroup& g) {
 
 hipError_t launch_plane_group(const PlaneLaunch& l, hipStream_t stream) {
   const PlaneGroup& g = l.g;
+  for (int i = 0; i < g.n_inst && i < kPlaneMaxInst; ++i)   // (means are of averages: run_pool)
+    if (g.inst[i].mean_ext >= 0 && (g.inst[i].kind != PLANE_POOL || g.inst[i].is_max)) return hipErrorInvalidValue;
   if (g.n_inst <= 0 || g.n_inst > kPlaneMaxInst || g.N <= 0 || g.C <= 0 || g.planes <= 0 || g.threads < 64 || g.threads > 1024 ||
       g.lds_bytes > kPlaneLdsMax || (int64_t)g.N * g.chunks > 0x7fffffff || (int64_t)g.planes * g.chunks < g.C)
     return hipErrorInvalidValue;

@@ -3442,8 +3442,9 @@ bool Planner::lower_plane_group(int seed) {
         I.kh = (int)n.i[2]; I.kw = (int)n.i[3]; I.sh = (int)n.i[4]; I.sw = (int)n.i[5];
         I.ph = (int)n.i[6]; I.pw = (int)n.i[7];
         I.count_pad = n.i[10] != 0;
-        // a pool whose only reader is the mean over its planes is not stored
-        if (!out->is_output && consumers_[out->index].size() == 1) {
+        // an average whose only reader is the mean over its planes is not stored (the kernel sums
+        // the results of averages only: a maximum stays in LDS for an instruction of its own)
+        if (!I.is_max && !out->is_output && consumers_[out->index].size() == 1) {
           const int ci = consumers_[out->index][0];
           if (in_group.count(ci) && comp_->nodes[ci].op == OP_REDUCE) {
             folded.insert(ci);

@@ -53,6 +53,21 @@ def test_windows(kind, window, step, pad, mode):
 
 
 @pytest.mark.parametrize("mode", KW)
+@pytest.mark.parametrize("kind,window,step,pad", WINDOWS)
+def test_mean_of_a_pool_that_nothing_else_reads(kind, window, step, pad, mode):
+    """The pool's own result is no result of the plan."""
+    for n, c, h, w in ((1, 1, 6, 5), (2, 3, 9, 7), (1, 37, 8, 11), (3, 130, 6, 6)):
+        announce("plane mean %s %s %s %s" % (mode, kind, window, (n, c, h, w)))
+
+        def build(b):
+            pool = b.maxpool if kind == "max" else b.avgpool
+            y = pool(b.leaky_relu(b.arg("x", (n, c, h, w)), 0.25, name="a"), window, step, (pad,) * 4, name="p")
+            b.output(b.reduce_mean(y, (2, 3), True, name="m"), "mean")
+
+        check(build, {"x": image(n, c, h, w)}, mode, 1)
+
+
+@pytest.mark.parametrize("mode", KW)
 @pytest.mark.parametrize("kind", ["max", "avg"])
 @pytest.mark.parametrize("window,step", [(1, 11), (1, 12), (1, 22), (2, 11), (2, 12)])
 def test_steps_beyond_ten(kind, window, step, mode):
