@@ -1050,12 +1050,17 @@ int wreg_k_groups(const IgemmParams& p, const int rows32, const int64_t workgrou
 // 103 MB 80.7 -> 83.9; with a transcendental activation 100 MB still gain (above).  The line of 48 MB lies where
 // the first layers lose, which are those of few columns: 1x1 into 256 channels, fp16, results of 35 MB (128 -> 256 over
 // 104 x 104) 40.6 -> 36.2, 51 MB (512 -> 256, 1024 -> 256 over 28 x 28) 51.0 -> 48.9 and 86.5 -> 89.3, 77 MB 75 -> 79, 103 MB 93 -> 98.6;
-// 256 -> 1024 over 14 x 14 would gain at every size: 26 MB 22.9 -> 20.5, 51 MB 34.1 -> 30.0, 103 MB 55.7 -> 50.4.  Reading
-// a residual in pieces needs the whole K loop to hide behind: with more workgroups than are resident at
-// once, 14 x 14 x 1024 at batch 256, 61 -> 84 us.
+// 256 -> 1024 over 14 x 14 would gain at every size: 26 MB 22.9 -> 20.5, 51 MB 34.1 -> 30.0, 103 MB 55.7 -> 50.4.  Results of
+// four bytes stop at two workgroups per unit: bf16 operands, fp32 results, 4096 x 2304 x 768 28.4 -> 29.1, K = 3072
+// 77.8 -> 78.7, K = 256 20.0 -> 19.6 (up to 512 workgroups 0.98 of the time over 25 shapes, 0.93 over 75 of up to 256).
+// Reading a residual in pieces pays where a workgroup has a compute unit to itself, and nothing else covers
+// its round trip: by rows -> ahead, over 95 shapes of up to 256 workgroups 0.97 of the time in 2-byte and in
+// 4-byte results (K 128 .. 3072), over 25 of 257 .. 512 1.03 and 1.07 (8192 x 256 x 768, fp32, 16.6 -> 18.8;
+// 2614 x 768 x 3072 26.6 -> 29.2), and 1.0 .. 1.3 beyond (14 x 14 x 1024 at batch 256, 61 -> 84 us).
 int wreg_direct(const IgemmParams& p, const int epi_vec, const int64_t workgroups, const bool rich) {
   if (p.Kout % 32 != 0 || (epi_vec & 1) == 0 || p.stream_out) return 0;
-  if (p.residual != nullptr) return !rich && workgroups <= 512 ? 2 : 0;
+  if (p.residual != nullptr) return !rich && workgroups <= 256 ? 2 : 0;
+  if (!rich && p.out_dt == DT_F32 && workgroups > 512) return 0;
   const int64_t bytes = (int64_t)p.N * p.Ho * p.Wo * p.Kout * p.batch * dtype_size(p.out_dt);
   return bytes <= ((int64_t)(rich ? 128 : 48) << 20) ? 1 : 0;
 }

@@ -79,9 +79,9 @@ def test_residual_and_activation_in_either_order(mode, rows, groups, monkeypatch
             assert np.max(np.abs(got[key] - want[key])) <= tolerance(mode, k, want[key]), (m, n, k, key)
 
 
-@pytest.mark.parametrize("batch", [8, 9])
+@pytest.mark.parametrize("batch", [4, 5, 8, 9])
 def test_residual_on_either_side_of_the_resident_workgroups(batch, monkeypatch):
-    """512 workgroups (the accumulator layout) and more (by rows)."""
+    """256 workgroups, one per compute unit (residual ahead, in the accumulator layout), and more (by rows)."""
     monkeypatch.setenv("ODLA_HIP_IGEMM_TILE", "wreg")
     r = np.random.default_rng(7)
     x = r.standard_normal((batch, 64, 91, 90)).astype(np.float32)
@@ -94,7 +94,7 @@ def test_residual_on_either_side_of_the_resident_workgroups(batch, monkeypatch):
 
     (got, want), seen = run_logged(lambda: run_both(build, {"x": x, "res": res}, fp16=True))
     form = tile_forms(seen)
-    assert form and all(s.endswith("residual ahead" if batch == 8 else "results by rows") for s in form), form
+    assert form and all(s.endswith("residual ahead" if batch == 4 else "results by rows") for s in form), form
     assert np.max(np.abs(got["o"] - want["o"])) <= tolerance("fp16", 64, want["o"])
 
 
