@@ -679,6 +679,117 @@ __device__ __forceinline__ void fused_walks(const FusedGroup* __restrict__ g, co
   }
 }
 
+// U points of a chain, from point i2 of the walk on: their loads, the operators on the values in
+// hand, their stores.
+template <typename T, int U>
+__device__ __forceinline__ void fused_chain_points(const FusedInstr* prog, const int first, const int last, const FusedViewAt<uint32_t>& in_view,
+                                                   const FusedViewAt<uint32_t>& out_view, const uint32_t in_at, const uint32_t out_at,
+                                                   const uint32_t i2, const bool live, const int once0, const float o0, const float o1,
+                                                   const bool best_of, float& best, int& best_at) {
+  float x[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) x[u] = live ? Store<T>::ld(fused_at<const T, uint32_t>(in_view.base, in_at + (i2 + u) * in_view.st[2])) : 0.f;
+  for (int k = first; k < last; ++k) {
+    const FusedInstr in = fused_uniform(prog[k]);
+#define CHAIN_EACH(EXPR) _Pragma("unroll") for (int u = 0; u < U; ++u) x[u] = EXPR; break
+    if (in.op == FOP_UNARY) {
+      switch ((ActKind)in.kind) {
+        case ACT_SIGMOID: CHAIN_EACH(fused_act<T>(x[u], ACT_SIGMOID, 0.f, 0.f));
+        case ACT_EXP: CHAIN_EACH(fused_act<T>(x[u], ACT_EXP, 0.f, 0.f));
+        case ACT_TANH: CHAIN_EACH(fused_act<T>(x[u], ACT_TANH, 0.f, 0.f));
+        default: CHAIN_EACH(fused_act<T>(x[u], ACT_RELU, 0.f, 0.f));
+      }
+    } else {
+      // (the other operand: an immediate or what the walk does not change; `pad[0]`: it is the left one)
+      const int reg = in.pad[0] ? in.a : in.b;
+      const float y = reg < 0 ? in.fa : reg == once0 ? o0 : o1;
+      switch ((BinKind)in.kind) {
+        case BIN_ADD: CHAIN_EACH(x[u] + y);
+        case BIN_MUL: CHAIN_EACH(x[u] * y);
+        default:
+          if (in.pad[0]) { CHAIN_EACH(y - x[u]); }
+          CHAIN_EACH(x[u] - y);
+      }
+    }
+#undef CHAIN_EACH
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    T t;
+    Store<T>::st(&t, x[u]);
+    if (live) *fused_at<T, uint32_t>(out_view.base, out_at + (i2 + u) * out_view.st[2]) = t;
+    if (best_of) {
+      const float v = Store<T>::ld(&t);
+      if (v > best || i2 + u == 0) { best = v; best_at = (int)i2 + u; }
+    }
+  }
+}
+
+// A chain (FusedGroup::chain): the values of a walk stay in vector registers, up to eight points at a
+// time, and only the once section uses the registers in LDS, one point each.  64 consecutive points
+// across the walks per wavefront; the four wavefronts of a workgroup share a walk between them, and
+// workgroups do where there would be few.  A workgroup goes through several such groups of points, so
+// that its copy of the program (3 us behind the start of the launch) is paid once and in one round.
+// With best_of the class scores of a detector leave with each box's best one: the launch that read
+// all of them again (14 us for 16 images) is gone.
+// Class scores of 16 images (13.6 M points, 116 MB) beside the boxes: 45.0 -> 33.6 us, what is left
+// being mostly the sigmoids (some 45 vector instructions a point); 20 points at a time 38.2, half the
+// workgroups 39.4, the same number of turns for all of them 34.4.
+template <typename T>
+__device__ __forceinline__ void fused_chain(const FusedGroup* __restrict__ g, const FusedInstr* prog, const FusedViewAt<uint32_t>* views,
+                                            float* r, const uint32_t block, const uint32_t blocks, float* __restrict__ best_ws,
+                                            int32_t* __restrict__ at_ws) {
+  __shared__ float s_best[4][64];
+  __shared__ int s_at[4][64];
+  const uint32_t d0 = (uint32_t)g->dims[0], d1 = (uint32_t)g->dims[1], d2 = (uint32_t)g->dims[2], d3 = (uint32_t)g->dims[3];
+  const uint32_t cols = d0 * d1 * d3, walk = (uint32_t)g->walk, split = (uint32_t)g->chain;
+  const int once_loads = g->n_once_loads, loads_end = once_loads + 1, once_end = loads_end + g->n_once, last = g->n_instr - 1;
+  const bool best_of = g->best_of != 0;
+  const int once0 = g->chain_once[0], once1 = g->chain_once[1];
+  const FusedViewAt<uint32_t> vin = fused_uniform(views[prog[once_loads].a]), vout = fused_uniform(views[prog[last].dst]);
+  const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t turns = (cols + 63) / 64 * split;
+  for (uint32_t t = block; t < turns; t += blocks) {
+    const uint32_t group = split == 1 ? t : t / split, piece = (split == 1 ? 0 : t - group * split) * 4 + part;
+    const uint32_t c = group * 64 + lane, col = c < cols ? c : cols - 1;
+    const bool live = c < cols;
+    const uint32_t q = fast_div(col, g->magic[0], g->shift[0]), i3 = col - q * d3;
+    const uint32_t i0 = fast_div(q, g->magic[2], g->shift[2]), i1 = q - i0 * d1;
+    for (int k = 0; k < once_loads; ++k) {
+      const FusedInstr in = fused_uniform(prog[k]);
+      const FusedViewAt<uint32_t> v = fused_uniform(views[in.a]);
+      r[in.dst * kThreads] = Store<T>::ld(fused_at<const T, uint32_t>(v.base, v.off + i0 * v.st[0] + i1 * v.st[1] + i3 * v.st[3]));
+    }
+    for (int k = loads_end; k < once_end; ++k) fused_op<T, 1, 1>(fused_uniform(prog[k]), r);
+    const float o0 = r[once0 * kThreads], o1 = r[once1 * kThreads];
+    const uint32_t in_at = vin.off + i0 * vin.st[0] + i1 * vin.st[1] + i3 * vin.st[3];
+    const uint32_t out_at = vout.off + i0 * vout.st[0] + i1 * vout.st[1] + i3 * vout.st[3];
+    const uint32_t from = piece * walk, end = from + walk < d2 ? from + walk : d2;
+    float best = -INFINITY;
+    int best_at = (int)(from < d2 ? from : 0);
+    uint32_t i2 = from;
+#define CHAIN_POINTS(U) fused_chain_points<T, U>(prog, once_end, last, vin, vout, in_at, out_at, i2, live, once0, o0, o1, best_of, best, best_at)
+    for (; i2 + 8 <= end; i2 += 8) CHAIN_POINTS(8);
+    if (i2 + 4 <= end) { CHAIN_POINTS(4); i2 += 4; }
+    for (; i2 < end; ++i2) CHAIN_POINTS(1);
+#undef CHAIN_POINTS
+    if (best_of) {   // (uniform over the workgroup)
+      s_best[part][lane] = best;
+      s_at[part][lane] = best_at;
+      __syncthreads();
+      if (part == 0 && live) {
+#pragma unroll
+        for (int w = 1; w < 4; ++w)
+          if (s_best[w][lane] > best) { best = s_best[w][lane]; best_at = s_at[w][lane]; }
+        const int64_t to = g->best_off + i0 * g->best_st[0] + i1 * g->best_st[1] + i3 * g->best_st[2];
+        best_ws[to] = best;
+        at_ws[to] = best_at;
+      }
+      __syncthreads();
+    }
+  }
+}
+
 template <typename T, typename I>
 __global__ void __launch_bounds__(kThreads) fused_eltwise_kernel(const FusedLaunch l) {
   extern __shared__ float fused_regs[];
@@ -707,6 +818,12 @@ __global__ void __launch_bounds__(kThreads) fused_eltwise_kernel(const FusedLaun
   }
   __syncthreads();
   float* r = fused_regs + threadIdx.x;
+  if constexpr (sizeof(I) == 4) {
+    if (g->chain > 0) {
+      fused_chain<T>(g, s_prog, s_view, r, blockIdx.x - l.block0[n], l.block0[n + 1] - l.block0[n], l.best, l.best_at);
+      return;
+    }
+  }
   const int64_t first = (int64_t)((int)blockIdx.x - l.block0[n]) * kThreads + threadIdx.x;
   const int64_t stride = (int64_t)(l.block0[n + 1] - l.block0[n]) * kThreads;
   if (g->points == 8) fused_walks<T, 8, I>(g, s_prog, s_view, r, first, stride);
@@ -973,6 +1090,8 @@ hipError_t launch_fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t stream)
   return hipGetLastError();
 }
 
+constexpr int kChainBlocks = 256 * 6;   // workgroups of a chain
+
 bool fused_prepare(FusedGroup* g, int* blocks, size_t* lds_bytes, bool* wide) {
   if (g->n_instr <= 0 || g->n_instr > kFusedMaxInstr || g->n_views < 0 || g->n_views > kFusedMaxViews) return false;
   if (g->n_once_loads < 0 || g->n_loads < 0 || g->n_once < 0) return false;
@@ -1001,6 +1120,39 @@ bool fused_prepare(FusedGroup* g, int* blocks, size_t* lds_bytes, bool* wide) {
     if (is_bin && (in.b >= kFusedMaxRegs || (in.a < 0 && in.b < 0))) return false;
     if (!is_store && in.dst + 1 > n_regs) n_regs = in.dst + 1;
   }
+  // A chain: behind the once section one load, operators on the value in hand (the other operand: an
+  // immediate or one of at most two results of the once section), one store.  Walks of fewer than 16
+  // points and launches of fewer than two wavefronts of neighbouring points stay on the general path.
+  const int64_t cols = g->dims[0] * g->dims[1] * g->dims[3];
+  bool chain = g->n_loads == 1 && g->n_instr > once_end && g->prog[g->n_instr - 1].op == FOP_STORE && g->dims[2] >= 16 && cols >= 128;
+  if (chain) {
+    unsigned once_regs = 0;
+    for (int k = 0; k < once_end; ++k)
+      if (k != g->n_once_loads) once_regs |= 1u << g->prog[k].dst;
+    int used = 0, once[2] = {0, 0}, value = g->prog[g->n_once_loads].dst;
+    for (int k = once_end; k + 1 < g->n_instr && chain; ++k) {
+      FusedInstr& in = g->prog[k];
+      if (in.op == FOP_UNARY) {
+        chain = in.a == value && (in.kind == ACT_SIGMOID || in.kind == ACT_EXP || in.kind == ACT_TANH || in.kind == ACT_RELU);
+      } else if (in.op == FOP_BINARY) {
+        const bool right = in.b == value;
+        const int other = right ? in.a : in.b;
+        chain = (in.a == value) != right && (in.kind == BIN_ADD || in.kind == BIN_SUB || in.kind == BIN_MUL);
+        if (chain && other >= 0 && !(used > 0 && once[0] == other) && !(used > 1 && once[1] == other)) {
+          chain = (once_regs >> other & 1u) != 0 && used < 2;
+          if (chain) once[used++] = other;
+        }
+        in.pad[0] = right ? 1 : 0;
+      } else {
+        chain = false;
+      }
+      value = in.dst;
+      chain = chain && (once_regs >> value & 1u) == 0;
+    }
+    chain = chain && g->prog[g->n_instr - 1].a == value;
+    g->chain_once[0] = once[0];
+    g->chain_once[1] = used > 1 ? once[1] : once[0];
+  }
   // points of the walk per instruction: as many as 32 KiB of LDS registers allow
   g->points = (walk >= 8 && n_regs * 8 <= 32) ? 8 : (walk >= 4 && n_regs * 4 <= 32) ? 4 : ((walk >= 2 && n_regs * 2 <= 32) ? 2 : 1);
   *lds_bytes = (size_t)n_regs * g->points * kThreads * sizeof(float);
@@ -1017,8 +1169,22 @@ bool fused_prepare(FusedGroup* g, int* blocks, size_t* lds_bytes, bool* wide) {
     if (far >= ((int64_t)1 << 29)) small = false;   // (bytes)
   }
   *wide = !small;
+  g->chain = 0;
+  if (chain && small) {
+    // a workgroup's four wavefronts deal a walk between them, several workgroups where there are few
+    const int64_t groups = (cols + 63) / 64;
+    int64_t split = (1024 + groups - 1) / groups;
+    if (split > g->dims[2] / 16) split = g->dims[2] / 16;
+    if (g->best_of) split = 1;
+    g->chain = (int)split;
+    g->walk = ((g->dims[2] + 4 * split - 1) / (4 * split) + 3) / 4 * 4;
+    g->points = 1;
+    *lds_bytes = (size_t)n_regs * kThreads * sizeof(float);
+    *blocks = (int)(groups * split < kChainBlocks ? groups * split : kChainBlocks);
+  }
+  const int64_t per = g->walk > 0 ? g->walk : g->dims[2];
   for (int v : {0, 1, 2}) {   // (32-bit walks: divisors of the thread number and what is left of it)
-    const int64_t d = v == 0 ? g->dims[3] : v == 1 ? (g->dims[2] + walk - 1) / walk : g->dims[1];
+    const int64_t d = v == 0 ? g->dims[3] : v == 1 ? (g->dims[2] + per - 1) / per : g->dims[1];
     if (small) div_magic((int)d, &g->magic[v], &g->shift[v]);
   }
   return true;

@@ -386,10 +386,19 @@ struct FusedGroup {
   int64_t walk = 0;    // points of dims[2] per thread (0: all of them); short walks give more threads
   unsigned magic[3] = {0, 0, 0};
   int shift[3] = {0, 0, 0};
+  // Behind its once section a chain is one load, operators on the value in hand and one store (see
+  // fused_chain).  0: no chain; otherwise a walk of dims[2] is dealt to 4 * chain wavefronts, `walk` points each.
+  int chain = 0;
+  int chain_once[2] = {0, 0};   // the registers of the once section that its operators read
+  // Where best_of is set, a whole walk meets in one workgroup and leaves its largest stored value and
+  // that value's place (the first of equals; a NaN only as the first of all) in FusedLaunch::best /
+  // best_at, at the point's own offset: best_off + i0 * best_st[0] + i1 * best_st[1] + i3 * best_st[2].
+  int best_of = 0;
+  int64_t best_off = 0, best_st[3] = {0, 0, 0};
   FusedView view[kFusedMaxViews];
   FusedInstr prog[kFusedMaxInstr];
 };
-// Checks a group and sets `points`; *blocks: the workgroups it takes, *lds_bytes: its registers,
+// Checks a group and sets `points` and what a chain needs; *blocks: the workgroups it takes, *lds_bytes: its registers,
 // *wide: its offsets need 64 bits.
 bool fused_prepare(FusedGroup* g, int* blocks, size_t* lds_bytes, bool* wide);
 // One launch of up to kFusedMaxGroups groups that do not depend on each other.
@@ -402,6 +411,8 @@ struct FusedLaunch {
   int block0[kFusedMaxGroups + 1] = {0};   // first workgroup of a group; behind the last: the grid
   int view0[kFusedMaxGroups + 1] = {0};    // a group's first view in base[]
   const FusedGroup* group[kFusedMaxGroups] = {nullptr};
+  float* best = nullptr;
+  int32_t* best_at = nullptr;
   const void* base[kFusedMaxBases] = {nullptr};   // per view (stores cast the const away)
 };
 hipError_t launch_fused_eltwise(const FusedLaunch& l, hipStream_t stream);
@@ -615,10 +626,14 @@ hipError_t launch_rownorm(const void* x, void* y, DType dt, int64_t rows, int64_
 // out int32 [N][max_out][3] = {image, class, box}, -1 padded.
 // workspace: at least nms_workspace_bytes(N, B) bytes of device memory.
 size_t nms_workspace_bytes(int N, int B);
+// Where in the workspace the best class score of each box ([N][B] floats) and its class ([N][B] int32) lie.
+size_t nms_best_offset(int N, int B);
+size_t nms_class_offset(int N, int B);
+// best_ready: both are there already (the launch that made the scores left them), and the scores are not read.
 // boxes / scores are read in their storage type (DT_F32, DT_F16 or DT_BF16).
 hipError_t launch_nms(const void* boxes, DType boxes_dt, const void* scores, DType scores_dt, int N, int C, int B,
                       int max_out, float iou_thr, float score_thr, int32_t* out,
-                      void* workspace, hipStream_t stream, int image_base = 0);
+                      void* workspace, hipStream_t stream, int image_base = 0, bool best_ready = false);
 
 // YOLOv3 post-processing of one image: decode of three heads [3*(5+classes)][dim][dim]
 // (fp32, channels first) into `boxes` [total][4] (y min, x min, y max, x max in

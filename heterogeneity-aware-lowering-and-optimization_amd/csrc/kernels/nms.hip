@@ -348,7 +348,7 @@ __device__ __forceinline__ void nms_on_cu(const TB* __restrict__ bx, const int32
 template <typename TB>
 __global__ void __launch_bounds__(kNmsThreads)
 nms_kernel(const TB* __restrict__ boxes, const float* __restrict__ best_ws, int B,
-           int max_out, float iou_thr, const unsigned long long* __restrict__ mask_ws, int32_t* __restrict__ out,
+           int max_out, float iou_thr, float score_thr, const unsigned long long* __restrict__ mask_ws, int32_t* __restrict__ out,
            unsigned long long* keys_ws, const int32_t* cls_ws, unsigned char* sup_ws, int64_t bpad,
            int lds_slots, int image_base) {
   const int n = blockIdx.x;
@@ -366,26 +366,67 @@ nms_kernel(const TB* __restrict__ boxes, const float* __restrict__ best_ws, int 
   for (int i = tid; i < max_out * 3; i += kNmsThreads) o[i] = -1;
   __syncthreads();
 
-  // ---- phase 1 (second half): the boxes above the threshold, in no order; then their keys ----
-  const int words = (B + 63) / 64;
-  for (int w = tid; w < words; w += kNmsThreads) {
-    unsigned long long mask = mask_ws[(int64_t)n * words + w];
-    if (mask == 0) continue;
-    int slot = atomicAdd(&s_count, __popcll(mask));
-    for (; mask != 0; mask &= mask - 1, ++slot) {
-      const unsigned b = (unsigned)w * 64 + (unsigned)(__ffsll(mask) - 1);
-      (slot < lds_slots ? lds_keys : keys)[slot] = b;
+  // ---- phase 1 (second half): the boxes above the threshold, in no order, and their keys ----
+  auto key_of = [](const float score, const unsigned b) {
+    unsigned w = __float_as_uint(score);
+    w = (w & 0x80000000u) ? ~w : (w | 0x80000000u);  // ascending in w == ascending in value
+    return ((unsigned long long)(~w) << 32) | b;     // score desc, then box asc
+  };
+  if (mask_ws == nullptr) {
+    // no words of decisions: the scores themselves, up to 24 per thread in flight (all boxes of a
+    // 608 x 608 image at once; eight at a time took 3 us more there), and the keys at once
+    constexpr int kAhead = 24;
+    for (int b0 = 0; b0 < B; b0 += kAhead * kNmsThreads) {
+      float v[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int b = b0 + u * kNmsThreads + tid;
+        if (b0 + u * kNmsThreads < B) v[u] = bestv[b < B ? b : B - 1];
+      }
+      // (one place in the list per wavefront for all of them: an atomic each took 3 us)
+      unsigned long long mask[kAhead];
+      int mine = 0;
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        mask[u] = 0;
+        if (b0 + u * kNmsThreads < B) mask[u] = __ballot(b0 + u * kNmsThreads + tid < B && v[u] > score_thr);
+        mine += __popcll(mask[u]);
+      }
+      if (mine == 0) continue;
+      int slot = 0;
+      if ((tid & 63) == 0) slot = atomicAdd(&s_count, mine);
+      slot = __builtin_amdgcn_readfirstlane(slot);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int at = slot + __popcll(mask[u] & ((1ull << (tid & 63)) - 1));
+        if ((mask[u] >> (tid & 63)) & 1ull) (at < lds_slots ? lds_keys : keys)[at] = key_of(v[u], (unsigned)(b0 + u * kNmsThreads + tid));
+        slot += __popcll(mask[u]);
+      }
+    }
+  } else {
+    const int words = (B + 63) / 64;
+    for (int w = tid; w < words; w += kNmsThreads) {
+      unsigned long long mask = mask_ws[(int64_t)n * words + w];
+      if (mask == 0) continue;
+      int slot = atomicAdd(&s_count, __popcll(mask));
+      for (; mask != 0; mask &= mask - 1, ++slot) {
+        const unsigned b = (unsigned)w * 64 + (unsigned)(__ffsll(mask) - 1);
+        (slot < lds_slots ? lds_keys : keys)[slot] = b;
+      }
     }
   }
   __syncthreads();
   const int M = s_count;
   if (M == 0 || max_out == 0) return;
   const bool on_cu = M <= lds_slots;   // (lds_slots is a power of two: the padded list fits as well)
-  for (int i = tid; i < M; i += kNmsThreads) {
-    const unsigned b = (unsigned)(i < lds_slots ? lds_keys : keys)[i];
-    unsigned w = __float_as_uint(bestv[b]);
-    w = (w & 0x80000000u) ? ~w : (w | 0x80000000u);  // ascending in w == ascending in value
-    (on_cu ? lds_keys : keys)[i] = ((unsigned long long)(~w) << 32) | b;  // score desc, then box asc
+  if (mask_ws == nullptr) {
+    if (!on_cu)
+      for (int i = tid; i < lds_slots; i += kNmsThreads) keys[i] = lds_keys[i];
+  } else {
+    for (int i = tid; i < M; i += kNmsThreads) {
+      const unsigned b = (unsigned)(i < lds_slots ? lds_keys : keys)[i];
+      (on_cu ? lds_keys : keys)[i] = key_of(bestv[b], b);
+    }
   }
   __syncthreads();
   const int P = (int)next_pow2(M);
@@ -455,8 +496,11 @@ size_t nms_workspace_bytes(int N, int B) {
   return (bytes + 255) & ~(size_t)255;
 }
 
+size_t nms_class_offset(int N, int B) { return ((size_t)N * next_pow2(B) + (size_t)N * ((B + 63) / 64)) * 8; }
+size_t nms_best_offset(int N, int B) { return nms_class_offset(N, B) + (size_t)N * B * 4; }
+
 template <typename TB>
-static hipError_t launch_nms_kernel(const void* boxes, const float* best, int N, int B, int max_out, float iou_thr,
+static hipError_t launch_nms_kernel(const void* boxes, const float* best, int N, int B, int max_out, float iou_thr, float score_thr,
                                     const unsigned long long* masks, int32_t* out, unsigned long long* keys, const int32_t* cls,
                                     unsigned char* sup, int64_t bpad, int image_base, hipStream_t stream) {
   // candidate list on the compute unit - first the keys (two exchange buffers of 8 B per
@@ -467,13 +511,13 @@ static hipError_t launch_nms_kernel(const void* boxes, const float* best, int N,
   const hipError_t e = limit.raise(reinterpret_cast<const void*>(nms_kernel<TB>), 8192 * 17);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(nms_kernel<TB>, dim3(N), dim3(kNmsThreads), lds_bytes, stream, (const TB*)boxes, best, B, max_out,
-                     iou_thr, masks, out, keys, cls, sup, bpad, lds_slots, image_base);
+                     iou_thr, score_thr, masks, out, keys, cls, sup, bpad, lds_slots, image_base);
   return hipGetLastError();
 }
 
 hipError_t launch_nms(const void* boxes, DType boxes_dt, const void* scores, DType scores_dt, int N, int C, int B,
                       int max_out, float iou_thr, float score_thr, int32_t* out, void* workspace,
-                      hipStream_t stream, int image_base) {
+                      hipStream_t stream, int image_base, bool best_ready) {
   if (!boxes || !scores || !out || !workspace || N <= 0 || C <= 0 || B <= 0 || max_out < 0)
     return hipErrorInvalidValue;
   if ((reinterpret_cast<uintptr_t>(workspace) & 7u) != 0) return hipErrorInvalidValue;
@@ -481,21 +525,21 @@ hipError_t launch_nms(const void* boxes, DType boxes_dt, const void* scores, DTy
   if (bpad > (1 << 24)) return hipErrorInvalidValue;
   unsigned long long* keys = reinterpret_cast<unsigned long long*>(workspace);
   unsigned long long* masks = keys + (int64_t)N * bpad;
-  int32_t* cls = reinterpret_cast<int32_t*>(masks + (int64_t)N * ((B + 63) / 64));
-  float* best = reinterpret_cast<float*>(cls + (int64_t)N * B);
+  int32_t* cls = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + nms_class_offset(N, B));
+  float* best = reinterpret_cast<float*>(static_cast<char*>(workspace) + nms_best_offset(N, B));
   unsigned char* sup = reinterpret_cast<unsigned char*>(best + (int64_t)N * B);
   if (N > 65535) return hipErrorInvalidValue;
   const dim3 grid1((unsigned)((B + 63) / 64), (unsigned)N);
-  switch (scores_dt) {
+  if (!best_ready) switch (scores_dt) {
     case DT_F32: hipLaunchKernelGGL(nms_best_class_kernel<float>, grid1, dim3(256), 0, stream, (const float*)scores, C, B, score_thr, best, cls, masks); break;
     case DT_F16: hipLaunchKernelGGL(nms_best_class_kernel<f16_t>, grid1, dim3(256), 0, stream, (const f16_t*)scores, C, B, score_thr, best, cls, masks); break;
     case DT_BF16: hipLaunchKernelGGL(nms_best_class_kernel<bf16_t>, grid1, dim3(256), 0, stream, (const bf16_t*)scores, C, B, score_thr, best, cls, masks); break;
     default: return hipErrorInvalidValue;
   }
   switch (boxes_dt) {
-    case DT_F32: return launch_nms_kernel<float>(boxes, best, N, B, max_out, iou_thr, masks, out, keys, cls, sup, bpad, image_base, stream);
-    case DT_F16: return launch_nms_kernel<f16_t>(boxes, best, N, B, max_out, iou_thr, masks, out, keys, cls, sup, bpad, image_base, stream);
-    case DT_BF16: return launch_nms_kernel<bf16_t>(boxes, best, N, B, max_out, iou_thr, masks, out, keys, cls, sup, bpad, image_base, stream);
+    case DT_F32: return launch_nms_kernel<float>(boxes, best, N, B, max_out, iou_thr, score_thr, best_ready ? nullptr : masks, out, keys, cls, sup, bpad, image_base, stream);
+    case DT_F16: return launch_nms_kernel<f16_t>(boxes, best, N, B, max_out, iou_thr, score_thr, best_ready ? nullptr : masks, out, keys, cls, sup, bpad, image_base, stream);
+    case DT_BF16: return launch_nms_kernel<bf16_t>(boxes, best, N, B, max_out, iou_thr, score_thr, best_ready ? nullptr : masks, out, keys, cls, sup, bpad, image_base, stream);
     default: return hipErrorInvalidValue;
   }
 }

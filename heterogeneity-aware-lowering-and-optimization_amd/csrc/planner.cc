@@ -648,8 +648,26 @@ class Planner {
   bool available(const _odla_value* v) const {
     return v->kind != _odla_value::TEMP || vs_[v->index].main >= 0 || strided_.count(v->index) != 0;
   }
+  // The value is the scores of a NonMaxSuppression, or a part of them.
+  bool scores_of_nms(const _odla_value* v, const bool part = true) const {
+    for (int c : consumers_[v->index]) {
+      const Node& n = comp_->nodes[c];
+      if (n.op == OP_NMS && n.in[1] == v) return true;
+      if (part && n.op == OP_CONCAT && scores_of_nms(n.out, false)) return true;
+    }
+    return false;
+  }
   // The launches of element-wise groups so far (later groups may join one).
-  struct FusedStep { int step = 0, n_ops = 0; FusedGroup model; FusedLaunch launch; std::vector<Ref> groups, bases; };
+  struct FusedPart { FusedGroup group; int blocks = 0, tensor = -1; size_t blob = 0; };   // tensor: the last store's
+  struct FusedStep {
+    int step = 0, n_ops = 0;
+    FusedGroup model;
+    FusedLaunch launch;
+    std::vector<Ref> groups, bases;
+    std::vector<FusedPart> parts;
+    Ref best{nullptr, -1};   // where the best values go (FusedGroup::best_of), if anywhere
+    size_t best_off = 0, best_at_off = 0;
+  };
   std::vector<std::shared_ptr<FusedStep>> fused_steps_;
   // A Transpose (and Reshapes behind it) whose readers all look like members of element-wise groups
   // stays a description of where its elements lie: extents and source strides, outermost first, of
@@ -734,6 +752,7 @@ class Planner {
   void lower_transpose(int ni);
   void lower_qdq(int ni);
   void lower_nms(int ni);
+  bool best_scores_from_groups(int ts, int tw, int64_t N, int64_t C, int64_t B);
   void lower_ewise(int ni);
   void lower_argext(int ni);
   void lower_copynd(int ni);
@@ -3184,13 +3203,22 @@ bool Planner::lower_fused_group(int seed, int from) {
   gs.rank = 1;
   gs.d[0] = (int64_t)raw.size();
   const Ref rg = ref(const_from_host(DT_U8, gs, nullptr, &raw));
+  FusedPart part;
+  part.group = fp;
+  part.blocks = blocks;
+  part.tensor = views.back().tensor;
+  part.blob = plan_->blobs.size() - 1;
   const std::string name = "fused:" + comp_->nodes[members.back()].out->name + "(" + std::to_string(members.size()) + ")";
   // A group whose operands were finished before an earlier one goes into its launch (every writer of
   // them, not the first one: the parts of a Concat arrive by several launches), if it repeats that one's program (the decode of another head: each is a short launch that hides none of its latency)
   // or brings a workgroup for every compute unit (the class scores beside the boxes): its traffic then
-  // runs beside the chain of the other.  Box decode and class scores of 16 images: 13 + 42 us as two
+  // runs beside the chain of the other.  (The scores of a NonMaxSuppression do so with fewer, too: the parts
+  // of the other heads follow the first, and one image of 608 x 608 takes 62 us a call with the scores in a launch
+  // of their own, 55 without.)  Box decode and class scores of 16 images: 13 + 42 us as two
   // launches, 45 us as one.  With the LDS of its hungriest group up to 32 KiB a compute unit still
   // holds five workgroups.
+  bool for_nms = fp.chain > 0;
+  for (const Sink& sk : sinks) for_nms = for_nms && scores_of_nms(comp_->nodes[sk.node].out);
   FusedStep* join = nullptr;
   for (auto& f : fused_steps_) {
     const FusedLaunch& l = f->launch;
@@ -3200,7 +3228,7 @@ bool Planner::lower_fused_group(int seed, int from) {
       same = x.op == y.op && x.kind == y.kind && x.dst == y.dst && x.a == y.a && x.b == y.b;
     }
     bool ok = l.dt == dt && l.n_groups < kFusedMaxGroups && l.view0[l.n_groups] + fp.n_views <= kFusedMaxBases &&
-              (same || (blocks >= 256 && std::max(lds, l.lds_bytes) <= 32 * 1024));
+              (same || ((blocks >= 256 || for_nms) && std::max(lds, l.lds_bytes) <= 32 * 1024));
     for (int t : read_tensors) {
       const auto w = last_write_.find(root(t));
       ok = ok && (w == last_write_.end() || w->second < f->step);
@@ -3215,6 +3243,7 @@ bool Planner::lower_fused_group(int seed, int from) {
     l.lds_bytes = std::max(l.lds_bytes, lds);
     l.wide = l.wide || wide;
     f->groups.push_back(rg);
+    f->parts.push_back(part);
     for (const View& vw : views) f->bases.push_back(ref(vw.tensor));
   };
   if (join != nullptr) {
@@ -3232,6 +3261,10 @@ bool Planner::lower_fused_group(int seed, int from) {
       FusedLaunch l = f->launch;
       for (size_t k = 0; k < f->groups.size(); ++k) l.group[k] = (const FusedGroup*)f->groups[k](e);
       for (size_t k = 0; k < f->bases.size(); ++k) l.base[k] = f->bases[k](e);
+      if (f->best.t >= 0) {
+        l.best = (float*)(f->best(e) + f->best_off);
+        l.best_at = (int32_t*)(f->best(e) + f->best_at_off);
+      }
       return launch_fused_eltwise(l, st);
     }, kReads16 | kWrites16);
   }
@@ -4439,6 +4472,53 @@ void Planner::lower_qdq(int ni) {
 }
 
 // ----------------------------------------------------------------- NMS ----
+// The scores [N][C][B] in tensor `ts` all come from chains of element-wise launches that walk the
+// classes (the parts of a Concat, each of which stores some boxes of every image): those launches
+// then leave every box's best score and its class in the workspace, and nothing reads the scores again.
+bool Planner::best_scores_from_groups(int ts, int tw, int64_t N, int64_t C, int64_t B) {
+  std::vector<std::pair<FusedStep*, size_t>> from;
+  int64_t boxes = 0;
+  for (auto& f : fused_steps_) {
+    for (size_t k = 0; k < f->parts.size(); ++k) {
+      const FusedPart& p = f->parts[k];
+      if (root(p.tensor) != root(ts)) continue;
+      const FusedGroup& g = p.group;
+      if (p.tensor != ts || g.chain == 0 || f->launch.wide || f->best.t >= 0) return false;
+      const FusedView& v = g.view[g.prog[g.n_instr - 1].dst];
+      int64_t last = v.off, images = 1, mine = 1;
+      for (int q : {0, 1, 3}) {
+        if (g.dims[q] == 1) continue;
+        if (v.st[q] == C * B) images *= g.dims[q];
+        else { last += (g.dims[q] - 1) * v.st[q]; mine *= g.dims[q]; }
+      }
+      if (g.dims[2] != C || v.st[2] != B || images != N || v.off < 0 || last >= B) return false;
+      boxes += mine;
+      from.push_back({f.get(), k});
+    }
+  }
+  if (boxes != B) return false;   // (parts of a Concat do not overlap: every box is one part's)
+  for (auto& fk : from) {
+    FusedStep* f = fk.first;
+    FusedPart& p = f->parts[fk.second];
+    FusedGroup& g = p.group;
+    const FusedView& v = g.view[g.prog[g.n_instr - 1].dst];
+    g.best_of = 1;
+    g.best_off = v.off;
+    int s = 0;
+    for (int q : {0, 1, 3}) g.best_st[s++] = g.dims[q] == 1 ? 0 : v.st[q] == C * B ? B : v.st[q];
+    size_t lds = 0;
+    bool wide = false;
+    if (!fused_prepare(&g, &p.blocks, &lds, &wide) || g.chain != 1 || wide) fail(ODLA_INTERNAL_LOGIC_ERR, "best scores of an element-wise group");
+    memcpy(plan_->blobs[p.blob].owned.data(), &g, sizeof(FusedGroup));
+    f->best = ref(tw);
+    f->best_off = nms_best_offset((int)N, (int)B);
+    f->best_at_off = nms_class_offset((int)N, (int)B);
+    for (size_t k = 0; k < f->parts.size(); ++k) f->launch.block0[k + 1] = f->launch.block0[k] + f->parts[k].blocks;
+    touch(f->step, {}, {tw}, kReads16 | kWrites16);
+  }
+  return true;
+}
+
 void Planner::lower_nms(int ni) {
   Node& n = comp_->nodes[ni];
   const _odla_value* boxes = n.in[0];
@@ -4463,8 +4543,11 @@ void Planner::lower_nms(int ni) {
   Shape o32 = n.out->shape;
   const int ty = new_tensor(DT_I32, L_ROWMAJOR, o32, 0, SP_ARENA);
   const Ref rb = ref(tb), rs = ref(ts), rw = ref(tw), ry = ref(ty);
-  emit("nms:" + n.out->name, {tb, ts, tw}, {ty, tw}, [=](const ExecEnv& e, hipStream_t st) {
-    return launch_nms(rb(e), bdt, rs(e), sdt, N, C, B, max_out, iou, thr, (int32_t*)ry(e), rw(e), st, e.image_base);
+  const bool best = best_scores_from_groups(ts, tw, N, C, B);
+  std::vector<int> reads = {tb, tw};
+  if (!best) reads.push_back(ts);
+  emit_lists(std::string(best ? "nms.best:" : "nms:") + n.out->name, reads, {ty, tw}, [=](const ExecEnv& e, hipStream_t st) {
+    return launch_nms(rb(e), bdt, rs(e), sdt, N, C, B, max_out, iou, thr, (int32_t*)ry(e), rw(e), st, e.image_base, best);
   }, kReads16 | kWrites16);
   if (dtype_from_odla(n.out->etype) == DT_I64) {
     const int t64 = new_tensor(DT_I64, L_ROWMAJOR, o32, 0, SP_ARENA);
