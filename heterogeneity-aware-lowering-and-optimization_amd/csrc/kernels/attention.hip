@@ -11,8 +11,11 @@
 // are one tile; longer sequences walk tiles of 128 keys with a running maximum and sum per query
 // (the next tile's rows travel in registers while the current one is used).  BERT-base in
 // accuracy mode at 8 x 384 tokens: product, Softmax, transposition and product took 22 + 20 + 7 +
-// 14 us per layer, this launch 15 us; at 1 x 41 tokens (keys that fill no block) nine launches
-// became one.  k goes through
+// 14 us per layer, this launch 15.3 (18.4 with
+// v^T stored value by value; 64 x 128 tokens 13.5 -> 12.3, 16 x 512 35.6 -> 30.0); at 1 x 41 tokens (keys that fill no block) nine launches
+// became one.  A launch of few workgroups is a chain of tiles with one wavefront per SIMD: there two groups of four
+// wavefronts take every other tile each, and the second group's maxima, sums and contexts join the first's
+// through LDS (1 x 512 tokens 13.2 -> 11.4 us; a chip that is full loses, 16 x 512 30 -> 37, 8 x 384 15.4 -> 19.9).  k goes through
 // LDS once (rows padded to 144 bytes), v is transposed on its way into LDS, q
 // comes straight from global memory into MFMA operand registers.
 //   scores  C[key][query] = k . q^T  (v_mfma_f32_32x32x16): a lane then holds, for
@@ -34,6 +37,7 @@ namespace ohip {
 namespace {
 
 constexpr int kAttnD = 64;            // head size
+constexpr float kLog2e = 1.44269504f;  // scores and mask are kept in units of log 2: the hardware exponential takes them as they are
 constexpr int kKPitch = 144;          // bytes per staged k row (128 + 16: conflict-free 16-byte fragment reads)
 constexpr int kVPitch = 272;          // bytes per staged v^T row (128 keys x 2 + 16)
 
@@ -72,23 +76,30 @@ __device__ __forceinline__ int slot_of_key(const int key) {
   return kb * 32 + (q >> 1) * 16 + s * 8 + (q & 1) * 4 + r;
 }
 
-// NKB: 32-key blocks of a tile; NKB wavefronts.  LOOP: more than one tile (NKB = 4).
-template <typename T, int NKB, bool LOOP>
-__global__ void __launch_bounds__(NKB * 64, 2)
-attention_kernel(const AttentionParams p) {
-  constexpr int TS = NKB * 32, NT = NKB * 64;
-  __shared__ __attribute__((aligned(16))) unsigned char smem[TS * kKPitch + kAttnD * kVPitch + TS * 4];
-  unsigned char* ks = smem;
-  unsigned char* vts = smem + TS * kKPitch;
-  float* ms = reinterpret_cast<float*>(smem + TS * kKPitch + kAttnD * kVPitch);
+// The 64-byte groups of v^T row `row` (0 .. 63) lie at their places XOR this.
+__device__ __forceinline__ int vt_group(const int row) { return ((row >> 3) & 3) << 6; }
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+// NKB: 32-key blocks of a tile; QW: wavefronts of a group, 32 queries each; LOOP: more than one tile; KG: groups that
+// share the tiles.
+template <typename T, int NKB, int QW, bool LOOP, int KG>
+__global__ void __launch_bounds__(QW * KG * 64, 2)
+attention_kernel(const AttentionParams p) {
+  constexpr int TS = NKB * 32, QS = QW * 32, NT = QW * 64;
+  constexpr int TILE = TS * kKPitch + kAttnD * kVPitch + TS * 4;
+  static_assert(KG == 1 || KG * TILE >= QW * 34 * 256, "room for the second group's maxima, sums and contexts");
+  __shared__ __attribute__((aligned(16))) unsigned char smem[KG * TILE];
+  const int group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
+  unsigned char* ks = smem + group * TILE;
+  unsigned char* vts = ks + TS * kKPitch;
+  float* ms = reinterpret_cast<float*>(vts + kAttnD * kVPitch);
+
+  const int tid = threadIdx.x - group * NT, wave = tid >> 6, lane = tid & 63;
   const int l32 = lane & 31, lg = lane >> 5;
   const int S = p.S;
-  const int q_tiles = LOOP ? (S + TS - 1) / TS : 1;
+  const int q_tiles = LOOP ? (S + QS - 1) / QS : 1;
   const int bh = blockIdx.x / q_tiles, qt = blockIdx.x - bh * q_tiles;
   const int b = bh / p.heads, h = bh - b * p.heads;
-  const int query = qt * TS + wave * 32 + l32;   // (may lie behind the last one: computed from the last row, never stored)
+  const int query = qt * QS + wave * 32 + l32;   // (may lie behind the last one: computed from the last row, never stored)
   const T* q = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_bs + (int64_t)h * p.q_hs;
   const T* k = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_bs + (int64_t)h * p.k_hs;
   const T* v = reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_bs + (int64_t)h * p.v_hs;
@@ -102,20 +113,30 @@ attention_kernel(const AttentionParams p) {
   }
   // ---- a tile of k and v rows and mask values: requested into registers, parked in LDS.  Keys
   // behind the last one are zero rows with the mask value -inf.
-  constexpr int RPT = TS * 8 / NT;   // rows per thread
-  const int c = tid & 7;             // 16-byte chunk of the row
-  uintx4 kr[RPT], vr[RPT];
+  // A thread takes one 16-byte chunk of four neighbouring keys, which are neighbours in a v^T row too: eight
+  // stores of 8 bytes, in a wavefront 64 bytes of each of 8 rows of each chunk, and the 64-byte groups of a row
+  // change places with its number so that these fall into all banks (as 2-byte stores, 32 a thread and eight lanes
+  // to a bank, the transposition was most of the launch).
+  const int c = tid & 7, key4 = (tid >> 3) * 4;
+  const bool stages = NT == TS * 2 || key4 < TS;   // (three blocks of keys, four wavefronts)
+  constexpr int RPT = TS * 8 / NT;   // k rows of a thread, NT / 8 apart
+  uintx4 kr[RPT], vr[4];
   float mr = 0.f;
   auto request = [&](const int key0) __attribute__((always_inline)) {
+    const uintx4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
       const int row = key0 + (tid >> 3) + i * (NT / 8);
-      const int rc = row < S ? row : S - 1;
-      const uintx4 kv = *(reinterpret_cast<const uintx4*>(k + (int64_t)rc * p.k_rs) + c);
-      const uintx4 vv = *(reinterpret_cast<const uintx4*>(v + (int64_t)rc * p.v_rs) + c);
-      const uintx4 zero = {0u, 0u, 0u, 0u};
+      const uintx4 kv = *(reinterpret_cast<const uintx4*>(k + (int64_t)(row < S ? row : S - 1) * p.k_rs) + c);
       kr[i] = row < S ? kv : zero;
-      vr[i] = row < S ? vv : zero;
+    }
+    if (stages) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = key0 + key4 + i;
+        const uintx4 vv = *(reinterpret_cast<const uintx4*>(v + (int64_t)(row < S ? row : S - 1) * p.v_rs) + c);
+        vr[i] = row < S ? vv : zero;
+      }
     }
     if (tid < TS) {
       const int key = key0 + tid;
@@ -129,18 +150,24 @@ attention_kernel(const AttentionParams p) {
   // k rows of 128 bytes, padded; v^T with the keys in slot order; the mask as fp32
   auto park = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-      const int row = (tid >> 3) + i * (NT / 8);
-      *reinterpret_cast<uintx4*>(ks + row * kKPitch + c * 16) = kr[i];
-      const unsigned w[4] = {vr[i].x, vr[i].y, vr[i].z, vr[i].w};
-      unsigned char* dst = vts + slot_of_key(row) * 2;
+    for (int i = 0; i < RPT; ++i) *reinterpret_cast<uintx4*>(ks + ((tid >> 3) + i * (NT / 8)) * kKPitch + c * 16) = kr[i];
+    if (stages) {
+      unsigned char* dst = vts + c * 8 * kVPitch + ((slot_of_key(key4) * 2) ^ vt_group(c * 8));
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        *reinterpret_cast<unsigned short*>(dst + (c * 8 + e) * kVPitch) = (unsigned short)(w[e >> 1] >> (16 * (e & 1)));
+      for (int w = 0; w < 4; ++w) {
+        const unsigned k0 = vr[0][w], k1 = vr[1][w], k2 = vr[2][w], k3 = vr[3][w];
+        *reinterpret_cast<uintx2*>(dst + (2 * w) * kVPitch) = uintx2{__builtin_amdgcn_perm(k1, k0, 0x05040100u), __builtin_amdgcn_perm(k3, k2, 0x05040100u)};
+        *reinterpret_cast<uintx2*>(dst + (2 * w + 1) * kVPitch) = uintx2{__builtin_amdgcn_perm(k1, k0, 0x07060302u), __builtin_amdgcn_perm(k3, k2, 0x07060302u)};
+      }
     }
-    if (tid < TS) ms[tid] = mr;
+    if (tid < TS) {
+      // (a mask of the type's lowest value stays finite: a row of nothing else is a plain mean)
+      const float m2 = mr * kLog2e;
+      ms[tid] = __builtin_isinf(m2) && !__builtin_isinf(mr) ? __builtin_copysignf(3.402823466e38f, mr) : m2;
+    }
   };
 
+  const float scale = p.scale * kLog2e;
   floatx16 o[2];
 #pragma unroll
   for (int dvb = 0; dvb < 2; ++dvb)
@@ -148,12 +175,14 @@ attention_kernel(const AttentionParams p) {
     for (int e = 0; e < 16; ++e) o[dvb][e] = 0.f;
   float run_max = -INFINITY, run_sum = 0.f;
 
-  request(0);
-  for (int key0 = 0; LOOP ? key0 < S : key0 == 0; key0 += TS) {
-    if (LOOP && key0 > 0) __syncthreads();   // everyone has used the tile before
+  // (both groups walk as often as the first, whose share is the longer one: a tile behind the last key holds
+  // nothing but keys with the mask value -inf)
+  request(group * TS);
+  for (int t0 = 0; LOOP ? t0 < S : t0 == 0; t0 += KG * TS) {
+    if (LOOP && t0 > 0) __syncthreads();   // everyone has used the tile before
     park();
     __syncthreads();
-    if (LOOP && key0 + TS < S) request(key0 + TS);
+    if (LOOP && t0 + KG * TS < S) request(t0 + KG * TS + group * TS);
 
     // ---- scores: acc[kb][q*4 + r] = k[kb*32 + q*8 + lg*4 + r] . q[query]
     floatx16 acc[NKB];
@@ -175,10 +204,10 @@ attention_kernel(const AttentionParams p) {
 #pragma unroll
       for (int qq = 0; qq < 4; ++qq) {
         const floatx4 m4 = *reinterpret_cast<const floatx4*>(ms + kb * 32 + qq * 8 + lg * 4);
-        acc[kb][qq * 4 + 0] = __builtin_fmaf(acc[kb][qq * 4 + 0], p.scale, m4.x);
-        acc[kb][qq * 4 + 1] = __builtin_fmaf(acc[kb][qq * 4 + 1], p.scale, m4.y);
-        acc[kb][qq * 4 + 2] = __builtin_fmaf(acc[kb][qq * 4 + 2], p.scale, m4.z);
-        acc[kb][qq * 4 + 3] = __builtin_fmaf(acc[kb][qq * 4 + 3], p.scale, m4.w);
+        acc[kb][qq * 4 + 0] = __builtin_fmaf(acc[kb][qq * 4 + 0], scale, m4.x);
+        acc[kb][qq * 4 + 1] = __builtin_fmaf(acc[kb][qq * 4 + 1], scale, m4.y);
+        acc[kb][qq * 4 + 2] = __builtin_fmaf(acc[kb][qq * 4 + 2], scale, m4.z);
+        acc[kb][qq * 4 + 3] = __builtin_fmaf(acc[kb][qq * 4 + 3], scale, m4.w);
 #pragma unroll
         for (int r = 0; r < 4; ++r) mx = fmaxf(mx, acc[kb][qq * 4 + r]);
       }
@@ -191,7 +220,7 @@ attention_kernel(const AttentionParams p) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         // (the result keeps 8 or 11 significant bits: the hardware exponential, 1 ulp, stands in for the library's)
-        const float ex = __expf(acc[kb][e] - ref);
+        const float ex = __builtin_amdgcn_exp2f(acc[kb][e] - ref);
         acc[kb][e] = ex;
         sum += ex;
       }
@@ -199,7 +228,7 @@ attention_kernel(const AttentionParams p) {
     float inv = 1.f;
     if constexpr (LOOP) {
       // what the tiles before contributed, in terms of the new maximum
-      const float keep = __expf(run_max - ref);
+      const float keep = __builtin_amdgcn_exp2f(run_max - ref);
       run_sum = __builtin_fmaf(run_sum, keep, sum);
       run_max = mx;
 #pragma unroll
@@ -224,17 +253,43 @@ attention_kernel(const AttentionParams p) {
         const uintx4 pf = pack8_rne<T>(pv);
 #pragma unroll
         for (int dvb = 0; dvb < 2; ++dvb) {
-          const uintx4 a = *reinterpret_cast<const uintx4*>(vts + (dvb * 32 + l32) * kVPitch + (kb * 32 + hh * 16 + lg * 8) * 2);
+          const int row = dvb * 32 + l32;
+          const uintx4 a = *reinterpret_cast<const uintx4*>(vts + row * kVPitch + (((kb * 32 + hh * 16 + lg * 8) * 2) ^ vt_group(row)));
           o[dvb] = Mma<T>::run(a, pf, o[dvb]);
         }
       }
   }
-  if constexpr (LOOP) {
+  if constexpr (LOOP && KG == 1) {
     const float inv = 1.0f / run_sum;
 #pragma unroll
     for (int dvb = 0; dvb < 2; ++dvb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) o[dvb][e] *= inv;
+  }
+  if constexpr (KG > 1) {
+    // the second group's part, a lane's values 64 places apart
+    float* part = reinterpret_cast<float*>(smem) + wave * (34 * 64) + lane;
+    __syncthreads();
+    if (group == 1) {
+#pragma unroll
+      for (int dvb = 0; dvb < 2; ++dvb)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) part[(dvb * 16 + e) * 64] = o[dvb][e];
+      part[32 * 64] = run_max;
+      part[33 * 64] = run_sum;
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float other_max = part[32 * 64], mx = fmaxf(run_max, other_max);
+    const float ref = mx == -INFINITY ? 0.f : mx;
+    float mine = __builtin_amdgcn_exp2f(run_max - ref), other = __builtin_amdgcn_exp2f(other_max - ref);
+    const float inv = 1.0f / __builtin_fmaf(run_sum, mine, part[33 * 64] * other);
+    mine *= inv;
+    other *= inv;
+#pragma unroll
+    for (int dvb = 0; dvb < 2; ++dvb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[dvb][e] = __builtin_fmaf(part[(dvb * 16 + e) * 64], other, o[dvb][e] * mine);
   }
 
   // ---- result rows: lane (query, lg) holds, per 32-value block, the groups (q, lg) of four
@@ -290,19 +345,26 @@ hipError_t launch_attention(const AttentionParams& p, hipStream_t stream) {
     return hipErrorInvalidValue;
   auto al16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
   if (!al16(p.q) || !al16(p.k) || !al16(p.v) || !al16(p.out)) return hipErrorInvalidValue;
-  // more than 128 keys: tiles of 128 keys and of 128 queries
-  const int nkb = p.S > 128 ? 5 : (p.S + 31) / 32;
-  const dim3 grid((unsigned)((int64_t)p.B * p.heads * (p.S > 128 ? (p.S + 127) / 128 : 1)));
-#define ATTN_CASE(T_, NKB_)                                                                                \
-  if (nkb == NKB_) {                                                                                       \
-    hipLaunchKernelGGL((attention_kernel<T_, (NKB_ > 4 ? 4 : NKB_), (NKB_ > 4)>), grid, dim3((NKB_ > 4 ? 4 : NKB_) * 64), 0, stream, p); \
+  // More than 128 keys: 128 queries a workgroup.  Where every workgroup has two compute units' worth of room, two groups, in tiles of
+  // 96 keys where the longer share is then shorter than in tiles of 128.
+  const int64_t q_tiles = p.S > 128 ? (p.S + 127) / 128 : 1, workgroups = (int64_t)p.B * p.heads * q_tiles;
+  const auto share = [&](const int ts) { return (p.S + 2 * ts - 1) / (2 * ts) * ts; };
+  const int nkb = p.S <= 128 ? (p.S + 31) / 32 : workgroups > 128 ? 5 : share(96) < share(128) ? 7 : 6;
+  const dim3 grid((unsigned)workgroups);
+#define ATTN_CASE(T_, CASE_, NKB_, QW_, LOOP_, KG_)                                                        \
+  if (nkb == CASE_) {                                                                                      \
+    hipLaunchKernelGGL((attention_kernel<T_, NKB_, QW_, LOOP_, KG_>), grid, dim3(QW_ * KG_ * 64), 0, stream, p); \
     return hipGetLastError();                                                                              \
   }
+#define ATTN_CASES(T_)                                                                                     \
+  ATTN_CASE(T_, 1, 1, 1, false, 1) ATTN_CASE(T_, 2, 2, 2, false, 1) ATTN_CASE(T_, 3, 3, 3, false, 1) ATTN_CASE(T_, 4, 4, 4, false, 1) \
+  ATTN_CASE(T_, 5, 4, 4, true, 1) ATTN_CASE(T_, 6, 4, 4, true, 2) ATTN_CASE(T_, 7, 3, 4, true, 2)
   if (p.dt == DT_BF16) {
-    ATTN_CASE(bf16_t, 1) ATTN_CASE(bf16_t, 2) ATTN_CASE(bf16_t, 3) ATTN_CASE(bf16_t, 4) ATTN_CASE(bf16_t, 5)
+    ATTN_CASES(bf16_t)
   } else {
-    ATTN_CASE(f16_t, 1) ATTN_CASE(f16_t, 2) ATTN_CASE(f16_t, 3) ATTN_CASE(f16_t, 4) ATTN_CASE(f16_t, 5)
+    ATTN_CASES(f16_t)
   }
+#undef ATTN_CASES
 #undef ATTN_CASE
   return hipErrorInvalidValue;
 }
