@@ -295,6 +295,8 @@ struct S2dParams {
 };
 hipError_t launch_nchw_to_s2d(const S2dParams& p, hipStream_t stream);
 hipError_t launch_nhwc_to_nchw(const LayoutParams& p, hipStream_t stream);
+// `bytes` from `src` (device or page-locked host memory) to `dst`, both 16-byte aligned.
+hipError_t launch_copy_pieces(const void* src, void* dst, int64_t bytes, hipStream_t stream);
 
 // Flat conversions -------------------------------------------------------
 hipError_t launch_cast(const void* src, DType sdt, void* dst, DType ddt, int64_t n,

@@ -515,6 +515,13 @@ gather_rows_kernel(const unsigned char* __restrict__ x, const IDX* __restrict__ 
 
 struct b16 { uintx4 v; };
 
+// Bytes as they are, 16 to a lane and one piece each, so that all of them are under way at once.
+__global__ void __launch_bounds__(kThreads) copy_pieces_kernel(const unsigned char* src, unsigned char* dst, int64_t n) {
+  const int64_t at = (blockIdx.x * (int64_t)kThreads + threadIdx.x) * 16;
+  if (at + 16 <= n) *reinterpret_cast<uintx4*>(dst + at) = *reinterpret_cast<const uintx4*>(src + at);
+  else for (int64_t i = at; i < n; ++i) dst[i] = src[i];
+}
+
 }  // namespace
 
 #define LAYOUT_PAIR_DISPATCH(KERNEL, ...)                                                      \
@@ -909,6 +916,15 @@ hipError_t launch_gather_rows(const void* x, const void* idx, DType idx_dt, void
                        n_src_rows, n_idx, row_bytes, vec);
   else
     return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_pieces(const void* src, void* dst, int64_t bytes, hipStream_t stream) {
+  if (bytes <= 0) return bytes == 0 ? hipSuccess : hipErrorInvalidValue;
+  if (!src || !dst || ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15u) != 0) return hipErrorInvalidValue;
+  const int64_t grid = (bytes + 16 * kThreads - 1) / (16 * kThreads);
+  if (grid > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(copy_pieces_kernel, dim3((unsigned)grid), dim3(kThreads), 0, stream, (const unsigned char*)src, (unsigned char*)dst, bytes);
   return hipGetLastError();
 }
 
