@@ -298,6 +298,29 @@ hipError_t launch_nhwc_to_nchw(const LayoutParams& p, hipStream_t stream);
 // `bytes` from `src` (device or page-locked host memory) to `dst`, both 16-byte aligned.
 hipError_t launch_copy_pieces(const void* src, void* dst, int64_t bytes, hipStream_t stream);
 
+// A 7x7 / stride 2 convolution over a three-channel NCHW fp32 image into 64 channels, ReLU, and the 3x3 / stride 2 /
+// padding 1 maximum of that (stem_pool.hip).  The convolution is the 4x4 / stride 1 one over the image's
+// space-to-depth form whose fragment-ordered weights w_frag holds (ph, pw: its padding there).  dt: type of operands and
+// result, which is channels-last without padding; DT_I8: scale, zp quantise the image, bias is int32, qmul / q_add / q_lo
+// requantise as in IgemmParams.
+struct StemPoolParams {
+  const float* x = nullptr;
+  void* y = nullptr;
+  const void* w_frag = nullptr;
+  const void* bias = nullptr;
+  const float* qmul = nullptr;
+  DType dt = DT_F16;
+  int wf_chunks = 0;
+  int N = 0, H = 0, W = 0;     // the image
+  int Ho = 0, Wo = 0;          // the convolution's result
+  int Po = 0, Qo = 0;          // the pool's
+  int ph = 0, pw = 0;
+  float scale = 1.f; int zp = 0;
+  float q_add = 0.f, q_lo = 0.f;
+};
+bool stem_pool_supported(const StemPoolParams& p);
+hipError_t launch_stem_pool(const StemPoolParams& p, hipStream_t stream);
+
 // Flat conversions -------------------------------------------------------
 hipError_t launch_cast(const void* src, DType sdt, void* dst, DType ddt, int64_t n,
                        hipStream_t stream);

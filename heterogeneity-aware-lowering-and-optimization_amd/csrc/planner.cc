@@ -784,7 +784,9 @@ class Planner {
   int pack_weights(const _odla_value* kernel, DType dst_dt, int G, int Og, int Cg, int R, int S, int Cp,
                    int64_t so, int64_t si, int64_t sr, int64_t ss, const std::vector<float>& row_scale,
                    int* w_rs_out, const std::vector<float>* wq_scale, int dense_groups = 0);
-  int make_wfrag(const std::string& name, IgemmParams* ip, int tw);
+  int make_wfrag(const std::string& name, IgemmParams* ip, int tw, bool always = false);
+  int stem_pool_behind(const Epilogue& ep, int O, int R, int S, DType from, DType dt, bool q8, StemPoolParams* sp);
+  void emit_stem_pool(const _odla_value* conv, int pool, StemPoolParams sp, IgemmParams ip, int from, int tw, int tb, int tm, int ty);
   // Debug-level log line "<launch>: kernel <variant>" (the device pointers that the
   // choice looks at are replaced by stand-ins: only their presence matters).
   void log_igemm_choice(const std::string& name, IgemmParams ip, bool has_wfrag, bool has_residual) {
@@ -1383,8 +1385,8 @@ int Planner::strided_copy_step(const std::string& name, int src, int dst, const 
 // Constant weights of layers that use the weights-in-registers kernel get a
 // second copy in MFMA fragment order, built once at initialisation.  Returns
 // the tensor (and fills ip->wf_*), or -1 when the layer does not use one.
-int Planner::make_wfrag(const std::string& name, IgemmParams* ip, int tw) {
-  if (T(tw).space != SP_CONST || !igemm_wants_wfrag(*ip)) return -1;
+int Planner::make_wfrag(const std::string& name, IgemmParams* ip, int tw, bool always) {
+  if (T(tw).space != SP_CONST || !(always || igemm_wants_wfrag(*ip))) return -1;
   if (ip->batch != 1 && (int64_t)ip->w_bs != (int64_t)ip->w_rows * ip->w_rs) return -1;
   const int es = dtype_size(ip->in_dt);
   WfragPackParams fp;
@@ -1483,6 +1485,43 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
 }
 
 // ---------------------------------------------------------------- Conv ----
+// The 3x3 / stride 2 / padding 1 maximum that alone reads a 7x7 / stride 2 network stem with ReLU
+// (folded operators `ep`), where one launch computes both: its node, or -1.
+int Planner::stem_pool_behind(const Epilogue& ep, int O, int R, int S, DType from, DType dt, bool q8, StemPoolParams* sp) {
+  const _odla_value* v = ep.final_value;
+  if (calib_ || in_init_ || v == nullptr || v->is_output || consumers_[v->index].size() != 1) return -1;
+  if (O != 64 || R != 7 || S != 7 || from != DT_F32 || (dt != DT_F16 && dt != DT_BF16 && dt != DT_I8)) return -1;
+  if (ep.act != ACT_RELU || ep.residual != nullptr || ep.scalar != 1.f) return -1;
+  if (q8 ? qentry(v) == nullptr : result_dtype(v) != dt) return -1;
+  const int pi = consumers_[v->index][0];
+  const Node& pool = comp_->nodes[pi];
+  if (pool.op != OP_POOL || pool.absorbed || pool.i[0] == ODLA_CHANNELS_LAST || pool.i[1] == 0) return -1;
+  for (int k = 2; k < 6; ++k) if (pool.i[k] != (k < 4 ? 3 : 2)) return -1;
+  if (pool.i[6] != 1 || pool.i[7] != 1 || (!q8 && storage_dtype(pool.out) != dt)) return -1;
+  const Shape& os = pool.out->shape;
+  sp->dt = dt;
+  sp->Po = (int)os.d[2];
+  sp->Qo = (int)os.d[3];
+  return pi;
+}
+
+void Planner::emit_stem_pool(const _odla_value* conv, int pool, StemPoolParams sp, IgemmParams ip, int from, int tw, int tb, int tm, int ty) {
+  const int tf = make_wfrag("conv:" + conv->name, &ip, tw, true);
+  Node& pn = comp_->nodes[pool];
+  if (tf < 0 || T(ty).cs != 64) fail(ODLA_INTERNAL_LOGIC_ERR, "weights or result of the stem '%s'", conv->name.c_str());
+  sp.wf_chunks = ip.wf_chunks;
+  const bool hm = tm >= 0;
+  const Ref rx = ref(from), rf = ref(tf), rb = ref(tb), rm = ref(hm ? tm : tb), ry = ref(ty);
+  emit("stem:" + conv->name + "+" + pn.out->name, {from}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
+    StemPoolParams p = sp;
+    p.x = (const float*)rx(e); p.y = ry(e); p.w_frag = rf(e); p.bias = rb(e);
+    p.qmul = hm ? (const float*)rm(e) : nullptr;
+    return launch_stem_pool(p, st);
+  }, kReadsAny);
+  pn.absorbed = true;
+  set_main(pn.out, ty);
+}
+
 void Planner::lower_conv(int ni) {
   Node& n = comp_->nodes[ni];
   const _odla_value* x = n.in[0];
@@ -1542,6 +1581,9 @@ void Planner::lower_conv(int ni) {
   const _odla_value* kpack = k;  // the kernel tensor that is packed
   _odla_value k_s2d;
   int tx_s2d = -1;
+  int stem_pool = -1;            // the pool behind the convolution, where one launch computes both (stem_pool.hip)
+  StemPoolParams stem;
+  int stem_from = -1;
   {
     const VState& xv = vs_[x->index];
     const bool src_ok = xv.main >= 0 && T(xv.main).layout == L_ROWMAJOR && !T(xv.main).quant;
@@ -1593,8 +1635,16 @@ void Planner::lower_conv(int ni) {
         set_quant(tx_s2d, true, qx->scale, qx->zp);
       }
       const int from = xv.main;
+      stem_pool = stem_pool_behind(ep, (int)O, (int)R, (int)S, T(from).dt, fdt, q8, &stem);
+      stem_from = from;
+      stem.N = (int)N; stem.H = (int)H; stem.W = (int)W;
+      stem.Ho = (int)Ho; stem.Wo = (int)Wo;
+      stem.ph = -dy0; stem.pw = -dx0;
+      stem.scale = sp.scale; stem.zp = sp.zp;
+      if (stem_pool >= 0 && (C != 3 || R2 != 4 || S2 != 4 || cs != 16 || !stem_pool_supported(stem))) stem_pool = -1;
       const Ref a = ref(from), b = ref(tx_s2d);
-      emit("to_s2d:" + x->name, {from}, {tx_s2d}, [=](const ExecEnv& e, hipStream_t st) {
+      if (stem_pool >= 0) T(tx_s2d).bytes = 0;   // (never made)
+      else emit("to_s2d:" + x->name, {from}, {tx_s2d}, [=](const ExecEnv& e, hipStream_t st) {
         S2dParams p = sp; p.src = a(e); p.dst = b(e);
         return launch_nchw_to_s2d(p, st);
       }, kReadsAny | kReadsOnce);
@@ -1690,6 +1740,15 @@ void Planner::lower_conv(int ni) {
       const QuantEntry* qy = qentry(outv);
       ip.r_mul = T(tr).qscale / qy->scale;
       ip.r_add = (float)qy->zp - (float)T(tr).qzp * ip.r_mul;
+    }
+    if (stem_pool >= 0) {
+      if (ip.out_dt != DT_I8) fail(ODLA_INTERNAL_LOGIC_ERR, "stem '%s' without 8-bit results", outv->name.c_str());
+      stem.q_add = ip.q_add; stem.q_lo = ip.q_lo;
+      const int tyq = new_tensor(DT_I8, L_NHWC, comp_->nodes[stem_pool].out->shape, (int)O, SP_ARENA);
+      set_quant(tyq, true, T(ty).qscale, T(ty).qzp);
+      T(ty).bytes = 0;   // (never made)
+      emit_stem_pool(outv, stem_pool, stem, ip, stem_from, tw, tb, tm, tyq);
+      return;
     }
     ip.stream_out = T(ty).bytes >= stream_out_bytes();
     const int tf = make_wfrag("conv.i8:" + outv->name, &ip, tw);
@@ -1806,6 +1865,13 @@ void Planner::lower_conv(int ni) {
   if (Ge > 1) { ip.x_bs = Cg; ip.w_bs = (int64_t)Og * w_rs; ip.y_bs = Og; ip.r_bs = Og; ip.bias_bs = Og; }
   ip.ycs = (int)O;
 
+  if (stem_pool >= 0) {
+    std::vector<float> b = ep.bias;
+    b.resize((size_t)O, 0.f);
+    _odla_value* pooled = comp_->nodes[stem_pool].out;
+    emit_stem_pool(outv, stem_pool, stem, ip, stem_from, tw, const_vector<float>(DT_F32, b), -1, channels_last_result(pooled, odt));
+    return;
+  }
   int ty;
   if (cl) ty = new_tensor(odt, L_ROWMAJOR, outv->shape, 0, SP_ARENA);
   else ty = channels_last_result(outv, odt);
