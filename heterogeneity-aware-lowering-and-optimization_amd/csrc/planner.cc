@@ -2291,7 +2291,7 @@ void Planner::lower_gemm(int ni) {
         const int64_t inner = rows * Nn;
         emit("gemm.sum:" + outv->name, {tp}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
           return launch_reduce(rp(e), ry(e), DT_F32, odt, 1, splits, inner, RED_SUM, st);
-        });
+        }, kWrites16);
         set_main(outv, ty);
         return;
       }
@@ -4087,7 +4087,7 @@ void Planner::lower_softmax(int ni) {
   const bool has_add = tadd >= 0;
   emit("softmax:" + n.out->name, {tx, tadd}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
     return launch_softmax(a(e), b(e), dt, odt, outer, len, inner, logsm, st, has_add ? m(e) : nullptr, add_div);
-  }, kWrites16);
+  }, kReads16 | kWrites16);
   set_main(n.out, ty);
 }
 
