@@ -570,10 +570,18 @@ hipError_t launch_softmax(const void* x, void* y, DType in_dt, DType out_dt, int
                           const void* add = nullptr, int64_t add_div = 1);
 // y = (x - mean) * rsqrt(var + eps) * gamma + beta over the last `len` elements.
 // y2 (optional): a second copy of the result in y2_dt (DT_F16 / DT_BF16), written by the same
-// launch - for fp32 rows that layernorm_dual_ok accepts.
+// launch - for fp32 rows that layernorm_dual_ok accepts; of 2-byte rows that layernorm_rows_ok accepts one in DT_F32 (then
+// y may be null).
+// emb (optional, rows that layernorm_rows_ok accepts): row r is row idx[r] of the table x, plus row r % pos_rows of pos.
+struct EmbedRows {
+  const int32_t* idx = nullptr;
+  const void* pos = nullptr;
+  int64_t n_src = 0, pos_rows = 1;
+};
 hipError_t launch_layernorm(const void* x, void* y, DType dt, int64_t rows, int64_t len,
                             const float* gamma, const float* beta, float eps,
-                            hipStream_t stream, void* y2 = nullptr, DType y2_dt = DT_F32);
+                            hipStream_t stream, void* y2 = nullptr, DType y2_dt = DT_F32, const EmbedRows* emb = nullptr);
+bool layernorm_rows_ok(DType dt, int64_t len);
 bool layernorm_dual_ok(DType dt, int64_t len);
 
 // ---------------------------------------------------------------------------

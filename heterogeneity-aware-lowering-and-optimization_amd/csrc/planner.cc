@@ -173,7 +173,7 @@ class Planner {
   // in place of that step (finish_igemm).
   struct LastNorm {
     int tx = -1, ty = -1, t2 = -1, tg = -1, tb = -1;
-    int64_t len = 0;
+    int64_t rows = 0, len = 0;
     float eps = 0.f;
     DType dt = DT_F32;
   } last_norm_;
@@ -739,7 +739,10 @@ class Planner {
   void lower_binary(int ni);
   void lower_unary(int ni);
   void lower_batchnorm(int ni);
-  void lower_layernorm(int ni);
+  // Rows of a table, picked by an index each, plus rows of `pos` in turn.
+  struct EmbedSource { int table = -1, idx = -1, pos = -1; int64_t n_src = 0, pos_rows = 1; };
+  void lower_layernorm(int ni, const EmbedSource* emb = nullptr);
+  int norm_behind_gather(const _odla_value* rows, const _odla_value** pos) const;
   void lower_pool(int ni);
   void lower_reduce(int ni);
   void lower_softmax(int ni);
@@ -991,6 +994,21 @@ void Planner::run() {
       }, kWrites16);
     } else {
       t = get(ov, L_ROWMAJOR, FORM_FLOAT);
+    }
+    const LastNorm ln = last_norm_;
+    if (!calib_ && !in_init_ && want == DT_F32 && T(t).dt != want && t == ln.ty && ln.t2 < 0 && consumers_[ov->index].empty() &&
+        std::count(comp_->outputs.begin(), comp_->outputs.end(), ov) == 1 && dtype_size(ln.dt) == 2 && layernorm_rows_ok(ln.dt, ln.len)) {
+      // the step right in front normalised these rows and nothing else reads them: it writes them in the declared type
+      plan_->steps.pop_back();
+      T(t).bytes = 0;   // (never made)
+      const int dst = new_tensor(want, L_ROWMAJOR, ov->shape, 0, SP_ARENA);
+      const bool hg = ln.tg >= 0, hb = ln.tb >= 0;
+      const Ref a = ref(ln.tx), b = ref(dst), rg = ref(hg ? ln.tg : ln.tx), rb = ref(hb ? ln.tb : ln.tx);
+      emit("layernorm:" + ov->name, {ln.tx}, {dst}, [=](const ExecEnv& e, hipStream_t st) {
+        return launch_layernorm(a(e), nullptr, ln.dt, ln.rows, ln.len, hg ? (const float*)rg(e) : nullptr,
+                                hb ? (const float*)rb(e) : nullptr, ln.eps, st, b(e), DT_F32);
+      }, kWrites16);
+      t = dst;
     }
     if (T(t).dt != want) {
       const int dst = new_tensor(want, L_ROWMAJOR, ov->shape, 0, SP_ARENA);
@@ -3844,10 +3862,11 @@ void Planner::lower_batchnorm(int ni) {
 }
 
 // ----------------------------------------------------------- LayerNorm ----
-void Planner::lower_layernorm(int ni) {
+// emb: the rows come from a table (lower_gather), not from the value in front.
+void Planner::lower_layernorm(int ni, const EmbedSource* emb) {
   Node& n = comp_->nodes[ni];
   const _odla_value* x = n.in[0];
-  const int tx = get(x, L_ROWMAJOR, FORM_FLOAT);
+  const int tx = emb != nullptr ? emb->table : get(x, L_ROWMAJOR, FORM_FLOAT);
   const Shape& xs = x->shape;
   const int na = (int)n.i[0];
   int64_t len = 1;
@@ -3875,11 +3894,22 @@ void Planner::lower_layernorm(int ni) {
   const Ref b2 = ref(t2 >= 0 ? t2 : ty);
   const bool dual = t2 >= 0;
   const DType dt2 = op_dt_;
-  emit("layernorm:" + n.out->name, {tx}, {ty, t2}, [=](const ExecEnv& e, hipStream_t st) {
-    return launch_layernorm(a(e), b(e), dt, rows, len, hg ? (const float*)rg(e) : nullptr,
-                            hb ? (const float*)rb(e) : nullptr, eps, st, dual ? b2(e) : nullptr, dt2);
-  }, kWrites16);
-  if (!calib_ && !in_init_) last_norm_ = {tx, ty, t2, tg, tb, len, eps, dt};
+  if (emb != nullptr) {
+    const Ref ri = ref(emb->idx), rp = ref(emb->pos);
+    const EmbedSource src = *emb;
+    emit("embed+layernorm:" + n.out->name, {tx, emb->idx, emb->pos}, {ty, t2}, [=](const ExecEnv& e, hipStream_t st) {
+      EmbedRows er;
+      er.idx = (const int32_t*)ri(e); er.pos = rp(e); er.n_src = src.n_src; er.pos_rows = src.pos_rows;
+      return launch_layernorm(a(e), b(e), dt, rows, len, hg ? (const float*)rg(e) : nullptr,
+                              hb ? (const float*)rb(e) : nullptr, eps, st, dual ? b2(e) : nullptr, dt2, &er);
+    }, kReads16 | kWrites16);
+  } else {
+    emit("layernorm:" + n.out->name, {tx}, {ty, t2}, [=](const ExecEnv& e, hipStream_t st) {
+      return launch_layernorm(a(e), b(e), dt, rows, len, hg ? (const float*)rg(e) : nullptr,
+                              hb ? (const float*)rb(e) : nullptr, eps, st, dual ? b2(e) : nullptr, dt2);
+    }, kWrites16);
+  }
+  if (!calib_ && !in_init_ && emb == nullptr) last_norm_ = {tx, ty, t2, tg, tb, rows, len, eps, dt};
   set_main(n.out, ty);
   if (dual) vs_[n.out->index].slot[L_ROWMAJOR][FORM_OPERAND] = t2;
 }
@@ -4175,6 +4205,29 @@ void Planner::lower_concat(int ni) {
 }
 
 // -------------------------------------------------------------- Gather ----
+// The LayerNorm over single rows that alone reads gathered `rows` plus a constant whose rows repeat over them
+// (an embedding: words and positions): its node, or -1.
+int Planner::norm_behind_gather(const _odla_value* rows, const _odla_value** pos) const {
+  if (calib_ || in_init_ || comp_->opts.int8 || rows->is_output || consumers_[rows->index].size() != 1 || rows->shape.rank < 2) return -1;
+  const Node& add = comp_->nodes[consumers_[rows->index][0]];
+  if (add.op != OP_BINARY || add.absorbed || add.i[0] != BIN_ADD || !(add.out->shape == rows->shape)) return -1;
+  if (add.out->is_output || consumers_[add.out->index].size() != 1 || add.in[0] == add.in[1] || storage_dtype(add.out) != storage_dtype(rows)) return -1;
+  const _odla_value* p = add.in[0] == rows ? add.in[1] : add.in[0];
+  if (p->kind != _odla_value::CONSTANT || storage_dtype(p) != storage_dtype(rows)) return -1;
+  // the last dims of p are those of the rows, in front of them there are only ones
+  const Shape &ps = p->shape, &rs = rows->shape;
+  int lead = 0;
+  while (lead < ps.rank && ps.d[lead] == 1) ++lead;
+  if (ps.rank - lead > rs.rank || ps.rank == lead) return -1;
+  for (int i = lead; i < ps.rank; ++i)
+    if (ps.d[i] != rs.d[rs.rank - ps.rank + i]) return -1;
+  const Node& ln = comp_->nodes[consumers_[add.out->index][0]];
+  if (ln.op != OP_LAYERNORM || ln.absorbed || ln.in[0] != add.out || ln.i[0] != 1) return -1;
+  if ((ln.in[1] && ln.in[1]->kind != _odla_value::CONSTANT) || (ln.in[2] && ln.in[2]->kind != _odla_value::CONSTANT)) return -1;
+  *pos = p;
+  return consumers_[add.out->index][0];
+}
+
 void Planner::lower_gather(int ni) {
   Node& n = comp_->nodes[ni];
   const _odla_value* x = n.in[0];
@@ -4190,6 +4243,19 @@ void Planner::lower_gather(int ni) {
   const DType idt = T(ti).dt;
   const int64_t n_src = xs.d[axis], n_idx = idx->shape.numel();
   const int64_t row_bytes = inner * dtype_size(dt);
+  const _odla_value* pv = nullptr;
+  const int norm = axis == 0 && xs.rank == 2 && idt == DT_I32 && dt == storage_dtype(n.out) ? norm_behind_gather(n.out, &pv) : -1;
+  if (norm >= 0 && layernorm_rows_ok(dt, inner)) {
+    EmbedSource es;
+    es.table = tx; es.idx = ti; es.pos = get(pv, L_ROWMAJOR, FORM_FLOAT);
+    es.n_src = n_src; es.pos_rows = pv->shape.numel() / inner;
+    if (T(es.pos).dt == dt) {
+      comp_->nodes[consumers_[n.out->index][0]].absorbed = true;
+      comp_->nodes[norm].absorbed = true;
+      lower_layernorm(norm, &es);
+      return;
+    }
+  }
   const int ty = new_tensor(dt, L_ROWMAJOR, n.out->shape, 0, SP_ARENA);
   const Ref a = ref(tx), ri = ref(ti), b = ref(ty);
   emit("gather:" + n.out->name, {tx, ti}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
