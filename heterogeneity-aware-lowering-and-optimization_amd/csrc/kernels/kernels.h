@@ -324,6 +324,16 @@ hipError_t launch_stem_pool(const StemPoolParams& p, hipStream_t stream);
 // Flat conversions -------------------------------------------------------
 hipError_t launch_cast(const void* src, DType sdt, void* dst, DType ddt, int64_t n,
                        hipStream_t stream);
+// dst = the operators in turn on src converted to ddt (fp32 to a 2-byte type, or the type of src), constant k on the left where lhs[k]; every step is rounded to ddt.
+constexpr int kScalarChain = 4;
+struct ScalarChain {
+  int n = 0;
+  BinKind op[kScalarChain] = {};
+  bool lhs[kScalarChain] = {};
+  float c[kScalarChain] = {};
+};
+hipError_t launch_scalar_chain(const void* src, DType sdt, void* dst, DType ddt, int64_t n, const ScalarChain& s,
+                               hipStream_t stream);
 // q = sat(rne(x / scale[c]) + zp[c]); channel c = (i / inner) % channels.
 struct QuantParams {
   const void* src = nullptr; void* dst = nullptr;

@@ -768,6 +768,7 @@ class Planner {
   bool plane_candidate(const Node& n) const;
   bool lower_plane_group(int seed);
   bool fuse_slice_seed(int ni) const;
+  bool lower_scalar_chain(int ni);
   bool fuse_candidate(int ni) const;
   bool gemm_epilogue(int ni, Epilogue* ep);
   bool try_fused_attention(int ni);
@@ -2426,6 +2427,63 @@ void logical_strides(const PTensor& t, int64_t* st) {
 }
 }  // namespace
 
+// Operators with a single constant each that alone read each other, with the conversion of an fp32 argument in front:
+// one launch where that replaces at least two.
+bool Planner::lower_scalar_chain(int ni) {
+  if (calib_ || in_init_ || comp_->opts.int8) return false;
+  auto constant_of = [&](const Node& n, const _odla_value* x) -> const _odla_value* {
+    if (n.op != OP_BINARY || n.absorbed || n.in[0] == n.in[1] || (n.in[0] != x && n.in[1] != x)) return nullptr;
+    if (n.i[0] < BIN_ADD || n.i[0] > BIN_MIN || !(n.out->shape == x->shape)) return nullptr;
+    const _odla_value* c = n.in[0] == x ? n.in[1] : n.in[0];
+    return c->kind == _odla_value::CONSTANT && c->shape.numel() == 1 && dtype_is_float(dtype_from_odla(c->etype)) ? c : nullptr;
+  };
+  const Node& first = comp_->nodes[ni];
+  const DType dt = storage_dtype(first.out);
+  if (!dtype_is_float(dt) || first.out->shape.numel() <= 0) return false;
+  const _odla_value* x = first.in[0]->kind == _odla_value::CONSTANT ? first.in[1] : first.in[0];
+  if (x->kind == _odla_value::CONSTANT || storage_dtype(x) != dt) return false;
+
+  ScalarChain s;
+  std::vector<int> members;
+  _odla_value* last = nullptr;
+  const _odla_value* v = x;
+  for (int j = ni; s.n < kScalarChain;) {
+    Node& n = comp_->nodes[j];
+    const _odla_value* c = constant_of(n, v);
+    if (c == nullptr || storage_dtype(n.out) != dt || storage_dtype(c) != dt) break;
+    s.op[s.n] = (BinKind)n.i[0];
+    s.lhs[s.n] = n.in[0] == c;
+    s.c[s.n] = const_as_float(c)[0];
+    ++s.n;
+    members.push_back(j);
+    v = last = n.out;
+    if (last->is_output || consumers_[last->index].size() != 1) break;
+    j = consumers_[last->index][0];
+  }
+  if (last == nullptr || (last->shape.rank == 4 && feeds_channels_last(last))) return false;
+
+  const VState& xs = vs_[x->index];
+  int tx = xs.slot[L_ROWMAJOR][FORM_FLOAT];
+  bool converts = false;
+  if (tx < 0) {
+    if (dt == DT_F32 || x->kind != _odla_value::ARG || xs.main < 0 || T(xs.main).dt != DT_F32) return false;
+    tx = xs.main;
+    converts = true;
+  }
+  if (T(tx).layout != L_ROWMAJOR || T(tx).quant || (!converts && T(tx).dt != dt) || (xs.main >= 0 && T(xs.main).layout != L_ROWMAJOR)) return false;
+  if (s.n + (converts ? 1 : 0) < 2) return false;
+  const int ty = new_tensor(dt, L_ROWMAJOR, last->shape, 0, SP_ARENA);
+  const DType sdt = T(tx).dt;
+  const int64_t count = last->shape.numel();
+  const Ref a = ref(tx), b = ref(ty);
+  emit("scalars(" + std::to_string(s.n) + "):" + last->name, {tx}, {ty}, [=](const ExecEnv& e, hipStream_t st) {
+    return launch_scalar_chain(a(e), sdt, b(e), dt, count, s, st);
+  }, kReads16 | kWrites16 | kReadsOnce);
+  for (int j : members) comp_->nodes[j].absorbed = true;
+  set_main(last, ty);
+  return true;
+}
+
 void Planner::lower_binary(int ni) {
   Node& n = comp_->nodes[ni];
   const _odla_value* a = n.in[0];
@@ -2463,6 +2521,8 @@ void Planner::lower_binary(int ni) {
       }
     }
   }
+
+  if (lower_scalar_chain(ni)) return;
 
   // optional trailing activation
   ActKind act = ACT_NONE;
