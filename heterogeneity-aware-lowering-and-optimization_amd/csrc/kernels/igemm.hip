@@ -1420,6 +1420,7 @@ hipError_t launch_igemm(const IgemmParams& p_in, hipStream_t stream) {
     return hipErrorInvalidValue;
 
   const int epi_vec = epilogue_vectors(p);
+  if (p.f_y != nullptr && (p.in_dt == DT_F16 || p.in_dt == DT_BF16)) return launch_igemm_pair(p, stream);
   if (p.f_y != nullptr) {
     // a second layer rides in this launch: only the streaming row kernel computes it
     if (p.in_dt != DT_I8 || p.out_dt != DT_I8 || p.w_frag == nullptr || !(epi_vec & 2)) return hipErrorInvalidValue;

@@ -159,8 +159,8 @@ class Planner {
   std::unordered_set<int> arena_only_, aligned_only_, written_;
   std::unordered_map<int, int> reads_;   // by root tensor: passes over it (2 for a launch that may read it several times)
   std::unordered_map<int, int> last_write_;   // by root tensor: the last step so far that writes it (a Concat's result has several)
-  // The 8-bit convolution steps, kept so that a plain 1x1 layer over the result of one can ride in
-  // its launch (lower_conv; igemm_stream_q8_fusable decides).
+  // The convolution steps, kept so that a plain 1x1 layer over the result of one can ride in its launch
+  // (8-bit ones: lower_conv, igemm_stream_q8_fusable decides; 2-byte ones: finish_igemm, igemm_pair_fusable).
   struct FuseProducer {
     int step = -1;
     const _odla_value* out = nullptr;
@@ -820,7 +820,7 @@ class Planner {
   // The Transpose (0, 2, 1, 3) that is the only use of a rank-4 value, or -1.
   int head_merge_behind(const _odla_value* v) const;
   void finish_igemm(const std::string& name, IgemmParams ip, int tx, int tw, int ty, const Epilogue& ep,
-                    int64_t Kout_total);
+                    int64_t Kout_total, const _odla_value* xv = nullptr, const _odla_value* outv = nullptr);
   int strided_copy_step(const std::string& name, int src, int dst, const StridedCopyParams& cp_in);
   void assign_arena();
   void parse_quant_table();
@@ -1432,7 +1432,7 @@ int Planner::make_wfrag(const std::string& name, IgemmParams* ip, int tw, bool a
 // Common tail of Conv / Gemm lowering: bias / residual / activation wiring and
 // the launch step.  tx, tw, ty are the operand tensors.
 void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int tw, int ty,
-                           const Epilogue& ep, int64_t Kout_total) {
+                           const Epilogue& ep, int64_t Kout_total, const _odla_value* xv, const _odla_value* outv) {
   int tb = -1, tr = -1;
   if (ep.has_bias) {
     std::vector<float> b = ep.bias;
@@ -1452,8 +1452,39 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
   // A result much larger than the last-level cache cannot be kept there for its
   // consumer; written around the cache it leaves the lines of smaller tensors alone.
   ip.stream_out = T(ty).bytes >= stream_out_bytes();
-  const int tf = make_wfrag(name, &ip, tw);
+  // A pointwise layer that reads the result of a wide one before it can ride in that one's launch.
+  auto prod = xv != nullptr && !in_init_ && tr < 0 ? fuse_prods_.find(xv) : fuse_prods_.end();
+  bool rides = false;
+  if (prod != fuse_prods_.end() && prod->second.ty == tx && T(tw).space == SP_CONST && T(ty).alias_off == 0 && T(tx).alias_off == 0) {
+    IgemmParams b = ip;
+    b.wf_chunks = (int)(((int64_t)ip.R * ip.S * ip.C * dtype_size(ip.in_dt) + 127) / 128) * 4;
+    rides = igemm_pair_fusable(prod->second.ip, b);
+  }
+  const int tf = make_wfrag(name, &ip, tw, rides);
   const bool hf = tf >= 0;
+  if (rides && hf) {
+    const FuseProducer fp = prod->second;
+    fuse_prods_.erase(prod);   // (one rider per launch)
+    IgemmParams fa = fp.ip;
+    fa.f_kout = ip.Kout; fa.f_ycs = ip.ycs; fa.f_wf_chunks = ip.wf_chunks; fa.f_act = ip.act;
+    const Ref ax = ref(fp.tx), aw = ref(fp.tw), ay = ref(fp.ty), ab = ref(fp.tb >= 0 ? fp.tb : fp.tx), af = ref(fp.tf), ar = ref(fp.tr >= 0 ? fp.tr : fp.tx);
+    const Ref rf = ref(tf), ry = ref(ty), rb = ref(tb >= 0 ? tb : tx);
+    const bool ahb = fp.tb >= 0, ahr = fp.tr >= 0, hb = tb >= 0;
+    Step& sa = plan_->steps[(size_t)fp.step];
+    OHIP_INFO("'%s' is computed in the launch of '%s' (from its tiles in LDS)", name.c_str(), sa.name.c_str());
+    sa.name += "+" + name.substr(name.find(':') + 1);
+    sa.fn = [=](const ExecEnv& e, hipStream_t st) {
+      IgemmParams p = fa;
+      p.x = ax(e); p.w = aw(e); p.y = ay(e);
+      p.bias = ahb ? ab(e) : nullptr;
+      p.residual = ahr ? ar(e) : nullptr;
+      p.w_frag = af(e);
+      p.f_wfrag = rf(e); p.f_bias = hb ? rb(e) : nullptr; p.f_y = ry(e);
+      return launch_igemm(p, st);
+    };
+    touch(fp.step, {}, {ty}, 0);   // (the second result is written by that step)
+    return;
+  }
   ip.slim = igemm_slim_variant(ip, hf);
   log_igemm_choice(name, ip, hf, tr >= 0);
   const Ref rf = ref(hf ? tf : tx);
@@ -1501,6 +1532,13 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
     p.w_frag = hf ? rf(e) : nullptr;
     return launch_igemm(p, st);
   }, exact);
+  if (outv != nullptr && !in_init_ && !calib_ && hf && T(ty).alias_off == 0) {
+    FuseProducer& fp = fuse_prods_[outv];
+    fp.step = (int)plan_->steps.size() - 1;
+    fp.out = outv;
+    fp.ip = ip;
+    fp.tx = tx; fp.tw = tw; fp.ty = ty; fp.tb = tb; fp.tm = -1; fp.tr = tr; fp.tf = tf;
+  }
 }
 
 // ---------------------------------------------------------------- Conv ----
@@ -1908,7 +1946,7 @@ void Planner::lower_conv(int ni) {
       return launch_igemm(p, st);
     });
   } else {
-    finish_igemm("conv:" + outv->name, ip, tx, tw, ty, ep, O);
+    finish_igemm("conv:" + outv->name, ip, tx, tw, ty, ep, O, x, outv);
   }
   set_main(outv, ty);
 }

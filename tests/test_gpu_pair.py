@@ -1,0 +1,71 @@
+"""Two pointwise convolutions in one launch (64 channels to 128 or 256 with residual and activation, those to 64 or
+128) against the oracle and against the two launches: ragged pixel counts, one pixel, more tiles than wavefronts; the
+wide result is read elsewhere too; forms that stay apart."""
+import numpy as np
+import pytest
+
+from test_plan_layernorm_cpu import steps_of
+from util import announce, run_hip, run_ref
+
+pytestmark = pytest.mark.gpu
+
+MODES = {"fp16": ({"fp16": True}, 2.0 ** -11), "bf16": ({"bf16": "performance"}, 2.0 ** -8)}
+
+
+def builder(n, h, w, wide, narrow, residual, act, stride=1, narrow_residual=False):
+    r = np.random.default_rng(n * 31 + h * 7 + w + wide + narrow)
+    k1 = (r.standard_normal((wide, 64, 1, 1)) / 8).astype(np.float32)
+    k2 = (r.standard_normal((narrow, wide, 1, 1)) / 16).astype(np.float32)
+    b1, b2 = r.standard_normal(wide).astype(np.float32), r.standard_normal(narrow).astype(np.float32)
+    feeds = {"x": r.standard_normal((n, 64, h, w)).astype(np.float32)}
+    if residual:
+        feeds["r"] = r.standard_normal((n, wide, h, w)).astype(np.float32)
+
+    def build(b):
+        t = b.conv(b.arg("x", feeds["x"].shape), b.const("k1", k1), b.const("b1", b1), name="c1")
+        if residual:
+            t = b.add(t, b.arg("r", feeds["r"].shape), name="s")
+        if act[0]:
+            t = b.relu(t, name="y_act")
+        z = b.conv(t, b.const("k2", k2), b.const("b2", b2) if narrow != 64 else None, stride=(stride, stride), name="c2")
+        if act[1]:
+            z = b.relu(z, name="z_act")
+        b.output(t, "y")
+        b.output(z, "z")
+    return build, feeds
+
+
+def rides(odla, build, kw):
+    return any("+" in s for s in steps_of(odla, build, **kw) if s.startswith("conv:"))
+
+
+@pytest.mark.parametrize("mode", sorted(MODES))
+@pytest.mark.parametrize("n,h,w,wide,narrow,residual,act", [(1, 1, 1, 256, 64, True, (1, 1)), (2, 5, 7, 256, 128, True, (1, 1)), (1, 31, 33, 128, 64, False, (0, 1)), (3, 56, 56, 256, 64, True, (1, 1)),
+                                                            (7, 56, 55, 256, 128, False, (1, 0)), (30, 56, 56, 256, 64, True, (0, 0)), (25, 57, 60, 128, 128, True, (1, 1)), (600, 4, 4, 256, 64, False, (1, 1))])
+def test_two_layers_in_one_launch(odla, monkeypatch, mode, n, h, w, wide, narrow, residual, act):
+    announce("pair %s %d x %d x %d, %d then %d" % (mode, n, h, w, wide, narrow))
+    kw, eps = MODES[mode]
+    build, feeds = builder(n, h, w, wide, narrow, residual, act)
+    monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", "1")
+    assert rides(odla, build, kw)
+    got = run_hip(build, feeds, **kw)
+    monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", str(1 << 40))
+    assert not rides(odla, build, kw)
+    apart, want = run_hip(build, feeds, **kw), run_ref(build, feeds)
+    for name, k in (("y", 64), ("z", wide)):
+        # operands of k products and the result rounded once each (the second layer's operand is the first's result)
+        bound = eps * (2 * np.sqrt(k) + 4) * max(1.0, float(np.max(np.abs(want[name]))))
+        assert np.max(np.abs(got[name] - want[name])) <= bound
+        # the order of a sum may differ from that of another kernel: a rounding step of the result at most
+        assert np.max(np.abs(got[name] - apart[name])) <= 4 * eps * max(1.0, float(np.max(np.abs(want[name]))))
+
+
+@pytest.mark.parametrize("form", ["fp32", "accuracy", "stride", "wide_512", "narrow_96"])
+def test_forms_that_stay_apart(odla, monkeypatch, form):
+    monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", "1")
+    kw = {"fp32": {}, "accuracy": {"bf16": "accuracy"}}.get(form, {"fp16": True})
+    build, feeds = builder(2, 12, 10, 512 if form == "wide_512" else 256, 96 if form == "narrow_96" else 64, True, (1, 1), stride=2 if form == "stride" else 1)
+    assert not rides(odla, build, kw)
+    got, want = run_hip(build, feeds, **kw), run_ref(build, feeds)
+    for name in want:
+        assert np.max(np.abs(got[name] - want[name])) <= 3e-2 * max(1.0, float(np.max(np.abs(want[name]))))
