@@ -11,9 +11,11 @@
 //   - residual in, results out and the operand pass through 4 KiB of LDS of the wavefront (rows of 64 channels,
 //     16-byte pieces rotated by the pixel so that neither rows nor columns collide), so that memory sees whole 128-byte
 //     rows.  No barrier but the one behind the weights.
+// A residual that is a layer over 64 channels by itself (the shortcut of a first block) is computed here too, rounded as
+// it would be stored: it is neither written nor read.
 // The residual of the next two steps and the pixels of the next tile are under way during each step.
 // Measured, 64 -> 256 with residual -> 64 / 128 on 256 images of 56 x 56, fp16, two launches and now: 175 + 103 -> 194 - 202
-// us (5.2 TB/s over 1.03 GB), 175 + 110 -> 224.
+// us (5.2 TB/s over 1.03 GB), 175 + 110 -> 224; with the shortcut's layer 113 + 194 -> 165.
 #include "igemm_common.h"
 
 namespace ohip {
@@ -22,7 +24,9 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kRowsBytes = 32 * 128;                     // 32 pixels x 64 channels
 
-template <typename T, int N2T, bool RES>   // N2T: 32-channel blocks of the second result; RES: the first one has a residual
+enum { kNoResidual = 0, kResidual = 1, kResidualLayer = 2 };
+
+template <typename T, int N2T, int RES>   // N2T: 32-channel blocks of the second result; RES: the first one's residual
 __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmParams p, const int tiles) {
   using Acc = typename Mma<T>::Acc;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -33,7 +37,9 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
   float* b2 = b1 + n1;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lg = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  unsigned char* rows = reinterpret_cast<unsigned char*>(b2 + N2T * 32) + wave * kRowsBytes;
+  uintx4* w3 = reinterpret_cast<uintx4*>(b2 + N2T * 32);                // (the residual's layer: as w1 and b1)
+  float* b3 = reinterpret_cast<float*>(w3 + (RES == kResidualLayer ? blocks1 * 4 * 64 : 0));
+  unsigned char* rows = reinterpret_cast<unsigned char*>(b3 + (RES == kResidualLayer ? n1 : 0)) + wave * kRowsBytes;
   const int M = p.N * p.Ho * p.Wo;
 
   {
@@ -44,6 +50,11 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
       for (int i = tid; i < steps2 * 64; i += kWaves * 64) w2[j * steps2 * 64 + i] = f2[j * p.f_wf_chunks * 64 + i];
     for (int i = tid; i < n1; i += kWaves * 64) b1[i] = p.bias != nullptr ? reinterpret_cast<const float*>(p.bias)[i] : 0.f;
     for (int i = tid; i < N2T * 32; i += kWaves * 64) b2[i] = p.f_bias != nullptr ? reinterpret_cast<const float*>(p.f_bias)[i] : 0.f;
+    if constexpr (RES == kResidualLayer) {
+      const uintx4* f3 = reinterpret_cast<const uintx4*>(p.r_wfrag);
+      for (int i = tid; i < blocks1 * 4 * 64; i += kWaves * 64) w3[i] = f3[i];
+      for (int i = tid; i < n1; i += kWaves * 64) b3[i] = p.r_bias != nullptr ? reinterpret_cast<const float*>(p.r_bias)[i] : 0.f;
+    }
   }
   __syncthreads();
 
@@ -62,10 +73,10 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
   const T* x = reinterpret_cast<const T*>(p.x);
   const T* res = reinterpret_cast<const T*>(p.residual);
   // lane (l32, lg) supplies bytes [32 kk + 16 lg, +16) of pixel l32
-  auto load_x = [&](const int tile, uintx4 (&a)[4]) __attribute__((always_inline)) {
+  auto load_x = [&](const T* from, const int cs, const int tile, uintx4 (&a)[4]) __attribute__((always_inline)) {
     int m = tile * 32 + l32;
     m = m < M ? m : M - 1;
-    const uintx4* row = reinterpret_cast<const uintx4*>(x + (int64_t)m * p.xcs) + lg;
+    const uintx4* row = reinterpret_cast<const uintx4*>(from + (int64_t)m * cs) + lg;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) a[kk] = row[2 * kk];
   };
@@ -97,9 +108,12 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
 
   int tile = bid * kWaves + wave;
   if (tile >= tiles) return;
+  // (r0, r1: the residual of two steps; r0: the pixels of its layer)
   uintx4 a[4], a_next[4], r0[4], r1[4];
-  load_x(tile, a);
-  if constexpr (RES) {
+  load_x(x, p.xcs, tile, a);
+  const T* rx = reinterpret_cast<const T*>(p.r_x);
+  if constexpr (RES == kResidualLayer) load_x(rx, p.r_xcs, tile, r0);
+  if constexpr (RES == kResidual) {
     load_res(tile, 0, r0);
     load_res(tile, 1, r1);
   }
@@ -107,14 +121,14 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
   for (; tile < tiles; tile += stride) {
     const int next = tile + stride;
     const int ahead = next < tiles ? next : tile;   // (requested in any case: requests in flight can then be counted)
-    load_x(ahead, a_next);
+    load_x(x, p.xcs, ahead, a_next);
     Acc acc2[N2T];
 #pragma unroll
     for (int j = 0; j < N2T; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc2[j][e] = 0.f;
-    auto step = [&](const int h, uintx4 (&r)[4]) __attribute__((always_inline)) {
-      if constexpr (RES) {
+    auto step = [&](const int h, auto odd, uintx4 (&r)[4]) __attribute__((always_inline)) {
+      if constexpr (RES == kResidual) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) *reinterpret_cast<uintx4*>(mem_at + k * 1024) = r[k];
         // the step after the next one, of this tile or the next
@@ -122,6 +136,27 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
         load_res(same ? tile : ahead, same ? h + 2 : h + 2 - halves, r);
       }
       Acc acc[2];
+      uintx2 side[2][4];
+      if constexpr (RES == kResidualLayer) {   // the residual's layer, rounded as it would be stored
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[j] = Mma<T>::run(w3[((h * 2 + j) * 4 + kk) * 64 + lane], r0[kk], acc[j]);
+        // (the last step requests the next tile's: a second set of registers would not fit)
+        if constexpr (decltype(odd)::value) load_x(rx, p.r_xcs, h + 1 < halves ? tile : ahead, r0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const floatx4 b = *reinterpret_cast<const floatx4*>(b3 + h * 64 + j * 32 + q * 8 + lg * 4);
+            const Acc& v = acc[j];
+            side[j][q] = uintx2{pack2<T>(v[q * 4] + b.x, v[q * 4 + 1] + b.y), pack2<T>(v[q * 4 + 2] + b.z, v[q * 4 + 3] + b.w)};
+          }
+      }
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -140,8 +175,8 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
           float v[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) v[e] = acc[j][q * 4 + e] + b[e];
-          if constexpr (RES) {
-            const uintx2 t = *reinterpret_cast<const uintx2*>(at);
+          if constexpr (RES != kNoResidual) {
+            const uintx2 t = RES == kResidualLayer ? side[j][q] : *reinterpret_cast<const uintx2*>(at);
             const T* rt = reinterpret_cast<const T*>(&t);
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += Store<T>::ld(rt + e);
@@ -164,8 +199,8 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
     };
 #pragma unroll 1
     for (int h = 0; h < halves; h += 2) {
-      step(h, r0);
-      step(h + 1, r1);
+      step(h, std::false_type(), r0);
+      step(h + 1, std::true_type(), r1);
     }
     // the second result, 64 channels at a time
 #pragma unroll
@@ -188,50 +223,57 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
       ordered();
     }
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) a[kk] = a_next[kk];
+    for (int kk = 0; kk < 4; ++kk) {
+      a[kk] = a_next[kk];
+    }
   }
 }
 
-// Where one launch is the faster form.  Few pixels: below 2^15 the fetch of the weights and one tile's chain of
+// Where one launch is the faster form.  Few pixels: below 2^14 the fetch of the weights and one tile's chain of
 // latencies are all there is (15 - 20 us), up to one tile for every wavefront the launches count.  Then the wide result
-// stays in the last-level cache and the second layer reads it there, until it takes up three quarters of that.
-// All launches of ResNet-50, fp16, on n images of 3136 pixels, apart and in one launch: n = 2: 332 / 345 us, 4: 400 / 401,
-// 8: 474 / 475, 16: 610 / 591, 20: 657 / 627, 28: 783 / 774, 32: 839 / 823, 36: 899 / 901, 44: 1078 / 1082, 52: 1150 / 1173,
-// 64: 1342 / 1336, 90: 1759 / 1691.  Between one and 1.6 tiles a wavefront what one launch alone gains is lost where two
-// halves of a batch run side by side (24 images of each: 1067 / 1091; bf16, 50 of 1600 pixels: 1105 / 1129).
-constexpr int64_t kPairPixels = 1 << 15, kPairPixelsMost = 64 << 10, kPairWideBytes = 192ll << 20;
+// and the residual stay in the last-level cache (256 MB), where the second layer reads them, until both and what is
+// written beside them do not fit any more.
+// All launches of ResNet-50, fp16, on n images of 3136 pixels, apart and in one launch (two pairs, one with the shortcut's
+// layer): n = 2: 329 / 342 us, 4: 398 / 393, 6: 463 / 457, 8: 473 / 465, 16: 610 / 591, 20: 657 / 627, 36: 884 / 895,
+// 52: 1137 / 1129, 64: 1348 / 1319, 90: 1759 / 1691.  Between one and 1.6 tiles a wavefront what one launch alone gains is
+// lost where two halves of a batch run side by side (24 images of each: 1067 / 1091; bf16, 50 of 1600 pixels: 1105 / 1129).
+constexpr int64_t kPairPixels = 1 << 14, kPairPixelsMost = 64 << 10, kPairWideBytes = 96ll << 20;
 bool pair_pays(const int64_t pixels, const int64_t wide_bytes) {
   if (const char* e = getenv("ODLA_HIP_PAIR_MIN_PIXELS")) return pixels >= atoll(e);   // test aid
   return (pixels >= kPairPixels && pixels <= kPairPixelsMost) || wide_bytes >= kPairWideBytes;
 }
 
-int pair_lds(const int n1, const int n2) { return n1 * 128 + n2 * n1 * 2 + (n1 + n2) * 4 + kWaves * kRowsBytes; }
+int pair_lds(const int n1, const int n2, const bool layer) { return n1 * (layer ? 256 : 128) + n2 * n1 * 2 + (n1 * (layer ? 2 : 1) + n2) * 4 + kWaves * kRowsBytes; }
 
 template <typename T>
 hipError_t launch_typed(const IgemmParams& p, hipStream_t stream) {
   const int64_t M = (int64_t)p.N * p.Ho * p.Wo;
   const int tiles = (int)((M + 31) / 32);
-  const int lds = pair_lds(p.Kout, p.f_kout);
+  const int lds = pair_lds(p.Kout, p.f_kout, p.r_x != nullptr);
   int grid = (tiles + kWaves - 1) / kWaves;
   if (grid > 256) grid = 256;
   auto go = [&](auto kernel) -> hipError_t {
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kWaves * 64), (size_t)lds, stream, p, tiles);
     return hipGetLastError();
   };
-  if (p.residual != nullptr) return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, true>) : go(igemm_pair_kernel<T, 4, true>);
-  return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, false>) : go(igemm_pair_kernel<T, 4, false>);
+  if (p.r_x != nullptr) return go(igemm_pair_kernel<T, 2, kResidualLayer>);
+  if (p.residual != nullptr) return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, kResidual>) : go(igemm_pair_kernel<T, 4, kResidual>);
+  return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, kNoResidual>) : go(igemm_pair_kernel<T, 4, kNoResidual>);
 }
 
+}  // namespace
+
+namespace {
+bool pointwise(const IgemmParams& p) {
+  return p.R == 1 && p.S == 1 && p.sh == 1 && p.sw == 1 && p.ph == 0 && p.pw == 0 && p.batch == 1 && p.Ho == p.H && p.Wo == p.W &&
+         p.alpha == 1.f && (p.act == ACT_NONE || p.act == ACT_RELU) && p.y_rdiv == 0 && p.row_softmax == 0 && !p.ln && p.f_y == nullptr &&
+         p.wf_chunks * 16 == p.C;
+}
 }  // namespace
 
 // a: the wide layer, b: the one that reads its result; no pointer is looked at.
 bool igemm_pair_fusable(const IgemmParams& a, const IgemmParams& b) {
   if ((a.in_dt != DT_F16 && a.in_dt != DT_BF16) || a.out_dt != a.in_dt || b.in_dt != a.in_dt || b.out_dt != a.in_dt) return false;
-  auto pointwise = [](const IgemmParams& p) {
-    return p.R == 1 && p.S == 1 && p.sh == 1 && p.sw == 1 && p.ph == 0 && p.pw == 0 && p.batch == 1 && p.Ho == p.H && p.Wo == p.W &&
-           p.alpha == 1.f && (p.act == ACT_NONE || p.act == ACT_RELU) && p.y_rdiv == 0 && p.row_softmax == 0 && !p.ln && p.f_y == nullptr &&
-           p.wf_chunks * 16 == p.C;
-  };
   if (!pointwise(a) || !pointwise(b) || a.res_after_act) return false;
   if (a.C != 64 || (a.Kout != 128 && a.Kout != 256) || a.ycs != a.Kout || a.xcs % 8 != 0) return false;
   if (b.C != a.Kout || b.xcs != a.ycs || (b.Kout != 64 && b.Kout != 128) || b.ycs % 8 != 0) return false;
@@ -240,11 +282,18 @@ bool igemm_pair_fusable(const IgemmParams& a, const IgemmParams& b) {
   return M < (1ll << 30) && pair_pays(M, M * a.Kout * 2);
 }
 
+// r: the layer whose result is the residual of a (f_kout channels behind), and nothing else reads.
+bool igemm_pair_residual(const IgemmParams& a, const int f_kout, const IgemmParams& r) {
+  return f_kout == 64 && pointwise(r) && r.act == ACT_NONE && r.in_dt == a.in_dt && r.out_dt == a.in_dt && r.C == 64 && r.Kout == a.Kout && r.ycs == r.Kout && r.xcs % 8 == 0 &&
+         r.N == a.N && r.H == a.H && r.W == a.W;   // (128 channels behind: three sets of weights do not fit)
+}
+
 hipError_t launch_igemm_pair(const IgemmParams& p, hipStream_t stream) {
   auto al16 = [](const void* q) { return q != nullptr && (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
   if (p.C != 64 || (p.Kout != 128 && p.Kout != 256) || (p.f_kout != 64 && p.f_kout != 128) || p.wf_chunks != 4 || p.f_wf_chunks * 16 != p.Kout) return hipErrorInvalidValue;
   if (!al16(p.x) || !al16(p.y) || !al16(p.f_y) || !al16(p.w_frag) || !al16(p.f_wfrag) || (p.residual != nullptr && !al16(p.residual))) return hipErrorInvalidValue;
   if (p.xcs % 8 != 0 || p.ycs != p.Kout || p.f_ycs % 8 != 0 || p.f_ycs < p.f_kout || (p.residual != nullptr && (p.rcs % 8 != 0 || p.rcs < p.Kout))) return hipErrorInvalidValue;
+  if (p.r_x != nullptr && (p.residual != nullptr || !al16(p.r_x) || !al16(p.r_wfrag) || p.r_xcs % 8 != 0 || p.r_xcs < 64 || p.f_kout != 64)) return hipErrorInvalidValue;
   if ((int64_t)p.N * p.Ho * p.Wo <= 0 || (int64_t)p.N * p.Ho * p.Wo >= (1ll << 30)) return hipErrorInvalidValue;
   return p.in_dt == DT_F16 ? launch_typed<f16_t>(p, stream) : p.in_dt == DT_BF16 ? launch_typed<bf16_t>(p, stream) : hipErrorInvalidValue;
 }

@@ -161,6 +161,11 @@ struct IgemmParams {
   float f_q_add = 0.f, f_q_lo = 0.f;
   // (2-byte types, igemm_pair_fusable: y2 = act2(y . w2 + bias2), bias2 in fp32)
   ActKind f_act = ACT_NONE;
+  // (with it, instead of `residual`: a layer over 64 channels of r_x with its own fragment-ordered weights and bias)
+  const void* r_x = nullptr;
+  const void* r_wfrag = nullptr;
+  const void* r_bias = nullptr;
+  int r_xcs = 0;
   // A LayerNorm over the C channels of every pixel in front of the product (igemm_slim_ln_ok says
   // where): rows of ln_dt at ln_x, C elements apart, are normalised, become the operand (x is not
   // read) and leave as ln_y (ln_dt) and, where asked for, as ln_y2 (in_dt).
@@ -211,6 +216,7 @@ bool igemm_stream_q8_fusable(const IgemmParams& a, const IgemmParams& b);
 hipError_t launch_igemm_stream_q8(const IgemmParams& p, hipStream_t stream);
 // The same of 2-byte types (igemm_pair.hip).
 bool igemm_pair_fusable(const IgemmParams& a, const IgemmParams& b);
+bool igemm_pair_residual(const IgemmParams& a, int f_kout, const IgemmParams& r);
 hipError_t launch_igemm_pair(const IgemmParams& p, hipStream_t stream);
 // 3x3, stride 1, padding 1 with the input patch of a tile held in LDS (igemm_c3.hip): whether
 // the layer is one of its shapes, and its launch (called by launch_igemm with its epi_vec).

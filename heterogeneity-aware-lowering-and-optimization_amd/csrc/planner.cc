@@ -168,6 +168,7 @@ class Planner {
     int tx = -1, tw = -1, ty = -1, tb = -1, tm = -1, tr = -1, tf = -1;
   };
   std::unordered_map<const _odla_value*, FuseProducer> fuse_prods_;   // by result value
+  std::vector<int> dead_steps_;   // steps whose results a later one computes itself: they leave the plan when it is complete
   // The LayerNorm whose launch is the last step of the plan (ty < 0: the last step is something
   // else; every emitted step clears it): a product of few rows that comes next computes it itself
   // in place of that step (finish_igemm).
@@ -1058,6 +1059,8 @@ void Planner::run() {
     }
   }
   assign_arena();
+  std::sort(dead_steps_.begin(), dead_steps_.end());
+  for (auto it = dead_steps_.rbegin(); it != dead_steps_.rend(); ++it) plan_->steps.erase(plan_->steps.begin() + *it);
 }
 
 // Staged arguments whose declared type differs from the storage type have no
@@ -1472,14 +1475,31 @@ void Planner::finish_igemm(const std::string& name, IgemmParams ip, int tx, int 
     const bool ahb = fp.tb >= 0, ahr = fp.tr >= 0, hb = tb >= 0;
     Step& sa = plan_->steps[(size_t)fp.step];
     OHIP_INFO("'%s' is computed in the launch of '%s' (from its tiles in LDS)", name.c_str(), sa.name.c_str());
+    // its residual, where that is a layer of the same kind that nothing else reads
+    FuseProducer side;
+    for (const auto& f : fuse_prods_) {
+      const FuseProducer& r = f.second;
+      if (ahr && r.ty == fp.tr && r.tr < 0 && !r.out->is_output && consumers_[r.out->index].size() == 1 && igemm_pair_residual(fa, ip.Kout, r.ip)) side = r;
+    }
+    if (side.step >= 0) {
+      sa.name += "+" + plan_->steps[(size_t)side.step].name.substr(5);   // (behind "conv:")
+      dead_steps_.push_back(side.step);
+      T(side.ty).bytes = 0;   // (never made)
+      fuse_prods_.erase(side.out);
+      touch(fp.step, {side.tx}, {}, 0);
+      fa.r_xcs = side.ip.xcs;
+    }
     sa.name += "+" + name.substr(name.find(':') + 1);
+    const bool hs = side.step >= 0, hsb = side.tb >= 0;
+    const Ref sx = ref(hs ? side.tx : fp.tx), sf = ref(hs ? side.tf : fp.tx), sb = ref(hsb ? side.tb : fp.tx);
     sa.fn = [=](const ExecEnv& e, hipStream_t st) {
       IgemmParams p = fa;
       p.x = ax(e); p.w = aw(e); p.y = ay(e);
       p.bias = ahb ? ab(e) : nullptr;
-      p.residual = ahr ? ar(e) : nullptr;
+      p.residual = ahr && !hs ? ar(e) : nullptr;
       p.w_frag = af(e);
       p.f_wfrag = rf(e); p.f_bias = hb ? rb(e) : nullptr; p.f_y = ry(e);
+      if (hs) { p.r_x = sx(e); p.r_wfrag = sf(e); p.r_bias = hsb ? sb(e) : nullptr; }
       return launch_igemm(p, st);
     };
     touch(fp.step, {}, {ty}, 0);   // (the second result is written by that step)

@@ -60,6 +60,49 @@ def test_two_layers_in_one_launch(odla, monkeypatch, mode, n, h, w, wide, narrow
         assert np.max(np.abs(got[name] - apart[name])) <= 4 * eps * max(1.0, float(np.max(np.abs(want[name]))))
 
 
+def shortcut(n, h, w, wide, narrow, act=False, twice=False):
+    r = np.random.default_rng(n * 13 + h + w + wide)
+    shape = (n, 64, h, w)
+    ks = [(r.standard_normal((c, i, 1, 1)) * s).astype(np.float32) for c, i, s in ((wide, 64, 0.1), (64, 64, 0.12), (wide, 64, 0.1), (narrow, wide, 0.06))]
+    bs = [r.standard_normal(k.shape[0]).astype(np.float32) for k in ks]
+
+    def build(b):
+        x = b.arg("x", shape)
+        x = b.relu(b.maxpool(x, (3, 3), (1, 1), (1, 1, 1, 1), name="front"), name="front_act")
+        conv = lambda t, k, name: b.conv(t, b.const("k%d" % k, ks[k]), b.const("b%d" % k, bs[k]), name=name)
+        s = conv(x, 0, "short")
+        if act:
+            s = b.relu(s, name="short_act")
+        t = b.relu(conv(x, 1, "c1"), name="c1_act")
+        y = b.relu(b.add(conv(t, 2, "c2"), s, name="sum"), name="y_act")
+        b.output(y, "y")
+        b.output(b.relu(conv(y, 3, "c3"), name="z_act"), "z")
+        if twice:
+            b.output(b.relu(s, name="s2"), "s")
+    return build, {"x": r.standard_normal(shape).astype(np.float32)}
+
+
+@pytest.mark.parametrize("mode", sorted(MODES))
+@pytest.mark.parametrize("n,h,w,wide,narrow,form", [(1, 1, 1, 256, 64, ""), (2, 5, 7, 128, 64, ""), (3, 56, 56, 256, 64, ""), (23, 57, 55, 256, 64, ""), (41, 45, 47, 128, 64, ""),
+                                                    (2, 20, 21, 256, 128, "apart"), (2, 20, 21, 256, 64, "act"), (2, 20, 21, 256, 64, "twice")])
+def test_the_residual_is_a_layer_too(odla, monkeypatch, mode, n, h, w, wide, narrow, form):
+    """Three layers in one launch; apart (the residual is written and read) where it does not fit or is read elsewhere."""
+    announce("pair with shortcut %s %d x %d x %d, %d then %d %s" % (mode, n, h, w, wide, narrow, form))
+    kw, eps = MODES[mode]
+    build, feeds = shortcut(n, h, w, wide, narrow, form == "act", form == "twice")
+    monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", "1")
+    names = steps_of(odla, build, **kw)
+    assert any(s.count("+") == (1 if form else 2) for s in names if s.startswith("conv:")) and ("conv:short" in names) == (form in ("apart", "twice"))
+    got = run_hip(build, feeds, **kw)
+    monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", str(1 << 40))
+    apart, want = run_hip(build, feeds, **kw), run_ref(build, feeds)
+    for name in want:
+        size = max(1.0, float(np.max(np.abs(want[name]))))
+        # three roundings of operands and results in a row
+        assert np.max(np.abs(got[name] - want[name])) <= 3 * eps * (2 * np.sqrt(wide) + 4) * size
+        assert np.max(np.abs(got[name] - apart[name])) <= 4 * eps * size
+
+
 @pytest.mark.parametrize("form", ["fp32", "accuracy", "stride", "wide_512", "narrow_96"])
 def test_forms_that_stay_apart(odla, monkeypatch, form):
     monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", "1")
