@@ -229,15 +229,17 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
   }
 }
 
-// Where one launch is the faster form.  Few pixels: below 2^14 the fetch of the weights and one tile's chain of
-// latencies are all there is (15 - 20 us), up to one tile for every wavefront the launches count.  Then the wide result
+// Where one launch is the faster form.  Few pixels: below 2^13 the fetch of the weights and one tile's chain of
+// latencies are all there is (15 - 20 us) and the launches apart are faster, up to 2^15 one launch gains 1 - 2 % of a
+// network (there the layers stay steps of their own, which a plan of few images shows and the profiler times one by one),
+// up to one tile for every wavefront the launches count.  Then the wide result
 // and the residual stay in the last-level cache (256 MB), where the second layer reads them, until both and what is
 // written beside them do not fit any more.
 // All launches of ResNet-50, fp16, on n images of 3136 pixels, apart and in one launch (two pairs, one with the shortcut's
 // layer): n = 2: 329 / 342 us, 4: 398 / 393, 6: 463 / 457, 8: 473 / 465, 16: 610 / 591, 20: 657 / 627, 36: 884 / 895,
 // 52: 1137 / 1129, 64: 1348 / 1319, 90: 1759 / 1691.  Between one and 1.6 tiles a wavefront what one launch alone gains is
 // lost where two halves of a batch run side by side (24 images of each: 1067 / 1091; bf16, 50 of 1600 pixels: 1105 / 1129).
-constexpr int64_t kPairPixels = 1 << 14, kPairPixelsMost = 64 << 10, kPairWideBytes = 96ll << 20;
+constexpr int64_t kPairPixels = 1 << 15, kPairPixelsMost = 64 << 10, kPairWideBytes = 96ll << 20;
 bool pair_pays(const int64_t pixels, const int64_t wide_bytes) {
   if (const char* e = getenv("ODLA_HIP_PAIR_MIN_PIXELS")) return pixels >= atoll(e);   // test aid
   return (pixels >= kPairPixels && pixels <= kPairPixelsMost) || wide_bytes >= kPairWideBytes;
