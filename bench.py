@@ -410,7 +410,7 @@ def profile_roofline(L, sess, wl, dump_path=None):
     for i in range(n.value):
         name = buf[i].name.decode()
         total_ms += buf[i].ms
-        if name.startswith("conv") or name.startswith("gemm"):
+        if name.startswith(("conv", "gemm", "stem")):   # (stem: the first convolution with what stands around it)
             mm_ms += buf[i].ms
             if not name.startswith("gemm.sum"):   # the reduction behind a split-K GEMM belongs to that GEMM
                 launches += 1
@@ -419,7 +419,7 @@ def profile_roofline(L, sess, wl, dump_path=None):
     roof = {"bound": "mfma", "achieved": round(achieved, 2), "peak": peak,
             "unit": "TOP/s" if wl.mode == "int8" else "TFLOP/s",
             "frac": round(achieved / peak, 4), "traffic": measured_traffic(wl.name),
-            "kernel": "igemm_wreg_kernel / igemm_kernel / igemm_lean_kernel / igemm_taps_kernel / igemm_stream_q8_kernel / igemm_c3_kernel (all %d conv/gemm launches of one step, avg %.1f us, "
+            "kernel": "igemm_wreg_kernel / igemm_kernel / igemm_lean_kernel / igemm_taps_kernel / igemm_stream_q8_kernel / igemm_c3_kernel / igemm_pair_kernel / stem_pool_kernel (all %d conv/gemm launches of one step, avg %.1f us, "
                       "avg %.2f GFLOP per launch)" % (launches, 1e3 * mm_ms / max(launches, 1),
                                                      wl.flop / 1e9 / max(launches, 1)),
             "mm_ms_per_step": round(mm_ms, 4), "all_kernels_ms_per_step": round(total_ms, 4),
@@ -438,13 +438,16 @@ def profile_roofline(L, sess, wl, dump_path=None):
         bound_ms = meas_ms = nbytes = 0.0
         hbm_bound = 0
         # a launch that computes a second layer from the first layer's tiles ("a+b") is priced as
-        # one launch: the operations and bytes of both, less the second layer's read of its input
+        # one launch: the operations and bytes of both, less the second layer's read of its input (a
+        # shortcut that is computed there: less its result's write and the read of it as a residual)
         priced = {}
         for key in t_by:
             parts = key.split("+")
             if all(k in wl.conv_elements for k in parts):
                 fl = sum(wl.conv_elements[k][0] for k in parts)
-                act = sum(wl.conv_elements[k][1] for k in parts) - sum(wl.conv_elements[k][3] for k in parts[1:])
+                act = sum(wl.conv_elements[k][1] for k in parts)
+                for k in parts[1:]:
+                    act -= 2 * (wl.conv_elements[k][1] - wl.conv_elements[k][3]) if k.endswith("ds") else wl.conv_elements[k][3]
                 wt = sum(wl.conv_elements[k][2] for k in parts)
                 priced[key] = (fl, act, wt)
         for key, (fl, act, wt) in priced.items():
