@@ -1245,6 +1245,7 @@ hipError_t launch_fused_eltwise(const FusedLaunch& l, hipStream_t stream) {
     if (l.group[k] == nullptr || l.block0[k + 1] <= l.block0[k] || l.view0[k + 1] < l.view0[k]) return hipErrorInvalidValue;
   for (int k = 0; k < l.view0[l.n_groups]; ++k)
     if (l.base[k] == nullptr) return hipErrorInvalidValue;
+  if (l.best != nullptr && (l.wide || l.best_at == nullptr)) return hipErrorInvalidValue;   // (only chains leave them)
   const dim3 grid((unsigned)l.block0[l.n_groups]);
   if (l.wide) { FLOAT_DISPATCH(l.dt, hipLaunchKernelGGL((fused_eltwise_kernel<T, int64_t>), grid, dim3(kThreads), l.lds_bytes, stream, l)); }
   else { FLOAT_DISPATCH(l.dt, hipLaunchKernelGGL((fused_eltwise_kernel<T, uint32_t>), grid, dim3(kThreads), l.lds_bytes, stream, l)); }

@@ -3431,6 +3431,8 @@ bool Planner::lower_fused_group(int seed, int from) {
     }
     bool ok = l.dt == dt && l.n_groups < kFusedMaxGroups && l.view0[l.n_groups] + fp.n_views <= kFusedMaxBases &&
               (same || ((blocks >= 256 || for_nms) && std::max(lds, l.lds_bytes) <= 32 * 1024));
+    // (best scores are left by launches of 32-bit offsets alone, see fused_eltwise_kernel)
+    ok = ok && !(wide && f->best.t >= 0);
     for (int t : read_tensors) {
       const auto w = last_write_.find(root(t));
       ok = ok && (w == last_write_.end() || w->second < f->step);
