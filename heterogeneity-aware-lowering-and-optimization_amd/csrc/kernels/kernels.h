@@ -312,7 +312,7 @@ hipError_t launch_copy_pieces(const void* src, void* dst, int64_t bytes, hipStre
 // A 7x7 / stride 2 convolution over a three-channel NCHW fp32 image into 64 channels, ReLU, and the 3x3 / stride 2 /
 // padding 1 maximum of that (stem_pool.hip).  The convolution is the 4x4 / stride 1 one over the image's
 // space-to-depth form whose fragment-ordered weights w_frag holds (ph, pw: its padding there).  dt: type of operands and
-// result, which is channels-last without padding; DT_I8: scale, zp quantise the image, bias is int32, qmul / q_add / q_lo
+// result, whose pixels lie ycs elements apart (64, or the pitch of the tensor it is a channel slice of); DT_I8: scale, zp quantise the image, bias is int32, qmul / q_add / q_lo
 // requantise as in IgemmParams.
 struct StemPoolParams {
   const float* x = nullptr;
@@ -325,6 +325,7 @@ struct StemPoolParams {
   int N = 0, H = 0, W = 0;     // the image
   int Ho = 0, Wo = 0;          // the convolution's result
   int Po = 0, Qo = 0;          // the pool's
+  int ycs = 64;
   int ph = 0, pw = 0;
   float scale = 1.f; int zp = 0;
   float q_add = 0.f, q_lo = 0.f;

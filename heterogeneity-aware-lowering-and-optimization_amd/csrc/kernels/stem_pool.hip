@@ -16,7 +16,8 @@
 //     a pooled one sit in one row of 16 lanes.  The maximum over rows is one of registers, the one over columns two
 //     lane shifts, on 16-bit results as they are stored, two at a time, or on 8-bit ones' sums: bias, ReLU,
 //     rounding and requantisation keep the order of values;
-//   - 14 pooled pixels of 64 channels, contiguous in the result, leave as 16-byte vectors.
+//   - 14 pooled pixels of 64 channels leave as 16-byte vectors, contiguous in a result of its own (one whose only reader is
+//     a Concat along the channels is a slice of that one's: its pixels lie a larger pitch apart).
 // No barrier: wavefronts drift apart, one in its matrix instructions while the other of its SIMD converts and
 // stores (a workgroup of four that filled a patch first and then computed took 251 us).  Bound by both together:
 // the matrix instructions alone are 50 us, the vector ones about as much, memory traffic 52 us.
@@ -256,13 +257,13 @@ __global__ void __launch_bounds__(64, 2) stem_pool_kernel(const StemPoolParams p
           else *reinterpret_cast<uintx2*>(out + (j * 32 + q * 8) * 2) = uintx2{m[j][q][0], m[j][q][1]};
     }
     ordered();
-    T* y = reinterpret_cast<T*>(p.y) + (((int64_t)n * p.Po + prow) * p.Qo + q0) * 64 + c0;
+    T* y = reinterpret_cast<T*>(p.y) + (((int64_t)n * p.Po + prow) * p.Qo + q0) * p.ycs + c0;
     constexpr int CH = NJ * 32 * ES / 16;                // 16-byte pieces of a pixel
 #pragma unroll
     for (int k = 0; k < (kCols * CH + 63) / 64; ++k) {
       const int piece = k * 64 + lane, px = piece / CH, c = piece % CH;
       if (piece < kCols * CH && q0 + px < p.Qo)
-        *reinterpret_cast<uintx4*>(reinterpret_cast<unsigned char*>(y) + px * (64 * ES) + c * 16) = *reinterpret_cast<const uintx4*>(stage + px * OPITCH + c * 16);
+        *reinterpret_cast<uintx4*>(reinterpret_cast<unsigned char*>(y) + px * p.ycs * ES + c * 16) = *reinterpret_cast<const uintx4*>(stage + px * OPITCH + c * 16);
     }
     ordered();
   };
@@ -342,6 +343,8 @@ bool stem_pool_supported(const StemPoolParams& p) {
   if (p.dt != DT_F16 && p.dt != DT_BF16 && p.dt != DT_I8) return false;
   if (p.N <= 0 || p.H < 2 || p.W < 2 || p.Ho <= 0 || p.Wo <= 0 || p.Po <= 0 || p.Qo <= 0) return false;
   if (p.dt == DT_I8 && !(p.scale >= kScaleLeast && p.scale <= kScaleMost)) return false;
+  // whole 16-byte vectors of a result pixel
+  if (p.ycs < 64 || p.ycs > (1 << 24) || p.ycs % (16 / dtype_size(p.dt)) != 0) return false;
   // every pooled value covers a convolution value; source coordinates and one image's elements in 32 bits
   if (2 * ((int64_t)p.Po - 1) - 1 >= p.Ho || 2 * ((int64_t)p.Qo - 1) - 1 >= p.Wo) return false;
   return (int64_t)p.H * p.W < (1ll << 29) && p.ph >= 0 && p.ph < 4 && p.pw >= 0 && p.pw < 4;

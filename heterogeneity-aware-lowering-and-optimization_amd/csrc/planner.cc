@@ -1585,7 +1585,7 @@ int Planner::stem_pool_behind(const Epilogue& ep, int O, int R, int S, DType fro
 void Planner::emit_stem_pool(const _odla_value* conv, int pool, StemPoolParams sp, IgemmParams ip, int from, int tw, int tb, int tm, int ty) {
   const int tf = make_wfrag("conv:" + conv->name, &ip, tw, true);
   Node& pn = comp_->nodes[pool];
-  if (tf < 0 || T(ty).cs != 64) fail(ODLA_INTERNAL_LOGIC_ERR, "weights or result of the stem '%s'", conv->name.c_str());
+  if (tf < 0) fail(ODLA_INTERNAL_LOGIC_ERR, "weights of the stem '%s'", conv->name.c_str());
   sp.wf_chunks = ip.wf_chunks;
   const bool hm = tm >= 0;
   const Ref rx = ref(from), rf = ref(tf), rb = ref(tb), rm = ref(hm ? tm : tb), ry = ref(ty);
@@ -1660,7 +1660,7 @@ void Planner::lower_conv(int ni) {
   int tx_s2d = -1;
   int stem_pool = -1;            // the pool behind the convolution, where one launch computes both (stem_pool.hip)
   StemPoolParams stem;
-  int stem_from = -1;
+  int stem_from = -1, stem_ty = -1;
   {
     const VState& xv = vs_[x->index];
     const bool src_ok = xv.main >= 0 && T(xv.main).layout == L_ROWMAJOR && !T(xv.main).quant;
@@ -1718,7 +1718,17 @@ void Planner::lower_conv(int ni) {
       stem.Ho = (int)Ho; stem.Wo = (int)Wo;
       stem.ph = -dy0; stem.pw = -dx0;
       stem.scale = sp.scale; stem.zp = sp.zp;
-      if (stem_pool >= 0 && (C != 3 || R2 != 4 || S2 != 4 || cs != 16 || !stem_pool_supported(stem))) stem_pool = -1;
+      if (stem_pool >= 0 && (C != 3 || R2 != 4 || S2 != 4 || cs != 16)) stem_pool = -1;
+      if (stem_pool >= 0) {
+        // (8-bit results and those in front of anything but a Concat are tensors of their own)
+        const _odla_value* pooled = comp_->nodes[stem_pool].out;
+        stem_ty = q8 ? new_tensor(DT_I8, L_NHWC, pooled->shape, (int)O, SP_ARENA) : channels_last_result(pooled, fdt);
+        stem.ycs = T(stem_ty).cs;
+        if (T(stem_ty).alias_off % 16 != 0 || !stem_pool_supported(stem)) {
+          if (T(stem_ty).alias_of < 0) T(stem_ty).bytes = 0;   // (never made)
+          stem_pool = -1;
+        }
+      }
       const Ref a = ref(from), b = ref(tx_s2d);
       if (stem_pool >= 0) T(tx_s2d).bytes = 0;   // (never made)
       else emit("to_s2d:" + x->name, {from}, {tx_s2d}, [=](const ExecEnv& e, hipStream_t st) {
@@ -1821,10 +1831,9 @@ void Planner::lower_conv(int ni) {
     if (stem_pool >= 0) {
       if (ip.out_dt != DT_I8) fail(ODLA_INTERNAL_LOGIC_ERR, "stem '%s' without 8-bit results", outv->name.c_str());
       stem.q_add = ip.q_add; stem.q_lo = ip.q_lo;
-      const int tyq = new_tensor(DT_I8, L_NHWC, comp_->nodes[stem_pool].out->shape, (int)O, SP_ARENA);
-      set_quant(tyq, true, T(ty).qscale, T(ty).qzp);
+      set_quant(stem_ty, true, T(ty).qscale, T(ty).qzp);
       T(ty).bytes = 0;   // (never made)
-      emit_stem_pool(outv, stem_pool, stem, ip, stem_from, tw, tb, tm, tyq);
+      emit_stem_pool(outv, stem_pool, stem, ip, stem_from, tw, tb, tm, stem_ty);
       return;
     }
     ip.stream_out = T(ty).bytes >= stream_out_bytes();
@@ -1945,8 +1954,7 @@ void Planner::lower_conv(int ni) {
   if (stem_pool >= 0) {
     std::vector<float> b = ep.bias;
     b.resize((size_t)O, 0.f);
-    _odla_value* pooled = comp_->nodes[stem_pool].out;
-    emit_stem_pool(outv, stem_pool, stem, ip, stem_from, tw, const_vector<float>(DT_F32, b), -1, channels_last_result(pooled, odt));
+    emit_stem_pool(outv, stem_pool, stem, ip, stem_from, tw, const_vector<float>(DT_F32, b), -1, stem_ty);
     return;
   }
   int ty;

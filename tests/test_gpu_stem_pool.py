@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import __graft_entry__ as entry
+from stem_concat_graphs import CONCATS, concat_graph
 from test_plan_layernorm_cpu import steps_of
 from util import announce, run_hip, run_ref
 
@@ -131,3 +132,18 @@ def test_the_convolution_is_read_elsewhere_too(odla):
         got, want = run_hip(build, {"x": x}, fp16=True), run_ref(build, {"x": x})
         for name in want:
             assert np.max(np.abs(got[name] - want[name])) <= 2e-2 * max(1.0, float(np.max(np.abs(want[name]))))
+
+
+@pytest.mark.parametrize("mode", ["fp16", "bf16"])
+@pytest.mark.parametrize("n,h,w", [(1, 3, 7), (2, 45, 37), (40, 97, 96)])
+@pytest.mark.parametrize("parts,one", CONCATS)
+def test_stem_pool_as_a_part_of_a_concat(odla, parts, one, n, h, w, mode):
+    """The pooled pixels are a slice of the Concat's, in front of, behind and between other parts."""
+    announce("stem and pool in a concat %s %d x %d x %d %s" % (mode, n, h, w, parts))
+    kw = {"fp16": {"fp16": True}, "bf16": {"bf16": "performance"}}[mode]
+    build, feeds = concat_graph(n, h, w, parts)
+    assert one_launch(odla, build, **kw) == one
+    got, want = run_hip(build, feeds, **kw)["out"], run_ref(build, feeds)["out"]
+    # operands of 147 products and the result rounded once each, largest of nine
+    eps = 2.0 ** -11 if mode == "fp16" else 2.0 ** -8
+    assert np.max(np.abs(got - want)) <= eps * (2 * np.sqrt(147) + 1) * max(1.0, float(np.max(np.abs(want))))
