@@ -17,6 +17,7 @@
 // Measured, 64 -> 256 with residual -> 64 / 128 on 256 images of 56 x 56, fp16, two launches and now: 175 + 103 -> 194 - 202
 // us (5.2 TB/s over 1.03 GB), 175 + 110 -> 224; with the shortcut's layer 113 + 194 -> 165.
 #include "igemm_common.h"
+#include "lds_limit.h"
 
 namespace ohip {
 namespace {
@@ -245,7 +246,9 @@ bool pair_pays(const int64_t pixels, const int64_t wide_bytes) {
   return (pixels >= kPairPixels && pixels <= kPairPixelsMost) || wide_bytes >= kPairWideBytes;
 }
 
-int pair_lds(const int n1, const int n2, const bool layer) { return n1 * (layer ? 256 : 128) + n2 * n1 * 2 + (n1 * (layer ? 2 : 1) + n2) * 4 + kWaves * kRowsBytes; }
+constexpr int pair_lds(const int n1, const int n2, const bool layer) { return n1 * (layer ? 256 : 128) + n2 * n1 * 2 + (n1 * (layer ? 2 : 1) + n2) * 4 + kWaves * kRowsBytes; }
+constexpr int kMostLds = pair_lds(256, 64, true) > pair_lds(256, 128, false) ? pair_lds(256, 64, true) : pair_lds(256, 128, false);
+static_assert(kMostLds <= 160 * 1024, "LDS of a compute unit");
 
 template <typename T>
 hipError_t launch_typed(const IgemmParams& p, hipStream_t stream) {
@@ -254,13 +257,16 @@ hipError_t launch_typed(const IgemmParams& p, hipStream_t stream) {
   const int lds = pair_lds(p.Kout, p.f_kout, p.r_x != nullptr);
   int grid = (tiles + kWaves - 1) / kWaves;
   if (grid > 256) grid = 256;
-  auto go = [&](auto kernel) -> hipError_t {
+  auto go = [&](auto kernel, LdsLimit& limit) -> hipError_t {
+    const hipError_t e = limit.raise(reinterpret_cast<const void*>(kernel), kMostLds);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kWaves * 64), (size_t)lds, stream, p, tiles);
     return hipGetLastError();
   };
-  if (p.r_x != nullptr) return go(igemm_pair_kernel<T, 2, kResidualLayer>);
-  if (p.residual != nullptr) return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, kResidual>) : go(igemm_pair_kernel<T, 4, kResidual>);
-  return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, kNoResidual>) : go(igemm_pair_kernel<T, 4, kNoResidual>);
+  static LdsLimit limits[5];   // (of this type's instances, in the order below)
+  if (p.r_x != nullptr) return go(igemm_pair_kernel<T, 2, kResidualLayer>, limits[0]);
+  if (p.residual != nullptr) return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, kResidual>, limits[1]) : go(igemm_pair_kernel<T, 4, kResidual>, limits[2]);
+  return p.f_kout == 64 ? go(igemm_pair_kernel<T, 2, kNoResidual>, limits[3]) : go(igemm_pair_kernel<T, 4, kNoResidual>, limits[4]);
 }
 
 }  // namespace
