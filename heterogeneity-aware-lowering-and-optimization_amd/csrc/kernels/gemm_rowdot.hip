@@ -12,7 +12,9 @@
 // thread requests up to four pieces of its row, and the weights for the first of them, before it
 // waits for anything.  64 x 784 x 10 with the rows in host memory: 10.0 us in the kernel trace and
 // 27.1 us a call with one wavefront per row, whose turns of one piece each waited for one another;
-// 8.4 and 25.2 us now (an empty launch takes 1.9).
+// 8.4 and 25.2 us now (an empty launch takes 1.9).  From a wavefront per SIMD on (1024 rows: more than the
+// room in host memory holds, but for the shortest) the trips hide each other and several wavefronts a row only repeat the lane
+// exchanges: there a row keeps one wavefront (rule at the launch).
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
@@ -119,13 +121,18 @@ hipError_t launch_gemm_rowdot(const IgemmParams& p, hipStream_t stream) {
   if (!gemm_rowdot_shape(p) || p.x == nullptr || p.w == nullptr || p.y == nullptr || !al16(p.x) || !al16(p.w))
     return hipErrorInvalidValue;
   const dim3 grid((unsigned)((int64_t)p.N * p.Ho * p.Wo));
-  // as many wavefronts as have pieces, up to four; one request per thread where they reach
+  // As many wavefronts as have pieces, up to four; one request per thread where they reach.  Of many rows one
+  // wavefront each, as long as it has at most eight pieces a lane: 16 columns, rows in device memory, several
+  // wavefronts / one, us a launch: 1024 rows of 512 5.4 / 5.1, of 1024 7.0 / 6.2, of 2048 9.1 / 8.3; 4096 rows of 1024
+  // 13.1 / 11.7; 10 columns, 4096 rows of 784 10.6 / 9.9.  (Longer rows or fewer of them: 1024 of 4096, 10 columns 10.7 /
+  // 12.7; 512 of 1024 and 16 columns 5.6 / 5.8.)
+  const bool many = grid.x >= 1024 && p.C <= 2048;
 #define ROWDOT(NB_)                                                                                              \
   do {                                                                                                           \
-    if (p.C > 1024) hipLaunchKernelGGL((gemm_rowdot_kernel<NB_, 4, 4>), grid, dim3(256), 0, stream, p);          \
+    if (many || p.C <= 256) hipLaunchKernelGGL((gemm_rowdot_kernel<NB_, 1, 1>), grid, dim3(64), 0, stream, p);   \
+    else if (p.C > 1024) hipLaunchKernelGGL((gemm_rowdot_kernel<NB_, 4, 4>), grid, dim3(256), 0, stream, p);          \
     else if (p.C > 512) hipLaunchKernelGGL((gemm_rowdot_kernel<NB_, 4, 1>), grid, dim3(256), 0, stream, p);      \
-    else if (p.C > 256) hipLaunchKernelGGL((gemm_rowdot_kernel<NB_, 2, 1>), grid, dim3(128), 0, stream, p);      \
-    else hipLaunchKernelGGL((gemm_rowdot_kernel<NB_, 1, 1>), grid, dim3(64), 0, stream, p);                      \
+    else hipLaunchKernelGGL((gemm_rowdot_kernel<NB_, 2, 1>), grid, dim3(128), 0, stream, p);                     \
   } while (0)
   if (p.Kout <= 4) ROWDOT(4);
   else if (p.Kout <= 8) ROWDOT(8);

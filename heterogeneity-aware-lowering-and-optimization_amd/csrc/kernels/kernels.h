@@ -131,7 +131,7 @@ struct IgemmParams {
   // the plan relies on then holds whatever the environment says later); -1: the launch asks itself.
   int slim = -1;
   // Softmax (1) or LogSoftmax (2) over the Kout columns of every result row, behind bias and
-  // activation: only the one-wavefront-per-row kernel computes it (gemm_rowdot_shape).
+  // activation: only the row kernel computes it (gemm_rowdot_shape).
   int row_softmax = 0;
   // int8 only -----------------------------------------------------------
   // acc = int32 accumulator + int32 bias; fma = one fused multiply-add in fp32
@@ -188,7 +188,7 @@ struct WregForm { int rows, slices, groups, epilogue; };
 WregForm igemm_wreg_form(const IgemmParams& p);
 
 // Products with at most 16 output columns, a long reduction and few rows (gemm_rowdot.hip): one
-// wavefront per output row.  Whether the shape qualifies, and the launch (launch_igemm uses both).
+// to four wavefronts per output row.  Whether the shape qualifies, and the launch (launch_igemm uses both).
 bool gemm_rowdot_shape(const IgemmParams& p);
 hipError_t launch_gemm_rowdot(const IgemmParams& p, hipStream_t stream);
 
