@@ -2526,7 +2526,18 @@ bool Planner::lower_scalar_chain(int ni) {
     if (last->is_output || consumers_[last->index].size() != 1) break;
     j = consumers_[last->index][0];
   }
-  if (last == nullptr || (last->shape.rank == 4 && feeds_channels_last(last))) return false;
+  if (last == nullptr) return false;
+  // An activation behind the last operator belongs into that one's launch, on the sum as it is before it is rounded
+  // (lower_binary): the chain ends in front of it.
+  if (!last->is_output && consumers_[last->index].size() == 1) {
+    const Node& nx = comp_->nodes[consumers_[last->index][0]];
+    if (nx.op == OP_UNARY && !nx.absorbed && (nx.i[0] == ACT_RELU || nx.i[0] == ACT_LEAKY || nx.i[0] == ACT_CLAMP)) {
+      if (--s.n == 0) return false;
+      members.pop_back();
+      last = comp_->nodes[members.back()].out;
+    }
+  }
+  if (last->shape.rank == 4 && feeds_channels_last(last)) return false;
 
   const VState& xs = vs_[x->index];
   int tx = xs.slot[L_ROWMAJOR][FORM_FLOAT];

@@ -71,3 +71,30 @@ def test_a_step_that_is_read_elsewhere_ends_the_launch(odla, mode):
     got = run_hip(builder(x.shape, chain, also=(1, 2)), {"x": x}, **kw)
     for k in (1, 2, 4):
         np.testing.assert_array_equal(got["y%d" % k], expected(x, chain[:k + 1], dtype))
+
+
+@pytest.mark.parametrize("mode", sorted(MODES))
+@pytest.mark.parametrize("act", ["relu", "leaky", "clamp"])
+@pytest.mark.parametrize("n", [1, 2, 5])
+def test_an_activation_takes_the_value_before_it_is_rounded(odla, n, act, mode):
+    announce("scalar chain and activation %s %d %s" % (mode, n, act))
+    kw, dtype = MODES[mode]
+    chain = CHAINS["five"][:n]
+    x = np.random.default_rng(n).standard_normal((3, 2, 50, 41)).astype(np.float32)
+
+    def build(b):
+        t = b.arg("x", x.shape)
+        for k, (op, c, lhs) in enumerate(chain):
+            cv = b.const("c%d" % k, np.full((1,), c, np.float32))
+            t = getattr(b, op)(cv, t, name="t%d" % k) if lhs else getattr(b, op)(t, cv, name="t%d" % k)
+        b.output({"relu": lambda: b.relu(t, name="act"), "leaky": lambda: b.leaky_relu(t, 0.3, name="act"),
+                  "clamp": lambda: b.clamp(t, -0.4, 0.4, name="act")}[act](), "y")
+
+    v = torch.from_numpy(expected(x, chain[:-1], dtype)) if n > 1 else torch.from_numpy(x).to(dtype).float()
+    op, c, lhs = chain[-1]
+    cv = torch.tensor(c).to(dtype).float()
+    l, r = (cv, v) if lhs else (v, cv)
+    v = {"add": torch.add, "sub": torch.sub, "mul": torch.mul, "div": torch.div}[op](l, r)
+    v = {"relu": lambda: torch.relu(v), "leaky": lambda: torch.where(v > 0, v, v * torch.tensor(0.3)),
+         "clamp": lambda: torch.clamp(v, -0.4, 0.4)}[act]()
+    np.testing.assert_array_equal(run_hip(build, {"x": x}, **kw)["y"], v.to(dtype).float().numpy())
