@@ -161,9 +161,10 @@ attention_kernel(const AttentionParams p) {
       }
     }
     if (tid < TS) {
-      // (a mask of the type's lowest value stays finite: a row of nothing else is a plain mean)
-      const float m2 = mr * kLog2e;
-      ms[tid] = __builtin_isinf(m2) && !__builtin_isinf(mr) ? __builtin_copysignf(3.402823466e38f, mr) : m2;
+      // Mask values beyond 2^126 keep their order and stay finite: whatever such values differ by decides alone, and a
+      // row of nothing but the type's lowest value is a plain mean.
+      const float far = 0x1p+126f, m = __builtin_fabsf(mr);
+      ms[tid] = m < far ? mr * kLog2e : __builtin_copysignf(__builtin_fmaf(m, 0.5f, far), mr);
     }
   };
 

@@ -50,3 +50,25 @@ def test_tiles(B, heads, S, mask, mode):
     assert np.all(np.isfinite(got))
     # probabilities and the result are rounded once each; |v| stays below 5
     assert np.max(np.abs(got - want)) <= 3 * eps * 5
+
+
+@pytest.mark.parametrize("mode", ["bf16", "bf16acc"])
+@pytest.mark.parametrize("B,heads,S", [(2, 2, 31), (2, 2, 128), (2, 2, 300), (11, 12, 300)])
+def test_masks_near_the_lowest_value_differ(B, heads, S, mode):
+    """Two mask values, both below what a product with log2(e) leaves finite: the larger one decides."""
+    print("attention mask near the lowest value", B, heads, S, mode, flush=True)
+    r = np.random.default_rng(S)
+    f = {n: r.standard_normal((B, heads, S, 64)).astype(np.float32) for n in ("q", "k", "v")}
+    keep = r.random((B, 1, 1, S)) < 0.3
+    keep[..., -1] = True
+    for low, high in ((-3.3e38, -2.5e38), (-2.5e38, -8e37), (-1e38, -8e37), (2.5e38, 3.3e38)):
+        f["mask"] = np.where(keep, high, low).astype(np.float32)
+        kw = {"bf16": {"bf16": "performance"}, "bf16acc": {"bf16": "accuracy"}}[mode]
+        got = run_hip(build_attention(B, heads, S, 64, "div", True, True, True), f, **kw)["out"]
+        # (no score shows beside such a mask in 32 bits)
+        v = torch.from_numpy(f["v"]).to(torch.bfloat16).double().numpy()
+        w = keep[:, :, 0, :, None] / keep.sum(-1)[..., None]
+        mean = (v * w).sum(2)                                     # [B, heads, 64]
+        want = np.maximum(np.broadcast_to(mean.reshape(B, 1, heads * 64), got.shape), 0)
+        # probabilities and the result are rounded once each; |v| stays below 5
+        assert np.max(np.abs(got - want)) <= 3 * 2.0 ** -8 * 5
