@@ -75,7 +75,7 @@ def test_a_step_that_is_read_elsewhere_ends_the_launch(odla, mode):
 
 @pytest.mark.parametrize("mode", sorted(MODES))
 @pytest.mark.parametrize("act", ["relu", "leaky", "clamp"])
-@pytest.mark.parametrize("n", [1, 2, 5])
+@pytest.mark.parametrize("n", [1, 2, 3, 5])
 def test_an_activation_takes_the_value_before_it_is_rounded(odla, n, act, mode):
     announce("scalar chain and activation %s %d %s" % (mode, n, act))
     kw, dtype = MODES[mode]
