@@ -230,20 +230,24 @@ __global__ void __launch_bounds__(kWaves * 64, 2) igemm_pair_kernel(const IgemmP
   }
 }
 
-// Where one launch is the faster form.  Few pixels: below 2^13 the fetch of the weights and one tile's chain of
-// latencies are all there is (15 - 20 us) and the launches apart are faster, up to 2^15 one launch gains 1 - 2 % of a
-// network (there the layers stay steps of their own, which a plan of few images shows and the profiler times one by one),
-// up to one tile for every wavefront the launches count.  Then the wide result
-// and the residual stay in the last-level cache (256 MB), where the second layer reads them, until both and what is
-// written beside them do not fit any more.
-// All launches of ResNet-50, fp16, on n images of 3136 pixels, apart and in one launch (two pairs, one with the shortcut's
-// layer): n = 2: 329 / 342 us, 4: 398 / 393, 6: 463 / 457, 8: 473 / 465, 16: 610 / 591, 20: 657 / 627, 36: 884 / 895,
-// 52: 1137 / 1129, 64: 1348 / 1319, 90: 1759 / 1691.  Between one and 1.6 tiles a wavefront what one launch alone gains is
-// lost where two halves of a batch run side by side (24 images of each: 1067 / 1091; bf16, 50 of 1600 pixels: 1105 / 1129).
-constexpr int64_t kPairPixels = 1 << 15, kPairPixelsMost = 64 << 10, kPairWideBytes = 96ll << 20;
-bool pair_pays(const int64_t pixels, const int64_t wide_bytes) {
+// Where one launch is the faster form.  The 2048 wavefronts of the launch take one tile each up to 2^16 pixels.
+// Measured as four blocks of a first stage (3x3 layers and pairs, a mean behind them), fp16, launches apart / one launch,
+// n images of 3136 pixels: 64 -> 256 -> 64, 64 -> 256 -> 128, 64 -> 128 -> 64, 64 -> 256 -> 64 with the shortcut's layer:
+//   n = 2: 111 / 126, 122 / 144, 102 / 108, 112 / 125 us   (fetch of the weights and one tile's chain of latencies)
+//   8: 158 / 163, 175 / 177, 134 / 138, 161 / 160     10: 161 / 164, 176 / 183, 144 / 143, 162 / 156
+//   14: 204 / 190, 219 / 214, 179 / 168, 206 / 178    20: 241 / 213, 273 / 246, 200 / 189, 242 / 198
+//   21: 247 / 242, 289 / 292, 209 / 209, 248 / 227    26: 264 / 256, 318 / 308, 217 / 217, 267 / 245
+//   28: 279 / 267, 329 / 317, 230 / 226, 282 / 256    40: 343 / 310, 407 / 366, 273 / 251, 342 / 288
+//   64: 473 / 420, 617 / 588, 364 / 327, 475 / 396    128: 903 / 808, 1156 / 1018, 614 / 572, 910 / 757
+// Below 2^15 pixels only the form with the shortcut's layer gains, which is not known yet when the pair is (all of
+// ResNet-50 fp16, which has one of these among its three pairs, at 8 images: 492 / 478).  Between one and 1.3 tiles a
+// wavefront little is gained alone, and more is lost where two halves of a batch run side by side: all of ResNet-50 fp16,
+// halves of 22 images 966 / 1020, of 24 1028 / 1052, of 26 1085 / 1094, of 28 1155 / 1145, of 30 1207 / 1189, of 36 1366 / 1311,
+// of 48 1685 / 1631 (and of 20 920 / 938, where 20 images alone take 655 / 622).
+constexpr int64_t kPairPixels = 1 << 15, kOneTile = 64 << 10, kTwoTiles = 84 << 10;
+bool pair_pays(const int64_t pixels) {
   if (const char* e = getenv("ODLA_HIP_PAIR_MIN_PIXELS")) return pixels >= atoll(e);   // test aid
-  return (pixels >= kPairPixels && pixels <= kPairPixelsMost) || wide_bytes >= kPairWideBytes;
+  return pixels >= kPairPixels && (pixels <= kOneTile || pixels >= kTwoTiles);
 }
 
 constexpr int pair_lds(const int n1, const int n2, const bool layer) { return n1 * (layer ? 256 : 128) + n2 * n1 * 2 + (n1 * (layer ? 2 : 1) + n2) * 4 + kWaves * kRowsBytes; }
@@ -287,7 +291,7 @@ bool igemm_pair_fusable(const IgemmParams& a, const IgemmParams& b) {
   if (b.C != a.Kout || b.xcs != a.ycs || (b.Kout != 64 && b.Kout != 128) || b.ycs % 8 != 0) return false;
   if (b.N != a.N || b.H != a.Ho || b.W != a.Wo) return false;
   const int64_t M = (int64_t)a.N * a.Ho * a.Wo;
-  return M < (1ll << 30) && pair_pays(M, M * a.Kout * 2);
+  return M < (1ll << 30) && pair_pays(M);
 }
 
 // r: the layer whose result is the residual of a (f_kout channels behind), and nothing else reads.
