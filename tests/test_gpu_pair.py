@@ -1,5 +1,5 @@
 """Two pointwise convolutions in one launch (64 channels to 128 or 256 with residual and activation, those to 64 or
-128) against the oracle and against the two launches: ragged pixel counts, one pixel, more tiles than wavefronts; the
+128) against the oracle and, to the bit, against the two launches: ragged pixel counts, one pixel, more tiles than wavefronts; the
 wide result is read elsewhere too; forms that stay apart."""
 import numpy as np
 import pytest
@@ -35,6 +35,13 @@ def builder(n, h, w, wide, narrow, residual, act, stride=1, narrow_residual=Fals
     return build, feeds
 
 
+def one_order(monkeypatch, pixels):
+    """Fewer pixels than one launch is ever taken for: the layers' own launches would be small tiles, which split K
+    between wavefronts.  The tiles that walk K in one order, as one launch of both does, stand in for them."""
+    if pixels < 1 << 15:
+        monkeypatch.setenv("ODLA_HIP_WREG_KSPLIT", "0")
+
+
 def rides(odla, build, kw):
     return any("+" in s for s in steps_of(odla, build, **kw) if s.startswith("conv:"))
 
@@ -45,6 +52,7 @@ def rides(odla, build, kw):
 def test_two_layers_in_one_launch(odla, monkeypatch, mode, n, h, w, wide, narrow, residual, act):
     announce("pair %s %d x %d x %d, %d then %d" % (mode, n, h, w, wide, narrow))
     kw, eps = MODES[mode]
+    one_order(monkeypatch, n * h * w)
     build, feeds = builder(n, h, w, wide, narrow, residual, act)
     monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", "1")
     assert rides(odla, build, kw)
@@ -56,8 +64,7 @@ def test_two_layers_in_one_launch(odla, monkeypatch, mode, n, h, w, wide, narrow
         # operands of k products and the result rounded once each (the second layer's operand is the first's result)
         bound = eps * (2 * np.sqrt(k) + 4) * max(1.0, float(np.max(np.abs(want[name]))))
         assert np.max(np.abs(got[name] - want[name])) <= bound
-        # the order of a sum may differ from that of another kernel: a rounding step of the result at most
-        assert np.max(np.abs(got[name] - apart[name])) <= 4 * eps * max(1.0, float(np.max(np.abs(want[name]))))
+        np.testing.assert_array_equal(got[name], apart[name])
 
 
 def shortcut(n, h, w, wide, narrow, act=False, twice=False):
@@ -89,6 +96,7 @@ def test_the_residual_is_a_layer_too(odla, monkeypatch, mode, n, h, w, wide, nar
     """Three layers in one launch; apart (the residual is written and read) where it does not fit or is read elsewhere."""
     announce("pair with shortcut %s %d x %d x %d, %d then %d %s" % (mode, n, h, w, wide, narrow, form))
     kw, eps = MODES[mode]
+    one_order(monkeypatch, n * h * w)
     build, feeds = shortcut(n, h, w, wide, narrow, form == "act", form == "twice")
     monkeypatch.setenv("ODLA_HIP_PAIR_MIN_PIXELS", "1")
     names = steps_of(odla, build, **kw)
@@ -100,7 +108,7 @@ def test_the_residual_is_a_layer_too(odla, monkeypatch, mode, n, h, w, wide, nar
         size = max(1.0, float(np.max(np.abs(want[name]))))
         # three roundings of operands and results in a row
         assert np.max(np.abs(got[name] - want[name])) <= 3 * eps * (2 * np.sqrt(wide) + 4) * size
-        assert np.max(np.abs(got[name] - apart[name])) <= 4 * eps * size
+        np.testing.assert_array_equal(got[name], apart[name])
 
 
 @pytest.mark.parametrize("form", ["fp32", "accuracy", "stride", "wide_512", "narrow_96"])
