@@ -339,6 +339,7 @@ odla_status stage_inputs(_odla_context* ctx, const Plan& plan, char* arena, std:
       }
       if (!ctx->in_place_off && in_place_args_enabled() && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
         (*ext)[plan.inputs.size() + plan.outputs.size() + k] = room;
+        OHIP_DEBUG("argument '%s' is copied by the first launches", io.v->name.c_str());
         continue;
       }
       src = room;
