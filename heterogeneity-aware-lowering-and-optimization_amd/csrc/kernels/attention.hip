@@ -2,22 +2,25 @@
 //
 //   out[b, h] = softmax(scale * q[b, h] . k[b, h]^T + mask[b]) . v[b, h]
 //
-// for 16-bit operands (bf16 / fp16) and head size 64 - the block that an encoder layer otherwise runs as matrix product, Softmax, transposition
-// of v and matrix product, each with its own pass over a [B, heads, S, S] tensor
+// for 16-bit operands (bf16 / fp16) and head size 64 - the block that an encoder layer otherwise
+// runs as matrix product, Softmax, transposition of v and matrix product, each with its own pass
+// over a [B, heads, S, S] tensor
 // [ref: the reference compiler matches the same block as one instruction,
 //  lib/transforms/fusion.cc:315-348].
 //
 // One workgroup per (batch, head) and 128 queries, one wavefront per 32 queries.  Up to 128 keys
 // are one tile; longer sequences walk tiles of 128 keys with a running maximum and sum per query
-// (the next tile's rows travel in registers while the current one is used).  BERT-base in
-// accuracy mode at 8 x 384 tokens: product, Softmax, transposition and product took 22 + 20 + 7 +
-// 14 us per layer, this launch 15.3 (18.4 with
-// v^T stored value by value; 64 x 128 tokens 13.5 -> 12.3, 16 x 512 35.6 -> 30.0); at 1 x 41 tokens (keys that fill no block) nine launches
-// became one.  A launch of few workgroups is a chain of tiles with one wavefront per SIMD: there two groups of four
-// wavefronts take every other tile each, and the second group's maxima, sums and contexts join the first's
-// through LDS (1 x 512 tokens 13.2 -> 11.4 us; a chip that is full loses, 16 x 512 30 -> 37, 8 x 384 15.4 -> 19.9).  k goes through
-// LDS once (rows padded to 144 bytes), v is transposed on its way into LDS, q
-// comes straight from global memory into MFMA operand registers.
+// (the next tile's rows travel in registers while the current one is used).  k goes through LDS
+// once (rows padded to 144 bytes), v is transposed on its way into LDS, q comes straight from
+// global memory into MFMA operand registers.  A launch of few workgroups is a chain of tiles with
+// one wavefront per SIMD: there two groups of four wavefronts take every other tile each, and the
+// second group's maxima, sums and contexts join the first's through LDS (a chip that is full
+// loses: 16 x 512 tokens 30 -> 37 us, 8 x 384 15.4 -> 19.9).
+// BERT-base in accuracy mode at 8 x 384 tokens: product, Softmax, transposition and product took
+// 22 + 20 + 7 + 14 us per layer, this launch 15.3; at 1 x 41 tokens (keys that fill no block) nine
+// launches became one.  With v^T stored value by value, the library's exponential and one group
+// throughout / now, us a launch: 8 x 384 18.2 / 15.3, 64 x 128 13.8 / 12.7, 16 x 512 36.6 / 30.7,
+// 1 x 512 15.3 / 10.9, 1 x 41 4.2 / 3.9.
 //   scores  C[key][query] = k . q^T  (v_mfma_f32_32x32x16): a lane then holds, for
 //           ITS query, 16 keys of every 32-key block, so the Softmax over the keys
 //           is a reduction inside the lane plus one exchange with lane + 32;

@@ -11,7 +11,7 @@
 //     (py * 2 + px) * 3 + channel, the order of the packed weights) in a ring of eight rows in LDS; the rows of the
 //     next but one step are on their way while a step computes;
 //   - the fragment-ordered weights stay in registers and every convolution row is 2 x 16 (8-bit: 2 x 8) matrix
-//     instructions on operands straight from LDS, requested three steps ahead (without that: 146 us for 115);
+//     instructions on operands straight from LDS, requested three steps ahead (without that: 146 us where this takes 115);
 //   - lane l of a half wavefront holds convolution column 14 (l / 16) + l % 16 of 29, so that the three columns of
 //     a pooled one sit in one row of 16 lanes.  The maximum over rows is one of registers, the one over columns two
 //     lane shifts, on 16-bit results as they are stored, two at a time, or on 8-bit ones' sums: bias, ReLU,
@@ -20,9 +20,10 @@
 //     a Concat along the channels is a slice of that one's: its pixels lie a larger pitch apart).
 // No barrier: wavefronts drift apart, one in its matrix instructions while the other of its SIMD converts and
 // stores (a workgroup of four that filled a patch first and then computed took 251 us).  Bound by both together:
-// the matrix instructions alone are 50 us, the vector ones about as much, memory traffic 52 us.
-// Measured, launches before and now: 256 x 224 x 224 fp16 43 + 203 + 98 us -> 115 us, 8 bit 38 + 109 + 55 -> 85;
-// one image fp16 4.3 + 8.9 + 4.1 -> 6.8; 13 x 237 x 237 8 bit 7.2 + 16.2 + 5.2 -> 12.3.
+// at 256 fp16 images the matrix cores are busy for 44 % of the time, vector instructions are 72 % of what is issued, and
+// 257 MB take 52 us (8 bit: 28 %, 80 %).
+// Measured, launches before and now: 256 x 224 x 224 fp16 43 + 203 + 98 us -> 110 - 121 us from card to card, 8 bit
+// 38 + 109 + 55 -> 85; one image fp16 4.3 + 8.9 + 4.1 -> 6.8; 13 x 237 x 237 8 bit 7.2 + 16.2 + 5.2 -> 12.3.
 #include "igemm_common.h"
 
 namespace ohip {
