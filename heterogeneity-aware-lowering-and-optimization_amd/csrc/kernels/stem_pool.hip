@@ -24,6 +24,9 @@
 // 257 MB take 52 us (8 bit: 28 %, 80 %).
 // Measured, launches before and now: 256 x 224 x 224 fp16 43 + 203 + 98 us -> 110 - 121 us from card to card, 8 bit
 // 38 + 109 + 55 -> 85; one image fp16 4.3 + 8.9 + 4.1 -> 6.8; 13 x 237 x 237 8 bit 7.2 + 16.2 + 5.2 -> 12.3.
+// Strips read the rows between them twice, so that a small image in host memory, which the conversion read in place, is
+// copied by a launch first: still 2 - 8 us of a call less (one fp16 image into ResNet-50, 96 x 96 280 -> 272 us, 224 x 224
+// 336 -> 333, 288 x 288 386 -> 384).
 #include "igemm_common.h"
 
 namespace ohip {
